@@ -282,6 +282,115 @@ __device__ __forceinline__ float Exp2Int(int e)
     return e >= -126 ? __uint_as_float(static_cast<uint32_t>(e + 127) << 23) : __uint_as_float(0x00400000u);
 }
 
+// ---- MXFP8 through the scaled converts -------------------------------------------------------------------------------
+//
+// A block is 32 columns: the four words (eight elements) of a lane and those of the three other lanes of its quad.  The
+// scaled converts take packed 16-bit elements as they are, divide by 2^e exactly and round once, two elements per
+// instruction; an exhaustive comparison on gfx950 (every 16-bit pattern x every scale exponent, bf16 and fp16, e4m3 and
+// e5m2) found them equal to Fp8Encode(ldexpf(x, -e)) wherever the quotient does not pass the largest finite code, and the
+// convert back, code x scale, equal to Fp8Decode(code) * 2^e for every code that is not a NaN or an infinity, subnormal
+// results and the scale 2^-127 included.  The software codec costs about forty instructions per element, this about
+// three.  What the converts do not do is saturate: elements beyond 1.75 * 2^emax times the scale are brought down to
+// that value, which has the largest finite code, beforehand, as 16-bit magnitudes.
+// Blocks that hold an infinity or a NaN take the software codec (MxScaling::plain is false).
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+typedef short s16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+
+constexpr uint32_t kPackedMagnitude = 0x7fff7fffu;
+
+__device__ __forceinline__ uint32_t PackedMaxU16(uint32_t a, uint32_t b)
+{
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, a), __builtin_bit_cast(u16x2, b)));
+}
+
+__device__ __forceinline__ uint32_t PackedMinU16(uint32_t a, uint32_t b)
+{
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(u16x2, a), __builtin_bit_cast(u16x2, b)));
+}
+
+// Largest magnitude of the lane's block, as its 16-bit pattern (magnitudes of one format order like their patterns; a
+// NaN is above the infinity).  All four lanes of the quad have to be active.
+__device__ __forceinline__ uint32_t MxBlockMaxBits(const u32x4 &v)
+{
+    uint32_t m = PackedMaxU16(PackedMaxU16(v[0] & kPackedMagnitude, v[1] & kPackedMagnitude),
+        PackedMaxU16(v[2] & kPackedMagnitude, v[3] & kPackedMagnitude));
+    constexpr int kQuadSwap1 = 0xb1;        // lanes 1 0 3 2
+    constexpr int kQuadSwap2 = 0x4e;        // lanes 2 3 0 1
+    m = PackedMaxU16(m, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(m), kQuadSwap1, 0xf, 0xf, true)));
+    m = PackedMaxU16(m, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(m), kQuadSwap2, 0xf, 0xf, true)));
+    const uint32_t lo = m & 0xffffu;
+    const uint32_t hi = m >> 16;
+    return lo > hi ? lo : hi;
+}
+
+struct MxScaling {
+    int exponent;           // MxSharedExponent of the block
+    float scale;            // 2^exponent, the operand of the scaled converts
+    uint32_t limit;         // magnitude that has the largest finite code, in both halves
+    bool plain;             // every element is finite
+};
+
+template <bool BF16, bool E5M2>
+__device__ __forceinline__ MxScaling MxScalingOf(uint32_t maxBits)
+{
+    constexpr int kEmax = E5M2 ? 15 : 8;
+    MxScaling s;
+    int biased;             // exponent field of the scale
+    if (BF16) {
+        // an exponent field below emax means a shared exponent clamped at -127, where nothing can saturate
+        int e = static_cast<int>(maxBits >> 7);
+        e = e < kEmax ? kEmax : e;
+        biased = e - kEmax;
+        const uint32_t one = (static_cast<uint32_t>(e) << 7) | 0x60u;
+        s.limit = one | (one << 16);
+        s.plain = maxBits < 0x7f80u;
+    } else {
+        const uint32_t bits = __float_as_uint(Decode16<false>(maxBits));
+        biased = static_cast<int>(bits >> 23) - kEmax;          // at least 127 - 24 - emax, or below zero for a block of zeros
+        biased = biased < 0 ? 0 : biased;
+        // rounded down where it is a subnormal fp16: no magnitude lies between the two
+        const float one = __uint_as_float((bits & 0x7f800000u) | 0x00600000u);
+        s.limit = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(one, one));
+        s.plain = maxBits < 0x7c00u;
+    }
+    s.exponent = biased - 127;
+    // 2^-127 is a subnormal fp32
+    const uint32_t bits = static_cast<uint32_t>(biased) << 23;
+    s.scale = __uint_as_float(bits < 0x00400000u ? 0x00400000u : bits);
+    return s;
+}
+
+// Two elements of a plain block -> two codes in the upper or lower half of `old`.
+template <bool BF16, bool E5M2, bool UPPER>
+__device__ __forceinline__ uint32_t MxEncodePair(uint32_t old, uint32_t pair, const MxScaling &s)
+{
+    const uint32_t clamped = PackedMinU16(pair & kPackedMagnitude, s.limit) | (pair & ~kPackedMagnitude);
+    const s16x2 to = __builtin_bit_cast(s16x2, old);
+    s16x2 r;
+    if constexpr (BF16 && E5M2) {
+        r = __builtin_amdgcn_cvt_scalef32_pk_bf8_bf16(to, __builtin_bit_cast(bf16x2, clamped), s.scale, UPPER);
+    } else if constexpr (BF16) {
+        r = __builtin_amdgcn_cvt_scalef32_pk_fp8_bf16(to, __builtin_bit_cast(bf16x2, clamped), s.scale, UPPER);
+    } else if constexpr (E5M2) {
+        r = __builtin_amdgcn_cvt_scalef32_pk_bf8_f16(to, __builtin_bit_cast(f16x2, clamped), s.scale, UPPER);
+    } else {
+        r = __builtin_amdgcn_cvt_scalef32_pk_fp8_f16(to, __builtin_bit_cast(f16x2, clamped), s.scale, UPPER);
+    }
+    return __builtin_bit_cast(uint32_t, r);
+}
+
+// The two codes in the lower half of `codes`, each times the block's scale.
+template <bool E5M2>
+__device__ __forceinline__ f32x2 MxDecodePair(uint32_t codes, const MxScaling &s)
+{
+    if constexpr (E5M2) {
+        return __builtin_amdgcn_cvt_scalef32_pk_f32_bf8(codes, s.scale, false);
+    } else {
+        return __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(codes, s.scale, false);
+    }
+}
+
 } // namespace TileXREp
 
 #endif // TILEXR_AMD_EP_NUMERICS_HIP_H

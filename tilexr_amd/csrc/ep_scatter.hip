@@ -277,58 +277,74 @@ __global__ __launch_bounds__(kThreads) void ep_scatter_vec_kernel(ScatterArgs a)
             }
             uint32_t bytes[8];
             uint32_t fp8Words[2] = {0u, 0u};
-            if (QMODE == TILEXR_EP_QUANT_MXFP8 || QMODE == TILEXR_EP_QUANT_FP8_BLOCK128) {
+            if (QMODE == TILEXR_EP_QUANT_MXFP8) {
+                const MxScaling mx = MxScalingOf<BF16, E5M2>(MxBlockMaxBits(v[j]));
+                sharedExp[j] = mx.exponent;
+                if (__all(mx.plain ? 1 : 0)) {
+                    fp8Words[0] = MxEncodePair<BF16, E5M2, true>(MxEncodePair<BF16, E5M2, false>(0u, v[j][0], mx), v[j][1], mx);
+                    fp8Words[1] = MxEncodePair<BF16, E5M2, true>(MxEncodePair<BF16, E5M2, false>(0u, v[j][2], mx), v[j][3], mx);
+                } else {
+                    // infinities and NaNs: the codec that defines what becomes of them
+                    float amax = 0.0f;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        amax = fmaxf(amax, fabsf(f[e]));
+                    }
+                    amax = fmaxf(amax, __shfl_xor(amax, 1));
+                    amax = fmaxf(amax, __shfl_xor(amax, 2));
+                    const int se = MxSharedExponent<E5M2>(amax);
+                    sharedExp[j] = se;
+#pragma unroll 1
+                    for (int e = 0; e < 8; ++e) {
+                        const uint32_t pair = e < 4 ? (e < 2 ? v[j][0] : v[j][1]) : (e < 6 ? v[j][2] : v[j][3]);
+                        const float one = Decode16<BF16>((e & 1) != 0 ? pair >> 16 : pair & 0xffffu);
+                        const uint32_t code = Fp8Encode<E5M2>(ldexpf(one, -se)) << (8 * (e % 4));
+                        fp8Words[0] |= e < 4 ? code : 0u;
+                        fp8Words[1] |= e < 4 ? 0u : code;
+                    }
+                }
+            } else if (QMODE == TILEXR_EP_QUANT_FP8_BLOCK128) {
                 float amax = 0.0f;
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
                     amax = fmaxf(amax, fabsf(f[e]));
                 }
-                // 32 columns = 4 neighbouring lanes, 128 columns = 16 neighbouring lanes
-                constexpr int kSpan = QMODE == TILEXR_EP_QUANT_MXFP8 ? 4 : 16;
+                // 128 columns = 16 neighbouring lanes
 #pragma unroll
-                for (int off = 1; off < kSpan; off <<= 1) {
+                for (int off = 1; off < 16; off <<= 1) {
                     amax = fmaxf(amax, __shfl_xor(amax, off));
                 }
-                if (QMODE == TILEXR_EP_QUANT_MXFP8) {
-                    const int se = MxSharedExponent<E5M2>(amax);
-                    sharedExp[j] = se;
+                const float sc = amax > 0.0f ? __fdiv_rn(amax, 448.0f) : 1.0f;
+                blockScale[j] = sc;
+                // eight quotients by one divisor: what depends on the divisor alone is done once (ep_numerics.hip.h)
+                float quot[8];
+                const bool shortForm = __all(SharedReciprocalHolds(sc) ? 1 : 0) != 0;
+                if (shortForm) {
+                    const float y = SharedReciprocal(sc);
 #pragma unroll
                     for (int e = 0; e < 8; ++e) {
-                        bytes[e] = Fp8Encode<E5M2>(ldexpf(f[e], -se));
+                        quot[e] = DivideByShared(f[e], sc, y);
                     }
                 } else {
-                    const float sc = amax > 0.0f ? __fdiv_rn(amax, 448.0f) : 1.0f;
-                    blockScale[j] = sc;
-                    // eight quotients by one divisor: what depends on the divisor alone is done once (ep_numerics.hip.h)
-                    float quot[8];
-                    const bool shortForm = __all(SharedReciprocalHolds(sc) ? 1 : 0) != 0;
-                    if (shortForm) {
-                        const float y = SharedReciprocal(sc);
 #pragma unroll
-                        for (int e = 0; e < 8; ++e) {
-                            quot[e] = DivideByShared(f[e], sc, y);
-                        }
-                    } else {
-#pragma unroll
-                        for (int e = 0; e < 8; ++e) {
-                            quot[e] = __fdiv_rn(f[e], sc);
-                        }
+                    for (int e = 0; e < 8; ++e) {
+                        quot[e] = __fdiv_rn(f[e], sc);
                     }
-                    bool anyNan = false;
+                }
+                bool anyNan = false;
 #pragma unroll
-                    for (int e = 0; e < 8; e += 2) {
-                        anyNan |= __builtin_isunordered(quot[e], quot[e + 1]);
-                    }
-                    if (!anyNan) {
-                        // four codes per word straight from the converts: the second one fills the word's upper half
-                        fp8Words[0] = Fp8E4m3EncodeFourSat(quot[0], quot[1], quot[2], quot[3]);
-                        fp8Words[1] = Fp8E4m3EncodeFourSat(quot[4], quot[5], quot[6], quot[7]);
-                    } else {
+                for (int e = 0; e < 8; e += 2) {
+                    anyNan |= __builtin_isunordered(quot[e], quot[e + 1]);
+                }
+                if (!anyNan) {
+                    // four codes per word straight from the converts: the second one fills the word's upper half
+                    fp8Words[0] = Fp8E4m3EncodeFourSat(quot[0], quot[1], quot[2], quot[3]);
+                    fp8Words[1] = Fp8E4m3EncodeFourSat(quot[4], quot[5], quot[6], quot[7]);
+                } else {
 #pragma unroll
-                        for (int e = 0; e < 8; e += 4) {
-                            fp8Words[e / 4] = Fp8E4m3EncodePairSat(quot[e], quot[e + 1]) |
-                                (Fp8E4m3EncodePairSat(quot[e + 2], quot[e + 3]) << 16);
-                        }
+                    for (int e = 0; e < 8; e += 4) {
+                        fp8Words[e / 4] = Fp8E4m3EncodePairSat(quot[e], quot[e + 1]) |
+                            (Fp8E4m3EncodePairSat(quot[e + 2], quot[e + 3]) << 16);
                     }
                 }
             } else {
@@ -337,7 +353,7 @@ __global__ __launch_bounds__(kThreads) void ep_scatter_vec_kernel(ScatterArgs a)
                     bytes[e] = static_cast<uint32_t>(ClampInt8(__fmul_rn(f[e], rowScaleInv))) & 0xffu;
                 }
             }
-            if (QMODE == TILEXR_EP_QUANT_FP8_BLOCK128) {
+            if (QMODE == TILEXR_EP_QUANT_MXFP8 || QMODE == TILEXR_EP_QUANT_FP8_BLOCK128) {
                 q[j][0] = fp8Words[0];
                 q[j][1] = fp8Words[1];
             } else {
