@@ -60,7 +60,13 @@ int RunDispatchSingle(EpComm *comm, const EpDispatchParams &p, bool memoryRoute,
             return TileXR::TILEXR_ERROR_MKIRT;
         }
     }
-    if (memoryRoute && p.quantMode == TILEXR_EP_QUANT_NONE && p.xActiveMask == nullptr && p.metaReadyEvent == nullptr) {
+    int maskMode = kMaskNone;
+    if (p.xActiveMask != nullptr && !memoryRoute) {
+        maskMode = kMaskPerToken;              // reference: tilexr_ep_dispatch_helpers.h:3-21
+    } else if (p.xActiveMask != nullptr) {
+        maskMode = p.activeMaskType == TILEXR_EP_ACTIVE_MASK_EXPERT ? kMaskPerRoute : kMaskTokenPrefix;
+    }
+    if (memoryRoute && p.quantMode == TILEXR_EP_QUANT_NONE && p.metaReadyEvent == nullptr) {
         // decode-sized calls: one launch instead of count + scatter (a consumer that is to run beside the dispatch needs
         // the row map ahead of the rows, which takes the separate launches)
         SmallDispatchLaunch small {};
@@ -70,6 +76,8 @@ int RunDispatchSingle(EpComm *comm, const EpDispatchParams &p, bool memoryRoute,
         small.h = p.h;
         small.topK = p.topK;
         small.numExperts = experts;
+        small.mask = reinterpret_cast<const uint8_t *>(p.xActiveMask);
+        small.maskMode = maskMode;
         small.capacity = p.expertCapacity;
         small.srcRank = comm->rank;
         small.expertIdBias = static_cast<int32_t>(p.sharedExpertNum);
@@ -102,12 +110,6 @@ int RunDispatchSingle(EpComm *comm, const EpDispatchParams &p, bool memoryRoute,
         }
     }
     const CountScratchLayout plan = PlanCountScratch(n, numKeys, experts, expertHist);
-    int maskMode = kMaskNone;
-    if (p.xActiveMask != nullptr && !memoryRoute) {
-        maskMode = kMaskPerToken;              // reference: tilexr_ep_dispatch_helpers.h:3-21
-    } else if (p.xActiveMask != nullptr) {
-        maskMode = p.activeMaskType == TILEXR_EP_ACTIVE_MASK_EXPERT ? kMaskPerRoute : kMaskTokenPrefix;
-    }
     // One launch resolves every route's row where every expert's workgroup can afford to read the whole id table
     // (ep_rows.hip); otherwise count (ticket, last workgroup scans) and place, the latter folded into the scatter
     // unless something needs the rows ahead of it.

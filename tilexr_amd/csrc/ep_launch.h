@@ -219,6 +219,8 @@ struct SmallDispatchLaunch {
     int64_t h;
     int64_t topK;
     int64_t numExperts;
+    const uint8_t *mask;         // nullptr with kMaskNone
+    int maskMode;                // kMaskNone, kMaskPerRoute or kMaskTokenPrefix
     int64_t capacity;
     int32_t srcRank;
     int32_t expertIdBias;

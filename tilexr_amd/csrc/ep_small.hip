@@ -30,6 +30,8 @@ struct SmallArgs {
     int h;
     int topK;
     int numExperts;
+    const uint8_t *mask;         // masked kernels: [bs] or [bs, topK]
+    int maskPerRoute;            // 1: route live iff mask[token, k]; 0: iff token < sum(mask)
     int capacity;
     int32_t srcRank;
     int32_t expertIdBias;
@@ -54,9 +56,46 @@ __device__ __forceinline__ void SmallRowStore(const u32x4 &v, u32x4 *dst, __amdg
     }
 }
 
-template <int V, bool WT>
+// Masked calls: first route that a token-prefix mask leaves out (n for a mask per route).  The mask is read beside the id
+// table, four bytes of it in flight per lane (1024 tokens), and one LDS exchange between the waves adds it up.  All lanes
+// of the workgroup call it.
+constexpr int kMaskBatch = 4;
+__device__ __forceinline__ int SmallLiveLimit(const SmallArgs &a, int n, int *s_live)
+{
+    if (a.maskPerRoute != 0) {
+        return n;
+    }
+    // bytes beyond the mask's end read as zero
+    const __amdgpu_buffer_rsrc_t mask = RowResource(a.mask, a.bs);
+    int live = 0;
+    for (int first = 0; first < a.bs; first += kMaskBatch * kThreads) {
+        uint8_t m[kMaskBatch];
+#pragma unroll
+        for (int u = 0; u < kMaskBatch; ++u) {
+            m[u] = __builtin_amdgcn_raw_buffer_load_b8(mask, first + u * kThreads + static_cast<int>(threadIdx.x), 0, 0);
+        }
+#pragma unroll
+        for (int u = 0; u < kMaskBatch; ++u) {
+            live += __popcll(__ballot(m[u] != 0));
+        }
+    }
+    if ((threadIdx.x & (kWave - 1)) == 0) {
+        s_live[threadIdx.x / kWave] = live;
+    }
+    __syncthreads();
+    return (s_live[0] + s_live[1] + s_live[2] + s_live[3]) * a.topK;
+}
+
+// Whether a route below `n` is dispatched.
+__device__ __forceinline__ bool SmallRouteLive(const SmallArgs &a, int route, int limit)
+{
+    return a.maskPerRoute != 0 ? a.mask[route] != 0 : route < limit;
+}
+
+template <int V, bool WT, bool MASKED>
 __global__ __launch_bounds__(kThreads) void ep_dispatch_small_kernel(SmallArgs a)
 {
+    __shared__ int s_live[kWavesPerBlock];
     __shared__ int s_hist[kMaxKeys];     // routes per expert, then exclusive row offsets
     __shared__ int s_kept[kMaxKeys];
     __shared__ int s_rank[kMaxTopK];
@@ -87,9 +126,19 @@ __global__ __launch_bounds__(kThreads) void ep_dispatch_small_kernel(SmallArgs a
     for (int k = tid; k < a.numExperts; k += kThreads) {
         s_hist[k] = 0;
     }
+    const int ownId = tid < a.topK ? a.ids[token * a.topK + tid] : -1;
+    int limit = n;
+    if (MASKED) {
+        limit = SmallLiveLimit(a, n, s_live);
+#pragma unroll
+        for (int j = 0; j < kIdsPerLane; ++j) {
+            const int i = j * kThreads + tid;
+            e[j] = i < n && SmallRouteLive(a, i, limit) ? e[j] : -1;
+        }
+    }
     if (tid < a.topK) {
-        const int id = a.ids[token * a.topK + tid];
-        s_key[tid] = (id >= 0 && id < a.numExperts) ? id : -1;
+        const bool live = !MASKED || SmallRouteLive(a, token * a.topK + tid, limit);
+        s_key[tid] = (live && ownId >= 0 && ownId < a.numExperts) ? ownId : -1;
         s_rank[tid] = 0;
     }
     __syncthreads();
@@ -184,9 +233,14 @@ __global__ __launch_bounds__(kThreads) void ep_dispatch_small_kernel(SmallArgs a
 // instruction every 4 ns or so.  So every lane counts its own ids with compares and adds (no ballot and scalar count
 // per id), the four sets share two registers (16 bits each: at most 2048 ids), one pair of reductions per wave and one
 // LDS exchange between the four waves finish it.  IDS = ids per lane (4: up to 1024 routes, 8: up to 2048).
-template <int V, bool WT, int IDS>
+//
+// MASKED: the routes a mask leaves out are dropped from the counts like ids outside [0, E) (token-prefix mask: one more
+// LDS exchange, for the number of active tokens).  200 tokens x 7168 x top-8 of 256 with a token mask: 6.7 us, 13.3 us
+// for the count and scatter launches such calls took before.
+template <int V, bool WT, int IDS, bool MASKED>
 __global__ __launch_bounds__(kThreads) void ep_dispatch_small_route_kernel(SmallArgs a)
 {
+    __shared__ int s_live[kWavesPerBlock];
     __shared__ int s_sum[kWavesPerBlock][3];     // per wave: smaller | earlier equal << 16, equal to blockIdx | not above << 16, valid
 
     const int tid = threadIdx.x;
@@ -218,7 +272,17 @@ __global__ __launch_bounds__(kThreads) void ep_dispatch_small_route_kernel(Small
     }
     const int mine = a.ids[route];
     const unsigned experts = static_cast<unsigned>(a.numExperts);
-    const int key = hasRoute && static_cast<unsigned>(mine) < experts ? mine : -1;       // ids outside [0, E) are skipped, not errors
+    bool live = hasRoute;
+    if (MASKED) {
+        const int limit = SmallLiveLimit(a, n, s_live);
+#pragma unroll
+        for (int j = 0; j < IDS; ++j) {
+            const int i = j * kThreads + tid;
+            e[j] = i < n && SmallRouteLive(a, i, limit) ? e[j] : -1;
+        }
+        live = hasRoute && SmallRouteLive(a, route, limit);
+    }
+    const int key = live && static_cast<unsigned>(mine) < experts ? mine : -1;       // ids outside [0, E) are skipped, not errors
     const int expert = blockIdx.x;       // the expert this workgroup counts for the outputs (if there is one)
     int rowCounts = 0;      // valid ids below the key | earlier ids equal to it << 16
     int outCounts = 0;      // ids equal to `expert` | valid ids not above it << 16
@@ -296,7 +360,8 @@ __global__ __launch_bounds__(kThreads) void ep_dispatch_small_route_kernel(Small
 bool SmallDispatchFits(const SmallDispatchLaunch &l)
 {
     return l.bs * l.topK <= kSmallRoutes && l.numExperts <= kMaxKeys && l.topK <= kMaxTopK && l.h % 8 == 0 &&
-        l.h / 8 <= 8 * kThreads && Aligned16(l.x) && Aligned16(l.out);
+        l.h / 8 <= 8 * kThreads && Aligned16(l.x) && Aligned16(l.out) &&
+        (l.maskMode == kMaskNone || (l.mask != nullptr && (l.maskMode == kMaskPerRoute || l.maskMode == kMaskTokenPrefix)));
 }
 
 hipError_t LaunchSmallDispatch(const SmallDispatchLaunch &l)
@@ -308,6 +373,8 @@ hipError_t LaunchSmallDispatch(const SmallDispatchLaunch &l)
     a.h = static_cast<int>(l.h);
     a.topK = static_cast<int>(l.topK);
     a.numExperts = static_cast<int>(l.numExperts);
+    a.mask = l.mask;
+    a.maskPerRoute = l.maskMode == kMaskPerRoute ? 1 : 0;
     a.capacity = static_cast<int>(l.capacity);
     a.srcRank = l.srcRank;
     a.expertIdBias = l.expertIdBias;
@@ -335,12 +402,22 @@ hipError_t LaunchSmallDispatch(const SmallDispatchLaunch &l)
         }
         const dim3 routes(static_cast<unsigned>(XcdPlacedUnits(static_cast<int>(l.bs), static_cast<int>(l.topK))));
         const bool few = l.bs * l.topK <= 4 * kThreads;
-        auto pick = [&](auto vecsPerLane) {
+        auto pickMasked = [&](auto vecsPerLane, auto masked) {
             constexpr int kV = decltype(vecsPerLane)::value;
+            constexpr bool kMasked = decltype(masked)::value;
             if (few) {
-                flags ? launch(ep_dispatch_small_route_kernel<kV, true, 4>, routes) : launch(ep_dispatch_small_route_kernel<kV, false, 4>, routes);
+                flags ? launch(ep_dispatch_small_route_kernel<kV, true, 4, kMasked>, routes) :
+                        launch(ep_dispatch_small_route_kernel<kV, false, 4, kMasked>, routes);
             } else {
-                flags ? launch(ep_dispatch_small_route_kernel<kV, true, kIdsPerLane>, routes) : launch(ep_dispatch_small_route_kernel<kV, false, kIdsPerLane>, routes);
+                flags ? launch(ep_dispatch_small_route_kernel<kV, true, kIdsPerLane, kMasked>, routes) :
+                        launch(ep_dispatch_small_route_kernel<kV, false, kIdsPerLane, kMasked>, routes);
+            }
+        };
+        auto pick = [&](auto vecsPerLane) {
+            if (l.maskMode != kMaskNone) {
+                pickMasked(vecsPerLane, std::true_type {});
+            } else {
+                pickMasked(vecsPerLane, std::false_type {});
             }
         };
         if (v == 2) {
@@ -356,12 +433,20 @@ hipError_t LaunchSmallDispatch(const SmallDispatchLaunch &l)
     if (l.kernelNameOut != nullptr) {
         *l.kernelNameOut = "ep_dispatch_small_kernel";
     }
+    auto pick = [&](auto vecsPerLane) {
+        constexpr int kV = decltype(vecsPerLane)::value;
+        if (l.maskMode != kMaskNone) {
+            flags ? launch(ep_dispatch_small_kernel<kV, true, true>, grid) : launch(ep_dispatch_small_kernel<kV, false, true>, grid);
+        } else {
+            flags ? launch(ep_dispatch_small_kernel<kV, true, false>, grid) : launch(ep_dispatch_small_kernel<kV, false, false>, grid);
+        }
+    };
     if (v == 2) {
-        flags ? launch(ep_dispatch_small_kernel<2, true>, grid) : launch(ep_dispatch_small_kernel<2, false>, grid);
+        pick(std::integral_constant<int, 2>{});
     } else if (v == 4) {
-        flags ? launch(ep_dispatch_small_kernel<4, true>, grid) : launch(ep_dispatch_small_kernel<4, false>, grid);
+        pick(std::integral_constant<int, 4>{});
     } else {
-        flags ? launch(ep_dispatch_small_kernel<8, true>, grid) : launch(ep_dispatch_small_kernel<8, false>, grid);
+        pick(std::integral_constant<int, 8>{});
     }
     return hipGetLastError();
 }
