@@ -55,8 +55,21 @@ inline PlaceArgs MakePlaceArgs(const RoutePlaceLaunch &l)
     return a;
 }
 
-// Resolves route i (< a.n), writes its assist tuple and rowOf entry, returns the row or -1.
-__device__ __forceinline__ int PlaceRoute(const PlaceArgs &a, int i)
+// The assist tuple of route i, which goes to `row` and names expert `e`.
+__device__ __forceinline__ void WriteTuple(const PlaceArgs &a, int i, int row, int e)
+{
+    int32_t *tuple = a.assist + static_cast<int64_t>(row) * 4;
+    const int pos = i % a.topK;
+    tuple[0] = a.srcRank;
+    tuple[1] = i / a.topK;
+    // shared routes come first in a token's row and report the slots after the routed ones
+    // (reference: src/ep/kernels/tilexr_ep_dispatch_kernel.cpp:536-568)
+    tuple[2] = pos < a.sharedNum ? a.topK - a.sharedNum + pos : pos - a.sharedNum;
+    tuple[3] = a.tupleExperts != nullptr ? a.tupleExperts[i] : e + a.expertIdBias;
+}
+
+// Resolves route i (< a.n) and returns its row or -1; `record`: writes its assist tuple and rowOf entry as well.
+__device__ __forceinline__ int PlaceRoute(const PlaceArgs &a, int i, bool record = true)
 {
     // both loads at once: the id is there for every route, whether it is live or not
     const int lr = a.localRank[i];
@@ -67,17 +80,12 @@ __device__ __forceinline__ int PlaceRoute(const PlaceArgs &a, int i)
         const int within = a.chunkBase[static_cast<int64_t>(i >> a.chunkShift) * a.numKeys + key] + lr;
         if (a.capacity <= 0 || within < a.capacity) {
             row = a.keyOffset[key] + within;
-            int32_t *tuple = a.assist + static_cast<int64_t>(row) * 4;
-            const int pos = i % a.topK;
-            tuple[0] = a.srcRank;
-            tuple[1] = i / a.topK;
-            // shared routes come first in a token's row and report the slots after the routed ones
-            // (reference: src/ep/kernels/tilexr_ep_dispatch_kernel.cpp:536-568)
-            tuple[2] = pos < a.sharedNum ? a.topK - a.sharedNum + pos : pos - a.sharedNum;
-            tuple[3] = a.tupleExperts != nullptr ? a.tupleExperts[i] : e + a.expertIdBias;
+            if (record) {
+                WriteTuple(a, i, row, e);
+            }
         }
     }
-    if (a.rowOf != nullptr) {
+    if (record && a.rowOf != nullptr) {
         a.rowOf[i] = row;
     }
     return row;

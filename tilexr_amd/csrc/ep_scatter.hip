@@ -65,9 +65,8 @@ __device__ __forceinline__ float GroupMax(float v, float *red, int lane)
         if ((lane & (kWave - 1)) == 0) {
             red[lane / kWave] = v;
         }
-        __syncthreads();
+        LdsBarrier();
         v = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-        __syncthreads();
     }
     return v;
 }
@@ -200,8 +199,182 @@ __global__ __launch_bounds__(THREADS) void ep_scatter_route_kernel(ScatterArgs a
     }
 }
 
-template <int G, int V, int QMODE, bool BF16, bool E5M2, bool WT>
-__global__ __launch_bounds__(kThreads) void ep_scatter_vec_kernel(ScatterArgs a)
+// A row's payload and scales, as the lanes of its group hold them: eight bytes per 16-byte vector.
+template <int V>
+struct QuantisedRow {
+    u32x2 q[V];
+    float blockScale[V];        // fp8: scale of the vector's 128 columns
+    int sharedExp[V];           // MXFP8: exponent of the vector's 32 columns
+    float rowScale;             // int8
+};
+
+template <int G, int V, int QMODE, bool BF16, bool E5M2>
+__device__ __forceinline__ void QuantiseRow(const ScatterArgs &a, const u32x4 (&v)[V], float *red, int lane, QuantisedRow<V> &out)
+{
+    out.rowScale = 1.0f;
+    // per-row / per-block scale, then 8 output bytes per input vector
+    float rowScaleInv = 1.0f;
+    if (QMODE == TILEXR_EP_QUANT_STATIC_INT8) {
+        rowScaleInv = a.staticScale[0];
+    }
+    if (QMODE == TILEXR_EP_QUANT_TOKEN_INT8) {
+        float amax = 0.0f;
+#pragma unroll
+        for (int j = 0; j < V; ++j) {
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                amax = fmaxf(amax, fabsf(Decode16<BF16>(v[j][w] & 0xffffu)));
+                amax = fmaxf(amax, fabsf(Decode16<BF16>(v[j][w] >> 16)));
+            }
+        }
+        amax = GroupMax<G>(amax, red, lane);
+        out.rowScale = amax > 0.0f ? __fdiv_rn(amax, 127.0f) : 1.0f;
+        rowScaleInv = out.rowScale > 0.0f ? __fdiv_rn(1.0f, out.rowScale) : 1.0f;
+    }
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+        float f[8];
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            f[2 * w] = Decode16<BF16>(v[j][w] & 0xffffu);
+            f[2 * w + 1] = Decode16<BF16>(v[j][w] >> 16);
+        }
+        uint32_t bytes[8];
+        uint32_t fp8Words[2] = {0u, 0u};
+        if (QMODE == TILEXR_EP_QUANT_MXFP8) {
+            const MxScaling mx = MxScalingOf<BF16, E5M2>(MxBlockMaxBits(v[j]));
+            out.sharedExp[j] = mx.exponent;
+            if (__all(mx.plain ? 1 : 0)) {
+                fp8Words[0] = MxEncodePair<BF16, E5M2, true>(MxEncodePair<BF16, E5M2, false>(0u, v[j][0], mx), v[j][1], mx);
+                fp8Words[1] = MxEncodePair<BF16, E5M2, true>(MxEncodePair<BF16, E5M2, false>(0u, v[j][2], mx), v[j][3], mx);
+            } else {
+                // infinities and NaNs: the codec that defines what becomes of them
+                float amax = 0.0f;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    amax = fmaxf(amax, fabsf(f[e]));
+                }
+                amax = fmaxf(amax, __shfl_xor(amax, 1));
+                amax = fmaxf(amax, __shfl_xor(amax, 2));
+                const int se = MxSharedExponent<E5M2>(amax);
+                out.sharedExp[j] = se;
+#pragma unroll 1
+                for (int e = 0; e < 8; ++e) {
+                    const uint32_t pair = e < 4 ? (e < 2 ? v[j][0] : v[j][1]) : (e < 6 ? v[j][2] : v[j][3]);
+                    const float one = Decode16<BF16>((e & 1) != 0 ? pair >> 16 : pair & 0xffffu);
+                    const uint32_t code = Fp8Encode<E5M2>(ldexpf(one, -se)) << (8 * (e % 4));
+                    fp8Words[0] |= e < 4 ? code : 0u;
+                    fp8Words[1] |= e < 4 ? 0u : code;
+                }
+            }
+        } else if (QMODE == TILEXR_EP_QUANT_FP8_BLOCK128) {
+            float amax = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                amax = fmaxf(amax, fabsf(f[e]));
+            }
+            // 128 columns = 16 neighbouring lanes
+#pragma unroll
+            for (int off = 1; off < 16; off <<= 1) {
+                amax = fmaxf(amax, __shfl_xor(amax, off));
+            }
+            const float sc = amax > 0.0f ? __fdiv_rn(amax, 448.0f) : 1.0f;
+            out.blockScale[j] = sc;
+            // eight quotients by one divisor: what depends on the divisor alone is done once (ep_numerics.hip.h)
+            float quot[8];
+            const bool shortForm = __all(SharedReciprocalHolds(sc) ? 1 : 0) != 0;
+            if (shortForm) {
+                const float y = SharedReciprocal(sc);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    quot[e] = DivideByShared(f[e], sc, y);
+                }
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    quot[e] = __fdiv_rn(f[e], sc);
+                }
+            }
+            bool anyNan = false;
+#pragma unroll
+            for (int e = 0; e < 8; e += 2) {
+                anyNan |= __builtin_isunordered(quot[e], quot[e + 1]);
+            }
+            if (!anyNan) {
+                // four codes per word straight from the converts: the second one fills the word's upper half
+                fp8Words[0] = Fp8E4m3EncodeFourSat(quot[0], quot[1], quot[2], quot[3]);
+                fp8Words[1] = Fp8E4m3EncodeFourSat(quot[4], quot[5], quot[6], quot[7]);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; e += 4) {
+                    fp8Words[e / 4] = Fp8E4m3EncodePairSat(quot[e], quot[e + 1]) |
+                        (Fp8E4m3EncodePairSat(quot[e + 2], quot[e + 3]) << 16);
+                }
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                bytes[e] = static_cast<uint32_t>(ClampInt8(__fmul_rn(f[e], rowScaleInv))) & 0xffu;
+            }
+        }
+        if (QMODE == TILEXR_EP_QUANT_MXFP8 || QMODE == TILEXR_EP_QUANT_FP8_BLOCK128) {
+            out.q[j][0] = fp8Words[0];
+            out.q[j][1] = fp8Words[1];
+        } else {
+            out.q[j][0] = bytes[0] | (bytes[1] << 8) | (bytes[2] << 16) | (bytes[3] << 24);
+            out.q[j][1] = bytes[4] | (bytes[5] << 8) | (bytes[6] << 16) | (bytes[7] << 24);
+        }
+    }
+}
+
+// Writes the row (or its payload and scales) held by the group's lanes to row `row` of the outputs.
+template <int G, int V, int QMODE, bool WT>
+__device__ __forceinline__ void StoreRow(const ScatterArgs &a, int row, const u32x4 (&v)[V], const QuantisedRow<V> &out, int lane)
+{
+    const int vecs = a.h / 8;
+    if (QMODE == TILEXR_EP_QUANT_NONE) {
+        char *dst = static_cast<char *>(a.out) + static_cast<int64_t>(row) * a.h * 2;
+        const __amdgpu_buffer_rsrc_t rsrc = RowResource(dst, vecs * 16);
+#pragma unroll
+        for (int j = 0; j < V; ++j) {
+            const int idx = j * G + lane;
+            if (idx < vecs) {
+                RowStore<WT>(v[j], dst, rsrc, idx * 16);
+            }
+        }
+        return;
+    }
+    const int mxBlocks = (a.h + 31) / 32;
+    const int mxScales = (mxBlocks + 1) / 2 * 2;
+    const int b128 = (a.h + 127) / 128;
+    char *dst = static_cast<char *>(a.out) + static_cast<int64_t>(row) * a.h;
+    const __amdgpu_buffer_rsrc_t rsrc = RowResource(dst, vecs * 8);
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+        const int idx = j * G + lane;
+        if (idx < vecs) {
+            RowStore<WT>(out.q[j], dst, rsrc, idx * 8);
+            if (QMODE == TILEXR_EP_QUANT_MXFP8 && (idx & 3) == 0) {
+                uint8_t *sc = static_cast<uint8_t *>(a.scalesOut) + static_cast<int64_t>(row) * mxScales;
+                ScalarStore<WT>(sc + (idx >> 2), static_cast<uint8_t>(out.sharedExp[j] + 127));
+                if ((idx >> 2) + 1 == mxBlocks && mxBlocks < mxScales) {
+                    ScalarStore<WT>(sc + mxBlocks, static_cast<uint8_t>(0));    // padding byte of an odd block count
+                }
+            }
+            if (QMODE == TILEXR_EP_QUANT_FP8_BLOCK128 && (idx & 15) == 0) {
+                ScalarStore<WT>(static_cast<float *>(a.scalesOut) + static_cast<int64_t>(row) * b128 + (idx >> 4),
+                    out.blockScale[j]);
+            }
+        }
+    }
+    if (QMODE == TILEXR_EP_QUANT_TOKEN_INT8 && lane == 0) {
+        ScalarStore<WT>(static_cast<float *>(a.scalesOut) + row, out.rowScale);
+    }
+}
+
+// Publishing launches: one token per group, because a group stays until its own stores have landed.
+template <int G, int V, int QMODE, bool BF16, bool E5M2>
+__device__ __forceinline__ void ScatterAndPublish(const ScatterArgs &a)
 {
     constexpr int kTokens = kThreads / G;
     __shared__ int s_pos[kTokens][kMaxTopK];
@@ -225,177 +398,72 @@ __global__ __launch_bounds__(kThreads) void ep_scatter_vec_kernel(ScatterArgs a)
         v[j] = (tokOk && idx < vecs) ? src[idx] : u32x4{0u, 0u, 0u, 0u};
     }
     __syncthreads();
-
-    if (QMODE == TILEXR_EP_QUANT_NONE) {
-        for (int k = 0; k < a.topK; ++k) {
-            // the lanes of a wave share one token, so the row is wave-uniform
-            const int row = __builtin_amdgcn_readfirstlane(s_pos[tg][k]);
-            if (row < 0) {
-                continue;
-            }
-            char *dst = static_cast<char *>(a.out) + static_cast<int64_t>(row) * a.h * 2;
-            const __amdgpu_buffer_rsrc_t rsrc = RowResource(dst, vecs * 16);
-#pragma unroll
-            for (int j = 0; j < V; ++j) {
-                const int idx = j * G + lane;
-                if (idx < vecs) {
-                    RowStore<WT>(v[j], dst, rsrc, idx * 16);
-                }
-            }
-        }
-    } else {
-        // per-row / per-block scale, then 8 output bytes per input vector
-        float rowScaleInv = 1.0f;
-        float rowScale = 1.0f;
-        if (QMODE == TILEXR_EP_QUANT_STATIC_INT8) {
-            rowScaleInv = a.staticScale[0];
-        }
-        if (QMODE == TILEXR_EP_QUANT_TOKEN_INT8) {
-            float amax = 0.0f;
-#pragma unroll
-            for (int j = 0; j < V; ++j) {
-#pragma unroll
-                for (int w = 0; w < 4; ++w) {
-                    amax = fmaxf(amax, fabsf(Decode16<BF16>(v[j][w] & 0xffffu)));
-                    amax = fmaxf(amax, fabsf(Decode16<BF16>(v[j][w] >> 16)));
-                }
-            }
-            amax = GroupMax<G>(amax, s_red[tg], lane);
-            rowScale = amax > 0.0f ? __fdiv_rn(amax, 127.0f) : 1.0f;
-            rowScaleInv = rowScale > 0.0f ? __fdiv_rn(1.0f, rowScale) : 1.0f;
-        }
-        u32x2 q[V];
-        float blockScale[V];
-        int sharedExp[V];
-#pragma unroll
-        for (int j = 0; j < V; ++j) {
-            float f[8];
-#pragma unroll
-            for (int w = 0; w < 4; ++w) {
-                f[2 * w] = Decode16<BF16>(v[j][w] & 0xffffu);
-                f[2 * w + 1] = Decode16<BF16>(v[j][w] >> 16);
-            }
-            uint32_t bytes[8];
-            uint32_t fp8Words[2] = {0u, 0u};
-            if (QMODE == TILEXR_EP_QUANT_MXFP8) {
-                const MxScaling mx = MxScalingOf<BF16, E5M2>(MxBlockMaxBits(v[j]));
-                sharedExp[j] = mx.exponent;
-                if (__all(mx.plain ? 1 : 0)) {
-                    fp8Words[0] = MxEncodePair<BF16, E5M2, true>(MxEncodePair<BF16, E5M2, false>(0u, v[j][0], mx), v[j][1], mx);
-                    fp8Words[1] = MxEncodePair<BF16, E5M2, true>(MxEncodePair<BF16, E5M2, false>(0u, v[j][2], mx), v[j][3], mx);
-                } else {
-                    // infinities and NaNs: the codec that defines what becomes of them
-                    float amax = 0.0f;
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        amax = fmaxf(amax, fabsf(f[e]));
-                    }
-                    amax = fmaxf(amax, __shfl_xor(amax, 1));
-                    amax = fmaxf(amax, __shfl_xor(amax, 2));
-                    const int se = MxSharedExponent<E5M2>(amax);
-                    sharedExp[j] = se;
-#pragma unroll 1
-                    for (int e = 0; e < 8; ++e) {
-                        const uint32_t pair = e < 4 ? (e < 2 ? v[j][0] : v[j][1]) : (e < 6 ? v[j][2] : v[j][3]);
-                        const float one = Decode16<BF16>((e & 1) != 0 ? pair >> 16 : pair & 0xffffu);
-                        const uint32_t code = Fp8Encode<E5M2>(ldexpf(one, -se)) << (8 * (e % 4));
-                        fp8Words[0] |= e < 4 ? code : 0u;
-                        fp8Words[1] |= e < 4 ? 0u : code;
-                    }
-                }
-            } else if (QMODE == TILEXR_EP_QUANT_FP8_BLOCK128) {
-                float amax = 0.0f;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    amax = fmaxf(amax, fabsf(f[e]));
-                }
-                // 128 columns = 16 neighbouring lanes
-#pragma unroll
-                for (int off = 1; off < 16; off <<= 1) {
-                    amax = fmaxf(amax, __shfl_xor(amax, off));
-                }
-                const float sc = amax > 0.0f ? __fdiv_rn(amax, 448.0f) : 1.0f;
-                blockScale[j] = sc;
-                // eight quotients by one divisor: what depends on the divisor alone is done once (ep_numerics.hip.h)
-                float quot[8];
-                const bool shortForm = __all(SharedReciprocalHolds(sc) ? 1 : 0) != 0;
-                if (shortForm) {
-                    const float y = SharedReciprocal(sc);
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        quot[e] = DivideByShared(f[e], sc, y);
-                    }
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        quot[e] = __fdiv_rn(f[e], sc);
-                    }
-                }
-                bool anyNan = false;
-#pragma unroll
-                for (int e = 0; e < 8; e += 2) {
-                    anyNan |= __builtin_isunordered(quot[e], quot[e + 1]);
-                }
-                if (!anyNan) {
-                    // four codes per word straight from the converts: the second one fills the word's upper half
-                    fp8Words[0] = Fp8E4m3EncodeFourSat(quot[0], quot[1], quot[2], quot[3]);
-                    fp8Words[1] = Fp8E4m3EncodeFourSat(quot[4], quot[5], quot[6], quot[7]);
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 8; e += 4) {
-                        fp8Words[e / 4] = Fp8E4m3EncodePairSat(quot[e], quot[e + 1]) |
-                            (Fp8E4m3EncodePairSat(quot[e + 2], quot[e + 3]) << 16);
-                    }
-                }
-            } else {
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    bytes[e] = static_cast<uint32_t>(ClampInt8(__fmul_rn(f[e], rowScaleInv))) & 0xffu;
-                }
-            }
-            if (QMODE == TILEXR_EP_QUANT_MXFP8 || QMODE == TILEXR_EP_QUANT_FP8_BLOCK128) {
-                q[j][0] = fp8Words[0];
-                q[j][1] = fp8Words[1];
-            } else {
-                q[j][0] = bytes[0] | (bytes[1] << 8) | (bytes[2] << 16) | (bytes[3] << 24);
-                q[j][1] = bytes[4] | (bytes[5] << 8) | (bytes[6] << 16) | (bytes[7] << 24);
-            }
-        }
-        const int mxBlocks = (a.h + 31) / 32;
-        const int mxScales = (mxBlocks + 1) / 2 * 2;
-        const int b128 = (a.h + 127) / 128;
-        for (int k = 0; k < a.topK; ++k) {
-            const int row = __builtin_amdgcn_readfirstlane(s_pos[tg][k]);
-            if (row < 0) {
-                continue;
-            }
-            char *dst = static_cast<char *>(a.out) + static_cast<int64_t>(row) * a.h;
-            const __amdgpu_buffer_rsrc_t rsrc = RowResource(dst, vecs * 8);
-#pragma unroll
-            for (int j = 0; j < V; ++j) {
-                const int idx = j * G + lane;
-                if (idx < vecs) {
-                    RowStore<WT>(q[j], dst, rsrc, idx * 8);
-                    if (QMODE == TILEXR_EP_QUANT_MXFP8 && (idx & 3) == 0) {
-                        uint8_t *sc = static_cast<uint8_t *>(a.scalesOut) + static_cast<int64_t>(row) * mxScales;
-                        ScalarStore<WT>(sc + (idx >> 2), static_cast<uint8_t>(sharedExp[j] + 127));
-                        if ((idx >> 2) + 1 == mxBlocks && mxBlocks < mxScales) {
-                            ScalarStore<WT>(sc + mxBlocks, static_cast<uint8_t>(0));    // padding byte of an odd block count
-                        }
-                    }
-                    if (QMODE == TILEXR_EP_QUANT_FP8_BLOCK128 && (idx & 15) == 0) {
-                        ScalarStore<WT>(static_cast<float *>(a.scalesOut) + static_cast<int64_t>(row) * b128 + (idx >> 4),
-                            blockScale[j]);
-                    }
-                }
-            }
-            if (QMODE == TILEXR_EP_QUANT_TOKEN_INT8 && lane == 0) {
-                ScalarStore<WT>(static_cast<float *>(a.scalesOut) + row, rowScale);
-            }
+    QuantisedRow<V> out;
+    if (QMODE != TILEXR_EP_QUANT_NONE) {
+        QuantiseRow<G, V, QMODE, BF16, E5M2>(a, v, s_red[tg], lane, out);
+    }
+    for (int k = 0; k < a.topK; ++k) {
+        // the lanes of a wave share one token, so the row is wave-uniform
+        const int row = __builtin_amdgcn_readfirstlane(s_pos[tg][k]);
+        if (row >= 0) {
+            StoreRow<G, V, QMODE, true>(a, row, v, out, lane);
         }
     }
-    if (WT && a.tileFlags != nullptr) {
+    if (a.tileFlags != nullptr) {
         PublishRows<true>(a, s_pos[tg], lane, G);
+    }
+}
+
+// Everything else.  Nothing is shared between the waves of a group but the int8 maximum: lane k of every wave works out the
+// row of route (token, k) for itself, so no wave waits at a barrier between its loads and its stores (16384 x 7168 bf16
+// x top-8 from HBM: 400 us = 5.3 TB/s, 426 us with the rows handed round through LDS).  Bound by memory: with token rows
+// that come from HBM the reads and the writes share it, and no kernel of this mix was measured above 5.4 TB/s here (all
+// cache policies of the loads and stores, one to four tokens in flight per group, a token read ahead of the stores).
+template <int G, int V, int QMODE, bool BF16, bool E5M2>
+__device__ __forceinline__ void ScatterOnly(const ScatterArgs &a)
+{
+    constexpr int kTokens = kThreads / G;
+    __shared__ float s_red[kTokens][kWavesPerBlock];
+
+    const int tg = threadIdx.x / G;
+    const int lane = threadIdx.x % G;
+    const int waveLane = threadIdx.x % kWave;
+    const int token = static_cast<int>(blockIdx.x) * kTokens + tg;
+    if (token >= a.bs) {
+        return;                     // a group of several waves has the workgroup to itself: nobody is left at a barrier
+    }
+    const int vecs = a.h / 8;
+    int row = -1;
+    if (waveLane < a.topK) {
+        const int route = token * a.topK + waveLane;
+        row = a.place.ids != nullptr ? PlaceRoute(a.place, route, lane < kWave) : a.rowOf[route];
+    }
+    const u32x4 *src = reinterpret_cast<const u32x4 *>(static_cast<const char *>(a.x) + static_cast<int64_t>(token) * a.h * 2);
+    u32x4 v[V];
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+        const int idx = j * G + lane;
+        v[j] = idx < vecs ? src[idx] : u32x4{0u, 0u, 0u, 0u};
+    }
+    QuantisedRow<V> out;
+    if (QMODE != TILEXR_EP_QUANT_NONE) {
+        QuantiseRow<G, V, QMODE, BF16, E5M2>(a, v, s_red[tg], lane, out);
+    }
+    for (int k = 0; k < a.topK; ++k) {
+        const int rowOfK = __builtin_amdgcn_readlane(row, k);
+        if (rowOfK >= 0) {
+            StoreRow<G, V, QMODE, false>(a, rowOfK, v, out, lane);
+        }
+    }
+}
+
+template <int G, int V, int QMODE, bool BF16, bool E5M2, bool WT>
+__global__ __launch_bounds__(kThreads) void ep_scatter_vec_kernel(ScatterArgs a)
+{
+    if constexpr (WT) {
+        ScatterAndPublish<G, V, QMODE, BF16, E5M2>(a);
+    } else {
+        ScatterOnly<G, V, QMODE, BF16, E5M2>(a);
     }
 }
 
@@ -498,11 +566,16 @@ template <int G, int V, int QMODE, bool BF16, bool E5M2>
 void LaunchVec(const ScatterArgs &a, hipStream_t stream)
 {
     constexpr int kTokens = kThreads / G;
-    const int grid = (a.bs + kTokens - 1) / kTokens;
+    const int groups = (a.bs + kTokens - 1) / kTokens;
     if (WriteThrough(a)) {
-        hipLaunchKernelGGL((ep_scatter_vec_kernel<G, V, QMODE, BF16, E5M2, true>), dim3(grid), dim3(kThreads), 0, stream, a);
+        hipLaunchKernelGGL((ep_scatter_vec_kernel<G, V, QMODE, BF16, E5M2, true>), dim3(groups), dim3(kThreads), 0, stream, a);
     } else {
-        hipLaunchKernelGGL((ep_scatter_vec_kernel<G, V, QMODE, BF16, E5M2, false>), dim3(grid), dim3(kThreads), 0, stream, a);
+        // Eight workgroups per compute unit that each quantise a wide row and store it topK times oversubscribe the memory
+        // system like those of the per-route kernel; unused dynamic LDS caps them at five.  (8192 x 4096 int8 x top-6,
+        // microseconds at eight, six, five, four, three: 53.5, 50.1, 49.4, 49.9, 50.8; 2048 x 7168 MXFP8 27.3, 27.0, 25.9,
+        // 25.6, 25.5.  Copies, 16384 x 7168 x top-8: 402, 403, 417, 430, 436.  Rows a wave holds: no difference.)
+        const unsigned capLds = QMODE != TILEXR_EP_QUANT_NONE && G == kThreads ? kRouteCapLdsBytes : 0u;
+        hipLaunchKernelGGL((ep_scatter_vec_kernel<G, V, QMODE, BF16, E5M2, false>), dim3(groups), dim3(kThreads), capLds, stream, a);
     }
 }
 
