@@ -28,6 +28,10 @@ constexpr int kXcds = 8;
 constexpr int kRowVecs = 2;     // 16-byte vectors per lane per row slice
 
 std::atomic<int64_t> gCachedRowBytes {int64_t{256} << 20};     // TileXRMoonEpSetCachedRowBytes
+// Unused dynamic LDS of the copying workgroups: five of them fit a compute unit's 160 KiB.  Eight keep more stores in
+// flight than this memory system digests (4096 x 7168 x top-8, microseconds at eight, seven, six, five, four: 83, 79, 74,
+// 73, 81; five hold their time in both directions, built and saved plans).
+constexpr unsigned kScatterCapLdsBytes = 27 * 1024;
 constexpr int kFusedPlanChunks = 1024;  // chunks of 2048 rows per rank up to which the scatter launch builds a fresh plan
 constexpr int64_t kFusedPlanRowBytes = int64_t{256} << 20;     // ... and bytes of rows the world's routes write
 constexpr int kSelfPlanChunks = 8;      // ... and up to which its plan workgroups add up the earlier chunks themselves
@@ -187,10 +191,11 @@ __device__ __forceinline__ void WarmRows(const DispatchWorld &a, int rank, int64
 
 // Saved plans, one thread per route of source rank blockIdx.y: whether the source may write a duplicate's row itself
 // (see SourceWrites).  Done ahead of the scatter so that its workgroups find the answer with the route word, in one
-// round trip, instead of looking up the parent record after decoding it.  The workgroups from `routeBlocks` on read the
-// token rows ahead (WarmRows) when warmVecs is not zero: this launch waits on a few small loads and leaves the memory
-// system idle, so the read costs a saved-plan Dispatch no launch of its own.
-__global__ __launch_bounds__(kThreads) void moon_agree_kernel(DispatchWorld a, unsigned routeBlocks, int64_t warmVecs)
+// round trip, instead of looking up the parent record after decoding it.  Ahead of the per-route scatter (`records`) it
+// also writes what a route records, weight and row tag, and reports a route that names no rank.  The workgroups from
+// `routeBlocks` on read the token rows ahead (WarmRows) when warmVecs is not zero: this launch waits on a few small loads
+// and leaves the memory system idle, so the read costs a saved-plan Dispatch no launch of its own.
+__global__ __launch_bounds__(kThreads) void moon_agree_kernel(DispatchWorld a, unsigned routeBlocks, int64_t warmVecs, int records)
 {
     if (blockIdx.x >= routeBlocks) {
         WarmRows(a, blockIdx.y, static_cast<int64_t>(blockIdx.x - routeBlocks), warmVecs);
@@ -204,24 +209,36 @@ __global__ __launch_bounds__(kThreads) void moon_agree_kernel(DispatchWorld a, u
     const int K = static_cast<int>(a.k);
     const int k = static_cast<int>(route % K);
     const int32_t *words = a.dst[src] + route - k;
+    const float weight = records != 0 && a.weightsSk[src] != nullptr ? a.weightsSk[src][route] : 0.0f;
     uint8_t direct = 0;
     const Route r = Decode(words[k], a.nvS, a.world);
+    const int64_t at = static_cast<int64_t>(r.peer) * a.tables.stride + r.row;
     if (r.ok && r.duplicate) {
-        const uint64_t p = a.tables.parentTag[static_cast<int64_t>(r.peer) * a.tables.stride + r.row];
+        const uint64_t p = a.tables.parentTag[at];
         direct = Tagged(p, a.epoch) && static_cast<int>(p & 0xffffffffu) - 1 == OwnPrimaryRow(a, words, k, r.peer) ? 1 : 0;
     }
     a.tables.direct[static_cast<int64_t>(src) * a.tables.stride + route] = direct;
-}
-
-// The same read as a launch of its own, for a Dispatch that builds its plan: nothing runs ahead of its scatter.
-__global__ __launch_bounds__(kThreads) void moon_warm_rows_kernel(DispatchWorld a, int64_t vecs)
-{
-    WarmRows(a, blockIdx.y, static_cast<int64_t>(blockIdx.x), vecs);
+    if (records == 0) {
+        return;
+    }
+    if (!r.ok) {
+        RecordFailure(a.tables, src, a.epoch, kDispatchInvalidRoute);
+        return;
+    }
+    uint32_t tagBits = 0;
+    SourceWrites<false>(r, direct, &tagBits);
+    if (a.weightsSk[src] != nullptr) {
+        a.weightsNvs[r.peer][r.row] = weight;
+    }
+    a.tables.rowTag[at] = Tag(a.epoch, tagBits);
 }
 
 // Fresh plans, one thread per route of source rank blockIdx.y: everything a route records (RouteRecords) and the
-// failure of a route that names no rank, ahead of the scatter.  Nothing the plan is built from is then written by the
-// scatter launch, so extra workgroups of that launch build it (moon_scatter_kernel, PLAN) instead of launches after it.
+// failure of a route that names no rank, ahead of the per-route scatter, whose workgroups then only copy: with the records
+// in them they asked for route words, weights and the token's other routes between the copies of everybody else, and a
+// scatter on tables that were not cached took 110 us instead of 76 (4096 x 7168 x top-8).  Nothing the plan is built from
+// is written by the scatter launch, so for smaller worlds extra workgroups of that launch build it (moon_scatter_kernel,
+// PLAN) instead of launches after it.
 // The workgroups from `routeBlocks` on read the token rows ahead, as in moon_agree_kernel.
 __global__ __launch_bounds__(kThreads) void moon_records_kernel(DispatchWorld a, unsigned routeBlocks, int64_t warmVecs)
 {
@@ -281,9 +298,10 @@ template <bool SELF>
 __device__ __forceinline__ void DedupGroupsOfChunk(const DispatchWorld &a, int rank, int chunk, bool lastChunk,
     int (*s_part)[kThreads / kWave], int *s_base);
 
-// One workgroup per (token, route, slice of 512 vectors) of source rank blockIdx.y.
+// One workgroup per (token, route, slice of 512 vectors) of source rank blockIdx.y.  What the routes record was written
+// ahead, by moon_records_kernel or moon_agree_kernel.
 //
-// PLAN: a fresh plan whose records were written ahead (moon_records_kernel) is built here as well: the first `planBlocks` workgroups
+// PLAN: a fresh plan is built here as well: the first `planBlocks` workgroups
 // of the launch (a multiple of eight, so that the rest keep their XCDs) take one chunk of destination rank blockIdx.y
 // each.  They depend on nothing this launch writes and are done long before the rows are.  The totals of the chunks
 // before its own a workgroup adds up itself while the chunks are few (planSelf), a trip to memory per chunk, and those
@@ -294,7 +312,6 @@ __global__ __launch_bounds__(kThreads) void moon_scatter_kernel(DispatchWorld a,
     int planSelf)
 {
     static_assert(FRESH || !PLAN, "only a Dispatch that builds its plan has plan workgroups");
-    __shared__ int32_t s_dst[kMaxTopK];
     if (PLAN && blockIdx.x < planBlocks) {
         __shared__ int s_part[2][kThreads / kWave];
         __shared__ int s_base[2];
@@ -322,13 +339,9 @@ __global__ __launch_bounds__(kThreads) void moon_scatter_kernel(DispatchWorld a,
     const int h = static_cast<int>(a.h);
     const int vecs = h / 8;
     const int colBase = slice * (kRowVecs * kThreads);
-    const int32_t *words = a.dst[src] + static_cast<int64_t>(token) * K;
-    const bool records = slice == 0 && !PLAN;       // PLAN: written ahead by moon_records_kernel
-    if (FRESH && records && lane < K) {
-        s_dst[lane] = words[lane];
-    }
-    const int32_t encoded = words[k];
-    const uint8_t direct = FRESH ? 0 : a.tables.direct[static_cast<int64_t>(src) * a.tables.stride + static_cast<int64_t>(token) * K + k];
+    const int64_t route = static_cast<int64_t>(token) * K + k;
+    const int32_t encoded = a.dst[src][route];
+    const uint8_t direct = FRESH ? 0 : a.tables.direct[static_cast<int64_t>(src) * a.tables.stride + route];
     const u32x4 *srcRow = reinterpret_cast<const u32x4 *>(static_cast<const char *>(a.hiddenSh[src]) +
         static_cast<int64_t>(token) * h * 2);
     u32x4 v[kRowVecs];
@@ -338,14 +351,8 @@ __global__ __launch_bounds__(kThreads) void moon_scatter_kernel(DispatchWorld a,
         v[i] = idx < vecs ? srcRow[idx] : u32x4{0u, 0u, 0u, 0u};
     }
     const Route r = Decode(encoded, a.nvS, a.world);
-    if (!r.ok) {
-        if (records && lane == 0) {
-            RecordFailure(a.tables, src, a.epoch, kDispatchInvalidRoute);
-        }
-        return;
-    }
     uint32_t tagBits = 0;
-    if (SourceWrites<FRESH>(r, direct, &tagBits)) {
+    if (r.ok && SourceWrites<FRESH>(r, direct, &tagBits)) {
         u32x4 *dstRow = reinterpret_cast<u32x4 *>(static_cast<char *>(a.hiddenNvsh[r.peer]) + static_cast<int64_t>(r.row) * h * 2);
 #pragma unroll
         for (int i = 0; i < kRowVecs; ++i) {
@@ -353,14 +360,6 @@ __global__ __launch_bounds__(kThreads) void moon_scatter_kernel(DispatchWorld a,
             if (idx < vecs) {
                 __builtin_nontemporal_store(v[i], dstRow + idx);
             }
-        }
-    }
-    if (records) {
-        if (FRESH) {
-            TileXREp::LdsBarrier();
-        }
-        if (lane < kWave) {
-            RouteRecords<FRESH>(a, src, token, k, r, tagBits, s_dst);
         }
     }
 }
@@ -1321,11 +1320,11 @@ hipError_t LaunchMoonDispatch(const DispatchWorld &w, hipStream_t stream, const 
         static_cast<int64_t>(w.world) * w.s * w.k * w.h * 2 <= kFusedPlanRowBytes;
     const bool planSelf = planChunks <= kSelfPlanChunks;
     const unsigned planBlocks = planInScatter ? static_cast<unsigned>((planChunks + kXcds - 1) / kXcds * kXcds) : 0u;
-    if (planInScatter) {
+    if (w.fresh && perRoute) {
         hipLaunchKernelGGL(moon_records_kernel, dim3(routeBlocks + warmBlocks, R), dim3(kThreads), 0, stream, w, routeBlocks,
             warm ? rowVecs : int64_t{0});
         MOON_LAUNCH_CHECK();
-        if (!planSelf) {
+        if (planInScatter && !planSelf) {
             hipLaunchKernelGGL(moon_dedup_totals_kernel, dim3(static_cast<unsigned>(planChunks), R), dim3(kThreads), 0, stream, w);
             MOON_LAUNCH_CHECK();
         }
@@ -1333,10 +1332,7 @@ hipError_t LaunchMoonDispatch(const DispatchWorld &w, hipStream_t stream, const 
         hipLaunchKernelGGL(moon_group_walk_kernel, dim3(rowBlocks, R), dim3(kThreads), 0, stream, w);
         MOON_LAUNCH_CHECK();
         hipLaunchKernelGGL(moon_agree_kernel, dim3(routeBlocks + warmBlocks, R), dim3(kThreads), 0, stream, w, routeBlocks,
-            warm ? rowVecs : int64_t{0});
-        MOON_LAUNCH_CHECK();
-    } else if (warm) {
-        hipLaunchKernelGGL(moon_warm_rows_kernel, dim3(warmBlocks, R), dim3(kThreads), 0, stream, w, rowVecs);
+            warm ? rowVecs : int64_t{0}, perRoute ? 1 : 0);
         MOON_LAUNCH_CHECK();
     }
     hipError_t err = RecordIf(timing.start, stream);
@@ -1353,14 +1349,16 @@ hipError_t LaunchMoonDispatch(const DispatchWorld &w, hipStream_t stream, const 
         }
     } else if (perRoute) {
         gScatterName = "moon_scatter_kernel";
+        // narrow rows give a workgroup a few KiB to move: those need every workgroup that fits
+        const unsigned capLds = vecs > kThreads ? kScatterCapLdsBytes : 0u;
         const dim3 grid(static_cast<unsigned>(blocks) + planBlocks, R);
         if (planInScatter) {
             hipLaunchKernelGGL((moon_scatter_kernel<true, true>), grid, dim3(kThreads), 0, stream, w, colSlices, planBlocks,
                 planChunks, planSelf ? 1 : 0);
         } else if (w.fresh) {
-            hipLaunchKernelGGL((moon_scatter_kernel<true, false>), grid, dim3(kThreads), 0, stream, w, colSlices, 0u, 0, 0);
+            hipLaunchKernelGGL((moon_scatter_kernel<true, false>), grid, dim3(kThreads), capLds, stream, w, colSlices, 0u, 0, 0);
         } else {
-            hipLaunchKernelGGL((moon_scatter_kernel<false, false>), grid, dim3(kThreads), 0, stream, w, colSlices, 0u, 0, 0);
+            hipLaunchKernelGGL((moon_scatter_kernel<false, false>), grid, dim3(kThreads), capLds, stream, w, colSlices, 0u, 0, 0);
         }
     } else {
         gScatterName = "moon_scatter_generic_kernel";
