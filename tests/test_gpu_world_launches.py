@@ -1,0 +1,57 @@
+"""Logical worlds at the edges of their launches: more segments than a copying workgroup adds up itself, more ranks than
+one launch takes, rows on both sides of 4 KiB (a wave or a workgroup per row), sends of one launch and of two, every row
+on one rank (its workgroups go round again), and all ranks on one stream (no events between them)."""
+import numpy as np
+import pytest
+import torch
+
+import test_gpu_multi_rank as multi
+from oracle import ep as O
+from tilexr_amd import ep
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [
+    (2, 40, 64, 4, 256),         # 256 segments per rank: the most a copying workgroup adds up
+    (2, 40, 64, 4, 258),         # 258: a plan launch ahead
+    (17, 9, 64, 2, 34),          # one rank more than a launch takes
+    (2, 260, 2048, 8, 32),       # 2080 routes: send in two launches; rows of exactly 4 KiB
+    (3, 20, 2056, 2, 9),         # rows just wider
+]
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_memory_route_world(shape):
+    multi.test_memory_dispatch_and_combine_across_ranks(shape, ep.DT_BF16)
+
+
+@pytest.mark.parametrize("shape", [(2, 20, 64, 2, 514), (17, 9, 64, 2, 34), (3, 20, 2056, 2, 9)])
+def test_mvp_route_world(shape):
+    multi.test_mvp_dispatch_and_combine_across_ranks(shape)
+
+
+@pytest.mark.parametrize("one_stream", [False, True])
+def test_every_row_on_one_rank(one_stream):
+    R, bs, h, K, E = 4, 60, 136, 4, 32
+    rng = np.random.default_rng(5)
+    ids = np.stack([np.stack([rng.permutation(8)[:K] for _ in range(bs)]) for _ in range(R)]).astype(np.int32) + 8
+    xt, xb = multi.rand_x(rng, R, bs, h, ep.DT_BF16)
+    with multi.World(R) as w:
+        if one_stream:
+            w.streams = [w.streams[0]] * R
+        for _ in range(2):                       # the second exchange reuses the first one's staging
+            outs = multi.run_dispatch(w, True, xt, ids, bs, h, K, E, ep.DT_BF16)
+            case = O.Case(R, bs, h, K, E, token_nums_type=1)
+            for r in range(R):
+                multi.check_rank(outs[r], O.mem_dispatch(case, r, xb, ids), "send_counts")
+            ys = [torch.full((bs, h), 7.0, dtype=torch.bfloat16, device=multi.DEV) for _ in range(R)]
+            torch.cuda.synchronize()
+            for r in range(R):
+                assert ep.combine_memory_v2(outs[r]["expand_x"], outs[r]["assist"], outs[r]["counts"], w.comms[r], bs, h, K, E,
+                                            ys[r], ep.DT_BF16, w.streams[r]) == 0
+            w.sync()
+            eo = np.stack([o["expand_x"].cpu().numpy().view(np.uint16) for o in outs])
+            assist = np.stack([o["assist"].cpu().numpy() for o in outs])
+            counts = np.stack([o["counts"].cpu().numpy() for o in outs])
+            for r in range(R):
+                assert np.array_equal(multi.bits16(ys[r]), O.mem_combine(case, r, eo, assist, counts)), f"rank {r}"

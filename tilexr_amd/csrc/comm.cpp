@@ -28,16 +28,14 @@ void ReleaseWorld(EpWorld *world)
         (void)hipFree(world->flagArea);
     }
     for (DeviceBuffer *b : {&world->stageRows, &world->stageAux, &world->stageCounts, &world->combineSlots,
-             &world->combineMeta}) {
+             &world->combineMeta, &world->drainPlans}) {
         b->Release();
     }
-    for (auto *list : {&world->dispatchEvents, &world->combineEvents}) {
-        for (RankEvents &e : *list) {
-            if (e.sent != nullptr) {
-                (void)hipEventDestroy(e.sent);
-            }
-            if (e.drained != nullptr) {
-                (void)hipEventDestroy(e.drained);
+    for (ExchangeOrder *order : {&world->dispatchOrder, &world->combineOrder}) {
+        order->reached.push_back(order->done);
+        for (hipEvent_t e : order->reached) {
+            if (e != nullptr) {
+                (void)hipEventDestroy(e);
             }
         }
     }
@@ -52,8 +50,8 @@ EpWorld *CreateWorld(int rankSize)
     world->comms.assign(static_cast<size_t>(rankSize), nullptr);
     world->pendingDispatch.resize(static_cast<size_t>(rankSize));
     world->pendingCombine.resize(static_cast<size_t>(rankSize));
-    world->dispatchEvents.resize(static_cast<size_t>(rankSize));
-    world->combineEvents.resize(static_cast<size_t>(rankSize));
+    world->dispatchOrder.reached.assign(static_cast<size_t>(rankSize), nullptr);
+    world->combineOrder.reached.assign(static_cast<size_t>(rankSize), nullptr);
     int device = -1;
     if (hipGetDevice(&device) == hipSuccess) {
         world->device = device;
@@ -202,7 +200,6 @@ int TileXRCommDestroy(TileXRCommPtr comm)
     c->dispatchScratch.Release();
     c->combineScratch.Release();
     c->claimWord.Release();
-    c->drainScratch.Release();
     c->tileCounters.Release();
     if (c->dev != nullptr) {
         (void)hipFree(c->dev);

@@ -71,11 +71,13 @@ struct PendingCombine {
     EpCombineParams params {};
 };
 
-// Per-rank events of the two-half exchange; created on first use, `armed` once recorded.
-struct RankEvents {
-    hipEvent_t sent = nullptr;       // this rank's send half is enqueued
-    hipEvent_t drained = nullptr;    // this rank's drain half is enqueued (staging may be reused after it)
-    bool drainedArmed = false;
+// Order of a two-half exchange: the second half of every rank runs on the stream of the last rank to call, which first
+// waits for the first halves (`reached`, one per rank); the other ranks' streams then wait for `done`, and so does the
+// first half of the next exchange, which reuses the staging.
+struct ExchangeOrder {
+    std::vector<hipEvent_t> reached;     // by rank, created on first use
+    hipEvent_t done = nullptr;
+    bool doneArmed = false;              // recorded at least once
 };
 
 struct EpComm;
@@ -95,8 +97,9 @@ struct EpWorld {
     ExchangeShape combineShape {};
     std::vector<PendingDispatch> pendingDispatch;
     std::vector<PendingCombine> pendingCombine;
-    std::vector<RankEvents> dispatchEvents;
-    std::vector<RankEvents> combineEvents;
+    ExchangeOrder dispatchOrder;
+    ExchangeOrder combineOrder;
+    DeviceBuffer drainPlans;      // [R] segment offsets of worlds with more segments than a copying workgroup adds up itself
     uint64_t combineEpoch = 0;
     DeviceBuffer stageRows;       // [R] payload rows grouped by key
     DeviceBuffer stageAux;        // [R] assist tuples + per-row scales
@@ -116,7 +119,6 @@ struct EpComm {
     DeviceBuffer dispatchScratch;
     DeviceBuffer combineScratch;
     DeviceBuffer claimWord;           // token claims of a combine that waits on readiness flags
-    DeviceBuffer drainScratch;
     DeviceBuffer tileCounters;        // rows landed per readiness tile; all zero whenever no dispatch is in flight
     // The last dispatch of this communicator that published readiness flags: a combine on the same stream that waits for
     // the same words and epoch finds every tile published (stream order), so it needs no room left for a producer.

@@ -2,9 +2,11 @@
 //
 // A multi-rank dispatch is two halves.  The source rank's call groups its rows by destination into a staging area
 // (the same count / place / scatter kernels as the single-rank path, writing to staging instead of expandXOut).
-// Once every rank has sent, each destination rank's outputs are assembled ("drained") from all staging areas:
-//   plan   per-segment counts -> count outputs + exclusive offsets, one workgroup
-//   copy   one workgroup per output row: locate its segment, copy row, assist tuple and scales
+// Once every rank has sent, the outputs of all destination ranks are assembled ("drained") from all staging areas in one
+// launch:
+//   plan   per-segment counts -> count outputs + exclusive offsets, by every workgroup for itself (worlds with more
+//          segments per rank than a workgroup has lanes: one workgroup per rank in a launch ahead)
+//   copy   a wave or a workgroup per output row: locate its segment, copy row, assist tuple and scales
 // A multi-rank combine is the transpose: every expert rank returns its rows to per-(token, k) slots of the source
 // ranks ("return"), then each source rank runs the ordinary reduce kernel over its slots.
 #ifndef TILEXR_AMD_EP_EXCHANGE_H
@@ -50,40 +52,37 @@ struct AugmentLaunch {
     hipStream_t stream;
 };
 
-struct DrainPlanLaunch {
-    StageLayout stage;
-    int rankSize;
-    int dstRank;
-    int localExperts;        // keys per rank in the staging areas' key space
-    int outLocalExperts;     // memory route: segments per source on this rank (1 on a shared-expert rank)
-    int tokenNumsCount;      // entries of expertTokenNumsOut
-    int tp;                  // MVP route: lanes per tensor-parallel group (<= 1: none)
-    bool memoryRoute;        // segments (localExpert, src) with inclusive-sum counts, else (src) with plain counts
-    int32_t *planOffsets;    // [numSeg + 1] exclusive offsets (scratch of the destination rank)
+// What one destination rank of a drain wants, by value in the kernel's arguments.
+struct DrainTarget {
+    int32_t dstRank;
+    int32_t outLocalExperts;     // memory route: segments per source on this rank (1 on a shared-expert rank)
+    int32_t tokenNumsCount;      // entries of expertTokenNumsOut
+    int32_t tokenNumsType;
+    int32_t *planOffsets;        // [numSeg + 1] exclusive offsets: scratch of a drain whose plan is a launch of its own
     int32_t *countsOut;
-    int32_t *tpCountsOut;    // optional mirror of countsOut (MVP route)
+    int32_t *tpCountsOut;        // optional mirror of countsOut (MVP route)
     int64_t *expertTokenNumsOut;
-    int tokenNumsType;
-    hipStream_t stream;
+    char *expandXOut;
+    int32_t *assistOut;
+    char *scalesOut;
 };
+constexpr int kDrainTargets = 16;        // destination ranks one launch takes
 
-struct DrainCopyLaunch {
+struct DrainLaunch {
     StageLayout stage;
     int rankSize;
-    int dstRank;
-    int localExperts;
-    int outLocalExperts;
-    int tp;
-    bool memoryRoute;
-    const int32_t *planOffsets;
-    int64_t maxRows;
+    int localExperts;            // keys per rank in the staging areas' key space
+    int tp;                      // MVP route: lanes per tensor-parallel group (<= 1: none)
+    bool memoryRoute;            // segments (localExpert, src) with inclusive-sum counts, else (src) with plain counts
     int64_t rowBytes;
     int64_t scaleBytesPerRow;
-    void *expandXOut;
-    int32_t *assistOut;
-    void *scalesOut;
+    int64_t routesPerRank;       // rows a rank sends at most, and receives on average
+    int targets;
+    DrainTarget target[kDrainTargets];
     hipStream_t stream;
 };
+// Whether the copying workgroups of a drain add its segments up themselves (no plan launch, planOffsets unused).
+bool DrainPlansItself(int64_t segmentsPerRank, int64_t tokenNumsCount);
 
 struct ReturnRowsLaunch {
     const void *expertOut;
@@ -93,6 +92,7 @@ struct ReturnRowsLaunch {
     bool memoryRoute;
     int64_t maxCountPerEntry;
     int64_t maxRows;
+    int64_t routesPerRank;   // rows an expert rank holds on average
     int64_t rowBytes;
     int rankSize;
     int expertRank;          // the calling rank
@@ -107,8 +107,7 @@ struct ReturnRowsLaunch {
 };
 
 hipError_t LaunchAugment(const AugmentLaunch &l);
-hipError_t LaunchDrainPlan(const DrainPlanLaunch &l);
-hipError_t LaunchDrainCopy(const DrainCopyLaunch &l);
+hipError_t LaunchDrain(const DrainLaunch &l);
 hipError_t LaunchReturnRows(const ReturnRowsLaunch &l);
 
 } // namespace TileXREp

@@ -14,6 +14,7 @@
 #include "ep_exchange.h"
 #include "ep_kernel_common.hip.h"
 #include "ep_launch.h"
+#include "ep_numerics.hip.h"
 
 namespace TileXREp {
 namespace {
@@ -105,60 +106,65 @@ __global__ __launch_bounds__(kThreads) void ep_augment_kernel(AugmentArgs a)
     }
 }
 
-struct DrainPlanArgs {
+struct DrainArgs {
     StageLayout stage;
     int rankSize;
-    int dstRank;
     int localExperts;
-    int outLocalExperts;
-    int tokenNumsCount;
     int tp;
     int memoryRoute;
-    int32_t *planOffsets;
-    int32_t *countsOut;
-    int32_t *tpCountsOut;
-    int64_t *expertTokenNumsOut;
-    int tokenNumsType;
+    int64_t rowBytes;
+    int64_t scaleBytesPerRow;
+    DrainTarget target[kDrainTargets];
 };
 
-__global__ __launch_bounds__(kThreads) void ep_drain_plan_kernel(DrainPlanArgs a)
+__device__ __forceinline__ int SegmentsOf(const DrainArgs &a, const DrainTarget &d)
 {
-    __shared__ int s_cnt[kMaxKeys];
-    __shared__ int s_off[kMaxKeys];
-    __shared__ int s_tok[kMaxKeys];
-    __shared__ int s_part[kThreads];
+    return a.memoryRoute ? d.outLocalExperts * a.rankSize : a.rankSize;
+}
+
+// Rows of every segment of destination `d` and their exclusive offsets (s_off[numSeg] = all of them), in LDS.  s_base,
+// where given, receives each segment's first row within its source's staging area.  Ends with a barrier.
+__device__ __forceinline__ int SegmentOffsets(const DrainArgs &a, const DrainTarget &d, int numSeg, int *s_cnt, int *s_off, int *s_base,
+    int *s_part)
+{
     const int tid = threadIdx.x;
-    const int numSeg = a.memoryRoute ? a.outLocalExperts * a.rankSize : a.rankSize;
     for (int idx = tid; idx < numSeg; idx += kThreads) {
         int src, key;
-        SegmentOf(idx, a.rankSize, a.dstRank, a.localExperts, a.memoryRoute != 0, a.tp, &src, &key);
+        SegmentOf(idx, a.rankSize, d.dstRank, a.localExperts, a.memoryRoute != 0, a.tp, &src, &key);
         const int32_t *ko = a.stage.counts + static_cast<int64_t>(src) * a.stage.countsStride;
-        const int c = ko[key + 1] - ko[key];
+        const int first = ko[key];
+        const int c = ko[key + 1] - first;
         s_cnt[idx] = c;
         s_off[idx] = c;
+        if (s_base != nullptr) {
+            s_base[idx] = first;
+        }
     }
-    __syncthreads();
-    const int total = BlockExclusiveScan(s_off, numSeg, s_part);
+    LdsBarrier();
+    return BlockExclusiveScan(s_off, numSeg, s_part);
+}
+
+// The count outputs of destination `d`, by one workgroup that has its segments in LDS.
+__device__ __forceinline__ void DrainCounts(const DrainArgs &a, const DrainTarget &d, int numSeg, int *s_cnt, const int *s_off, int *s_tok,
+    int *s_part)
+{
+    const int tid = threadIdx.x;
     const int expertRanks = a.tp > 1 ? a.rankSize / a.tp : a.rankSize;
     for (int idx = tid; idx < numSeg; idx += kThreads) {
-        a.planOffsets[idx] = s_off[idx];
         if (a.memoryRoute) {
-            a.countsOut[idx] = s_off[idx] + s_cnt[idx];
+            d.countsOut[idx] = s_off[idx] + s_cnt[idx];
         } else if (idx < expertRanks) {
             // plain per-source counts, indexed by the source's rank; with tp lanes only the rank's own lane is
             // counted here and the other entries are left alone (reference: tilexr_ep_combine_helpers.h:92-95)
             int src, key;
-            SegmentOf(idx, a.rankSize, a.dstRank, a.localExperts, false, a.tp, &src, &key);
-            a.countsOut[src] = s_cnt[idx];
-            if (a.tpCountsOut != nullptr) {
-                a.tpCountsOut[src] = s_cnt[idx];
+            SegmentOf(idx, a.rankSize, d.dstRank, a.localExperts, false, a.tp, &src, &key);
+            d.countsOut[src] = s_cnt[idx];
+            if (d.tpCountsOut != nullptr) {
+                d.tpCountsOut[src] = s_cnt[idx];
             }
         }
     }
-    if (tid == 0) {
-        a.planOffsets[numSeg] = total;
-    }
-    if (a.tp > 1 && a.tpCountsOut != nullptr) {
+    if (a.tp > 1 && d.tpCountsOut != nullptr) {
         // afterwards the first tp entries become rows per lane (reference: tilexr_ep_dispatch_kernel.cpp:818-827)
         __syncthreads();
         if (tid < a.tp) {
@@ -166,13 +172,13 @@ __global__ __launch_bounds__(kThreads) void ep_drain_plan_kernel(DrainPlanArgs a
             for (int es = 0; es < expertRanks; ++es) {
                 rows += s_cnt[tid * expertRanks + es];
             }
-            const int myLane = a.dstRank % a.tp;
+            const int myLane = d.dstRank % a.tp;
             const int lane = tid == 0 ? myLane : (tid - 1 < myLane ? tid - 1 : tid);
-            a.tpCountsOut[lane] = rows;
+            d.tpCountsOut[lane] = rows;
         }
     }
     // rows per local expert
-    for (int le = tid; le < a.tokenNumsCount; le += kThreads) {
+    for (int le = tid; le < d.tokenNumsCount; le += kThreads) {
         int n = 0;
         if (a.memoryRoute) {
             for (int s = 0; s < a.rankSize; ++s) {
@@ -182,91 +188,155 @@ __global__ __launch_bounds__(kThreads) void ep_drain_plan_kernel(DrainPlanArgs a
             for (int s = 0; s < a.rankSize; ++s) {
                 const int32_t *et = a.stage.counts + static_cast<int64_t>(s) * a.stage.countsStride +
                     a.stage.expertTotalOffset;
-                n += et[(a.tp > 1 ? a.dstRank / a.tp : a.dstRank) * a.localExperts + le];
+                n += et[(a.tp > 1 ? d.dstRank / a.tp : d.dstRank) * a.localExperts + le];
             }
         }
         s_tok[le] = n;
     }
     __syncthreads();
-    if (a.tokenNumsType == 0) {
-        for (int le = tid; le < a.tokenNumsCount; le += kThreads) {
+    if (d.tokenNumsType == 0) {
+        for (int le = tid; le < d.tokenNumsCount; le += kThreads) {
             s_cnt[le] = s_tok[le];
         }
         __syncthreads();
-        BlockExclusiveScan(s_cnt, a.tokenNumsCount, s_part);
-        for (int le = tid; le < a.tokenNumsCount; le += kThreads) {
-            a.expertTokenNumsOut[le] = static_cast<int64_t>(s_cnt[le]) + s_tok[le];
+        BlockExclusiveScan(s_cnt, d.tokenNumsCount, s_part);
+        for (int le = tid; le < d.tokenNumsCount; le += kThreads) {
+            d.expertTokenNumsOut[le] = static_cast<int64_t>(s_cnt[le]) + s_tok[le];
         }
     } else {
-        for (int le = tid; le < a.tokenNumsCount; le += kThreads) {
-            a.expertTokenNumsOut[le] = s_tok[le];
+        for (int le = tid; le < d.tokenNumsCount; le += kThreads) {
+            d.expertTokenNumsOut[le] = s_tok[le];
         }
     }
 }
 
-__device__ __forceinline__ void CopyBytes(char *dst, const char *src, int64_t bytes, int tid)
+// One workgroup per destination rank, for worlds whose segments do not fit the copying workgroups' LDS.
+__global__ __launch_bounds__(kThreads) void ep_drain_plan_kernel(DrainArgs a)
+{
+    __shared__ int s_cnt[kMaxKeys];
+    __shared__ int s_off[kMaxKeys];
+    __shared__ int s_tok[kMaxKeys];
+    __shared__ int s_part[kThreads];
+    const DrainTarget &d = a.target[blockIdx.x];
+    const int numSeg = SegmentsOf(a, d);
+    const int total = SegmentOffsets(a, d, numSeg, s_cnt, s_off, nullptr, s_part);
+    for (int idx = threadIdx.x; idx < numSeg; idx += kThreads) {
+        d.planOffsets[idx] = s_off[idx];
+    }
+    if (threadIdx.x == 0) {
+        d.planOffsets[numSeg] = total;
+    }
+    DrainCounts(a, d, numSeg, s_cnt, s_off, s_tok, s_part);
+}
+
+__device__ __forceinline__ void CopyBytes(char *dst, const char *src, int64_t bytes, int tid, int threads)
 {
     if (((reinterpret_cast<uintptr_t>(dst) | reinterpret_cast<uintptr_t>(src) | static_cast<uintptr_t>(bytes)) & 15u) == 0) {
-        const uint4 *s = reinterpret_cast<const uint4 *>(src);
-        uint4 *d = reinterpret_cast<uint4 *>(dst);
-        for (int64_t i = tid; i < bytes / 16; i += kThreads) {
-            d[i] = s[i];
+        const u32x4 *s = reinterpret_cast<const u32x4 *>(src);
+        u32x4 *d = reinterpret_cast<u32x4 *>(dst);
+        constexpr int kAhead = 4;       // vectors a lane has in flight
+        const int vecs = static_cast<int>(bytes / 16);
+        for (int i = tid; i < vecs; i += kAhead * threads) {
+            u32x4 v[kAhead];
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) {
+                const int at = i + u * threads;
+                v[u] = s[at < vecs ? at : i];
+            }
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) {
+                const int at = i + u * threads;
+                if (at < vecs) {
+                    d[at] = v[u];
+                }
+            }
         }
     } else {
-        for (int64_t i = tid; i < bytes; i += kThreads) {
+        for (int64_t i = tid; i < bytes; i += threads) {
             dst[i] = src[i];
         }
     }
 }
 
-struct DrainCopyArgs {
-    StageLayout stage;
-    int rankSize;
-    int dstRank;
-    int localExperts;
-    int outLocalExperts;
-    int tp;
-    int memoryRoute;
-    const int32_t *planOffsets;
-    int64_t rowBytes;
-    int64_t scaleBytesPerRow;
-    char *expandXOut;
-    int32_t *assistOut;
-    char *scalesOut;
-};
+// Lanes that share a row: a wave for rows of up to 4 KiB, the workgroup for wider ones (a wave would take a 14 KiB row in
+// four trips to memory).
+constexpr int64_t kWaveRowBytes = 4096;
 
-__global__ __launch_bounds__(kThreads) void ep_drain_copy_kernel(DrainCopyArgs a)
+inline int LanesPerRow(int64_t rowBytes)
 {
-    const int numSeg = a.memoryRoute ? a.outLocalExperts * a.rankSize : a.rankSize;
-    const int row = blockIdx.x;
-    if (row >= a.planOffsets[numSeg]) {
-        return;
-    }
-    // last segment whose exclusive offset is <= row (empty segments share an offset with their successor)
-    int lo = 0;
-    int hi = numSeg - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) / 2;
-        if (a.planOffsets[mid] <= row) {
-            lo = mid;
+    return rowBytes <= kWaveRowBytes ? kWave : kThreads;
+}
+
+// The rows of destination rank blockIdx.y, G lanes per row: rows group, group + groups of the rank's workgroups, ...  What a
+// logical world moves is small, and a launch costs as much as the rows: hence one launch for all ranks, and (PLANNED =
+// false) no launch ahead that adds up the segments -- every workgroup does so for itself, two loads and a scan in LDS,
+// in less time than a launch takes to begin.  With the sends, the returns and the reduces put together the same way a
+// dispatch and a combine of 4 ranks with 128 x 1024 and 2 routes take 136 us (a plan and a copy launch per rank with a
+// workgroup per row: 203 us), of 8 ranks with 1000 x 4096 and 8 routes 721 us (898 us).
+template <bool PLANNED, int G>
+__global__ __launch_bounds__(kThreads) void ep_drain_rows_kernel(DrainArgs a)
+{
+    constexpr int kSeg = PLANNED ? 1 : kThreads;
+    constexpr int kRows = kThreads / G;
+    __shared__ int s_cnt[kSeg];
+    __shared__ int s_off[kSeg];
+    __shared__ int s_base[kSeg];
+    __shared__ int s_tok[kSeg];
+    __shared__ int s_part[kThreads];
+    const DrainTarget &d = a.target[blockIdx.y];
+    const int numSeg = SegmentsOf(a, d);
+    const int waveLane = threadIdx.x % kWave;
+    const int lane = threadIdx.x % G;
+    const int total = PLANNED ? d.planOffsets[numSeg] : SegmentOffsets(a, d, numSeg, s_cnt, s_off, s_base, s_part);
+    for (int row = static_cast<int>(blockIdx.x) * kRows + static_cast<int>(threadIdx.x) / G; row < total;
+         row += static_cast<int>(gridDim.x) * kRows) {
+        // last segment whose exclusive offset is <= row (empty segments share an offset with their successor)
+        int seg;
+        if (PLANNED) {
+            int lo = 0;
+            int hi = numSeg - 1;
+            while (lo < hi) {
+                const int mid = (lo + hi + 1) / 2;
+                if (d.planOffsets[mid] <= row) {
+                    lo = mid;
+                } else {
+                    hi = mid - 1;
+                }
+            }
+            seg = lo;
         } else {
-            hi = mid - 1;
+            seg = -1;
+            for (int first = 0; first < numSeg; first += kWave) {
+                seg += __popcll(__ballot(first + waveLane < numSeg && s_off[first + waveLane] <= row));
+            }
+        }
+        int src, key;
+        SegmentOf(seg, a.rankSize, d.dstRank, a.localExperts, a.memoryRoute != 0, a.tp, &src, &key);
+        int64_t srcRow;
+        if (PLANNED) {
+            srcRow = a.stage.counts[static_cast<int64_t>(src) * a.stage.countsStride + key] + (row - d.planOffsets[seg]);
+        } else {
+            srcRow = s_base[seg] + (row - s_off[seg]);
+        }
+        const char *rows = a.stage.rows + static_cast<int64_t>(src) * a.stage.rowsStride;
+        const char *aux = a.stage.aux + static_cast<int64_t>(src) * a.stage.auxStride;
+        int32_t word = 0;
+        if (lane < 4) {
+            word = reinterpret_cast<const int32_t *>(aux)[srcRow * 4 + lane];
+        }
+        CopyBytes(d.expandXOut + static_cast<int64_t>(row) * a.rowBytes, rows + srcRow * a.rowBytes, a.rowBytes, lane, G);
+        if (lane < 4) {
+            d.assistOut[static_cast<int64_t>(row) * 4 + lane] = word;
+        }
+        if (a.scaleBytesPerRow > 0) {
+            CopyBytes(d.scalesOut + static_cast<int64_t>(row) * a.scaleBytesPerRow,
+                aux + a.stage.scalesOffset + srcRow * a.scaleBytesPerRow, a.scaleBytesPerRow, lane, G);
         }
     }
-    int src, key;
-    SegmentOf(lo, a.rankSize, a.dstRank, a.localExperts, a.memoryRoute != 0, a.tp, &src, &key);
-    const int32_t *ko = a.stage.counts + static_cast<int64_t>(src) * a.stage.countsStride;
-    const int64_t srcRow = ko[key] + (row - a.planOffsets[lo]);
-    const char *rows = a.stage.rows + static_cast<int64_t>(src) * a.stage.rowsStride;
-    const char *aux = a.stage.aux + static_cast<int64_t>(src) * a.stage.auxStride;
-    const int tid = threadIdx.x;
-    CopyBytes(a.expandXOut + static_cast<int64_t>(row) * a.rowBytes, rows + srcRow * a.rowBytes, a.rowBytes, tid);
-    if (tid < 4) {
-        a.assistOut[static_cast<int64_t>(row) * 4 + tid] = reinterpret_cast<const int32_t *>(aux)[srcRow * 4 + tid];
-    }
-    if (a.scaleBytesPerRow > 0) {
-        CopyBytes(a.scalesOut + static_cast<int64_t>(row) * a.scaleBytesPerRow,
-            aux + a.stage.scalesOffset + srcRow * a.scaleBytesPerRow, a.scaleBytesPerRow, tid);
+    if (!PLANNED && blockIdx.x == gridDim.x - 1) {
+        // the last workgroup has the fewest rows
+        __syncthreads();
+        DrainCounts(a, d, numSeg, s_cnt, s_off, s_tok, s_part);
     }
 }
 
@@ -290,49 +360,52 @@ struct ReturnRowsArgs {
     int64_t metaStride;
 };
 
+// G lanes per row of the expert rank, for as many rows at once as it holds on average: rows group, group + groups, ...
+template <int G>
 __global__ __launch_bounds__(kThreads) void ep_return_rows_kernel(ReturnRowsArgs a)
 {
-    __shared__ int s_src;
-    __shared__ int s_total;
-    const int row = blockIdx.x;
-    if (threadIdx.x == 0) {
-        int src = -1;
-        int total = 0;
-        if (a.memoryRoute) {
-            total = a.counts[a.numCounts - 1];
-        } else {
-            // rows are grouped by the per-source counts; entries outside [0, max] read as 0
-            for (int s = 0; s < a.numCounts; ++s) {
-                int c = a.counts[s];
-                c = (c < 0 || c > a.maxCountPerEntry) ? 0 : c;
-                if (row >= total && row < total + c) {
-                    src = s;
-                }
-                total += c;
+    __shared__ int s_first[kThreads];       // MVP route: first row of every source's rows (at most 128 sources)
+    __shared__ int s_part[kThreads];
+    constexpr int kRows = kThreads / G;
+    const int waveLane = threadIdx.x % kWave;
+    const int lane = threadIdx.x % G;
+    int total;
+    if (a.memoryRoute) {
+        total = a.counts[a.numCounts - 1];
+    } else {
+        // rows are grouped by the per-source counts; entries outside [0, max] read as 0
+        for (int s = threadIdx.x; s < a.numCounts; s += kThreads) {
+            const int c = a.counts[s];
+            s_first[s] = (c < 0 || c > a.maxCountPerEntry) ? 0 : c;
+        }
+        LdsBarrier();
+        total = BlockExclusiveScan(s_first, a.numCounts, s_part);
+    }
+    total = total < 0 ? 0 : (total > a.maxRows ? a.maxRows : total);
+    for (int row = static_cast<int>(blockIdx.x) * kRows + static_cast<int>(threadIdx.x) / G; row < total;
+         row += static_cast<int>(gridDim.x) * kRows) {
+        const int32_t *t = a.assist + static_cast<int64_t>(row) * 4;
+        int src = t[0];
+        const int token = t[1];
+        const int k = t[2];
+        if (!a.memoryRoute) {
+            src = -1;
+            for (int first = 0; first < a.numCounts; first += kWave) {
+                src += __popcll(__ballot(first + waveLane < a.numCounts && s_first[first + waveLane] <= row));
             }
         }
-        s_src = src;
-        s_total = total < 0 ? 0 : (total > a.maxRows ? a.maxRows : total);
-    }
-    __syncthreads();
-    if (row >= s_total) {
-        return;
-    }
-    const int32_t *t = a.assist + static_cast<int64_t>(row) * 4;
-    const int src = a.memoryRoute ? t[0] : s_src;
-    const int token = t[1];
-    const int k = t[2];
-    if (src < 0 || src >= a.rankSize || token < 0 || token >= a.bs || k < 0 || k >= a.topK) {
-        return;
-    }
-    const int64_t slot = static_cast<int64_t>(token) * a.topK + k;
-    CopyBytes(a.slots + static_cast<int64_t>(src) * a.slotsStride + slot * a.rowBytes,
-        a.expertOut + static_cast<int64_t>(row) * a.rowBytes, a.rowBytes, threadIdx.x);
-    if (threadIdx.x == 0) {
-        uint64_t *meta = a.meta + static_cast<int64_t>(src) * a.metaStride;
-        meta[slot] = (a.epoch << 32) | static_cast<uint32_t>(slot);
-        meta[static_cast<int64_t>(a.bs) * a.topK + slot] =
-            (static_cast<uint64_t>(static_cast<uint32_t>(a.expertRank)) << 32) | static_cast<uint32_t>(row);
+        if (src < 0 || src >= a.rankSize || token < 0 || token >= a.bs || k < 0 || k >= a.topK) {
+            continue;
+        }
+        const int64_t slot = static_cast<int64_t>(token) * a.topK + k;
+        CopyBytes(a.slots + static_cast<int64_t>(src) * a.slotsStride + slot * a.rowBytes,
+            a.expertOut + static_cast<int64_t>(row) * a.rowBytes, a.rowBytes, lane, G);
+        if (lane == 0) {
+            uint64_t *meta = a.meta + static_cast<int64_t>(src) * a.metaStride;
+            meta[slot] = (a.epoch << 32) | static_cast<uint32_t>(slot);
+            meta[static_cast<int64_t>(a.bs) * a.topK + slot] =
+                (static_cast<uint64_t>(static_cast<uint32_t>(a.expertRank)) << 32) | static_cast<uint32_t>(row);
+        }
     }
 }
 
@@ -360,43 +433,48 @@ hipError_t LaunchAugment(const AugmentLaunch &l)
     return hipGetLastError();
 }
 
-hipError_t LaunchDrainPlan(const DrainPlanLaunch &l)
+bool DrainPlansItself(int64_t segmentsPerRank, int64_t tokenNumsCount)
 {
-    DrainPlanArgs a {};
-    a.stage = l.stage;
-    a.rankSize = l.rankSize;
-    a.dstRank = l.dstRank;
-    a.localExperts = l.localExperts;
-    a.outLocalExperts = l.outLocalExperts;
-    a.tokenNumsCount = l.tokenNumsCount;
-    a.tp = l.tp;
-    a.memoryRoute = l.memoryRoute ? 1 : 0;
-    a.planOffsets = l.planOffsets;
-    a.countsOut = l.countsOut;
-    a.tpCountsOut = l.tpCountsOut;
-    a.expertTokenNumsOut = l.expertTokenNumsOut;
-    a.tokenNumsType = l.tokenNumsType;
-    hipLaunchKernelGGL(ep_drain_plan_kernel, dim3(1), dim3(kThreads), 0, l.stream, a);
-    return hipGetLastError();
+    return segmentsPerRank <= kThreads && tokenNumsCount <= kThreads;       // their tables in a workgroup's LDS
 }
 
-hipError_t LaunchDrainCopy(const DrainCopyLaunch &l)
+hipError_t LaunchDrain(const DrainLaunch &l)
 {
-    DrainCopyArgs a {};
+    DrainArgs a {};
     a.stage = l.stage;
     a.rankSize = l.rankSize;
-    a.dstRank = l.dstRank;
     a.localExperts = l.localExperts;
-    a.outLocalExperts = l.outLocalExperts;
     a.tp = l.tp;
     a.memoryRoute = l.memoryRoute ? 1 : 0;
-    a.planOffsets = l.planOffsets;
     a.rowBytes = l.rowBytes;
     a.scaleBytesPerRow = l.scaleBytesPerRow;
-    a.expandXOut = static_cast<char *>(l.expandXOut);
-    a.assistOut = l.assistOut;
-    a.scalesOut = static_cast<char *>(l.scalesOut);
-    hipLaunchKernelGGL(ep_drain_copy_kernel, dim3(static_cast<unsigned>(l.maxRows)), dim3(kThreads), 0, l.stream, a);
+    bool planned = false;
+    for (int t = 0; t < l.targets; ++t) {
+        a.target[t] = l.target[t];
+        const int64_t segments = l.memoryRoute ? static_cast<int64_t>(l.target[t].outLocalExperts) * l.rankSize : l.rankSize;
+        planned = planned || !DrainPlansItself(segments, l.target[t].tokenNumsCount);
+    }
+    // room for the rows a rank receives on average; one that receives more has its workgroups go round again
+    const int lanes = LanesPerRow(l.rowBytes);
+    const int perGroup = kThreads / lanes;
+    const unsigned groups = static_cast<unsigned>((l.routesPerRank + perGroup - 1) / perGroup);
+    const dim3 grid(groups > 0 ? groups : 1, static_cast<unsigned>(l.targets));
+    if (planned) {
+        hipLaunchKernelGGL(ep_drain_plan_kernel, dim3(static_cast<unsigned>(l.targets)), dim3(kThreads), 0, l.stream, a);
+        const hipError_t err = hipGetLastError();
+        if (err != hipSuccess) {
+            return err;
+        }
+        if (lanes == kWave) {
+            hipLaunchKernelGGL((ep_drain_rows_kernel<true, kWave>), grid, dim3(kThreads), 0, l.stream, a);
+        } else {
+            hipLaunchKernelGGL((ep_drain_rows_kernel<true, kThreads>), grid, dim3(kThreads), 0, l.stream, a);
+        }
+    } else if (lanes == kWave) {
+        hipLaunchKernelGGL((ep_drain_rows_kernel<false, kWave>), grid, dim3(kThreads), 0, l.stream, a);
+    } else {
+        hipLaunchKernelGGL((ep_drain_rows_kernel<false, kThreads>), grid, dim3(kThreads), 0, l.stream, a);
+    }
     return hipGetLastError();
 }
 
@@ -420,7 +498,14 @@ hipError_t LaunchReturnRows(const ReturnRowsLaunch &l)
     a.slotsStride = l.slotsStride;
     a.meta = l.meta;
     a.metaStride = l.metaStride;
-    hipLaunchKernelGGL(ep_return_rows_kernel, dim3(static_cast<unsigned>(l.maxRows)), dim3(kThreads), 0, l.stream, a);
+    const int lanes = LanesPerRow(l.rowBytes);
+    const int perGroup = kThreads / lanes;
+    const unsigned groups = static_cast<unsigned>((l.routesPerRank + perGroup - 1) / perGroup);
+    if (lanes == kWave) {
+        hipLaunchKernelGGL(ep_return_rows_kernel<kWave>, dim3(groups > 0 ? groups : 1), dim3(kThreads), 0, l.stream, a);
+    } else {
+        hipLaunchKernelGGL(ep_return_rows_kernel<kThreads>, dim3(groups > 0 ? groups : 1), dim3(kThreads), 0, l.stream, a);
+    }
     return hipGetLastError();
 }
 

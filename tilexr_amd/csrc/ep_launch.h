@@ -86,6 +86,7 @@ struct RouteRowsLaunch {
     int32_t *assist;             // [rows, 4] out
     int32_t *totalRowsOut;       // [1] out: rows kept
     int32_t *sendCountsOut;      // optional [numKeys] inclusive sum of kept rows
+    int32_t *firstOffsetOut;     // optional: set to zero (as SmallDispatchLaunch)
     int64_t *expertTokenNumsOut; // optional [numKeys]
     int tokenNumsType;
     const void *warmRows;        // as RouteCountLaunch
@@ -209,8 +210,8 @@ struct ReduceLaunch {
 bool SmallReduceFits(const ReduceLaunch &l);
 hipError_t LaunchSmallReduce(const ReduceLaunch &l);
 
-// Memory-route dispatch of a small batch (plain copies, one rank, no mask, no readiness flags) in a single launch:
-// every workgroup counts the whole id table itself instead of waiting for a counting kernel.
+// Memory-route dispatch of a small batch (plain copies; the send half of a logical world's call among them) in a single
+// launch: every workgroup counts the whole id table itself instead of waiting for a counting kernel.
 constexpr int kSmallRoutes = 2048;
 struct SmallDispatchLaunch {
     const void *x;
@@ -228,6 +229,7 @@ struct SmallDispatchLaunch {
     int32_t *assist;
     int32_t *rowOf;                  // optional
     int32_t *sendCountsOut;
+    int32_t *firstOffsetOut;         // optional: set to zero (the word ahead of sendCountsOut, where the caller wants exclusive offsets)
     int64_t *expertTokenNumsOut;
     int tokenNumsType;
     uint64_t *tileFlags;             // optional: a readiness word per tile of rows, as LaunchScatter publishes them
@@ -249,6 +251,9 @@ hipError_t LaunchScatter(const ScatterLaunch &l);
 bool ScatterCopiesPerRoute(const void *x, const void *out, int64_t bs, int64_t h, int64_t topK, int quantMode);
 hipError_t LaunchInvert(const InvertLaunch &l);
 hipError_t LaunchReduce(const ReduceLaunch &l);
+// The reduces of several logical ranks of one shape (16-bit rows, at most 16 ranks) as one launch on ls[0].stream.
+bool ReduceWorldFits(const ReduceLaunch *ls, int ranks);
+hipError_t LaunchReduceWorld(const ReduceLaunch *ls, int ranks);
 
 // Bytes of CountScratch arrays for a problem (used by the host to carve one allocation).
 struct CountScratchLayout {

@@ -117,14 +117,14 @@ __global__ __launch_bounds__(kThreads) void ep_reduce_generic_kernel(ReduceArgs 
 }
 
 
-void LaunchVecKernels(int g, int v, const ReduceLaunch &l, const ReduceArgs &a, int gridLimit)
+void LaunchVecKernels(int g, int v, const ReduceLaunch &l, const ReduceArgs &a, int gridLimit, const WorldReduceArgs *world, int ranks)
 {
     // one workgroup per token is a geometry of the units with flags only
     const bool flags = a.tileFlags != nullptr || g == kThreads;
     if (l.bf16) {
-        (flags ? LaunchReduceVecBf16Flags : LaunchReduceVecBf16)(g, v, l, a, gridLimit);
+        (flags ? LaunchReduceVecBf16Flags : LaunchReduceVecBf16)(g, v, l, a, gridLimit, world, ranks);
     } else {
-        (flags ? LaunchReduceVecFp16Flags : LaunchReduceVecFp16)(g, v, l, a, gridLimit);
+        (flags ? LaunchReduceVecFp16Flags : LaunchReduceVecFp16)(g, v, l, a, gridLimit, world, ranks);
     }
 }
 
@@ -140,9 +140,7 @@ void LaunchQuantKernels(int g, int v, const ReduceLaunch &l, const ReduceArgs &a
     }
 }
 
-} // namespace
-
-hipError_t LaunchReduce(const ReduceLaunch &l)
+ReduceArgs ArgsOf(const ReduceLaunch &l)
 {
     ReduceArgs a {};
     a.expertOut = l.expertOut;
@@ -173,6 +171,57 @@ hipError_t LaunchReduce(const ReduceLaunch &l)
     a.flagsSettled = (l.tileFlags != nullptr && l.producerOrdered) ? 1 : 0;
     a.claim = l.claimWord;
     a.colSlices = 1;
+    return a;
+}
+
+// 16-bit rows the register-resident kernel takes.
+bool IsPlain(const ReduceLaunch &l)
+{
+    return l.inQuant == 0 && l.h % 8 == 0 && Aligned16(l.y) && l.h / 8 <= 8 * kThreads &&
+        Aligned16(l.expertOut) && l.rowBytes % 16 == 0 &&
+        (l.sharedExpertX == nullptr || Aligned16(l.sharedExpertX)) && (l.commQuant == 0 || l.h % 32 == 0);
+}
+
+// Narrow rows: a wave per token.  Wide ones are cut into slices of 128 vectors, one wave each (many small independent waves
+// with four rows in flight each reach the highest gather bandwidth here).
+int SlicesOf(int64_t vecs)
+{
+    return vecs <= 4 * kWave ? 1 : static_cast<int>((vecs + 2 * kWave - 1) / (2 * kWave));
+}
+
+} // namespace
+
+bool ReduceWorldFits(const ReduceLaunch *ls, int ranks)
+{
+    for (int r = 0; r < ranks; ++r) {
+        if (!IsPlain(ls[r]) || ls[r].tileFlags != nullptr || ls[r].bf16 != ls[0].bf16) {
+            return false;
+        }
+    }
+    return ranks > 0 && ranks <= kReduceRanks;
+}
+
+hipError_t LaunchReduceWorld(const ReduceLaunch *ls, int ranks)
+{
+    if (!ReduceWorldFits(ls, ranks)) {
+        return hipErrorInvalidValue;
+    }
+    const int64_t vecs = ls[0].h / 8;
+    WorldReduceArgs w {};
+    for (int r = 0; r < ranks; ++r) {
+        w.rank[r] = ArgsOf(ls[r]);
+        w.rank[r].colSlices = SlicesOf(vecs);
+        if (ls[r].kernelNameOut != nullptr) {
+            *ls[r].kernelNameOut = "ep_reduce_vec_world_kernel";
+        }
+    }
+    LaunchVecKernels(kWave, vecs > 2 * kWave && vecs <= 4 * kWave ? 4 : 2, ls[0], w.rank[0], 0, &w, ranks);
+    return hipGetLastError();
+}
+
+hipError_t LaunchReduce(const ReduceLaunch &l)
+{
+    ReduceArgs a = ArgsOf(l);
     // A kernel that waits on flags must never crowd out the producer it waits for: its waiting waves keep their
     // registers, and with three or more of these workgroups per compute unit a producer workgroup no longer fits
     // beside them (measured: flag waits expire at six).  Two workgroups per compute unit walk the tokens.
@@ -180,9 +229,7 @@ hipError_t LaunchReduce(const ReduceLaunch &l)
     const bool mayWait = l.tileFlags != nullptr && !l.producerOrdered;
     const int gridLimit = mayWait ? 2 * (l.numComputeUnits > 0 ? l.numComputeUnits : 256) : 0;
     const int64_t vecs = l.h / 8;
-    const bool plain = l.inQuant == 0 && l.h % 8 == 0 && Aligned16(l.y) && vecs <= 8 * kThreads &&
-        Aligned16(l.expertOut) && l.rowBytes % 16 == 0 &&
-        (l.sharedExpertX == nullptr || Aligned16(l.sharedExpertX)) && (l.commQuant == 0 || l.h % 32 == 0);
+    const bool plain = IsPlain(l);
     const int64_t qvecs = l.h / 16;
     const bool quant = l.inQuant != 0 && l.commQuant == 0 && l.reduceKind == kReduceFp32 && l.h % 16 == 0 &&
         qvecs <= 4 * kThreads && Aligned16(l.y) && Aligned16(l.expertOut) && l.rowBytes % 16 == 0 &&
@@ -203,26 +250,23 @@ hipError_t LaunchReduce(const ReduceLaunch &l)
             LaunchQuantKernels(kThreads, 4, l, a, gridLimit);
         }
     } else if (plain) {
-        // a wave per token for narrow rows; wide rows are cut into slices of 128 vectors, one wave each (many small
-        // independent waves with four rows in flight each reach the highest gather bandwidth here)
-        a.colSlices = 1;
         if (vecs <= 2 * kWave) {
-            LaunchVecKernels(kWave, 2, l, a, gridLimit);
+            LaunchVecKernels(kWave, 2, l, a, gridLimit, nullptr, 1);
         } else if (vecs <= 4 * kWave) {
-            LaunchVecKernels(kWave, 4, l, a, gridLimit);
+            LaunchVecKernels(kWave, 4, l, a, gridLimit, nullptr, 1);
         } else if (mayWait) {
             // readiness flags that may still be pending: one workgroup per token, so that one wave polls the token's
             // tiles instead of one per slice, and few enough workgroups that the producer fits beside them
             if (vecs <= 2 * kThreads) {
-                LaunchVecKernels(kThreads, 2, l, a, gridLimit);
+                LaunchVecKernels(kThreads, 2, l, a, gridLimit, nullptr, 1);
             } else if (vecs <= 4 * kThreads) {
-                LaunchVecKernels(kThreads, 4, l, a, gridLimit);
+                LaunchVecKernels(kThreads, 4, l, a, gridLimit, nullptr, 1);
             } else {
-                LaunchVecKernels(kThreads, 8, l, a, gridLimit);
+                LaunchVecKernels(kThreads, 8, l, a, gridLimit, nullptr, 1);
             }
         } else {
-            a.colSlices = static_cast<int>((vecs + 2 * kWave - 1) / (2 * kWave));
-            LaunchVecKernels(kWave, 2, l, a, gridLimit);
+            a.colSlices = SlicesOf(vecs);
+            LaunchVecKernels(kWave, 2, l, a, gridLimit, nullptr, 1);
         }
     } else {
         int grid = static_cast<int>(l.bs);

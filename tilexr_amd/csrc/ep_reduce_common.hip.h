@@ -46,13 +46,20 @@ struct ReduceArgs {
                                      // over (the next group nobody has claimed yet; workgroups that have left)
 };
 
+// The reduces of several logical ranks as one launch: blockIdx.y names the rank.  All have the same shape.
+constexpr int kReduceRanks = 16;
+struct WorldReduceArgs {
+    ReduceArgs rank[kReduceRanks];
+};
+
 // Launchers of the register-resident kernels, one translation unit per (element type, with / without readiness flags).
 // g, v: lanes per token (or per slice of a token's row) and 16-byte vectors per lane; a combination that a unit does
-// not hold is a programming error and launches nothing.
-void LaunchReduceVecBf16(int g, int v, const ReduceLaunch &l, const ReduceArgs &a, int gridLimit);
-void LaunchReduceVecBf16Flags(int g, int v, const ReduceLaunch &l, const ReduceArgs &a, int gridLimit);
-void LaunchReduceVecFp16(int g, int v, const ReduceLaunch &l, const ReduceArgs &a, int gridLimit);
-void LaunchReduceVecFp16Flags(int g, int v, const ReduceLaunch &l, const ReduceArgs &a, int gridLimit);
+// not hold is a programming error and launches nothing.  world (units without flags only): one launch for `ranks` ranks,
+// whose arguments it holds; `a` is then the first rank's, for the geometry.
+void LaunchReduceVecBf16(int g, int v, const ReduceLaunch &l, const ReduceArgs &a, int gridLimit, const WorldReduceArgs *world, int ranks);
+void LaunchReduceVecBf16Flags(int g, int v, const ReduceLaunch &l, const ReduceArgs &a, int gridLimit, const WorldReduceArgs *world, int ranks);
+void LaunchReduceVecFp16(int g, int v, const ReduceLaunch &l, const ReduceArgs &a, int gridLimit, const WorldReduceArgs *world, int ranks);
+void LaunchReduceVecFp16Flags(int g, int v, const ReduceLaunch &l, const ReduceArgs &a, int gridLimit, const WorldReduceArgs *world, int ranks);
 void LaunchReduceQuantBf16(int g, int v, const ReduceLaunch &l, const ReduceArgs &a, int gridLimit);
 void LaunchReduceQuantBf16Flags(int g, int v, const ReduceLaunch &l, const ReduceArgs &a, int gridLimit);
 void LaunchReduceQuantFp16(int g, int v, const ReduceLaunch &l, const ReduceArgs &a, int gridLimit);

@@ -51,8 +51,8 @@ __host__ __device__ inline bool PlacesByXcd(const ReduceArgs &a, int lanesPerUni
         static_cast<int64_t>(a.bs) * a.slots * a.rowBytes <= kPlacedRowBytes;
 }
 
-template <int G, int V, int KIND, bool BF16, int COMMQ, bool FL, bool WIDE = false>
-__global__ __launch_bounds__(kThreads) void ep_reduce_vec_kernel(ReduceArgs a)
+template <int G, int V, int KIND, bool BF16, int COMMQ, bool FL, bool WIDE>
+__device__ __forceinline__ void ReduceVec(const ReduceArgs &a)
 {
     constexpr int kTokens = kThreads / G;
     constexpr bool kMx = COMMQ != 0;
@@ -293,10 +293,23 @@ __global__ __launch_bounds__(kThreads) void ep_reduce_vec_kernel(ReduceArgs a)
 }
 
 
+template <int G, int V, int KIND, bool BF16, int COMMQ, bool FL, bool WIDE = false>
+__global__ __launch_bounds__(kThreads) void ep_reduce_vec_kernel(ReduceArgs a)
+{
+    ReduceVec<G, V, KIND, BF16, COMMQ, FL, WIDE>(a);
+}
+
+// The reduces of a logical world's ranks, which are small: one launch of all of them takes what one of them takes.
+template <int G, int V, int KIND, bool BF16, int COMMQ, bool WIDE>
+__global__ __launch_bounds__(kThreads) void ep_reduce_vec_world_kernel(WorldReduceArgs w)
+{
+    ReduceVec<G, V, KIND, BF16, COMMQ, false, WIDE>(w.rank[blockIdx.y]);
+}
+
 constexpr int64_t kWideReduceUnits = 2048;      // token slices (waves) up to which a launch takes the WIDE kernel
 
 template <int G, int V, int KIND, bool BF16, int COMMQ, bool FL>
-void LaunchVec(const ReduceArgs &a, int gridLimit, hipStream_t stream)
+void LaunchVec(const ReduceArgs &a, int gridLimit, const WorldReduceArgs *world, int ranks, hipStream_t stream)
 {
     if constexpr (G == kThreads) {
         // whole-workgroup tokens are only used for rows published through readiness flags
@@ -313,7 +326,7 @@ void LaunchVec(const ReduceArgs &a, int gridLimit, hipStream_t stream)
         int64_t units = static_cast<int64_t>(a.bs) * a.colSlices;
         bool wide = false;
         if constexpr (G == kWave && V == 2 && KIND == kReduceFp32 && COMMQ == 0 && !FL) {
-            wide = units <= kWideReduceUnits;
+            wide = units * ranks <= kWideReduceUnits;
         }
         if (PlacesByXcd<FL>(a, G)) {
             units = XcdPlacedUnits(a.bs, a.colSlices);
@@ -322,6 +335,21 @@ void LaunchVec(const ReduceArgs &a, int gridLimit, hipStream_t stream)
         if (gridLimit > 0 && grid > gridLimit * (kThreads / threads)) {
             // a multiple of eight, so that a workgroup's later units (blockIdx.x + i * gridDim.x) stay on its XCD
             grid = std::max(gridLimit * (kThreads / threads) / kXcdCount * kXcdCount, kXcdCount);
+        }
+        if constexpr (!FL) {
+            if (world != nullptr) {
+                const dim3 worldGrid(grid, ranks);
+                if constexpr (V == 2 && KIND == kReduceFp32 && COMMQ == 0) {
+                    if (wide) {
+                        hipLaunchKernelGGL((ep_reduce_vec_world_kernel<G, V, KIND, BF16, COMMQ, true>), worldGrid, dim3(threads), 0,
+                            stream, *world);
+                        return;
+                    }
+                }
+                hipLaunchKernelGGL((ep_reduce_vec_world_kernel<G, V, KIND, BF16, COMMQ, false>), worldGrid, dim3(threads), 0, stream,
+                    *world);
+                return;
+            }
         }
         if constexpr (G == kWave && V == 2 && KIND == kReduceFp32 && COMMQ == 0 && !FL) {
             if (wide) {
@@ -334,37 +362,37 @@ void LaunchVec(const ReduceArgs &a, int gridLimit, hipStream_t stream)
 }
 
 template <int G, int V, bool BF16, bool FL>
-void LaunchByMode(const ReduceLaunch &l, const ReduceArgs &a, int gridLimit)
+void LaunchByMode(const ReduceLaunch &l, const ReduceArgs &a, int gridLimit, const WorldReduceArgs *world, int ranks)
 {
     if (l.reduceKind == kReducePerAdd) {
-        LaunchVec<G, V, kReducePerAdd, BF16, 0, FL>(a, gridLimit, l.stream);
+        LaunchVec<G, V, kReducePerAdd, BF16, 0, FL>(a, gridLimit, world, ranks, l.stream);
     } else if (l.commQuant == TILEXR_EP_QUANT_COMM_MXFP8_E5M2) {
-        LaunchVec<G, V, kReduceFp32, BF16, TILEXR_EP_QUANT_COMM_MXFP8_E5M2, FL>(a, gridLimit, l.stream);
+        LaunchVec<G, V, kReduceFp32, BF16, TILEXR_EP_QUANT_COMM_MXFP8_E5M2, FL>(a, gridLimit, world, ranks, l.stream);
     } else if (l.commQuant == TILEXR_EP_QUANT_MXFP8) {
-        LaunchVec<G, V, kReduceFp32, BF16, TILEXR_EP_QUANT_MXFP8, FL>(a, gridLimit, l.stream);
+        LaunchVec<G, V, kReduceFp32, BF16, TILEXR_EP_QUANT_MXFP8, FL>(a, gridLimit, world, ranks, l.stream);
     } else {
-        LaunchVec<G, V, kReduceFp32, BF16, 0, FL>(a, gridLimit, l.stream);
+        LaunchVec<G, V, kReduceFp32, BF16, 0, FL>(a, gridLimit, world, ranks, l.stream);
     }
 }
 
 } // namespace
 
-void TILEXR_REDUCE_ENTRY(int g, int v, const ReduceLaunch &l, const ReduceArgs &a, int gridLimit)
+void TILEXR_REDUCE_ENTRY(int g, int v, const ReduceLaunch &l, const ReduceArgs &a, int gridLimit, const WorldReduceArgs *world, int ranks)
 {
     constexpr bool kBf16 = TILEXR_REDUCE_BF16;
     constexpr bool kFlags = TILEXR_REDUCE_FLAGS;
     if (g == kWave && v == 2) {
-        LaunchByMode<kWave, 2, kBf16, kFlags>(l, a, gridLimit);
+        LaunchByMode<kWave, 2, kBf16, kFlags>(l, a, gridLimit, world, ranks);
     } else if (g == kWave && v == 4) {
-        LaunchByMode<kWave, 4, kBf16, kFlags>(l, a, gridLimit);
+        LaunchByMode<kWave, 4, kBf16, kFlags>(l, a, gridLimit, world, ranks);
     }
     if constexpr (kFlags) {
         if (g == kThreads && v == 2) {
-            LaunchByMode<kThreads, 2, kBf16, true>(l, a, gridLimit);
+            LaunchByMode<kThreads, 2, kBf16, true>(l, a, gridLimit, world, ranks);
         } else if (g == kThreads && v == 4) {
-            LaunchByMode<kThreads, 4, kBf16, true>(l, a, gridLimit);
+            LaunchByMode<kThreads, 4, kBf16, true>(l, a, gridLimit, world, ranks);
         } else if (g == kThreads && v == 8) {
-            LaunchByMode<kThreads, 8, kBf16, true>(l, a, gridLimit);
+            LaunchByMode<kThreads, 8, kBf16, true>(l, a, gridLimit, world, ranks);
         }
     }
 }

@@ -57,6 +57,7 @@ struct RouteRowsArgs {
     int assistAligned;           // the tuples can go out as one 16-byte store each
     int32_t *totalRowsOut;       // device word: rows the dispatch keeps
     int32_t *sendCountsOut;
+    int32_t *firstOffsetOut;     // optional
     int64_t *expertTokenNumsOut;
     int tokenNumsType;
     const u32x4 *warmRows;
@@ -264,6 +265,9 @@ __global__ __launch_bounds__(kRowsThreads, 8) void ep_route_rows_kernel(RouteRow
         if (key == a.numKeys - 1) {
             *a.totalRowsOut = incl;
         }
+        if (key == 0 && a.firstOffsetOut != nullptr) {
+            *a.firstOffsetOut = 0;
+        }
     }
 }
 
@@ -330,6 +334,7 @@ hipError_t LaunchRouteRows(const RouteRowsLaunch &l)
     a.assistAligned = Aligned16(l.assist) ? 1 : 0;
     a.totalRowsOut = l.totalRowsOut;
     a.sendCountsOut = l.sendCountsOut;
+    a.firstOffsetOut = l.firstOffsetOut;
     a.expertTokenNumsOut = l.expertTokenNumsOut;
     a.tokenNumsType = l.tokenNumsType;
     // the keys' workgroups, one for the routes without an expert, then those that read token rows

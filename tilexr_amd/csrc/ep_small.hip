@@ -39,6 +39,7 @@ struct SmallArgs {
     int32_t *assist;
     int32_t *rowOf;              // optional [bs, topK]
     int32_t *sendCountsOut;
+    int32_t *firstOffsetOut;     // optional
     int64_t *expertTokenNumsOut;
     int tokenNumsType;
     TilePublishArgs tiles;       // flags == nullptr: none (totalRows is filled in by the kernels)
@@ -185,6 +186,9 @@ __global__ __launch_bounds__(kThreads) void ep_dispatch_small_kernel(SmallArgs a
         }
     }
     if (token == 0) {
+        if (tid == 0 && a.firstOffsetOut != nullptr) {
+            *a.firstOffsetOut = 0;
+        }
         for (int k = tid; k < a.numExperts; k += kThreads) {
             const int incl = s_hist[k] + s_kept[k];
             a.sendCountsOut[k] = incl;
@@ -323,6 +327,9 @@ __global__ __launch_bounds__(kThreads) void ep_dispatch_small_route_kernel(Small
         if (a.rowOf != nullptr && hasRoute) {
             a.rowOf[route] = row;
         }
+        if (expert == 0 && a.firstOffsetOut != nullptr) {
+            *a.firstOffsetOut = 0;
+        }
         if (expert < a.numExperts) {
             const int outSum = s_sum[0][1] + s_sum[1][1] + s_sum[2][1] + s_sum[3][1];
             a.sendCountsOut[expert] = outSum >> 16;
@@ -382,6 +389,7 @@ hipError_t LaunchSmallDispatch(const SmallDispatchLaunch &l)
     a.assist = l.assist;
     a.rowOf = l.rowOf;
     a.sendCountsOut = l.sendCountsOut;
+    a.firstOffsetOut = l.firstOffsetOut;
     a.expertTokenNumsOut = l.expertTokenNumsOut;
     a.tokenNumsType = l.tokenNumsType;
     const bool flags = l.tileFlags != nullptr;

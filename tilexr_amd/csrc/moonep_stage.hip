@@ -301,12 +301,12 @@ __device__ __forceinline__ void DedupGroupsOfChunk(const DispatchWorld &a, int r
 // One workgroup per (token, route, slice of 512 vectors) of source rank blockIdx.y.  What the routes record was written
 // ahead, by moon_records_kernel or moon_agree_kernel.
 //
-// PLAN: a fresh plan is built here as well: the first `planBlocks` workgroups
-// of the launch (a multiple of eight, so that the rest keep their XCDs) take one chunk of destination rank blockIdx.y
-// each.  They depend on nothing this launch writes and are done long before the rows are.  The totals of the chunks
-// before its own a workgroup adds up itself while the chunks are few (planSelf), a trip to memory per chunk, and those
-// trips are slow beside the scatter's traffic (measured: 5 us each; 32 chunks took longer than the rows); otherwise a
-// launch of moon_dedup_totals_kernel ahead of this one has left them.
+// PLAN: a fresh plan is built here as well: the first `planBlocks` workgroups of the launch (a multiple of eight, so
+// that the rest keep their XCDs) take one chunk of destination rank blockIdx.y each.  They depend on nothing this launch
+// writes and are done long before the rows are.  The totals of the chunks before its own a workgroup adds up itself
+// while the chunks are few (planSelf), a trip to memory per chunk, and those trips are slow beside the scatter's traffic
+// (measured: 5 us each; 32 chunks took longer than the rows); otherwise a launch of moon_dedup_totals_kernel ahead of
+// this one has left them.
 template <bool FRESH, bool PLAN>
 __global__ __launch_bounds__(kThreads) void moon_scatter_kernel(DispatchWorld a, int colSlices, unsigned planBlocks, int planChunks,
     int planSelf)

@@ -4,9 +4,10 @@
 // (src/ep/kernels/tilexr_ep_dispatch_kernel.cpp:700-836, tilexr_ep_dispatch_memory_kernel.h:1549-1562).  With every
 // rank in one process and on one device, spinning kernels could starve each other, so the exchange is ordered by
 // the host instead: a call enqueues its rank's SEND half on the caller's stream immediately; when the last rank of
-// the world has called, the DRAIN half of every rank is enqueued on that rank's own stream behind events of all
-// send halves.  A rank's outputs are therefore complete once every rank has made the call and the rank's stream
-// has been synchronised -- the same moment the reference's kernels would pass their barriers.
+// the world has called, the second half of all ranks (dispatch: one drain launch; combine: the reduces) is enqueued on
+// that last caller's stream, behind one event per other rank's stream and ahead of one that those streams wait for.
+// A rank's outputs are therefore complete once every rank has made the call and the rank's stream has been synchronised
+// -- the same moment the reference's kernels would pass their barriers.
 #include <algorithm>
 
 #include "ep_context.h"
@@ -20,6 +21,23 @@ namespace {
 
 constexpr int kOk = TileXR::TILEXR_SUCCESS;
 
+constexpr int kReduceBatch = 16;
+
+// Timed for one launch that works for `ranks` ranks from `first` on: every one of them records its events and stamps.
+template <typename Launch>
+int TimedForRanks(EpWorld *world, int first, int ranks, int kernel, hipStream_t stream, const char *what, Launch launch)
+{
+    if (ranks == 0) {
+        return LaunchStatus(launch(), what);
+    }
+    int inner = kOk;
+    const int outer = Timed(world->comms[static_cast<size_t>(first)], kernel, stream, what, [&] {
+        inner = TimedForRanks(world, first + 1, ranks - 1, kernel, stream, what, launch);
+        return hipSuccess;
+    });
+    return inner != kOk ? inner : outer;
+}
+
 int64_t Align256(int64_t v)
 {
     return (v + 255) / 256 * 256;
@@ -30,13 +48,54 @@ int64_t MxScaleBytes(int64_t h)
     return ((h + 31) / 32 + 1) / 2 * 2;
 }
 
-bool EnsureEvents(RankEvents *e)
+// What a call of a logical world mostly consists of is the runtime's price for ordering streams: a kernel launch costs
+// the calling thread 2.5 us, a wait for an event that another stream has just recorded 4 to 8 us, one for an event that
+// has been reached by now a few tenths.  Hence one launch per half, events recorded as early as they can be (a rank's
+// right behind its first half), and one wait per other rank's stream at the end of the exchange.
+bool EnsureEvent(hipEvent_t *e)
 {
-    if (e->sent == nullptr && hipEventCreateWithFlags(&e->sent, hipEventDisableTiming) != hipSuccess) {
+    return *e != nullptr || hipEventCreateWithFlags(e, hipEventDisableTiming) == hipSuccess;
+}
+
+// The first half of a call waits for the world's previous exchange, whose second half reads the staging it overwrites.
+bool AwaitPrevious(const ExchangeOrder &order, hipStream_t stream)
+{
+    return !order.doneArmed || hipStreamWaitEvent(stream, order.done, 0) == hipSuccess;
+}
+
+// Behind the first half of rank r's call.
+bool MarkSent(ExchangeOrder *order, int r, hipStream_t stream)
+{
+    hipEvent_t *e = &order->reached[static_cast<size_t>(r)];
+    return EnsureEvent(e) && hipEventRecord(*e, stream) == hipSuccess;
+}
+
+// `stream` waits for the first halves of all ranks.
+template <typename Pending>
+bool JoinStreams(const ExchangeOrder &order, const std::vector<Pending> &calls, hipStream_t stream)
+{
+    for (size_t r = 0; r < calls.size(); ++r) {
+        if (static_cast<hipStream_t>(calls[r].params.stream) != stream &&
+            hipStreamWaitEvent(stream, order.reached[r], 0) != hipSuccess) {
+            return false;
+        }
+    }
+    return true;
+}
+
+// Marks the end of the exchange on `stream` and makes the other ranks' streams wait for it.
+template <typename Pending>
+bool ReleaseStreams(ExchangeOrder *order, const std::vector<Pending> &calls, hipStream_t stream)
+{
+    if (!EnsureEvent(&order->done) || hipEventRecord(order->done, stream) != hipSuccess) {
         return false;
     }
-    if (e->drained == nullptr && hipEventCreateWithFlags(&e->drained, hipEventDisableTiming) != hipSuccess) {
-        return false;
+    order->doneArmed = true;
+    for (const Pending &c : calls) {
+        hipStream_t other = static_cast<hipStream_t>(c.params.stream);
+        if (other != stream && hipStreamWaitEvent(other, order->done, 0) != hipSuccess) {
+            return false;
+        }
     }
     return true;
 }
@@ -97,70 +156,198 @@ bool PlanStage(EpWorld *world, const ExchangeShape &shape, bool reserve, StagePl
     return true;
 }
 
-int DrainRank(EpWorld *world, int q, const ExchangeShape &shape, const StagePlan &plan)
+// The send half of a call of any size and kind: this rank's rows grouped by destination key in its staging area, in two
+// launches (three with shared experts).
+int SendRoutes(EpComm *comm, const EpDispatchParams &p, bool memoryRoute, const ExchangeShape &shape, const StagePlan &plan)
 {
-    EpComm *comm = world->comms[static_cast<size_t>(q)];
-    const EpDispatchParams &p = world->pendingDispatch[static_cast<size_t>(q)].params;
+    const int R = comm->world->rankSize;
+    const int r = comm->rank;
+    const int64_t shared = shape.sharedNum;
+    const int64_t tp = shape.tp;
+    const int64_t n = p.bs * plan.perToken;
     hipStream_t stream = static_cast<hipStream_t>(p.stream);
+    const CountScratchLayout cs = PlanCountScratch(n, plan.numKeys, plan.keySpace, plan.expertHist);
+    const int64_t tableBytes = shared > 0 ? Align256(n * 4) : 0;      // key ids, tuple expert ids, widened mask
+    if (!comm->dispatchScratch.Reserve(static_cast<size_t>(cs.totalBytes + 3 * tableBytes), true)) {
+        return TileXR::TILEXR_ERROR_INTERNAL;
+    }
+    const uint8_t *routeMask = reinterpret_cast<const uint8_t *>(p.xActiveMask);
+    CountScratch scratch = CarveCountScratch(comm->dispatchScratch.ptr, cs, plan.expertHist);
+    const int32_t *routeIds = p.expertIds;
+    const int32_t *tupleExperts = nullptr;
+    if (shared > 0) {
+        int32_t *keyIds = reinterpret_cast<int32_t *>(static_cast<char *>(comm->dispatchScratch.ptr) + cs.totalBytes);
+        int32_t *tuples = reinterpret_cast<int32_t *>(static_cast<char *>(comm->dispatchScratch.ptr) + cs.totalBytes +
+            tableBytes);
+        AugmentLaunch aug {};
+        aug.ids = p.expertIds;
+        aug.bs = p.bs;
+        aug.topK = p.topK;
+        aug.moeExpertNum = p.moeExpertNum;
+        aug.rankSize = R;
+        aug.srcRank = static_cast<int>(r / tp);      // the placement rules see the source's expert rank
+        aug.sharedNum = static_cast<int>(shared);
+        aug.sharedRanks = static_cast<int>(p.sharedExpertRankNum);
+        aug.localExperts = static_cast<int>(plan.localExperts);
+        aug.keysPerRank = static_cast<int>(plan.keysPerRank);
+        aug.sharedAtExpertId = !memoryRoute;
+        aug.keyIdsOut = keyIds;
+        aug.tupleExpertsOut = tuples;
+        if (memoryRoute && p.xActiveMask != nullptr && p.activeMaskType == TILEXR_EP_ACTIVE_MASK_EXPERT) {
+            uint8_t *wide = reinterpret_cast<uint8_t *>(static_cast<char *>(comm->dispatchScratch.ptr) + cs.totalBytes +
+                2 * tableBytes);
+            aug.routeMask = routeMask;
+            aug.routeMaskOut = wide;
+            routeMask = wide;
+        }
+        aug.stream = stream;
+        const int ar = LaunchStatus(LaunchAugment(aug), "route tables");
+        if (ar != kOk) {
+            return ar;
+        }
+        routeIds = keyIds;
+        tupleExperts = tuples;
+    }
+    int32_t *myCounts = plan.layout.counts + static_cast<int64_t>(r) * plan.layout.countsStride;
+    scratch.keyOffset = myCounts;
+    scratch.expertTotal = myCounts + plan.layout.expertTotalOffset;
+    int32_t *rowOf = reinterpret_cast<int32_t *>(static_cast<char *>(comm->dispatchScratch.ptr) + cs.rowOfOff);
+    char *myRows = plan.layout.rows + static_cast<int64_t>(r) * plan.layout.rowsStride;
+    char *myAux = plan.layout.aux + static_cast<int64_t>(r) * plan.layout.auxStride;
+
+    int maskMode = kMaskNone;
+    if (p.xActiveMask != nullptr) {
+        maskMode = !memoryRoute ? kMaskPerToken :
+            (p.activeMaskType == TILEXR_EP_ACTIVE_MASK_EXPERT ? kMaskPerRoute : kMaskTokenPrefix);
+    }
+    // as on a single rank (api.cpp): the rows resolved in one launch where that pays, else count and place, the latter
+    // folded into the scatter; the launch ahead of a scatter that copies per route reads the token rows ahead
+    const bool warm = ScatterCopiesPerRoute(p.x, myRows, p.bs, p.h, plan.perToken, static_cast<int>(p.quantMode));
+    const bool oneLaunch = memoryRoute && shared == 0 && comm->routing != EpComm::Routing::kLegacy &&
+        RouteRowsFits(routeIds, n, plan.numKeys, maskMode, 0) &&
+        (comm->routing == EpComm::Routing::kOneLaunch || RouteRowsPays(n, plan.numKeys, false, warm));
+    int ret = kOk;
+    RoutePlaceLaunch place {};
+    if (oneLaunch) {
+        RouteRowsLaunch rows {};
+        rows.ids = routeIds;
+        rows.bs = p.bs;
+        rows.topK = plan.perToken;
+        rows.numKeys = plan.numKeys;
+        rows.srcRank = r;
+        rows.rowOf = rowOf;
+        rows.assist = reinterpret_cast<int32_t *>(myAux);
+        // exclusive offsets of the keys: a zero, then the inclusive sums, the last of which is the total
+        rows.firstOffsetOut = myCounts;
+        rows.sendCountsOut = myCounts + 1;
+        rows.totalRowsOut = myCounts + plan.numKeys;
+        rows.tokenNumsType = static_cast<int>(p.expertTokenNumsType);
+        rows.warmRows = warm ? p.x : nullptr;
+        rows.warmBytes = p.bs * p.h * 2;
+        rows.stream = stream;
+        comm->lastKernel[kKernelCount] = "ep_route_rows_kernel";
+        ret = Timed(comm, kKernelCount, stream, "route rows", [&] { return LaunchRouteRows(rows); });
+    } else {
+        RouteCountLaunch count {};
+        count.ids = routeIds;
+        count.mask = routeMask;
+        count.maskMode = maskMode;
+        count.bs = p.bs;
+        count.topK = plan.perToken;
+        count.numExperts = plan.keySpace;
+        count.keyDiv = plan.keyDiv;
+        count.numKeys = plan.numKeys;
+        count.capacity = 0;
+        count.scratch = scratch;
+        count.tokenNumsType = static_cast<int>(p.expertTokenNumsType);
+        count.stream = stream;
+        count.warmRows = warm ? p.x : nullptr;
+        count.warmBytes = p.bs * p.h * 2;
+        comm->lastKernel[kKernelCount] = "ep_route_count_kernel";
+        ret = Timed(comm, kKernelCount, stream, "route count", [&] { return LaunchRouteCount(count); });
+        place.ids = routeIds;
+        place.bs = p.bs;
+        place.topK = plan.perToken;
+        place.keyDiv = plan.keyDiv;
+        place.numKeys = plan.numKeys;
+        place.scratch = scratch;
+        place.srcRank = r;
+        place.expertIdBias = 0;
+        place.sharedNum = static_cast<int32_t>(shared);
+        place.tupleExperts = tupleExperts;
+        place.rowOf = nullptr;          // the scatter resolves its own rows
+        place.assist = reinterpret_cast<int32_t *>(myAux);
+        place.stream = stream;
+    }
+    if (ret != kOk) {
+        return ret;
+    }
+    ScatterLaunch scatter {};
+    scatter.x = p.x;
+    scatter.rowOf = rowOf;
+    scatter.fusedPlace = oneLaunch ? nullptr : &place;
+    scatter.bs = p.bs;
+    scatter.h = p.h;
+    scatter.topK = plan.perToken;
+    scatter.quantMode = static_cast<int>(p.quantMode);
+    scatter.inputBf16 = memoryRoute && p.dtype == TileXR::TILEXR_DATA_TYPE_BFP16;
+    scatter.fp8E5m2 = p.expandXOutDtype == TileXR::TILEXR_DATA_TYPE_FP8E5M2;
+    scatter.staticScale = static_cast<const float *>(p.scales);
+    scatter.out = myRows;
+    scatter.scalesOut = myAux + plan.layout.scalesOffset;
+    scatter.stream = stream;
+    return Timed(comm, kKernelScatter, stream, "scatter", [&] { return LaunchScatter(scatter); });
+}
+
+// The drain of every rank of the world, on the stream of the last rank to call.
+int DrainWorld(EpWorld *world, const ExchangeShape &shape, const StagePlan &plan, hipStream_t stream)
+{
     const int R = world->rankSize;
-    const int localExperts = static_cast<int>(plan.keysPerRank);
-    // a shared-expert rank presents one local expert on the memory route
-    // (reference: src/ep/kernels/tilexr_ep_dispatch_memory_kernel.h:1153, tests/ep/demo/tilexr_ep_dispatch_demo.cpp:632-635)
-    const int outLocalExperts = q < shape.sharedRanks ? 1 : static_cast<int>(plan.localExperts);
-    const int64_t numSeg = shape.memoryRoute ? static_cast<int64_t>(outLocalExperts) * R : R;
-    for (int s = 0; s < R; ++s) {
-        if (hipStreamWaitEvent(stream, world->dispatchEvents[static_cast<size_t>(s)].sent, 0) != hipSuccess) {
-            return TileXR::TILEXR_ERROR_INTERNAL;
+    if (!JoinStreams(world->dispatchOrder, world->pendingDispatch, stream)) {
+        return TileXR::TILEXR_ERROR_INTERNAL;
+    }
+    const int64_t maxSegments = shape.memoryRoute ? std::max<int64_t>(plan.localExperts, 1) * R : R;
+    if (!DrainPlansItself(maxSegments, plan.localExperts) &&
+        !world->drainPlans.Reserve(static_cast<size_t>(R * (maxSegments + 1)) * 4, false)) {
+        return TileXR::TILEXR_ERROR_INTERNAL;
+    }
+    DrainLaunch drain {};
+    drain.stage = plan.layout;
+    drain.rankSize = R;
+    drain.localExperts = static_cast<int>(plan.keysPerRank);
+    drain.tp = static_cast<int>(shape.tp);
+    drain.memoryRoute = shape.memoryRoute;
+    drain.rowBytes = plan.rowBytes;
+    drain.scaleBytesPerRow = plan.scaleBytesPerRow;
+    drain.routesPerRank = shape.bs * plan.perToken;
+    drain.stream = stream;
+    for (int q = 0; q < R; ++q) {
+        const EpDispatchParams &p = world->pendingDispatch[static_cast<size_t>(q)].params;
+        DrainTarget &d = drain.target[drain.targets++];
+        d = DrainTarget {};
+        d.dstRank = q;
+        // a shared-expert rank presents one local expert on the memory route
+        // (reference: src/ep/kernels/tilexr_ep_dispatch_memory_kernel.h:1153, tests/ep/demo/tilexr_ep_dispatch_demo.cpp:632-635)
+        d.outLocalExperts = q < shape.sharedRanks ? 1 : static_cast<int>(plan.localExperts);
+        d.tokenNumsCount = shape.memoryRoute ? d.outLocalExperts : static_cast<int>(plan.localExperts);
+        d.tokenNumsType = static_cast<int>(p.expertTokenNumsType);
+        d.planOffsets = world->drainPlans.ptr == nullptr ? nullptr :
+            static_cast<int32_t *>(world->drainPlans.ptr) + q * (maxSegments + 1);
+        d.countsOut = p.epRecvCountsOut;
+        d.tpCountsOut = shape.memoryRoute ? nullptr : p.tpRecvCountsOut;
+        d.expertTokenNumsOut = p.expertTokenNumsOut;
+        d.expandXOut = static_cast<char *>(p.expandXOut);
+        d.assistOut = p.assistInfoForCombineOut;
+        d.scalesOut = static_cast<char *>(p.dynamicScalesOut);
+        if (drain.targets == kDrainTargets || q == R - 1) {
+            const int ret = LaunchStatus(LaunchDrain(drain), "drain");
+            if (ret != kOk) {
+                return ret;
+            }
+            drain.targets = 0;
         }
     }
-    if (!comm->drainScratch.Reserve(static_cast<size_t>(numSeg + 1) * 4, false)) {
-        return TileXR::TILEXR_ERROR_INTERNAL;
-    }
-    DrainPlanLaunch dp {};
-    dp.stage = plan.layout;
-    dp.rankSize = R;
-    dp.dstRank = q;
-    dp.localExperts = localExperts;
-    dp.outLocalExperts = outLocalExperts;
-    dp.tokenNumsCount = shape.memoryRoute ? outLocalExperts : static_cast<int>(plan.localExperts);
-    dp.tp = static_cast<int>(shape.tp);
-    dp.memoryRoute = shape.memoryRoute;
-    dp.planOffsets = static_cast<int32_t *>(comm->drainScratch.ptr);
-    dp.countsOut = p.epRecvCountsOut;
-    dp.tpCountsOut = shape.memoryRoute ? nullptr : p.tpRecvCountsOut;
-    dp.expertTokenNumsOut = p.expertTokenNumsOut;
-    dp.tokenNumsType = static_cast<int>(p.expertTokenNumsType);
-    dp.stream = stream;
-    int ret = LaunchStatus(LaunchDrainPlan(dp), "drain plan");
-    if (ret != kOk) {
-        return ret;
-    }
-    DrainCopyLaunch dc {};
-    dc.stage = plan.layout;
-    dc.rankSize = R;
-    dc.dstRank = q;
-    dc.localExperts = localExperts;
-    dc.outLocalExperts = outLocalExperts;
-    dc.tp = static_cast<int>(shape.tp);
-    dc.memoryRoute = shape.memoryRoute;
-    dc.planOffsets = dp.planOffsets;
-    dc.maxRows = static_cast<int64_t>(R) * shape.bs * plan.perToken;
-    dc.rowBytes = plan.rowBytes;
-    dc.scaleBytesPerRow = plan.scaleBytesPerRow;
-    dc.expandXOut = p.expandXOut;
-    dc.assistOut = p.assistInfoForCombineOut;
-    dc.scalesOut = p.dynamicScalesOut;
-    dc.stream = stream;
-    ret = LaunchStatus(LaunchDrainCopy(dc), "drain copy");
-    if (ret != kOk) {
-        return ret;
-    }
-    RankEvents &ev = world->dispatchEvents[static_cast<size_t>(q)];
-    if (hipEventRecord(ev.drained, stream) != hipSuccess) {
-        return TileXR::TILEXR_ERROR_INTERNAL;
-    }
-    ev.drainedArmed = true;
-    return kOk;
+    return ReleaseStreams(&world->dispatchOrder, world->pendingDispatch, stream) ? kOk : TileXR::TILEXR_ERROR_INTERNAL;
 }
 
 } // namespace
@@ -214,130 +401,43 @@ int RunDispatchMulti(EpComm *comm, const EpDispatchParams &p, bool memoryRoute, 
     if (!PlanStage(world, shape, first, &plan)) {
         return TileXR::TILEXR_ERROR_INTERNAL;
     }
-    RankEvents &mine = world->dispatchEvents[static_cast<size_t>(r)];
-    if (!EnsureEvents(&mine)) {
+    if (!AwaitPrevious(world->dispatchOrder, stream)) {
         return TileXR::TILEXR_ERROR_INTERNAL;
-    }
-    // the previous exchange's drains read the staging areas this send is about to overwrite
-    for (int q = 0; q < R; ++q) {
-        const RankEvents &ev = world->dispatchEvents[static_cast<size_t>(q)];
-        if (ev.drainedArmed && hipStreamWaitEvent(stream, ev.drained, 0) != hipSuccess) {
-            return TileXR::TILEXR_ERROR_INTERNAL;
-        }
     }
 
     // ---- send half: group this rank's rows by destination in its staging area ----
-    const int64_t n = p.bs * plan.perToken;
-    const CountScratchLayout cs = PlanCountScratch(n, plan.numKeys, plan.keySpace, plan.expertHist);
-    const int64_t tableBytes = shared > 0 ? Align256(n * 4) : 0;      // key ids, tuple expert ids, widened mask
-    if (!comm->dispatchScratch.Reserve(static_cast<size_t>(cs.totalBytes + 3 * tableBytes), true)) {
-        return TileXR::TILEXR_ERROR_INTERNAL;
+    int ret = kOk;
+    SmallDispatchLaunch small {};
+    if (memoryRoute && p.quantMode == TILEXR_EP_QUANT_NONE && shared == 0) {
+        // decode-sized: the same one launch that serves such a call on a single rank, into the staging area
+        small.x = p.x;
+        small.ids = p.expertIds;
+        small.bs = p.bs;
+        small.h = p.h;
+        small.topK = p.topK;
+        small.numExperts = plan.keySpace;
+        small.mask = reinterpret_cast<const uint8_t *>(p.xActiveMask);
+        small.maskMode = p.xActiveMask == nullptr ? kMaskNone :
+            (p.activeMaskType == TILEXR_EP_ACTIVE_MASK_EXPERT ? kMaskPerRoute : kMaskTokenPrefix);
+        small.srcRank = r;
+        small.out = plan.layout.rows + static_cast<int64_t>(r) * plan.layout.rowsStride;
+        small.assist = reinterpret_cast<int32_t *>(plan.layout.aux + static_cast<int64_t>(r) * plan.layout.auxStride);
+        // exclusive offsets of the keys: a zero, then the inclusive sums
+        small.firstOffsetOut = plan.layout.counts + static_cast<int64_t>(r) * plan.layout.countsStride;
+        small.sendCountsOut = small.firstOffsetOut + 1;
+        small.kernelNameOut = &comm->lastKernel[kKernelScatter];
+        small.stream = stream;
     }
-    const uint8_t *routeMask = reinterpret_cast<const uint8_t *>(p.xActiveMask);
-    CountScratch scratch = CarveCountScratch(comm->dispatchScratch.ptr, cs, plan.expertHist);
-    const int32_t *routeIds = p.expertIds;
-    const int32_t *tupleExperts = nullptr;
-    if (shared > 0) {
-        int32_t *keyIds = reinterpret_cast<int32_t *>(static_cast<char *>(comm->dispatchScratch.ptr) + cs.totalBytes);
-        int32_t *tuples = reinterpret_cast<int32_t *>(static_cast<char *>(comm->dispatchScratch.ptr) + cs.totalBytes +
-            tableBytes);
-        AugmentLaunch aug {};
-        aug.ids = p.expertIds;
-        aug.bs = p.bs;
-        aug.topK = p.topK;
-        aug.moeExpertNum = p.moeExpertNum;
-        aug.rankSize = R;
-        aug.srcRank = static_cast<int>(r / tp);      // the placement rules see the source's expert rank
-        aug.sharedNum = static_cast<int>(shared);
-        aug.sharedRanks = static_cast<int>(p.sharedExpertRankNum);
-        aug.localExperts = static_cast<int>(plan.localExperts);
-        aug.keysPerRank = static_cast<int>(plan.keysPerRank);
-        aug.sharedAtExpertId = !memoryRoute;
-        aug.keyIdsOut = keyIds;
-        aug.tupleExpertsOut = tuples;
-        if (memoryRoute && p.xActiveMask != nullptr && p.activeMaskType == TILEXR_EP_ACTIVE_MASK_EXPERT) {
-            uint8_t *wide = reinterpret_cast<uint8_t *>(static_cast<char *>(comm->dispatchScratch.ptr) + cs.totalBytes +
-                2 * tableBytes);
-            aug.routeMask = routeMask;
-            aug.routeMaskOut = wide;
-            routeMask = wide;
-        }
-        aug.stream = stream;
-        const int ar = LaunchStatus(LaunchAugment(aug), "route tables");
-        if (ar != kOk) {
-            return ar;
-        }
-        routeIds = keyIds;
-        tupleExperts = tuples;
-    }
-    int32_t *myCounts = plan.layout.counts + static_cast<int64_t>(r) * plan.layout.countsStride;
-    scratch.keyOffset = myCounts;
-    scratch.expertTotal = myCounts + plan.layout.expertTotalOffset;
-    int32_t *rowOf = reinterpret_cast<int32_t *>(static_cast<char *>(comm->dispatchScratch.ptr) + cs.rowOfOff);
-    char *myRows = plan.layout.rows + static_cast<int64_t>(r) * plan.layout.rowsStride;
-    char *myAux = plan.layout.aux + static_cast<int64_t>(r) * plan.layout.auxStride;
-
-    RouteCountLaunch count {};
-    count.ids = routeIds;
-    count.mask = routeMask;
-    if (p.xActiveMask == nullptr) {
-        count.maskMode = kMaskNone;
-    } else if (!memoryRoute) {
-        count.maskMode = kMaskPerToken;
+    if (small.x != nullptr && SmallDispatchFits(small)) {
+        ret = Timed(comm, kKernelScatter, stream, "small dispatch", [&] { return LaunchSmallDispatch(small); });
     } else {
-        count.maskMode = p.activeMaskType == TILEXR_EP_ACTIVE_MASK_EXPERT ? kMaskPerRoute : kMaskTokenPrefix;
+        ret = SendRoutes(comm, p, memoryRoute, shape, plan);
     }
-    count.bs = p.bs;
-    count.topK = plan.perToken;
-    count.numExperts = plan.keySpace;
-    count.keyDiv = plan.keyDiv;
-    count.numKeys = plan.numKeys;
-    count.capacity = 0;
-    count.scratch = scratch;
-    count.tokenNumsType = static_cast<int>(p.expertTokenNumsType);
-    count.stream = stream;
-    comm->lastKernel[kKernelCount] = "ep_route_count_kernel";
-    int ret = Timed(comm, kKernelCount, stream, "route count", [&] { return LaunchRouteCount(count); });
+    if (ret == kOk && !MarkSent(&world->dispatchOrder, r, stream)) {
+        ret = TileXR::TILEXR_ERROR_INTERNAL;
+    }
     if (ret != kOk) {
         return ret;
-    }
-    RoutePlaceLaunch place {};
-    place.ids = routeIds;
-    place.bs = p.bs;
-    place.topK = plan.perToken;
-    place.keyDiv = plan.keyDiv;
-    place.numKeys = plan.numKeys;
-    place.scratch = scratch;
-    place.srcRank = r;
-    place.expertIdBias = 0;
-    place.sharedNum = static_cast<int32_t>(shared);
-    place.tupleExperts = tupleExperts;
-    place.rowOf = rowOf;
-    place.assist = reinterpret_cast<int32_t *>(myAux);
-    place.stream = stream;
-    ret = Timed(comm, kKernelPlace, stream, "route place", [&] { return LaunchRoutePlace(place); });
-    if (ret != kOk) {
-        return ret;
-    }
-    ScatterLaunch scatter {};
-    scatter.x = p.x;
-    scatter.rowOf = rowOf;
-    scatter.bs = p.bs;
-    scatter.h = p.h;
-    scatter.topK = plan.perToken;
-    scatter.quantMode = static_cast<int>(p.quantMode);
-    scatter.inputBf16 = memoryRoute && p.dtype == TileXR::TILEXR_DATA_TYPE_BFP16;
-    scatter.fp8E5m2 = p.expandXOutDtype == TileXR::TILEXR_DATA_TYPE_FP8E5M2;
-    scatter.staticScale = static_cast<const float *>(p.scales);
-    scatter.out = myRows;
-    scatter.scalesOut = myAux + plan.layout.scalesOffset;
-    scatter.stream = stream;
-    ret = Timed(comm, kKernelScatter, stream, "scatter", [&] { return LaunchScatter(scatter); });
-    if (ret != kOk) {
-        return ret;
-    }
-    if (hipEventRecord(mine.sent, stream) != hipSuccess) {
-        return TileXR::TILEXR_ERROR_INTERNAL;
     }
     world->pendingDispatch[static_cast<size_t>(r)].present = true;
     world->pendingDispatch[static_cast<size_t>(r)].params = p;
@@ -348,22 +448,11 @@ int RunDispatchMulti(EpComm *comm, const EpDispatchParams &p, bool memoryRoute, 
             return kOk;
         }
     }
-    int status = kOk;
-    for (int q = 0; q < R; ++q) {
-        if (!EnsureEvents(&world->dispatchEvents[static_cast<size_t>(q)])) {
-            status = TileXR::TILEXR_ERROR_INTERNAL;
-            break;
-        }
-        const int dr = DrainRank(world, q, shape, plan);
-        if (dr != kOk) {
-            status = dr;
-            break;
-        }
-    }
+    ret = DrainWorld(world, shape, plan, stream);
     for (PendingDispatch &pd : world->pendingDispatch) {
         pd.present = false;
     }
-    return status;
+    return ret;
 }
 
 int RunCombineMulti(EpComm *comm, const EpCombineParams &p, bool memoryRoute, int64_t magic)
@@ -419,15 +508,8 @@ int RunCombineMulti(EpComm *comm, const EpCombineParams &p, bool memoryRoute, in
     } else if (!(shape == world->combineShape)) {
         return TileXR::TILEXR_ERROR_PARA_CHECK_FAIL;
     }
-    RankEvents &mine = world->combineEvents[static_cast<size_t>(er)];
-    if (!EnsureEvents(&mine)) {
+    if (!AwaitPrevious(world->combineOrder, stream)) {
         return TileXR::TILEXR_ERROR_INTERNAL;
-    }
-    for (int q = 0; q < R; ++q) {
-        const RankEvents &ev = world->combineEvents[static_cast<size_t>(q)];
-        if (ev.drainedArmed && hipStreamWaitEvent(stream, ev.drained, 0) != hipSuccess) {
-            return TileXR::TILEXR_ERROR_INTERNAL;
-        }
     }
     const uint64_t epoch = world->combineEpoch & 0xffffffffull;
 
@@ -443,6 +525,7 @@ int RunCombineMulti(EpComm *comm, const EpCombineParams &p, bool memoryRoute, in
     back.memoryRoute = memoryRoute;
     back.maxCountPerEntry = n;
     back.maxRows = static_cast<int64_t>(R) * n;
+    back.routesPerRank = n;
     back.rowBytes = rowBytes;
     back.rankSize = R;
     back.expertRank = er;
@@ -455,11 +538,11 @@ int RunCombineMulti(EpComm *comm, const EpCombineParams &p, bool memoryRoute, in
     back.metaStride = metaStride;
     back.stream = stream;
     int ret = LaunchStatus(LaunchReturnRows(back), "return rows");
+    if (ret == kOk && !MarkSent(&world->combineOrder, er, stream)) {
+        ret = TileXR::TILEXR_ERROR_INTERNAL;
+    }
     if (ret != kOk) {
         return ret;
-    }
-    if (hipEventRecord(mine.sent, stream) != hipSuccess) {
-        return TileXR::TILEXR_ERROR_INTERNAL;
     }
     world->pendingCombine[static_cast<size_t>(er)].present = true;
     world->pendingCombine[static_cast<size_t>(er)].params = p;
@@ -470,23 +553,12 @@ int RunCombineMulti(EpComm *comm, const EpCombineParams &p, bool memoryRoute, in
     }
 
     // ---- reduce halves ----
-    int status = kOk;
-    for (int r = 0; r < R && status == kOk; ++r) {
+    int status = JoinStreams(world->combineOrder, world->pendingCombine, stream) ? kOk : TileXR::TILEXR_ERROR_INTERNAL;
+    std::vector<ReduceLaunch> reduces(static_cast<size_t>(R));
+    for (int r = 0; r < R; ++r) {
         const EpCombineParams &rp = world->pendingCombine[static_cast<size_t>(r)].params;
-        EpComm *rc = world->comms[static_cast<size_t>(r)];
-        hipStream_t rs = static_cast<hipStream_t>(rp.stream);
-        RankEvents &ev = world->combineEvents[static_cast<size_t>(r)];
-        if (!EnsureEvents(&ev)) {
-            status = TileXR::TILEXR_ERROR_INTERNAL;
-            break;
-        }
-        for (int s = 0; s < R; ++s) {
-            if (hipStreamWaitEvent(rs, world->combineEvents[static_cast<size_t>(s)].sent, 0) != hipSuccess) {
-                status = TileXR::TILEXR_ERROR_INTERNAL;
-            }
-        }
         uint64_t *meta = static_cast<uint64_t *>(world->combineMeta.ptr) + static_cast<int64_t>(r) * metaStride;
-        ReduceLaunch red {};
+        ReduceLaunch &red = reduces[static_cast<size_t>(r)];
         red.expertOut = static_cast<char *>(world->combineSlots.ptr) + static_cast<int64_t>(r) * slotsStride;
         red.rowBytes = rowBytes;
         red.inverseTagged = meta;
@@ -504,16 +576,24 @@ int RunCombineMulti(EpComm *comm, const EpCombineParams &p, bool memoryRoute, in
         red.sharedSlots = shared;
         red.y = rp.yOut;
         red.numComputeUnits = world->numComputeUnits;
-        red.stream = rs;
-        if (status == kOk) {
-            status = Timed(rc, kKernelReduce, rs, "reduce", [&] { return LaunchReduce(red); });
-        }
-        if (status == kOk) {
-            if (hipEventRecord(ev.drained, rs) != hipSuccess) {
-                status = TileXR::TILEXR_ERROR_INTERNAL;
+        red.stream = stream;
+        red.kernelNameOut = &world->comms[static_cast<size_t>(r)]->lastKernel[kKernelReduce];
+    }
+    // batches of ranks in one launch each, or a launch per rank for rows that take another kernel
+    for (int first = 0; first < R && status == kOk; first += kReduceBatch) {
+        const int ranks = std::min(kReduceBatch, R - first);
+        const ReduceLaunch *batch = reduces.data() + first;
+        if (ReduceWorldFits(batch, ranks)) {
+            status = TimedForRanks(world, first, ranks, kKernelReduce, stream, "reduce", [&] { return LaunchReduceWorld(batch, ranks); });
+        } else {
+            for (int r = 0; r < ranks && status == kOk; ++r) {
+                status = Timed(world->comms[static_cast<size_t>(first + r)], kKernelReduce, stream, "reduce",
+                    [&] { return LaunchReduce(batch[r]); });
             }
-            ev.drainedArmed = true;
         }
+    }
+    if (status == kOk && !ReleaseStreams(&world->combineOrder, world->pendingCombine, stream)) {
+        status = TileXR::TILEXR_ERROR_INTERNAL;
     }
     for (PendingCombine &pc : world->pendingCombine) {
         pc.present = false;
