@@ -54,7 +54,7 @@ extern "C" {
 #endif
 
 #ifndef TILEXR_EP_HAVE_ACL_STREAM
-typedef void *aclrtStream;   /* holds a hipStream_t */
+typedef void *aclrtStream;   /* holds a hipStream_t; hipStreamLegacy names the default stream */
 #endif
 
 typedef void *TileXRCommPtr;

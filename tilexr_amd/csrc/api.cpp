@@ -33,7 +33,7 @@ int RunDispatchSingle(EpComm *comm, const EpDispatchParams &p, bool memoryRoute,
     if (!WithinKernelLimits(p.bs, p.h, p.topK, p.moeExpertNum)) {
         return TileXR::TILEXR_ERROR_NOT_SUPPORT;
     }
-    hipStream_t stream = static_cast<hipStream_t>(p.stream);
+    hipStream_t stream = StreamOf(p.stream);
     const int64_t n = p.bs * p.topK;
     const int64_t experts = p.moeExpertNum;
     const int64_t numKeys = memoryRoute ? experts : 1;
@@ -280,7 +280,7 @@ int RunCombineSingle(EpComm *comm, const EpCombineParams &p, bool memoryRoute, i
     if (!WithinKernelLimits(p.bs, p.h, p.topK, p.moeExpertNum)) {
         return TileXR::TILEXR_ERROR_NOT_SUPPORT;
     }
-    hipStream_t stream = static_cast<hipStream_t>(p.stream);
+    hipStream_t stream = StreamOf(p.stream);
     const int64_t n = p.bs * p.topK;
     std::lock_guard<std::mutex> lock(comm->mu);
     comm->debug.magic = magic;

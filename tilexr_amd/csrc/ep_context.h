@@ -32,6 +32,13 @@ namespace TileXREp {
 constexpr int64_t kFlagAreaBytesPerRank = 64 * 1024;
 constexpr uint32_t kCommTag = 0x54584550u;   // "TXEP"
 
+// The stream a call is to run on.  The default stream has to be named hipStreamLegacy, since a null stream is an error
+// of the calls; the runtime gets it as its null stream, which every version knows.
+inline hipStream_t StreamOf(aclrtStream stream)
+{
+    return stream == static_cast<void *>(hipStreamLegacy) ? nullptr : static_cast<hipStream_t>(stream);
+}
+
 // Grow-only device buffer.  Growing frees the old block (which synchronises the device) and allocates a new one.
 struct DeviceBuffer {
     void *ptr = nullptr;

@@ -474,7 +474,7 @@ int ValidateDispatch(const TileXRMoonEpDispatchArgsV1 *args, aclrtStream stream,
         return kInvalid;
     }
     FillCommon(call, args->plan, s, args->hiddenSh->shape[1], args->flags & TILEXR_MOONEP_FLAG_BUILD_DEDUP,
-        static_cast<hipStream_t>(stream));
+        TileXREp::StreamOf(stream));
     call->hiddenSh = args->hiddenSh->data;
     call->weightsSk = args->routeWeightsSk == nullptr ? nullptr : static_cast<const float *>(args->routeWeightsSk->data);
     call->hiddenNvsh = args->hiddenNvsh->data;
@@ -507,7 +507,7 @@ int ValidateCombine(const TileXRMoonEpCombineArgsV1 *args, aclrtStream stream, E
         !WeightsPairValid(args->routeWeightsSk, args->routeWeightsNvs, s, args->plan->k, args->plan->nvS)) {
         return kInvalid;
     }
-    FillCommon(call, args->plan, s, args->hiddenNvsh->shape[1], 0, static_cast<hipStream_t>(stream));
+    FillCommon(call, args->plan, s, args->hiddenNvsh->shape[1], 0, TileXREp::StreamOf(stream));
     call->dstLocal = args->dstLocal;
     call->hiddenNvsh = args->hiddenNvsh->data;
     call->weightsNvs = args->routeWeightsNvs == nullptr ? nullptr : static_cast<float *>(args->routeWeightsNvs->data);

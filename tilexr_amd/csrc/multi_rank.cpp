@@ -75,7 +75,7 @@ template <typename Pending>
 bool JoinStreams(const ExchangeOrder &order, const std::vector<Pending> &calls, hipStream_t stream)
 {
     for (size_t r = 0; r < calls.size(); ++r) {
-        if (static_cast<hipStream_t>(calls[r].params.stream) != stream &&
+        if (StreamOf(calls[r].params.stream) != stream &&
             hipStreamWaitEvent(stream, order.reached[r], 0) != hipSuccess) {
             return false;
         }
@@ -92,7 +92,7 @@ bool ReleaseStreams(ExchangeOrder *order, const std::vector<Pending> &calls, hip
     }
     order->doneArmed = true;
     for (const Pending &c : calls) {
-        hipStream_t other = static_cast<hipStream_t>(c.params.stream);
+        hipStream_t other = StreamOf(c.params.stream);
         if (other != stream && hipStreamWaitEvent(other, order->done, 0) != hipSuccess) {
             return false;
         }
@@ -165,7 +165,7 @@ int SendRoutes(EpComm *comm, const EpDispatchParams &p, bool memoryRoute, const 
     const int64_t shared = shape.sharedNum;
     const int64_t tp = shape.tp;
     const int64_t n = p.bs * plan.perToken;
-    hipStream_t stream = static_cast<hipStream_t>(p.stream);
+    hipStream_t stream = StreamOf(p.stream);
     const CountScratchLayout cs = PlanCountScratch(n, plan.numKeys, plan.keySpace, plan.expertHist);
     const int64_t tableBytes = shared > 0 ? Align256(n * 4) : 0;      // key ids, tuple expert ids, widened mask
     if (!comm->dispatchScratch.Reserve(static_cast<size_t>(cs.totalBytes + 3 * tableBytes), true)) {
@@ -364,7 +364,7 @@ int RunDispatchMulti(EpComm *comm, const EpDispatchParams &p, bool memoryRoute, 
     if (!WithinKernelLimits(p.bs, p.h, p.topK + shared, std::max(p.moeExpertNum, keySpaceBound), R) || p.extended) {
         return TileXR::TILEXR_ERROR_NOT_SUPPORT;
     }
-    hipStream_t stream = static_cast<hipStream_t>(p.stream);
+    hipStream_t stream = StreamOf(p.stream);
     ExchangeShape shape {};
     shape.bs = p.bs;
     shape.h = p.h;
@@ -468,7 +468,7 @@ int RunCombineMulti(EpComm *comm, const EpCombineParams &p, bool memoryRoute, in
     if (!WithinKernelLimits(p.bs, p.h, perToken, p.moeExpertNum, R) || p.extended) {
         return TileXR::TILEXR_ERROR_NOT_SUPPORT;
     }
-    hipStream_t stream = static_cast<hipStream_t>(p.stream);
+    hipStream_t stream = StreamOf(p.stream);
     ExchangeShape shape {};
     shape.bs = p.bs;
     shape.h = p.h;

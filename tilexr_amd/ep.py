@@ -1,7 +1,7 @@
 """ctypes binding of libtilexr-ep.so: the calls of include/tilexr_ep.h and include/tilexr_api.h for Python callers.
 
-Device memory is passed as torch tensors (or None for optional arguments); `stream` is a torch.cuda.Stream (the
-C ABI rejects a null stream, as the reference does, so the legacy default stream cannot be used).  Every function
+Device memory is passed as torch tensors (or None for optional arguments); `stream` is a torch.cuda.Stream or a stream
+handle (the C ABI rejects a null stream, as the reference does: the default stream is STREAM_LEGACY).  Every function
 returns the library's status code; `check()` turns a non-zero code into an exception.
 """
 import ctypes as C
@@ -17,6 +17,7 @@ SUCCESS, ERR_NOT_INITIALIZED, ERR_MKIRT, ERR_PARA_CHECK_FAIL, ERR_INTERNAL, ERR_
     ERR_NOT_FOUND = 0, -1, -2, -3, -4, -5, -6, -7
 # element types
 DT_INT8, DT_FP16, DT_FP32, DT_BF16, DT_FP8E4M3, DT_FP8E5M2, DT_RESERVED = 0, 3, 4, 11, 15, 16, 255
+STREAM_LEGACY = 1       # hipStreamLegacy
 # masks / quant modes
 MASK_NONE, MASK_TOKEN, MASK_EXPERT = 0, 1, 2
 Q_NONE, Q_STATIC_INT8, Q_TOKEN_INT8, Q_COMM_E5M2, Q_MXFP8, Q_FP8_BLOCK128 = 0, 1, 2, 3, 4, 5
