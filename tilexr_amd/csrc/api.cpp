@@ -111,14 +111,18 @@ int RunDispatchSingle(EpComm *comm, const EpDispatchParams &p, bool memoryRoute,
     }
     const CountScratchLayout plan = PlanCountScratch(n, numKeys, experts, expertHist);
     // One launch resolves every route's row where every expert's workgroup can afford to read the whole id table
-    // (ep_rows.hip); otherwise count (ticket, last workgroup scans) and place, the latter folded into the scatter
+    // (ep_rows.hip; the MVP route without a mask has no key and its own launch there); otherwise count (ticket, last workgroup scans) and place, the latter folded into the scatter
     // unless something needs the rows ahead of it.
     const bool rowsAhead = p.tileFlagsOut != nullptr || p.metaReadyEvent != nullptr;
     // the scatter kernel that copies per route wants the token rows close by: the routing launch reads them ahead
     const bool warm = ScatterCopiesPerRoute(p.x, p.expandXOut, p.bs, p.h, p.topK, static_cast<int>(p.quantMode));
-    const bool oneLaunch = memoryRoute && comm->routing != EpComm::Routing::kLegacy &&
+    const bool mayOneLaunch = comm->routing != EpComm::Routing::kLegacy;
+    const bool oneLaunchRows = mayOneLaunch && memoryRoute &&
         RouteRowsFits(p.expertIds, n, numKeys, maskMode, p.expertCapacity) &&
         (comm->routing == EpComm::Routing::kOneLaunch || RouteRowsPays(n, numKeys, rowsAhead, warm));
+    const bool oneLaunchCompact = mayOneLaunch && !memoryRoute && p.expertCapacity <= 0 &&
+        RouteCompactFits(p.expertIds, n, experts, maskMode);
+    const bool oneLaunch = oneLaunchRows || oneLaunchCompact;
     void *scratchBase = nullptr;
     if (p.noAlloc) {
         // this call may not allocate: the per-GPU static array or nothing
@@ -147,7 +151,26 @@ int RunDispatchSingle(EpComm *comm, const EpDispatchParams &p, bool memoryRoute,
     int ret = kOk;
     RoutePlaceLaunch place {};
     bool separatePlace = false;
-    if (oneLaunch) {
+    if (oneLaunchCompact) {
+        RouteCompactLaunch compact {};
+        compact.ids = p.expertIds;
+        compact.bs = p.bs;
+        compact.topK = p.topK;
+        compact.numExperts = experts;
+        compact.srcRank = comm->rank;
+        compact.expertIdBias = static_cast<int32_t>(p.sharedExpertNum);
+        compact.rowOf = rowOf;
+        compact.assist = p.assistInfoForCombineOut;
+        compact.totalRowsOut = scratch.keyOffset + numKeys;
+        compact.recvCountOut = p.epRecvCountsOut;
+        compact.expertTokenNumsOut = p.expertTokenNumsOut;
+        compact.tokenNumsType = static_cast<int>(p.expertTokenNumsType);
+        compact.warmRows = warm ? p.x : nullptr;
+        compact.warmBytes = p.bs * p.h * 2;
+        compact.stream = stream;
+        comm->lastKernel[kKernelCount] = "ep_route_compact_kernel";
+        ret = Timed(comm, kKernelCount, stream, "route compact", [&] { return LaunchRouteCompact(compact); });
+    } else if (oneLaunchRows) {
         RouteRowsLaunch rows {};
         rows.ids = p.expertIds;
         rows.bs = p.bs;
@@ -166,13 +189,6 @@ int RunDispatchSingle(EpComm *comm, const EpDispatchParams &p, bool memoryRoute,
         rows.stream = stream;
         comm->lastKernel[kKernelCount] = "ep_route_rows_kernel";
         ret = Timed(comm, kKernelCount, stream, "route rows", [&] { return LaunchRouteRows(rows); });
-        if (ret != kOk) {
-            return ret;
-        }
-        if (p.metaReadyEvent != nullptr &&
-            hipEventRecord(static_cast<hipEvent_t>(p.metaReadyEvent), stream) != hipSuccess) {
-            return TileXR::TILEXR_ERROR_INTERNAL;
-        }
     } else {
         RouteCountLaunch count {};
         count.ids = p.expertIds;
@@ -194,17 +210,23 @@ int RunDispatchSingle(EpComm *comm, const EpDispatchParams &p, bool memoryRoute,
         count.warmBytes = p.bs * p.h * 2;
         comm->lastKernel[kKernelCount] = "ep_route_count_kernel";
         ret = Timed(comm, kKernelCount, stream, "route count", [&] { return LaunchRouteCount(count); });
-        if (ret != kOk) {
-            return ret;
+    }
+    if (ret != kOk) {
+        return ret;
+    }
+    if (!memoryRoute && p.tpRecvCountsOut != nullptr) {
+        // reference: tilexr_ep_combine_helpers.h:93-95 mirrors the per-source count into tpRecvCounts
+        if (hipMemcpyAsync(p.tpRecvCountsOut, p.epRecvCountsOut, sizeof(int32_t), hipMemcpyDeviceToDevice, stream) !=
+            hipSuccess) {
+            return TileXR::TILEXR_ERROR_INTERNAL;
         }
-        if (!memoryRoute && p.tpRecvCountsOut != nullptr) {
-            // reference: tilexr_ep_combine_helpers.h:93-95 mirrors the per-source count into tpRecvCounts
-            if (hipMemcpyAsync(p.tpRecvCountsOut, p.epRecvCountsOut, sizeof(int32_t), hipMemcpyDeviceToDevice, stream) !=
-                hipSuccess) {
-                return TileXR::TILEXR_ERROR_INTERNAL;
-            }
+    }
+    if (oneLaunch) {
+        if (p.metaReadyEvent != nullptr &&
+            hipEventRecord(static_cast<hipEvent_t>(p.metaReadyEvent), stream) != hipSuccess) {
+            return TileXR::TILEXR_ERROR_INTERNAL;
         }
-
+    } else {
         place.ids = p.expertIds;
         place.bs = p.bs;
         place.topK = p.topK;

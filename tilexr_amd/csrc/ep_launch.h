@@ -97,6 +97,28 @@ bool RouteRowsPays(int64_t routes, int64_t numKeys, bool rowsAhead, bool readsRo
 bool RouteRowsFits(const int32_t *ids, int64_t routes, int64_t numKeys, int maskMode, int64_t capacity);
 hipError_t LaunchRouteRows(const RouteRowsLaunch &l);
 
+// MVP route, one rank, no mask: the compaction of all routes in one launch (ep_rows.hip).
+constexpr int kCompactTableRoutes = 131072;
+struct RouteCompactLaunch {
+    const int32_t *ids;
+    int64_t bs;
+    int64_t topK;
+    int64_t numExperts;
+    int32_t srcRank;
+    int32_t expertIdBias;
+    int32_t *rowOf;              // [n] out: row of each route, -1 = none
+    int32_t *assist;             // [rows, 4] out
+    int32_t *totalRowsOut;       // [1] out: rows kept
+    int32_t *recvCountOut;       // optional [1]: the same
+    int64_t *expertTokenNumsOut; // optional [numExperts]
+    int tokenNumsType;
+    const void *warmRows;        // as RouteCountLaunch
+    int64_t warmBytes;
+    hipStream_t stream;
+};
+bool RouteCompactFits(const int32_t *ids, int64_t routes, int64_t numExperts, int maskMode);
+hipError_t LaunchRouteCompact(const RouteCompactLaunch &l);
+
 struct RoutePlaceLaunch {
     const int32_t *ids;
     int64_t bs;
