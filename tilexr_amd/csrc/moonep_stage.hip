@@ -64,15 +64,19 @@ struct Route {
     bool ok;
 };
 
+// Plans keep world * nvS within 31 bits, so a word is taken apart in 32: a 64-bit division is a hundred-odd dependent
+// instructions, and where few waves run (prepare, walk, records) those were much of the launch.  With the group's words
+// and the sibling record asked for a round trip earlier (WalkGroup, moon_finish_kernel): a layer of 128 tokens x 1024,
+// top-8, 32.9 -> 31.8 us, 1024 x 7168 forward and backward 141.6 -> 139.9, 4096 x 7168 393.8 -> 391.9.
 __device__ __forceinline__ Route Decode(int32_t encoded, int64_t nvS, int world)
 {
-    const int64_t e = encoded;
-    const int64_t raw = e >= 0 ? e : -e - 1;
-    const int64_t peer = raw / nvS;
+    const uint32_t raw = static_cast<uint32_t>(encoded >= 0 ? encoded : ~encoded);
+    const uint32_t rows = static_cast<uint32_t>(nvS);
+    const uint32_t peer = raw / rows;
     Route r;
-    r.ok = peer < world;
+    r.ok = peer < static_cast<uint32_t>(world);
     r.peer = r.ok ? static_cast<int>(peer) : 0;
-    r.row = static_cast<int>(raw % nvS);
+    r.row = static_cast<int>(raw - peer * rows);
     r.duplicate = encoded < 0;
     return r;
 }
@@ -207,7 +211,7 @@ __global__ __launch_bounds__(kThreads) void moon_agree_kernel(DispatchWorld a, u
         return;
     }
     const int K = static_cast<int>(a.k);
-    const int k = static_cast<int>(route % K);
+    const int k = static_cast<int>(static_cast<uint32_t>(route) % static_cast<uint32_t>(K));
     const int32_t *words = a.dst[src] + route - k;
     const float weight = records != 0 && a.weightsSk[src] != nullptr ? a.weightsSk[src][route] : 0.0f;
     uint8_t direct = 0;
@@ -252,7 +256,7 @@ __global__ __launch_bounds__(kThreads) void moon_records_kernel(DispatchWorld a,
         return;
     }
     const int K = static_cast<int>(a.k);
-    const int k = static_cast<int>(route % K);
+    const int k = static_cast<int>(static_cast<uint32_t>(route) % static_cast<uint32_t>(K));
     const int32_t *words = a.dst[src] + route - k;
     const float weight = a.weightsSk[src] != nullptr ? a.weightsSk[src][route] : 0.0f;
     const Route r = Decode(words[k], a.nvS, a.world);
@@ -681,19 +685,28 @@ __device__ __forceinline__ int64_t SlotOfRow(const WalkArgs &a, int32_t row)
     if (encoded < 0) {
         return -1;
     }
-    const int64_t peer = encoded / a.nvS;
-    const int64_t target = encoded % a.nvS;
-    if (peer >= a.world || target >= a.n) {
-        return -1;
-    }
-    return peer * a.t.stride + target;
+    const Route r = Decode(encoded, a.nvS, a.world);
+    return r.ok && r.row < a.n ? r.peer * a.t.stride + r.row : -1;
 }
 
 constexpr int kWalkBatch = 8;    // entries of a group a thread has in flight
 
+__device__ __forceinline__ void LoadGroupEntries(const WalkArgs &a, int32_t start, int32_t count, int32_t i0, int32_t (&dup)[kWalkBatch])
+{
+#pragma unroll
+    for (int j = 0; j < kWalkBatch; ++j) {
+        dup[j] = i0 + j < count ? a.dupLoffs[start + i0 + j] : -1;
+    }
+}
+
 // One thread per group.  Checks follow the reference (dispatch kernel :428-457, combine kernel :307-345).
 __device__ __forceinline__ void WalkGroup(const WalkArgs &a, int64_t g)
 {
+    // the group's words are asked for with the counts that say whether there is such a group (the tensor holds nvS of them)
+    const int32_t *words = a.dupGroups + (g < a.nvS ? g : 0) * 3;
+    const int32_t primary = words[0];
+    const int32_t start = words[1];
+    const int32_t count = words[2];
     const int32_t groupCount = a.dupCounts[0];
     const int32_t duplicateCount = a.dupCounts[1];
     const int32_t invalid = a.combine ? kCombineInvalidRoute : kDispatchInvalidRoute;
@@ -706,9 +719,6 @@ __device__ __forceinline__ void WalkGroup(const WalkArgs &a, int64_t g)
     if (g >= groupCount) {
         return;
     }
-    const int32_t primary = a.dupGroups[g * 3];
-    const int32_t start = a.dupGroups[g * 3 + 1];
-    const int32_t count = a.dupGroups[g * 3 + 2];
     if (primary < 0 || primary >= a.nvS || start < 0 || count <= 0 || static_cast<int64_t>(start) + count > duplicateCount) {
         RecordFailure(a.t, a.rank, a.epoch, invalid);
         return;
@@ -718,12 +728,9 @@ __device__ __forceinline__ void WalkGroup(const WalkArgs &a, int64_t g)
     // one by one would sit out two dependent round trips per duplicate (entry, then the entry's dstLocal word).
     // Nothing is recorded for a group with a bad entry: the kernels that follow these records do not check them again.
     bool bad = false;
+    int32_t dup[kWalkBatch];
     for (int32_t i0 = 0; i0 < count; i0 += kWalkBatch) {
-        int32_t dup[kWalkBatch];
-#pragma unroll
-        for (int j = 0; j < kWalkBatch; ++j) {
-            dup[j] = i0 + j < count ? a.dupLoffs[start + i0 + j] : 0;
-        }
+        LoadGroupEntries(a, start, count, i0, dup);
 #pragma unroll
         for (int j = 0; j < kWalkBatch; ++j) {
             bad = bad || (i0 + j < count && (dup[j] < 0 || dup[j] >= a.nvS || (a.combine && dup[j] == primary)));
@@ -742,10 +749,8 @@ __device__ __forceinline__ void WalkGroup(const WalkArgs &a, int64_t g)
         }
     }
     for (int32_t i0 = 0; i0 < count; i0 += kWalkBatch) {
-        int32_t dup[kWalkBatch];
-#pragma unroll
-        for (int j = 0; j < kWalkBatch; ++j) {
-            dup[j] = i0 + j < count ? a.dupLoffs[start + i0 + j] : -1;
+        if (count > kWalkBatch) {
+            LoadGroupEntries(a, start, count, i0, dup);     // a group of one batch still has it
         }
         if (a.combine) {
             int64_t slot[kWalkBatch];
@@ -809,6 +814,7 @@ __global__ __launch_bounds__(kThreads) void moon_finish_kernel(DispatchWorld a)
             const bool written = tagged && (tag & kRowWritten) != 0;
             const bool direct = tagged && (tag & kRowDirect) != 0;
             const uint64_t p = a.tables.parentTag[base + row];
+            const uint32_t sibling = a.fresh ? a.tables.sibling[base + row] : 0u;
             if (!a.fresh && Tagged(p, a.epoch) && !direct) {
                 item = static_cast<int32_t>(row) | (kFillCopy << 30);
             } else if (!written) {
@@ -821,7 +827,7 @@ __global__ __launch_bounds__(kThreads) void moon_finish_kernel(DispatchWorld a)
                 // slot of this duplicate in its group's slice (dispatch kernel :393-419)
                 const uint64_t gs = a.tables.groupStart[base + static_cast<int64_t>(p & 0xffffffffu) - 1];
                 if (Tagged(gs, a.epoch)) {
-                    const int64_t at = static_cast<int64_t>(gs & 0xffffffffu) + (a.tables.sibling[base + row] & 0xffffu);
+                    const int64_t at = static_cast<int64_t>(gs & 0xffffffffu) + (sibling & 0xffffu);
                     if (at < a.nvS) {
                         a.dupLoffs[rank][at] = static_cast<int32_t>(row);
                     } else {
@@ -907,13 +913,12 @@ __global__ __launch_bounds__(kThreads) void moon_combine_prepare_kernel(CombineW
     if (encoded == -1) {
         return;
     }
-    const int64_t peer = encoded / a.nvS;
-    const int64_t target = encoded % a.nvS;
-    if (encoded < 0 || peer >= a.world || target >= a.s * a.k) {
+    const Route r = Decode(encoded, a.nvS, a.world);
+    if (r.duplicate || !r.ok || r.row >= a.s * a.k) {
         RecordFailure(a.tables, rank, a.epoch, kCombineInvalidRoute);
         return;
     }
-    a.tables.slotSrc[peer * a.tables.stride + target] = Tag(a.epoch, static_cast<uint32_t>(rank * a.nvS + row));
+    a.tables.slotSrc[r.peer * a.tables.stride + r.row] = Tag(a.epoch, static_cast<uint32_t>(rank * a.nvS + row));
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -978,8 +983,9 @@ __device__ __forceinline__ void LoadSlots(const CombineWorld &a, int rank, int t
     const int32_t groupCount = a.tables.slotCount[slot];
     const bool present = Tagged(w, a.epoch);
     const uint32_t low = static_cast<uint32_t>(w);
+    const uint32_t rows = static_cast<uint32_t>(a.nvS);
     if (writeWeights && a.weightsSk[rank] != nullptr) {
-        a.weightsSk[rank][static_cast<int64_t>(token) * K + lane] = present ? a.weightsNvs[low / a.nvS][low % a.nvS] : 0.0f;
+        a.weightsSk[rank][static_cast<int64_t>(token) * K + lane] = present ? a.weightsNvs[low / rows][low % rows] : 0.0f;
     }
     const bool travels = present && !Tagged(dup, a.epoch);
     const bool grouped = travels && Tagged(group, a.epoch);
