@@ -68,8 +68,11 @@ __device__ __forceinline__ void ReduceVec(const ReduceArgs &a)
     constexpr int KB = WIDE ? 8 : (G == kThreads ? 4 : (V <= 2 ? 4 : (V <= 4 ? 2 : 1)));
     const int vecs = a.h / 8;
     // a unit is one token, or -- for wide rows -- one slice of G * V vectors of a token
-    // the launch may use fewer waves per workgroup than kThreads / kWave (single-wave workgroups for sliced rows)
-    const int unitsPerGroup = static_cast<int>(blockDim.x) / G;
+    // A launch for sliced rows has single-wave workgroups, every other one kThreads lanes.  That is told from the slices and
+    // not from blockDim, which in a function that two kernels share is read from the implicit arguments: a scalar and then
+    // a vector load that everything below waits for (eight decode layers of 128 x 7168 in a graph: 101.7 us that way,
+    // 101.0 us this way).
+    const int unitsPerGroup = G == kThreads || a.colSlices > 1 ? 1 : kThreads / G;
     const bool byXcd = PlacesByXcd<FL>(a, G);
     const int units = byXcd ? XcdPlacedUnits(a.bs, a.colSlices) : a.bs * a.colSlices;
     const int groups = (units + unitsPerGroup - 1) / unitsPerGroup;
