@@ -46,6 +46,8 @@ struct ReduceArgs {
                                      // over (the next group nobody has claimed yet; workgroups that have left)
 };
 
+constexpr int64_t kWideReduceUnits = 2048;      // token slices (waves) up to which a launch takes the WIDE kernel
+
 // The reduces of several logical ranks as one launch: blockIdx.y names the rank.  All have the same shape.
 constexpr int kReduceRanks = 16;
 struct WorldReduceArgs {

@@ -309,8 +309,6 @@ __global__ __launch_bounds__(kThreads) void ep_reduce_vec_world_kernel(WorldRedu
     ReduceVec<G, V, KIND, BF16, COMMQ, false, WIDE>(w.rank[blockIdx.y]);
 }
 
-constexpr int64_t kWideReduceUnits = 2048;      // token slices (waves) up to which a launch takes the WIDE kernel
-
 template <int G, int V, int KIND, bool BF16, int COMMQ, bool FL>
 void LaunchVec(const ReduceArgs &a, int gridLimit, const WorldReduceArgs *world, int ranks, hipStream_t stream)
 {
