@@ -36,6 +36,11 @@ class Dispatched:
         return int(self.send_counts[-1].item())
 
 
+def _capturing(stream):
+    with torch.cuda.stream(stream):
+        return torch.cuda.is_current_stream_capturing()
+
+
 class _CallStream:
     """The stream of one call of a layer, and its order after the layer's previous call, whose scratch it shares:
 
@@ -51,7 +56,7 @@ class _CallStream:
     def __init__(self, device, own):
         self._device = device
         self._own = own
-        self._last = own
+        self._last = None           # stream of the last eager call
         self._waiting = None
         self._lock = threading.Lock()
 
@@ -65,9 +70,11 @@ class _CallStream:
                 self._waiting, run = current, self._own
                 run.wait_stream(current)
                 handle = run.cuda_stream
-            if run != self._last:
-                # a capture is not ordered behind what was enqueued before it, nor may it be
-                if not torch.cuda.is_current_stream_capturing():
+            # a capture is not ordered behind what was enqueued before it, nor may it be
+            if run != self._last and not torch.cuda.is_current_stream_capturing():
+                # a wait for a stream that is capturing by now would pull this one into the capture
+                # (torch.cuda.graph has synchronised the device before it began)
+                if self._last is not None and not _capturing(self._last):
                     run.wait_stream(self._last)
                 self._last = run
             return (handle if handle != 0 else ep.STREAM_LEGACY), current
