@@ -71,6 +71,45 @@ def test_captured_call_replays():
             check(*other, eager, out)
 
 
+def test_two_branches_of_one_capture():
+    """Two micro-batches on forked streams of one capture.  With a capacity limit a dispatch of this size takes the count
+    launch, which hands histograms and its ticket from workgroup to workgroup through the layer's scratch."""
+    batches = [inputs(31), inputs(32)]
+    capacity = BS * K // E
+    side = torch.cuda.Stream()
+
+    def step(moe, x, ids, weights):
+        d = moe.dispatch(x, ids, capacity=capacity)
+        return d, moe.combine(d.expand_x, d, weights)
+
+    def results(d, y):
+        rows = d.rows()
+        return [d.expand_x[:rows].clone(), d.assist[:rows].clone(), d.send_counts.clone(), d.token_nums.clone(), d.row_map.clone(),
+                y.clone()]
+
+    with layer.MoeEpLayer(E, K, H) as moe:
+        step(moe, *batches[0])                      # scratch of this size
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            main = torch.cuda.current_stream()
+            side.wait_stream(main)
+            first = step(moe, *batches[0])
+            with torch.cuda.stream(side):
+                second = step(moe, *batches[1])
+            main.wait_stream(side)
+        for replay in range(3):
+            for (x, _, _), seed in zip(batches, (40 + replay, 50 + replay)):
+                x.copy_(inputs(seed)[0])
+            eager = [results(*step(moe, *b)) for b in batches]
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            for (d, y), want in zip((first, second), eager):
+                for got, expected in zip(results(d, y), want):
+                    assert torch.equal(got, expected)
+
+
 def test_default_stream_handle_is_taken_and_null_is_not():
     x, ids, _ = inputs(3)
     n = BS * K

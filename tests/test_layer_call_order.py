@@ -19,10 +19,11 @@ class Stream:
         self.capture, self.behind = None, set()
 
     def wait_stream(self, other):
-        if self.capture is None:
+        if self.capture is None and self.name == "own":
+            self.capture = other.capture        # the layer's own stream, forked for a call on a wrapped one
+        elif self.capture is None:
             assert other.capture is None, f"eager {self.name} is pulled into the capture of {other.name}"
         else:
-            # a fork into the capture goes from a capturing stream to one that is not (the layer's own stream)
             assert other.capture == self.capture, f"the capture of {self.name} waits for {other.name}, which is not in it"
         self.behind |= {other.name} | other.behind
 
@@ -106,3 +107,47 @@ def test_capture_is_not_ordered_behind_what_ran_before_it(device):
     b.capture = 1
     device.call(b)
     assert "a" not in b.behind
+
+
+@pytest.mark.parametrize("eager_first", [None, "main", "side"])
+def test_calls_of_one_capture_are_ordered_on_whatever_branch(device, eager_first):
+    main, side, third = Stream("main", 10), Stream("side", 11), Stream("third", 12)
+    if eager_first is not None:
+        device.call({"main": main, "side": side}[eager_first])
+    for s in (main, side, third):
+        s.capture = 1
+    device.call(main)
+    device.call(side)
+    assert "main" in side.behind
+    device.call(third)
+    assert "side" in third.behind
+    device.call(main)
+    assert "third" in main.behind
+
+
+def test_calls_of_one_capture_are_ordered_around_an_eager_one(device):
+    main, side, beside = Stream("main", 10), Stream("side", 11), Stream("beside", 12)
+    device.call(main)
+    main.capture = side.capture = 1
+    device.call(main)
+    device.call(beside)
+    device.call(side)
+    assert "main" in side.behind
+
+
+def test_next_capture_does_not_wait_for_the_streams_of_the_one_before(device):
+    a, b = Stream("a", 10), Stream("b", 11)
+    a.capture = 1
+    device.call(a)
+    a.capture = None
+    b.capture = 2
+    device.call(b)
+    assert "a" not in b.behind
+
+
+def test_wrapped_streams_of_a_capture_share_the_layers_own(device):
+    wrapped, b = Stream("wrapped", 10, stream_id=10), Stream("b", 11)
+    wrapped.capture = b.capture = 1
+    assert device.call(wrapped) == device.own.cuda_stream
+    device.call(b)
+    assert {"own", "wrapped"} <= b.behind and "own" in wrapped.behind
