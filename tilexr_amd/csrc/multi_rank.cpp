@@ -63,6 +63,12 @@ bool AwaitPrevious(const ExchangeOrder &order, hipStream_t stream)
     return !order.doneArmed || hipStreamWaitEvent(stream, order.done, 0) == hipSuccess;
 }
 
+// hipStreamPerThread names another stream in every thread, so that two ranks with that handle are not on one stream.
+bool NamesOneStream(hipStream_t stream)
+{
+    return stream != hipStreamPerThread;
+}
+
 // Behind the first half of rank r's call.
 bool MarkSent(ExchangeOrder *order, int r, hipStream_t stream)
 {
@@ -75,7 +81,8 @@ template <typename Pending>
 bool JoinStreams(const ExchangeOrder &order, const std::vector<Pending> &calls, hipStream_t stream)
 {
     for (size_t r = 0; r < calls.size(); ++r) {
-        if (StreamOf(calls[r].params.stream) != stream &&
+        hipStream_t other = StreamOf(calls[r].params.stream);
+        if ((other != stream || !NamesOneStream(other)) &&
             hipStreamWaitEvent(stream, order.reached[r], 0) != hipSuccess) {
             return false;
         }
