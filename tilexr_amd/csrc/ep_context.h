@@ -79,8 +79,8 @@ struct PendingCombine {
 };
 
 // Order of a two-half exchange: the second half of every rank runs on the stream of the last rank to call, which first
-// waits for the first halves (`reached`, one per rank); the other ranks' streams then wait for `done`, and so does the
-// first half of the next exchange, which reuses the staging.
+// waits for the other ranks' streams (`reached`, one per rank); those then wait for `done`, and so does the first half of
+// the next exchange, which reuses the staging.
 struct ExchangeOrder {
     std::vector<hipEvent_t> reached;     // by rank, created on first use
     hipEvent_t done = nullptr;
