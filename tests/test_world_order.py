@@ -20,7 +20,7 @@ def check(tmp_path_factory):
 
 
 @pytest.mark.parametrize("half", ["dispatch", "combine"])
-@pytest.mark.parametrize("scenario", ["late-work", "next-exchange", "per-thread-streams"])
+@pytest.mark.parametrize("scenario", ["late-work", "next-exchange", "per-thread-streams", "failed-launch"])
 def test_order_of_a_worlds_calls(check, scenario, half):
     run = subprocess.run([check, scenario, half], capture_output=True, text=True, timeout=60)
     assert run.returncode == 0, run.stdout

@@ -100,7 +100,8 @@ bool JoinStreams(const ExchangeOrder &order, const std::vector<Pending> &calls, 
     return true;
 }
 
-// Marks the end of the exchange on `stream` and makes the other ranks' streams wait for it.
+// Marks the end of the exchange on `stream` and makes the other ranks' streams wait for it.  Also where a launch failed:
+// the ones ahead of it still read the staging that the next exchange overwrites.
 template <typename Pending>
 bool ReleaseStreams(ExchangeOrder *order, const std::vector<Pending> &calls, hipStream_t stream)
 {
@@ -338,7 +339,8 @@ int DrainWorld(EpWorld *world, const ExchangeShape &shape, const StagePlan &plan
     drain.scaleBytesPerRow = plan.scaleBytesPerRow;
     drain.routesPerRank = shape.bs * plan.perToken;
     drain.stream = stream;
-    for (int q = 0; q < R; ++q) {
+    int ret = kOk;
+    for (int q = 0; q < R && ret == kOk; ++q) {
         const EpDispatchParams &p = world->pendingDispatch[static_cast<size_t>(q)].params;
         DrainTarget &d = drain.target[drain.targets++];
         d = DrainTarget {};
@@ -357,14 +359,14 @@ int DrainWorld(EpWorld *world, const ExchangeShape &shape, const StagePlan &plan
         d.assistOut = p.assistInfoForCombineOut;
         d.scalesOut = static_cast<char *>(p.dynamicScalesOut);
         if (drain.targets == kDrainTargets || q == R - 1) {
-            const int ret = LaunchStatus(LaunchDrain(drain), "drain");
-            if (ret != kOk) {
-                return ret;
-            }
+            ret = LaunchStatus(LaunchDrain(drain), "drain");
             drain.targets = 0;
         }
     }
-    return ReleaseStreams(&world->dispatchOrder, world->pendingDispatch, stream) ? kOk : TileXR::TILEXR_ERROR_INTERNAL;
+    if (!ReleaseStreams(&world->dispatchOrder, world->pendingDispatch, stream) && ret == kOk) {
+        ret = TileXR::TILEXR_ERROR_INTERNAL;
+    }
+    return ret;
 }
 
 } // namespace
@@ -609,7 +611,7 @@ int RunCombineMulti(EpComm *comm, const EpCombineParams &p, bool memoryRoute, in
             }
         }
     }
-    if (status == kOk && !ReleaseStreams(&world->combineOrder, world->pendingCombine, stream)) {
+    if (!ReleaseStreams(&world->combineOrder, world->pendingCombine, stream) && status == kOk) {
         status = TileXR::TILEXR_ERROR_INTERNAL;
     }
     for (PendingCombine &pc : world->pendingCombine) {
