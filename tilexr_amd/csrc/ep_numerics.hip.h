@@ -286,11 +286,10 @@ __device__ __forceinline__ float Exp2Int(int e)
 //
 // A block is 32 columns: the four words (eight elements) of a lane and those of the three other lanes of its quad.  The
 // scaled converts take packed 16-bit elements as they are, divide by 2^e exactly and round once, two elements per
-// instruction; an exhaustive comparison on gfx950 (every 16-bit pattern x every scale exponent, bf16 and fp16, e4m3 and
-// e5m2) found them equal to Fp8Encode(ldexpf(x, -e)) wherever the quotient does not pass the largest finite code, and the
-// convert back, code x scale, equal to Fp8Decode(code) * 2^e for every code that is not a NaN or an infinity, subnormal
-// results and the scale 2^-127 included.  The software codec costs about forty instructions per element, this about
-// three.  What the converts do not do is saturate: elements beyond 1.75 * 2^emax times the scale are brought down to
+// instruction; an exhaustive comparison on gfx950 (tests/cxx/mx_convert_check.hip: every block maximum x every element
+// under it, bf16 and fp16, e4m3 and e5m2) finds the functions below equal to Fp8Encode(ldexpf(x, -e)) and, back,
+// code x scale, to Fp8Decode(code) * 2^e, subnormal results and the scale 2^-127 included.  The software codec costs about
+// forty instructions per element, this about three.  What the converts do not do is saturate: elements beyond 1.75 * 2^emax times the scale are brought down to
 // that value, which has the largest finite code, beforehand, as 16-bit magnitudes.
 // Blocks that hold an infinity or a NaN take the software codec (MxScaling::plain is false).
 typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
