@@ -34,7 +34,6 @@ def test_no_alloc_dispatch_matches_the_allocating_entry_point(legacy_routing):
     shapes = [(4096, 1024, 8, 256), (700, 512, 6, 48), (4096, 1024, 8, 256), (1031, 264, 4, 7)]
     rng = np.random.default_rng(20)
     with Session(legacy_routing=legacy_routing) as s:
-        free_before = None
         for call, (bs, h, K, E) in enumerate(shapes):
             ids = np.stack([rng.permutation(E)[:K] for _ in range(bs)]).astype(np.int32)
             ids[rng.random((bs, K)) < 0.03] = -1                       # a few routes without an expert
@@ -45,12 +44,12 @@ def test_no_alloc_dispatch_matches_the_allocating_entry_point(legacy_routing):
             print(f"no-alloc dispatch: call {call} shape {(bs, h, K, E)}", flush=True)
             assert _call(ep.dispatch_memory, s, x, d_ids, bs, h, K, E, want) == 0
             s.sync()
-            if call == 1:
-                free_before = torch.cuda.mem_get_info()[0]
+            free_before = torch.cuda.mem_get_info()[0]
             assert _call(ep.dispatch_memory_no_alloc, s, x, d_ids, bs, h, K, E, got) == 0
             s.sync()
             if call >= 1:
-                # the device's free memory did not shrink across the call (the first call may still load code)
+                # the device's free memory did not shrink across the call (the first call may still load code); it is read
+                # right ahead of each one, since torch's allocator grows for the comparisons in between
                 assert torch.cuda.mem_get_info()[0] >= free_before
             for name in want:
                 assert torch.equal(want[name].view(torch.int16) if name == "expand_x" else want[name],
