@@ -58,3 +58,22 @@ def test_one_launch_mvp_routing_matches_oracle(case, nums_type):
             got = fetch(out, "recv_counts", counts)
             check_dispatch(got, want)
             assert np.array_equal(got["recv_counts"], want["recv_counts"])
+
+
+@pytest.mark.parametrize("bs,K,E,kernel", [(2, 4, 1024, "ep_route_compact_kernel"), (2, 4, 1025, "ep_route_count_kernel"),
+                                           (2047, 1, 2048, "ep_route_count_kernel"), (256, 8, 2048, "ep_route_compact_kernel")])
+def test_many_experts_and_few_routes_keep_the_count_launch(bs, K, E, kernel):
+    rng = np.random.default_rng(bs + E)
+    ids = ids_for(rng, bs, K, E, invalid=0.1)
+    xt, xb = x_for(rng, bs, 64, ep.DT_FP16)
+    want = O.mvp_dispatch(O.Case(1, bs, 64, K, E, dtype=O.DT_FP16, token_nums_type=1), 0, xb[None], ids[None])
+    with Session() as s:
+        out = alloc_dispatch_outputs(bs, 64, K, E)
+        counts = torch.full((1,), -1, dtype=torch.int32, device=DEV)
+        ids_dev = to_dev(ids)
+        torch.cuda.synchronize()
+        assert ep.dispatch_v2(xt, ids_dev, s.comm, bs, 64, K, E, out["expand_x"], out["assist"], out["token_nums"], counts,
+                              ep.DT_FP16, s.stream, token_nums_type=1) == 0
+        s.sync()
+        assert ep.last_kernel_name(s.comm, ep.K_COUNT) == kernel
+        check_dispatch(fetch(out, "recv_counts", counts), want)

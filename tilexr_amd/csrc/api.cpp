@@ -111,8 +111,8 @@ int RunDispatchSingle(EpComm *comm, const EpDispatchParams &p, bool memoryRoute,
     }
     const CountScratchLayout plan = PlanCountScratch(n, numKeys, experts, expertHist);
     // One launch resolves every route's row where every expert's workgroup can afford to read the whole id table
-    // (ep_rows.hip; the MVP route without a mask has no key and its own launch there); otherwise count (ticket, last workgroup scans) and place, the latter folded into the scatter
-    // unless something needs the rows ahead of it.
+    // (ep_rows.hip; the MVP route without a mask has no key and its own launch there); otherwise count (ticket, last
+    // workgroup scans) and place, the latter folded into the scatter unless something needs the rows ahead of it.
     const bool rowsAhead = p.tileFlagsOut != nullptr || p.metaReadyEvent != nullptr;
     // the scatter kernel that copies per route wants the token rows close by: the routing launch reads them ahead
     const bool warm = ScatterCopiesPerRoute(p.x, p.expandXOut, p.bs, p.h, p.topK, static_cast<int>(p.quantMode));
@@ -121,7 +121,8 @@ int RunDispatchSingle(EpComm *comm, const EpDispatchParams &p, bool memoryRoute,
         RouteRowsFits(p.expertIds, n, numKeys, maskMode, p.expertCapacity) &&
         (comm->routing == EpComm::Routing::kOneLaunch || RouteRowsPays(n, numKeys, rowsAhead, warm));
     const bool oneLaunchCompact = mayOneLaunch && !memoryRoute && p.expertCapacity <= 0 &&
-        RouteCompactFits(p.expertIds, n, experts, maskMode);
+        RouteCompactFits(p.expertIds, n, experts, maskMode) &&
+        (comm->routing == EpComm::Routing::kOneLaunch || RouteCompactPays(n, experts));
     const bool oneLaunch = oneLaunchRows || oneLaunchCompact;
     void *scratchBase = nullptr;
     if (p.noAlloc) {

@@ -97,7 +97,8 @@ bool RouteRowsPays(int64_t routes, int64_t numKeys, bool rowsAhead, bool readsRo
 bool RouteRowsFits(const int32_t *ids, int64_t routes, int64_t numKeys, int maskMode, int64_t capacity);
 hipError_t LaunchRouteRows(const RouteRowsLaunch &l);
 
-// MVP route, one rank, no mask: the compaction of all routes in one launch (ep_rows.hip).
+// MVP route, one rank, no mask: the compaction of all routes in one launch (ep_rows.hip), for id tables up to the largest one
+// measured.
 constexpr int kCompactTableRoutes = 131072;
 struct RouteCompactLaunch {
     const int32_t *ids;
@@ -116,6 +117,7 @@ struct RouteCompactLaunch {
     int64_t warmBytes;
     hipStream_t stream;
 };
+bool RouteCompactPays(int64_t routes, int64_t numExperts);
 bool RouteCompactFits(const int32_t *ids, int64_t routes, int64_t numExperts, int maskMode);
 hipError_t LaunchRouteCompact(const RouteCompactLaunch &l);
 

@@ -484,12 +484,19 @@ hipError_t LaunchRouteRows(const RouteRowsLaunch &l)
     return hipGetLastError();
 }
 
-// Every call it fits: against the count launch, both forced in turn on the same buffers, dispatch + combine layers of
-// 512 .. 131 072 routes x 16 .. 1024 experts, 1024 and 4096 columns, plain and int8 rows took 1.5 us less at the smallest
-// and 20-110 us less at the largest, and no combination longer.  Beyond the largest measured table the count launch stays.
 bool RouteCompactFits(const int32_t *ids, int64_t routes, int64_t numExperts, int maskMode)
 {
     return routes > 0 && routes <= kCompactTableRoutes && numExperts > 0 && numExperts <= kMaxKeys && maskMode == kMaskNone && Aligned16(ids);
+}
+
+// Against the count launch, both forced in turn on the same buffers, us per dispatch + combine layer: up to 1024 experts no
+// combination of 4 .. 131 072 routes, 1024 to 7168 columns, plain and int8 rows took longer (512 experts, 8 routes x 1024
+// columns 11.8 -> 10.2; 1024 experts, 8 routes 12.0 -> 11.7, 131 072 routes 239 -> 132).  Beyond, each expert costs a
+// workgroup, which few routes do not pay for (8 routes: 1280 experts 12.3 -> 12.5, 2048 experts 12.8 -> 14.8; 1024 routes x
+// 2048 experts 15.5 -> 16.5) and 2048 or more do (2048 routes x 2048 experts 21.6 -> 17.7; 131 072 routes 355 -> 150).
+bool RouteCompactPays(int64_t routes, int64_t numExperts)
+{
+    return numExperts <= 1024 || routes >= 2048;
 }
 
 hipError_t LaunchRouteCompact(const RouteCompactLaunch &l)
