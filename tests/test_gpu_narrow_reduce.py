@@ -11,7 +11,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("dtype,torch_dtype", [(ep.DT_BF16, torch.bfloat16), (ep.DT_FP16, torch.float16)])
 @pytest.mark.parametrize("bs,h,K,E", [(1, 2048, 8, 16), (3, 1032, 8, 16), (7, 2040, 1, 8), (130, 1536, 9, 32), (1024, 2048, 2, 16),
-                                      (1025, 2048, 2, 16)])
+                                      (1025, 2048, 2, 16), (640, 1032, 2, 16), (641, 2048, 1, 16), (1024, 1032, 3, 16),
+                                      (1025, 2048, 3, 16)])
 def test_matches_sums_in_slot_order(bs, h, K, E, dtype, torch_dtype):
     gen = torch.Generator(device=DEV).manual_seed(bs + h)
     x = torch.randn(bs, h, device=DEV, generator=gen).to(torch_dtype)

@@ -25,6 +25,14 @@ def test_memory_route_world(shape):
     multi.test_memory_dispatch_and_combine_across_ranks(shape, ep.DT_BF16)
 
 
+@pytest.mark.parametrize("dtype", [ep.DT_BF16, ep.DT_FP16])
+@pytest.mark.parametrize("shape", [(3, 20, 1032, 4, 9), (2, 320, 2048, 2, 8), (2, 321, 1536, 2, 8), (2, 512, 1040, 3, 8),
+                                   (2, 513, 1040, 3, 8)])
+def test_rows_in_one_slice_and_in_two(shape, dtype):
+    """Combines of rows of 129 to 256 vectors on both sides of the numbers of tokens up to which they are cut."""
+    multi.test_memory_dispatch_and_combine_across_ranks(shape, dtype)
+
+
 @pytest.mark.parametrize("shape", [(2, 20, 64, 2, 514), (17, 9, 64, 2, 34), (3, 20, 2056, 2, 9)])
 def test_mvp_route_world(shape):
     multi.test_mvp_dispatch_and_combine_across_ranks(shape)

@@ -182,11 +182,33 @@ bool IsPlain(const ReduceLaunch &l)
         (l.sharedExpertX == nullptr || Aligned16(l.sharedExpertX)) && (l.commQuant == 0 || l.h % 32 == 0);
 }
 
-// Narrow rows: a wave per token.  Wide ones are cut into slices of 128 vectors, one wave each (many small independent waves
-// with four rows in flight each reach the highest gather bandwidth here).
-int SlicesOf(int64_t vecs)
+// Slices that a token's row is cut into by the plain kernels, a wave each; `ranks` reduces of this shape in the launch.
+// Narrow rows: a wave per token.  Wide ones: slices of 128 vectors (many small independent waves with four rows in flight
+// each reach the highest gather bandwidth here).  Rows of 129 to 256 vectors: a wave that has a token to itself keeps two
+// rows in flight; a launch of at most kWideReduceUnits waves with half a row each keeps eight.  Eight layers in a graph, us
+// with one slice and with two, 2048 columns, top-8: 16 tokens 92 -> 56, 512 tokens 150 -> 134, 1024 tokens 186 -> 171, 2048
+// tokens 280 and 278.  One or two rows arrive in one trip either way, and a second wave pays only while the waves are few:
+// top-2, 512 tokens 76.6 -> 72.6, 640 tokens 82.2 -> 79.6, 768 tokens 85.1 and 84.1 (1032 columns 80.7 and 81.7), 1024
+// tokens 95.5 and 96.1 (1032 columns 88.2 and 90.5).  The reduce of a logical world, us of its launch: 4 ranks x 128 tokens,
+// top-8 7.9 -> 5.7, 2 x 512 8.5 and 8.4, top-2 2 x 64 4.6 -> 4.4, 2 x 300 4.8 and 5.0.
+int SlicesOf(const ReduceLaunch &l, int ranks)
 {
-    return vecs <= 4 * kWave ? 1 : static_cast<int>((vecs + 2 * kWave - 1) / (2 * kWave));
+    constexpr int64_t kPairTokens = 640;
+    const int64_t vecs = l.h / 8;
+    const int slices = static_cast<int>((vecs + 2 * kWave - 1) / (2 * kWave));
+    if (vecs > 4 * kWave) {
+        return slices;
+    }
+    const int64_t tokens = l.bs * ranks;
+    const bool few = l.tileFlags == nullptr && l.reduceKind == kReduceFp32 && l.commQuant == 0 &&
+        tokens * slices <= kWideReduceUnits && (l.topK + l.sharedSlots > 2 || tokens <= kPairTokens);
+    return few ? slices : 1;
+}
+
+// 16-byte vectors per lane of a wave that takes one of `slices` slices.
+int VecsPerLane(int64_t vecs, int slices)
+{
+    return slices == 1 && vecs > 2 * kWave ? 4 : 2;
 }
 
 } // namespace
@@ -206,16 +228,16 @@ hipError_t LaunchReduceWorld(const ReduceLaunch *ls, int ranks)
     if (!ReduceWorldFits(ls, ranks)) {
         return hipErrorInvalidValue;
     }
-    const int64_t vecs = ls[0].h / 8;
+    const int slices = SlicesOf(ls[0], ranks);
     WorldReduceArgs w {};
     for (int r = 0; r < ranks; ++r) {
         w.rank[r] = ArgsOf(ls[r]);
-        w.rank[r].colSlices = SlicesOf(vecs);
+        w.rank[r].colSlices = slices;
         if (ls[r].kernelNameOut != nullptr) {
             *ls[r].kernelNameOut = "ep_reduce_vec_world_kernel";
         }
     }
-    LaunchVecKernels(kWave, vecs > 2 * kWave && vecs <= 4 * kWave ? 4 : 2, ls[0], w.rank[0], 0, &w, ranks);
+    LaunchVecKernels(kWave, VecsPerLane(ls[0].h / 8, slices), ls[0], w.rank[0], 0, &w, ranks);
     return hipGetLastError();
 }
 
@@ -250,15 +272,7 @@ hipError_t LaunchReduce(const ReduceLaunch &l)
             LaunchQuantKernels(kThreads, 4, l, a, gridLimit);
         }
     } else if (plain) {
-        // Few tokens of 129 to 256 vectors: a wave per token keeps two rows in flight, four round trips for eight rows; in
-        // two slices they all arrive in one.  Eight layers of 3 x 2048, top-8 of 16, in a graph: 85.1 -> 54.0 us.
-        const bool few = l.tileFlags == nullptr && l.reduceKind == kReduceFp32 && l.commQuant == 0 &&
-            l.bs * 2 <= kWideReduceUnits;
-        if (vecs <= 2 * kWave) {
-            LaunchVecKernels(kWave, 2, l, a, gridLimit, nullptr, 1);
-        } else if (vecs <= 4 * kWave && !few) {
-            LaunchVecKernels(kWave, 4, l, a, gridLimit, nullptr, 1);
-        } else if (mayWait) {
+        if (vecs > 4 * kWave && mayWait) {
             // readiness flags that may still be pending: one workgroup per token, so that one wave polls the token's
             // tiles instead of one per slice, and few enough workgroups that the producer fits beside them
             if (vecs <= 2 * kThreads) {
@@ -269,8 +283,8 @@ hipError_t LaunchReduce(const ReduceLaunch &l)
                 LaunchVecKernels(kThreads, 8, l, a, gridLimit, nullptr, 1);
             }
         } else {
-            a.colSlices = static_cast<int>((vecs + 2 * kWave - 1) / (2 * kWave));
-            LaunchVecKernels(kWave, 2, l, a, gridLimit, nullptr, 1);
+            a.colSlices = SlicesOf(l, 1);
+            LaunchVecKernels(kWave, VecsPerLane(vecs, a.colSlices), l, a, gridLimit, nullptr, 1);
         }
     } else {
         int grid = static_cast<int>(l.bs);
