@@ -573,8 +573,14 @@ void LaunchVec(const ScatterArgs &a, hipStream_t stream)
         // Eight workgroups per compute unit that each quantise a wide row and store it topK times oversubscribe the memory
         // system like those of the per-route kernel; unused dynamic LDS caps them at five.  (8192 x 4096 int8 x top-6,
         // microseconds at eight, six, five, four, three: 53.5, 50.1, 49.4, 49.9, 50.8; 2048 x 7168 MXFP8 27.3, 27.0, 25.9,
-        // 25.6, 25.5.  Copies, 16384 x 7168 x top-8: 402, 403, 417, 430, 436.  Rows a wave holds: no difference.)
-        const unsigned capLds = QMODE != TILEXR_EP_QUANT_NONE && G == kThreads ? kRouteCapLdsBytes : 0u;
+        // 25.6, 25.5.  Copies, 16384 x 7168 x top-8: 402, 403, 417, 430, 436.)  That takes rows that store enough: dispatch +
+        // combine at eight and at five, int8 or block fp8, 2048 x 7168 top-8 65.7 -> 62.3, 4096 x 7168 top-4 69.3 -> 67.1,
+        // 2048 x 8192 top-4 43.4 -> 42.1, 8192 x 4096 top-6 107.9 -> 105.5; but 2048 x 4096 top-2 20.4 and 21.4, 8192 x
+        // 2304 top-2 42.3 and 44.6, 16384 x 2304 top-8 181 and 201, 16384 x 3072 top-8 205 and 213, 16384 x 4096 top-5 181
+        // and 187, 2048 x 12288 top-2 46.8 and 48.6.  (Rows a wave holds: no difference.)
+        const int vecs = a.h / 8;
+        const bool capped = QMODE != TILEXR_EP_QUANT_NONE && vecs >= 2 * kThreads && a.topK >= 4 && vecs * a.topK >= 12 * kThreads;
+        const unsigned capLds = capped ? kRouteCapLdsBytes : 0u;
         hipLaunchKernelGGL((ep_scatter_vec_kernel<G, V, QMODE, BF16, E5M2, false>), dim3(groups), dim3(kThreads), capLds, stream, a);
     }
 }
