@@ -1,5 +1,7 @@
 """One layer called on one stream after another, torch's default stream, streams of torch's own, a wrapped one and a
 capturing one among them: every call sees the inputs its stream has written and the scratch of no other call."""
+import ctypes
+
 import pytest
 import torch
 
@@ -108,6 +110,28 @@ def test_two_branches_of_one_capture():
             for (d, y), want in zip((first, second), eager):
                 for got, expected in zip(results(d, y), want):
                     assert torch.equal(got, expected)
+
+
+def test_calls_of_one_capture_are_one_chain():
+    """Whether the two micro-batches of a capture are ordered, from the captured graph itself: it begins with one kernel,
+    where two unordered branches begin with two."""
+    hip = ctypes.CDLL("libamdhip64.so")
+    batches = [inputs(33), inputs(34)]
+    side = torch.cuda.Stream()
+    with layer.MoeEpLayer(E, K, H) as moe:
+        moe.dispatch(*batches[0][:2], capacity=8)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph(keep_graph=True)
+        with torch.cuda.graph(graph):
+            main = torch.cuda.current_stream()
+            side.wait_stream(main)
+            kept = [moe.dispatch(*batches[0][:2], capacity=8)]
+            with torch.cuda.stream(side):
+                kept.append(moe.dispatch(*batches[1][:2], capacity=8))
+            main.wait_stream(side)
+        roots = ctypes.c_size_t(0)
+        assert hip.hipGraphGetRootNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(roots)) == 0
+        assert roots.value == 1
 
 
 def test_default_stream_handle_is_taken_and_null_is_not():

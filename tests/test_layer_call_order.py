@@ -27,6 +27,15 @@ class Stream:
             assert other.capture == self.capture, f"the capture of {self.name} waits for {other.name}, which is not in it"
         self.behind |= {other.name} | other.behind
 
+    def __eq__(self, other):
+        return isinstance(other, Stream) and self is other
+
+    def __ne__(self, other):
+        # as torch's: anything that is no stream, None among it, is neither equal nor unequal to one
+        return isinstance(other, Stream) and self is not other
+
+    __hash__ = object.__hash__
+
     def __repr__(self):
         return self.name
 

@@ -71,7 +71,8 @@ class _CallStream:
                 self._waiting, run = current, self._own
                 run.wait_stream(current)
                 handle = run.cuda_stream
-            if run != self._last or self._captured is not None:
+            # (not `run != self._last`: torch's streams answer False to `!= None`)
+            if self._captured is not None or not run == self._last:
                 self._order(run)
             return (handle if handle != 0 else ep.STREAM_LEGACY), current
         except BaseException:
