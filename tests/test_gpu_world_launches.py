@@ -63,3 +63,46 @@ def test_every_row_on_one_rank(one_stream):
             counts = np.stack([o["counts"].cpu().numpy() for o in outs])
             for r in range(R):
                 assert np.array_equal(multi.bits16(ys[r]), O.mem_combine(case, r, eo, assist, counts)), f"rank {r}"
+
+
+def test_work_between_a_ranks_call_and_the_last_ones_runs_ahead_of_the_outputs():
+    """Rank 0 fills its outputs, and writes the combine weights, on its own stream after its call: the second half, which
+    the last caller's stream runs, comes behind that."""
+    R, bs, h, K, E = 2, 50, 256, 4, 8
+    rng = np.random.default_rng(8)
+    ids = multi.rand_ids(rng, R, bs, K, E)
+    xt, xb = multi.rand_x(rng, R, bs, h, ep.DT_BF16)
+    weights = rng.random((R, bs, K)).astype(np.float32)
+    case = O.Case(R, bs, h, K, E, token_nums_type=1)
+    wants = [O.mem_dispatch(case, r, xb, ids) for r in range(R)]
+    with multi.World(R) as w:
+        outs = multi.run_dispatch(w, True, xt, ids, bs, h, K, E, ep.DT_BF16)        # scratch of this size
+        dev_ids = [multi.to_dev(ids[r]) for r in range(R)]
+        dev_w = [torch.zeros((bs, K), device=multi.DEV) for _ in range(R)]
+        given = [multi.to_dev(weights[r]) for r in range(R)]
+        ys = [torch.full((bs, h), 7.0, dtype=torch.bfloat16, device=multi.DEV) for _ in range(R)]
+        torch.cuda.synchronize()
+        for r in range(R):
+            o = outs[r]
+            assert ep.dispatch_memory_v2(xt[r], dev_ids[r], w.comms[r], bs, h, K, E, o["expand_x"], o["assist"], o["token_nums"],
+                                         o["counts"], ep.DT_BF16, w.streams[r]) == 0
+            if r == 0:
+                with torch.cuda.stream(w.streams[0]):
+                    torch.cuda._sleep(2_000_000)
+                    for name in ("expand_x", "assist", "counts"):
+                        o[name].fill_(-77)
+        w.sync()
+        for r in range(R):
+            multi.check_rank(outs[r], wants[r], "send_counts")
+        for r in range(R):
+            assert ep.combine_memory_v2(outs[r]["expand_x"], outs[r]["assist"], outs[r]["counts"], w.comms[r], bs, h, K, E, ys[r],
+                                        ep.DT_BF16, w.streams[r], expert_scales=dev_w[r]) == 0
+            with torch.cuda.stream(w.streams[r]):
+                if r == 0:
+                    torch.cuda._sleep(2_000_000)
+                    dev_w[0].copy_(given[0])
+        w.sync()
+        eo = np.stack([o["expand_x"].cpu().numpy().view(np.uint16) for o in outs])
+        assist = np.stack([o["assist"].cpu().numpy() for o in outs])
+        counts = np.stack([o["counts"].cpu().numpy() for o in outs])
+        assert np.array_equal(multi.bits16(ys[0]), O.mem_combine(case, 0, eo, assist, counts, expert_scales=weights[0]))

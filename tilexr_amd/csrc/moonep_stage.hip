@@ -1355,7 +1355,10 @@ hipError_t LaunchMoonDispatch(const DispatchWorld &w, hipStream_t stream, const 
         }
     } else if (perRoute) {
         gScatterName = "moon_scatter_kernel";
-        // narrow rows give a workgroup a few KiB to move: those need every workgroup that fits
+        // The cap takes workgroups with both of their lanes' loads to do (four stages, top-8, us without and with it: 4096 x
+        // 4096 265 and 262, 4096 x 7168 436 and 415; up to 4096 x 2304 no difference beyond the runs' own).  The launch that
+        // builds the plan as well keeps eight: at five its narrow rows lose what its wide ones gain (forward stages, top-8:
+        // 4096 x 1024 76.0 and 77.6, 4096 x 2304 93.5 and 97.1; 1024 x 4096 53.1 and 51.1, 1024 x 7168 72.8 and 72.0).
         const unsigned capLds = vecs > kThreads ? kScatterCapLdsBytes : 0u;
         const dim3 grid(static_cast<unsigned>(blocks) + planBlocks, R);
         if (planInScatter) {
