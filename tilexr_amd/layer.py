@@ -57,6 +57,7 @@ class _CallStream:
         self._device = device
         self._own = own
         self._last = None           # stream of the last eager call
+        self._last_handle = None
         self._captured = None       # stream of the last call known to be captured
         self._waiting = None
         self._lock = threading.Lock()
@@ -71,8 +72,8 @@ class _CallStream:
                 self._waiting, run = current, self._own
                 run.wait_stream(current)
                 handle = run.cuda_stream
-            # (not `run != self._last`: torch's streams answer False to `!= None`)
-            if self._captured is not None or not run == self._last:
+            # by handle: torch's streams answer False to `!= None` (and torch's own, or the layer's, are never destroyed)
+            if handle != self._last_handle or self._captured is not None:
                 self._order(run)
             return (handle if handle != 0 else ep.STREAM_LEGACY), current
         except BaseException:
@@ -99,7 +100,7 @@ class _CallStream:
                 run.wait_stream(self._last)
             elif self._captured is None:
                 self._captured = self._last
-        self._last = run
+        self._last, self._last_handle = run, run.cuda_stream
 
     def __exit__(self, *exc):
         try:
