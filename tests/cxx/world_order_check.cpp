@@ -73,6 +73,43 @@ void ExpectOrder(const std::string &first, const std::string &then, int from = 0
     }
 }
 
+// Where the reduces of the calls so far found their tagged slot tables and their order keys.
+struct Range {
+    const char *first, *end;
+};
+std::vector<Range> gTagWords;
+std::vector<Range> gKeyWords;
+
+void NoteTables(const ReduceLaunch &l)
+{
+    const int64_t bytes = l.bs * (l.topK + l.sharedSlots) * 8;
+    const char *tags = reinterpret_cast<const char *>(l.inverseTagged);
+    gTagWords.push_back({tags, tags + bytes});
+    if (l.orderKeys != nullptr) {
+        const char *keys = reinterpret_cast<const char *>(l.orderKeys);
+        gKeyWords.push_back({keys, keys + bytes});
+    }
+}
+
+// A word that one call uses as an order key (a rank in its upper half) may not be one that another call takes for a slot's
+// tag (an epoch in its upper half).
+void ExpectTagsApartFromKeys()
+{
+    if (gTagWords.empty() || gKeyWords.empty()) {
+        std::printf("FAIL: no tables were seen\n");
+        ++gFailures;
+    }
+    for (const Range &t : gTagWords) {
+        for (const Range &k : gKeyWords) {
+            if (t.first < k.end && k.first < t.end) {
+                std::printf("FAIL: order keys of one call lie where another looks for tags\n");
+                ++gFailures;
+                return;
+            }
+        }
+    }
+}
+
 hipError_t SecondHalf(hipStream_t s, const char *name)
 {
     if (gLaunchesUntilFailure == 0) {
@@ -103,16 +140,16 @@ struct World {
             world.comms.push_back(&c);
         }
     }
-    int Call(bool combine, int r, hipStream_t stream)
+    int Call(bool combine, int r, hipStream_t stream, int64_t tokens = 4, bool memoryRoute = true)
     {
         static int32_t words[64] = {};
         EpComm *c = &comms[static_cast<size_t>(r)];
         if (combine) {
             EpCombineParams p {};
-            p.bs = 4, p.h = 64, p.topK = 2, p.moeExpertNum = world.rankSize;
+            p.bs = tokens, p.h = 64, p.topK = 2, p.moeExpertNum = world.rankSize;
             p.stream = stream;
             p.epRecvCounts = words;
-            return RunCombineMulti(c, p, true, 1);
+            return RunCombineMulti(c, p, memoryRoute, 1);
         }
         EpDispatchParams p {};
         p.x = words;
@@ -176,7 +213,9 @@ namespace TileXREp {
 
 bool DeviceBuffer::Reserve(size_t want, bool)
 {
-    ptr = reinterpret_cast<void *>(static_cast<uintptr_t>(0x100000));
+    // every buffer has addresses of its own, and room for whatever is asked of it
+    static std::map<DeviceBuffer *, uintptr_t> places;
+    ptr = reinterpret_cast<void *>(places.emplace(this, (places.size() + 1) << 40).first->second);
     bytes = want;
     return true;
 }
@@ -194,7 +233,13 @@ hipError_t LaunchReturnRows(const ReturnRowsLaunch &l)
     return hipSuccess;
 }
 bool ReduceWorldFits(const ReduceLaunch *, int) { return true; }
-hipError_t LaunchReduceWorld(const ReduceLaunch *ls, int) { return SecondHalf(ls[0].stream, "reduce"); }
+hipError_t LaunchReduceWorld(const ReduceLaunch *ls, int ranks)
+{
+    for (int r = 0; r < ranks; ++r) {
+        NoteTables(ls[r]);
+    }
+    return SecondHalf(ls[0].stream, "reduce");
+}
 // launches these calls do not make
 hipError_t LaunchReduce(const ReduceLaunch &) { return hipErrorUnknown; }
 hipError_t LaunchAugment(const AugmentLaunch &) { return hipErrorUnknown; }
@@ -267,6 +312,17 @@ int main(int argc, char **argv)
             ++gFailures;
         }
         NextExchange(w, combine);
+    } else if (scenario == "shapes") {
+        // combines of several sizes, on both routes, through one world's tables
+        World w(3);
+        for (const bool memoryRoute : {false, true}) {
+            for (const int64_t tokens : {4, 40, 7, 23}) {
+                for (int r = 0; r < 3; ++r) {
+                    gFailures += w.Call(true, r, StreamNo(r), tokens, memoryRoute) != 0 ? 1 : 0;
+                }
+            }
+        }
+        ExpectTagsApartFromKeys();
     } else {
         std::printf("unknown scenario\n");
         return 2;

@@ -65,6 +65,31 @@ def test_every_row_on_one_rank(one_stream):
                 assert np.array_equal(multi.bits16(ys[r]), O.mem_combine(case, r, eo, assist, counts)), f"rank {r}"
 
 
+@pytest.mark.parametrize("memory", [True, False])
+def test_sizes_in_turn_leave_no_rows_behind(memory):
+    """A large, a small and the large size again, the last with a rank whose routes name no expert: its outputs are zero,
+    whatever the small exchange, whose slots lie elsewhere in the same tables, has written there."""
+    R, h, K, E = 8, 64, 2, 16
+    rng = np.random.default_rng(12)
+    dtype, tdt = (ep.DT_BF16, torch.bfloat16) if memory else (ep.DT_FP16, torch.float16)
+    with multi.World(R) as w:
+        for round_ in range(3):
+            for bs in (64, 9, 64, 17, 64):
+                ids = multi.rand_ids(rng, R, bs, K, E)
+                ids[0] = -1
+                xt, _ = multi.rand_x(rng, R, bs, h, dtype)
+                outs = multi.run_dispatch(w, memory, xt, ids, bs, h, K, E, dtype)
+                ys = [torch.full((bs, h), 7.0, dtype=tdt, device=multi.DEV) for _ in range(R)]
+                torch.cuda.synchronize()
+                for r in range(R):
+                    call = ep.combine_memory_v2 if memory else ep.combine_v2
+                    assert call(outs[r]["expand_x"].view(tdt), outs[r]["assist"], outs[r]["counts"], w.comms[r], bs, h, K, E, ys[r],
+                                dtype, w.streams[r]) == 0
+                w.sync()
+                assert not ys[0].any()
+                assert ys[1].any()
+
+
 def test_work_between_a_ranks_call_and_the_last_ones_runs_ahead_of_the_outputs():
     """Rank 0 fills its outputs, and writes the combine weights, on its own stream after its call: the second half, which
     the last caller's stream runs, comes behind that."""

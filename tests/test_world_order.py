@@ -24,3 +24,9 @@ def check(tmp_path_factory):
 def test_order_of_a_worlds_calls(check, scenario, half):
     run = subprocess.run([check, scenario, half], capture_output=True, text=True, timeout=60)
     assert run.returncode == 0, run.stdout
+
+
+def test_tables_of_differently_sized_combines(check):
+    """Tags are told from stale words by their epoch: what is no tag may not lie where another size's tags do."""
+    run = subprocess.run([check, "shapes"], capture_output=True, text=True, timeout=60)
+    assert run.returncode == 0, run.stdout

@@ -28,7 +28,7 @@ void ReleaseWorld(EpWorld *world)
         (void)hipFree(world->flagArea);
     }
     for (DeviceBuffer *b : {&world->stageRows, &world->stageAux, &world->stageCounts, &world->combineSlots,
-             &world->combineMeta, &world->drainPlans}) {
+             &world->combineMeta, &world->combineKeys, &world->drainPlans}) {
         b->Release();
     }
     for (ExchangeOrder *order : {&world->dispatchOrder, &world->combineOrder}) {

@@ -112,7 +112,8 @@ struct EpWorld {
     DeviceBuffer stageAux;        // [R] assist tuples + per-row scales
     DeviceBuffer stageCounts;     // [R] keyOffset + expertTotal
     DeviceBuffer combineSlots;    // [R] [bs, topK] rows returned by the expert ranks
-    DeviceBuffer combineMeta;     // [R] tagged slot table + order keys
+    DeviceBuffer combineMeta;     // [R] slot tables, nothing but tagged words: a word another size left behind has an older tag
+    DeviceBuffer combineKeys;     // [R] order keys of the slots (MVP route)
     TileXRMoon::WorldState *moon = nullptr;   // created by the first plan-driven call of the world
 };
 

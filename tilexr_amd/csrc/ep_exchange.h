@@ -101,7 +101,8 @@ struct ReturnRowsLaunch {
     uint64_t epoch;
     char *slots;             // [R] x slotsStride: rows at slot token*topK + k of the source rank
     int64_t slotsStride;
-    uint64_t *meta;          // [R] x metaStride words: inverse (epoch << 32 | slot), then order keys
+    uint64_t *meta;          // [R] x metaStride words: inverse (epoch << 32 | slot)
+    uint64_t *orderKeys;     // optional, [R] x metaStride words: expert rank << 32 | row
     int64_t metaStride;      // in words
     hipStream_t stream;
 };

@@ -357,6 +357,7 @@ struct ReturnRowsArgs {
     char *slots;
     int64_t slotsStride;
     uint64_t *meta;
+    uint64_t *orderKeys;
     int64_t metaStride;
 };
 
@@ -401,10 +402,11 @@ __global__ __launch_bounds__(kThreads) void ep_return_rows_kernel(ReturnRowsArgs
         CopyBytes(a.slots + static_cast<int64_t>(src) * a.slotsStride + slot * a.rowBytes,
             a.expertOut + static_cast<int64_t>(row) * a.rowBytes, a.rowBytes, lane, G);
         if (lane == 0) {
-            uint64_t *meta = a.meta + static_cast<int64_t>(src) * a.metaStride;
-            meta[slot] = (a.epoch << 32) | static_cast<uint32_t>(slot);
-            meta[static_cast<int64_t>(a.bs) * a.topK + slot] =
-                (static_cast<uint64_t>(static_cast<uint32_t>(a.expertRank)) << 32) | static_cast<uint32_t>(row);
+            const int64_t at = static_cast<int64_t>(src) * a.metaStride + slot;
+            a.meta[at] = (a.epoch << 32) | static_cast<uint32_t>(slot);
+            if (a.orderKeys != nullptr) {
+                a.orderKeys[at] = (static_cast<uint64_t>(static_cast<uint32_t>(a.expertRank)) << 32) | static_cast<uint32_t>(row);
+            }
         }
     }
 }
@@ -497,6 +499,7 @@ hipError_t LaunchReturnRows(const ReturnRowsLaunch &l)
     a.slots = l.slots;
     a.slotsStride = l.slotsStride;
     a.meta = l.meta;
+    a.orderKeys = l.orderKeys;
     a.metaStride = l.metaStride;
     const int lanes = LanesPerRow(l.rowBytes);
     const int perGroup = kThreads / lanes;

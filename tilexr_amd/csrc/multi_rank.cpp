@@ -516,12 +516,13 @@ int RunCombineMulti(EpComm *comm, const EpCombineParams &p, bool memoryRoute, in
     const int64_t n = p.bs * perToken;
     const int64_t rowBytes = p.h * 2;
     const int64_t slotsStride = Align256(n * rowBytes);
-    const int64_t metaStride = (2 * n + 31) / 32 * 32;
+    const int64_t metaStride = (n + 31) / 32 * 32;
     if (first) {
         world->combineShape = shape;
         ++world->combineEpoch;
         if (!world->combineSlots.Reserve(static_cast<size_t>(R * slotsStride), false) ||
-            !world->combineMeta.Reserve(static_cast<size_t>(R * metaStride * 8), true)) {
+            !world->combineMeta.Reserve(static_cast<size_t>(R * metaStride * 8), true) ||
+            (!memoryRoute && !world->combineKeys.Reserve(static_cast<size_t>(R * metaStride * 8), false))) {
             return TileXR::TILEXR_ERROR_INTERNAL;
         }
     } else if (!(shape == world->combineShape)) {
@@ -554,6 +555,7 @@ int RunCombineMulti(EpComm *comm, const EpCombineParams &p, bool memoryRoute, in
     back.slots = static_cast<char *>(world->combineSlots.ptr);
     back.slotsStride = slotsStride;
     back.meta = static_cast<uint64_t *>(world->combineMeta.ptr);
+    back.orderKeys = memoryRoute ? nullptr : static_cast<uint64_t *>(world->combineKeys.ptr);
     back.metaStride = metaStride;
     back.stream = stream;
     int ret = LaunchStatus(LaunchReturnRows(back), "return rows");
@@ -576,13 +578,12 @@ int RunCombineMulti(EpComm *comm, const EpCombineParams &p, bool memoryRoute, in
     std::vector<ReduceLaunch> reduces(static_cast<size_t>(R));
     for (int r = 0; r < R; ++r) {
         const EpCombineParams &rp = world->pendingCombine[static_cast<size_t>(r)].params;
-        uint64_t *meta = static_cast<uint64_t *>(world->combineMeta.ptr) + static_cast<int64_t>(r) * metaStride;
         ReduceLaunch &red = reduces[static_cast<size_t>(r)];
         red.expertOut = static_cast<char *>(world->combineSlots.ptr) + static_cast<int64_t>(r) * slotsStride;
         red.rowBytes = rowBytes;
-        red.inverseTagged = meta;
+        red.inverseTagged = back.meta + static_cast<int64_t>(r) * metaStride;
         red.epoch = epoch;
-        red.orderKeys = memoryRoute ? nullptr : meta + n;
+        red.orderKeys = memoryRoute ? nullptr : back.orderKeys + static_cast<int64_t>(r) * metaStride;
         red.expertScales = memoryRoute ? rp.expertScales : nullptr;
         red.tokenMask = memoryRoute ? reinterpret_cast<const uint8_t *>(rp.xActiveMask) : nullptr;
         red.sharedExpertX = memoryRoute ? rp.sharedExpertX : nullptr;
