@@ -239,6 +239,33 @@ def test_random_shapes(seed, row_cache):
                 np.testing.assert_array_equal(cres[r]["wy"].cpu().numpy(), wy[r], err_msg=f"rank {r} routeWeightsSk")
 
 
+@pytest.mark.parametrize("world", [1, 3])
+def test_sizes_in_turn_through_one_world(world, row_cache):
+    """A large size again and again with small ones between: what another size keeps in the world's tables (duplicates per
+    group, chunk totals: small numbers, like those of the first exchanges) must not pass for words of the running one.
+    Rows that no route names come out as zeros."""
+    rng = np.random.default_rng(70 + world)
+    k, h = 8, 64
+    with World(world) as w:
+        for s, slack in ((600, 900), (70, 40), (600, 900), (9, 0), (600, 900), (150, 300), (33, 7), (600, 900)):
+            sh = M.Shape(world, s, k, h, s * k + slack)
+            dst = MC.random_dst(sh, rng, duplicates=True)
+            hidden = random_rows(rng, (world, s, h))
+            want = M.dispatch_world(sh, dst, hidden, None, flags=M.FLAG_BUILD_DEDUP)
+            plans = w.plan_tensors(sh, dst)
+            res = w.dispatch(sh, plans, hidden, None, flags=mp.FLAG_BUILD_DEDUP)
+            w.sync()
+            check_dispatch(sh, res, plans, want, fresh=True)
+            out, _, _, dup = want
+            dst_local = M.build_dst_local(sh, dst)
+            cres = w.combine(sh, plans, dst_local, [r["out"] for r in res], None)
+            w.sync()
+            y, _, cstatus = M.combine_world(sh, dst_local, dup, out, None)
+            for r in range(world):
+                assert int(plans[r]["status"][0].item()) == int(cstatus[r])
+                np.testing.assert_array_equal(host_bits16(cres[r]["y"]), y[r], err_msg=f"rank {r} hiddenSh")
+
+
 def test_home_plans_with_padding():
     """Plans as the reference's planner lays them out (expert groups padded to 8 rows, duplicates marked), fresh and
     saved, three exchanges back to back on one world without waiting in between."""

@@ -146,17 +146,19 @@ int Internal(hipError_t err, const char *what)
         }                                         \
     } while (0)
 
-// Sizes the world's per-row tables for this shape and returns views into them.  Entries carry their epoch, so a
-// change of layout needs no clearing: whatever an older call left behind has an older epoch.
+// Sizes the world's per-row tables for this shape and returns views into them.  Tagged words carry their epoch, so a
+// change of layout needs no clearing: whatever an older call left behind among them has an older epoch.  That holds for
+// tagged words only, hence a buffer of their own: a count or a rank that another shape left in the upper half of a word
+// could be the running epoch.
 bool PrepareTables(WorldState *st, int world, int64_t nvS, int64_t n, WorldTables *out)
 {
     const int64_t rows = nvS > n ? nvS : n;
     const int64_t stride = (rows + kTableAlign - 1) / kTableAlign * kTableAlign;
     const int64_t groups = (rows + kChunkRows - 1) / kChunkRows;
     const int64_t perRank8 = stride * 8;
-    // six 8-byte tables, two 4-byte tables, then the per-rank words
-    const int64_t bytes = world * (6 * perRank8 + 2 * stride * 4 + stride) + world * 8 + world * groups * 8 + 256;
-    if (!st->tables.Reserve(static_cast<size_t>(bytes), true)) {
+    // six 8-byte tables and the per-rank words; two 4-byte tables, the chunks' totals and a table of bytes
+    if (!st->tables.Reserve(static_cast<size_t>(world * (6 * perRank8 + 8)), true) ||
+        !st->plainTables.Reserve(static_cast<size_t>(world * (2 * stride * 4 + groups * 8 + stride)), true)) {
         return false;
     }
     char *p = static_cast<char *>(st->tables.ptr);
@@ -172,6 +174,7 @@ bool PrepareTables(WorldState *st, int world, int64_t nvS, int64_t n, WorldTable
     out->slotDup = reinterpret_cast<uint64_t *>(take(world * perRank8));
     out->slotGroup = reinterpret_cast<uint64_t *>(take(world * perRank8));
     out->fail = reinterpret_cast<uint64_t *>(take(world * 8));
+    p = static_cast<char *>(st->plainTables.ptr);
     out->sibling = reinterpret_cast<uint32_t *>(take(world * stride * 4));
     out->slotCount = reinterpret_cast<int32_t *>(take(world * stride * 4));
     out->chunkTotals = reinterpret_cast<int32_t *>(take(world * groups * 8));
@@ -424,6 +427,7 @@ void ReleaseWorldState(WorldState *st)
         return;
     }
     st->tables.Release();
+    st->plainTables.Release();
     for (RankEvents &e : st->events) {
         if (e.arrived != nullptr) {
             (void)hipEventDestroy(e.arrived);

@@ -39,7 +39,8 @@ struct RankEvents {
 
 struct WorldState {
     uint64_t epochCounter = 0;
-    TileXREp::DeviceBuffer tables;
+    TileXREp::DeviceBuffer tables;      // nothing but words that carry their epoch
+    TileXREp::DeviceBuffer plainTables; // the tables of other words
     std::vector<StageCall> dispatch;    // calls waiting for the rest of the world, by rank
     std::vector<StageCall> combine;
     std::vector<RankEvents> events;
