@@ -271,8 +271,8 @@ inline int LanesPerRow(int64_t rowBytes)
 // logical world moves is small, and a launch costs as much as the rows: hence one launch for all ranks, and (PLANNED =
 // false) no launch ahead that adds up the segments -- every workgroup does so for itself, two loads and a scan in LDS,
 // in less time than a launch takes to begin.  With the sends, the returns and the reduces put together the same way a
-// dispatch and a combine of 4 ranks with 128 x 1024 and 2 routes take 136 us (a plan and a copy launch per rank with a
-// workgroup per row: 203 us), of 8 ranks with 1000 x 4096 and 8 routes 721 us (898 us).
+// dispatch and a combine of 4 ranks with 128 x 1024 and 2 routes take 143 to 156 us (a plan and a copy launch per rank with a
+// workgroup per row: 203 us), of 8 ranks with 1000 x 4096 and 8 routes 760 us (898 us).
 template <bool PLANNED, int G>
 __global__ __launch_bounds__(kThreads) void ep_drain_rows_kernel(DrainArgs a)
 {
