@@ -53,6 +53,27 @@ def test_calls_on_changing_streams():
             check(x, ids, weights, got, out)
 
 
+def test_eager_calls_on_two_streams_run_one_after_the_other():
+    x, ids, weights = inputs(9)
+    other = inputs(10)
+    first, second = torch.cuda.Stream(), torch.cuda.Stream()
+    with layer.MoeEpLayer(E, K, H) as moe:
+        moe.dispatch(x, ids, capacity=8)            # scratch of this size
+        torch.cuda.synchronize()
+        reached = torch.cuda.Event()
+        with torch.cuda.stream(first):
+            torch.cuda._sleep(50_000_000)
+            a = moe.dispatch(x, ids, capacity=8)
+            reached.record()
+        with torch.cuda.stream(second):
+            b = moe.dispatch(*other[:2], capacity=8)
+        second.synchronize()
+        assert reached.query()                      # the first call, behind some 20 ms of sleep, has run
+        for d, given in ((a, ids), (b, other[1])):
+            want = torch.bincount(given.flatten().long(), minlength=E).clamp(max=8)
+            assert torch.equal(d.token_nums, want)
+
+
 def test_captured_call_replays():
     x, ids, weights = inputs(11)
     other = inputs(12)
