@@ -370,6 +370,14 @@ int RunCombineSingle(EpComm *comm, const EpCombineParams &p, bool memoryRoute, i
             return TileXR::TILEXR_ERROR_INTERNAL;
         }
         inv.inverse = static_cast<uint64_t *>(comm->combineScratch.ptr);
+        // A slot's word holds for the call that wrote it, told by the epoch.  Replays of a graph share the epoch of the
+        // captured call: a slot that has no row this time would keep that of an earlier replay.
+        if (IsCapturing(stream)) {
+            const int cleared = LaunchStatus(LaunchClearInverse(inv), "clear of the inverse table");
+            if (cleared != kOk) {
+                return cleared;
+            }
+        }
         const int ret = Timed(comm, kKernelInvert, stream, "invert", [&] { return LaunchInvert(inv); });
         if (ret != kOk) {
             return ret;

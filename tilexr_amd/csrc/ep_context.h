@@ -39,6 +39,13 @@ inline hipStream_t StreamOf(aclrtStream stream)
     return stream == static_cast<void *>(hipStreamLegacy) ? nullptr : static_cast<hipStream_t>(stream);
 }
 
+// Whether what a call enqueues is recorded into a graph.  (The default stream cannot be.)
+inline bool IsCapturing(hipStream_t stream)
+{
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    return stream != nullptr && hipStreamIsCapturing(stream, &status) == hipSuccess && status == hipStreamCaptureStatusActive;
+}
+
 // Grow-only device buffer.  Growing frees the old block (which synchronises the device) and allocates a new one.
 struct DeviceBuffer {
     void *ptr = nullptr;

@@ -274,6 +274,8 @@ hipError_t LaunchScatter(const ScatterLaunch &l);
 // what RouteCountLaunch::warmRows is for.
 bool ScatterCopiesPerRoute(const void *x, const void *out, int64_t bs, int64_t h, int64_t topK, int quantMode);
 hipError_t LaunchInvert(const InvertLaunch &l);
+// Empties the table that LaunchInvert fills, ahead of it: for calls that are captured, whose replays share one epoch.
+hipError_t LaunchClearInverse(const InvertLaunch &l);
 hipError_t LaunchReduce(const ReduceLaunch &l);
 // The reduces of several logical ranks of one shape (16-bit rows, at most 16 ranks) as one launch on ls[0].stream.
 bool ReduceWorldFits(const ReduceLaunch *ls, int ranks);
