@@ -130,6 +130,7 @@ bool DeviceBuffer::Reserve(size_t want, bool)
     return true;
 }
 void DeviceBuffer::Release() {}
+hipError_t LaunchClearTagged(uint64_t *, int64_t, hipStream_t) { return hipErrorUnknown; }
 EpComm *LookupComm(TileXRCommPtr comm) { return static_cast<EpComm *>(comm); }
 
 } // namespace TileXREp
@@ -169,6 +170,11 @@ hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned)
     return hipSuccess;
 }
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus *status)
+{
+    *status = hipStreamCaptureStatusNone;
+    return hipSuccess;
+}
 hipError_t hipDeviceSynchronize() { return hipSuccess; }
 hipError_t hipMemset(void *, int, size_t) { return hipSuccess; }
 const char *hipGetErrorString(hipError_t) { return "failure"; }

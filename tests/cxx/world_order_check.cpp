@@ -240,6 +240,7 @@ hipError_t LaunchReduceWorld(const ReduceLaunch *ls, int ranks)
     }
     return SecondHalf(ls[0].stream, "reduce");
 }
+hipError_t LaunchClearTagged(uint64_t *, int64_t, hipStream_t) { return hipErrorUnknown; }
 // launches these calls do not make
 hipError_t LaunchReduce(const ReduceLaunch &) { return hipErrorUnknown; }
 hipError_t LaunchAugment(const AugmentLaunch &) { return hipErrorUnknown; }
@@ -271,6 +272,11 @@ hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned)
 {
     const std::set<int> &reached = gEvents[reinterpret_cast<size_t>(e) - 1];
     Tail(s).insert(reached.begin(), reached.end());
+    return hipSuccess;
+}
+hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus *status)
+{
+    *status = hipStreamCaptureStatusNone;
     return hipSuccess;
 }
 const char *hipGetErrorString(hipError_t) { return "failure asked for"; }

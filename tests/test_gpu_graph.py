@@ -10,7 +10,7 @@ import pytest
 import torch
 
 from gpu_harness import DEV, Session
-from tilexr_amd import ep, workloads
+from tilexr_amd import ep, moonep as mp, workloads
 
 pytestmark = pytest.mark.gpu
 
@@ -132,3 +132,99 @@ def test_replays_without_a_row_map_forget_the_rows_of_the_replay_before(memory):
             torch.cuda.synchronize()
             for g, t in zip(got, layers):
                 assert torch.equal(g, t["y"])
+
+
+def test_replays_of_a_logical_world_forget_the_rows_of_the_replay_before():
+    """Two ranks on one captured stream (their eager calls are made on another one)."""
+    R, bs, h, K, E = 2, 60, 64, 2, 8
+    gen = torch.Generator(device=DEV).manual_seed(4)
+    new = lambda *shape, dtype=torch.int32: torch.empty(shape, dtype=dtype, device=DEV)
+    ranks = [dict(x=new(bs, h, dtype=torch.bfloat16), ids=new(bs, K), rows=new(R * bs * K, h, dtype=torch.bfloat16),
+                  assist=new(R * bs * K, 4), nums=new(E // R, dtype=torch.int64), counts=new(E), y=new(bs, h, dtype=torch.bfloat16))
+             for _ in range(R)]
+
+    def load():
+        for t in ranks:
+            t["x"].copy_(torch.randn(bs, h, device=DEV, generator=gen))
+            ids = torch.randint(0, E, (bs, K), device=DEV, generator=gen, dtype=torch.int32)
+            t["ids"].copy_(torch.where(torch.rand(bs, K, device=DEV, generator=gen) < 0.5, -1, ids))
+            t["y"].fill_(7)
+        torch.cuda.synchronize()
+
+    def step(comms, stream):
+        for c, t in zip(comms, ranks):
+            assert ep.dispatch_memory(t["x"], t["ids"], c, bs, h, K, E, t["rows"], t["nums"], t["counts"], t["assist"], ep.DT_BF16,
+                                      stream) == 0
+        for c, t in zip(comms, ranks):
+            assert ep.combine_memory(t["rows"], t["assist"], t["counts"], c, bs, h, K, E, t["y"], ep.DT_BF16, stream) == 0
+
+    torch.cuda.set_device(0)
+    captured, eager = [ep.Comm(R, r) for r in range(R)], [ep.Comm(R, r) for r in range(R)]
+    first, stream = torch.cuda.Stream(), torch.cuda.Stream()
+    load()
+    step(captured, first)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        step(captured, stream)
+    for _ in range(4):
+        load()
+        graph.replay()
+        torch.cuda.synchronize()
+        got = [t["y"].clone() for t in ranks]
+        step(eager, first)
+        torch.cuda.synchronize()
+        for g, t in zip(got, ranks):
+            assert torch.equal(g, t["y"])
+    for c in captured + eager:
+        c.destroy()
+
+
+def test_replays_of_plan_driven_stages_follow_the_plan_as_it_stands():
+    """One rank; the plan's words are rewritten between the replays, so that other rows are named, and rows that no route
+    names any more come out as zeros.  The expected outputs are torch's."""
+    S, K, H, NVS = 64, 4, 64, 400
+    gen = torch.Generator().manual_seed(5)
+    comm = ep.Comm(1, 0)
+    first, stream = torch.cuda.Stream(), torch.cuda.Stream()
+    dst, dst_local = torch.zeros(S * K, dtype=torch.int32, device=DEV), torch.zeros(NVS, dtype=torch.int32, device=DEV)
+    groups, loffs = torch.zeros((NVS, 3), dtype=torch.int32, device=DEV), torch.zeros(NVS, dtype=torch.int32, device=DEV)
+    counts, status = torch.zeros(2, dtype=torch.int32, device=DEV), torch.zeros(4, dtype=torch.int32, device=DEV)
+    x, rows = torch.zeros((S, H), dtype=torch.bfloat16, device=DEV), torch.zeros((NVS, H), dtype=torch.bfloat16, device=DEV)
+    y = torch.zeros((S, H), dtype=torch.bfloat16, device=DEV)
+    plan = mp.plan(S * K, 1, K, 1, NVS, K, dst, groups, loffs, counts, status)
+
+    def load():
+        at = torch.randperm(NVS, generator=gen)[:S * K].to(torch.int32)
+        words = at.clone().view(S, K)
+        words[:, 1:] = -words[:, 1:] - 1            # the later routes of a token are duplicates
+        dst.copy_(words.flatten().to(DEV))
+        back = torch.full((NVS,), -1, dtype=torch.int32)
+        back[at.long()] = torch.arange(S * K, dtype=torch.int32)
+        dst_local.copy_(back.to(DEV))
+        x.copy_(torch.randn(S, H, generator=gen).to(DEV))
+        for t in (rows, y):
+            t.fill_(7)
+        torch.cuda.synchronize()
+        return at.long().to(DEV)
+
+    def step(on):
+        tensors = [mp.tensor(t, mp.DT_BF16, tuple(t.shape)) for t in (x, rows, y)]
+        assert mp.dispatch_v1(comm, plan, tensors[0], tensors[1], on, flags=mp.FLAG_BUILD_DEDUP) == 0
+        assert mp.combine_v1(comm, plan, dst_local, tensors[1], tensors[2], on) == 0
+
+    load()
+    step(first)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        step(stream)
+    for _ in range(4):
+        at = load()
+        graph.replay()
+        torch.cuda.synchronize()
+        want = torch.zeros_like(rows)
+        want[at] = x.repeat_interleave(K, dim=0)
+        assert torch.equal(rows, want)
+        assert torch.equal(y, (K * x.float()).to(torch.bfloat16))      # K equal rows: a power of two times the row
+    comm.destroy()

@@ -373,7 +373,7 @@ int RunCombineSingle(EpComm *comm, const EpCombineParams &p, bool memoryRoute, i
         // A slot's word holds for the call that wrote it, told by the epoch.  Replays of a graph share the epoch of the
         // captured call: a slot that has no row this time would keep that of an earlier replay.
         if (IsCapturing(stream)) {
-            const int cleared = LaunchStatus(LaunchClearInverse(inv), "clear of the inverse table");
+            const int cleared = LaunchStatus(LaunchClearTagged(inv.inverse, n, stream), "clear of the inverse table");
             if (cleared != kOk) {
                 return cleared;
             }

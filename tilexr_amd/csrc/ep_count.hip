@@ -307,12 +307,12 @@ struct InvertArgs {
     uint64_t *inverse;
 };
 
-// Eight bytes a lane, as the slots are read and written: 262 KB for 32 768 routes, in a graph only (LaunchClearInverse).
-__global__ __launch_bounds__(kThreads) void ep_clear_inverse_kernel(uint64_t *inverse, int64_t words)
+// Eight bytes a lane: 262 KB for the slots of 32 768 routes, in graphs only (LaunchClearTagged).
+__global__ __launch_bounds__(kThreads) void ep_clear_tagged_kernel(uint64_t *words, int64_t count)
 {
     const int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
-    if (i < words) {
-        inverse[i] = 0;
+    if (i < count) {
+        words[i] = 0;
     }
 }
 
@@ -446,11 +446,10 @@ hipError_t LaunchRoutePlace(const RoutePlaceLaunch &l)
     return hipGetLastError();
 }
 
-hipError_t LaunchClearInverse(const InvertLaunch &l)
+hipError_t LaunchClearTagged(uint64_t *words, int64_t count, hipStream_t stream)
 {
-    const int64_t words = l.bs * l.topK;
-    hipLaunchKernelGGL(ep_clear_inverse_kernel, dim3(static_cast<unsigned>((words + kThreads - 1) / kThreads)), dim3(kThreads), 0,
-        l.stream, l.inverse, words);
+    hipLaunchKernelGGL(ep_clear_tagged_kernel, dim3(static_cast<unsigned>((count + kThreads - 1) / kThreads)), dim3(kThreads), 0,
+        stream, words, count);
     return hipGetLastError();
 }
 

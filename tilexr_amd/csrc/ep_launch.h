@@ -274,8 +274,9 @@ hipError_t LaunchScatter(const ScatterLaunch &l);
 // what RouteCountLaunch::warmRows is for.
 bool ScatterCopiesPerRoute(const void *x, const void *out, int64_t bs, int64_t h, int64_t topK, int quantMode);
 hipError_t LaunchInvert(const InvertLaunch &l);
-// Empties the table that LaunchInvert fills, ahead of it: for calls that are captured, whose replays share one epoch.
-hipError_t LaunchClearInverse(const InvertLaunch &l);
+// Empties a table of tagged words.  Such a table is otherwise never cleared: a word holds for the call whose epoch it
+// carries.  For calls that are captured, since replays share the epoch of the captured call.
+hipError_t LaunchClearTagged(uint64_t *words, int64_t count, hipStream_t stream);
 hipError_t LaunchReduce(const ReduceLaunch &l);
 // The reduces of several logical ranks of one shape (16-bit rows, at most 16 ranks) as one launch on ls[0].stream.
 bool ReduceWorldFits(const ReduceLaunch *ls, int ranks);

@@ -16,6 +16,7 @@
 #include <hip/hip_runtime_api.h>
 
 #include "ep_context.h"
+#include "ep_launch.h"
 #include "ep_run_common.h"
 #include "moonep_host.h"
 #include "moonep_stage.h"
@@ -157,7 +158,8 @@ bool PrepareTables(WorldState *st, int world, int64_t nvS, int64_t n, WorldTable
     const int64_t groups = (rows + kChunkRows - 1) / kChunkRows;
     const int64_t perRank8 = stride * 8;
     // six 8-byte tables and the per-rank words; two 4-byte tables, the chunks' totals and a table of bytes
-    if (!st->tables.Reserve(static_cast<size_t>(world * (6 * perRank8 + 8)), true) ||
+    st->taggedWords = world * (6 * stride + 1);
+    if (!st->tables.Reserve(static_cast<size_t>(st->taggedWords * 8), true) ||
         !st->plainTables.Reserve(static_cast<size_t>(world * (2 * stride * 4 + groups * 8 + stride)), true)) {
         return false;
     }
@@ -249,6 +251,10 @@ int BeginExchange(EpWorld *world, WorldState *st, const std::vector<StageCall> &
     }
     if (st->doneArmed) {
         MOON_TRY(hipStreamWaitEvent(*stream, st->done, 0), "waiting for the previous exchange");
+    }
+    if (TileXREp::IsCapturing(*stream)) {
+        // replays share this exchange's epoch: each begins with tables that hold nothing of the one before
+        MOON_TRY(TileXREp::LaunchClearTagged(static_cast<uint64_t *>(st->tables.ptr), st->taggedWords, *stream), "clearing the tables");
     }
     return kOk;
 }

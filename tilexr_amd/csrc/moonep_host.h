@@ -40,6 +40,7 @@ struct RankEvents {
 struct WorldState {
     uint64_t epochCounter = 0;
     TileXREp::DeviceBuffer tables;      // nothing but words that carry their epoch
+    int64_t taggedWords = 0;            // how many of them the tables of the last shape have
     TileXREp::DeviceBuffer plainTables; // the tables of other words
     std::vector<StageCall> dispatch;    // calls waiting for the rest of the world, by rank
     std::vector<StageCall> combine;

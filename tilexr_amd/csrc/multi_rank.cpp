@@ -612,6 +612,10 @@ int RunCombineMulti(EpComm *comm, const EpCombineParams &p, bool memoryRoute, in
             }
         }
     }
+    if (status == kOk && IsCapturing(stream)) {
+        // replays share this exchange's epoch: each finds the tables empty
+        status = LaunchStatus(LaunchClearTagged(back.meta, R * metaStride, stream), "clear of the slot tables");
+    }
     if (!ReleaseStreams(&world->combineOrder, world->pendingCombine, stream) && status == kOk) {
         status = TileXR::TILEXR_ERROR_INTERNAL;
     }
