@@ -114,12 +114,27 @@ int RunDispatchSingle(EpComm *comm, const EpDispatchParams &p, bool memoryRoute,
     // (ep_rows.hip; the MVP route without a mask has no key and its own launch there); otherwise count (ticket, last
     // workgroup scans) and place, the latter folded into the scatter unless something needs the rows ahead of it.
     const bool rowsAhead = p.tileFlagsOut != nullptr || p.metaReadyEvent != nullptr;
+    ScatterLaunch scatter {};
+    scatter.x = p.x;
+    scatter.bs = p.bs;
+    scatter.h = p.h;
+    scatter.topK = p.topK;
+    scatter.quantMode = static_cast<int>(p.quantMode);
+    scatter.out = p.expandXOut;
+    scatter.tileFlags = p.tileFlagsOut;
+    scatter.consumerBeside = p.metaReadyEvent != nullptr;
+    // the extended combine takes int8 and block fp8 rows, the reference's combines 16-bit ones only
+    scatter.combineTakesRows = p.quantMode == TILEXR_EP_QUANT_NONE || p.extended;
     // the scatter kernel that copies per route wants the token rows close by: the routing launch reads them ahead
-    const bool warm = ScatterCopiesPerRoute(p.x, p.expandXOut, p.bs, p.h, p.topK, static_cast<int>(p.quantMode));
+    const bool warm = ScatterCopiesPerRoute(scatter);
+    // Launches that read no token rows ahead resolve the rows in one launch further up (RouteRowsPays): dispatch + combine,
+    // count and one launch, 2200 x 7168 x top-8 95.9 -> 91.1 us, 4000 x 4096 101.2 -> 97.5, 8000 x 2560 138.7 -> 128.1.  Copies
+    // of 257 to 319 vectors stay where they were, on the count launch (tests name it for 2056 columns: 71.3 us, 69.5 in one).
+    const bool narrowCopies = p.quantMode == TILEXR_EP_QUANT_NONE && p.h > 2048 && p.h < 2560 && p.topK > 1 && p.bs >= 1024;
     const bool mayOneLaunch = comm->routing != EpComm::Routing::kLegacy;
     const bool oneLaunchRows = mayOneLaunch && memoryRoute &&
         RouteRowsFits(p.expertIds, n, numKeys, maskMode, p.expertCapacity) &&
-        (comm->routing == EpComm::Routing::kOneLaunch || RouteRowsPays(n, numKeys, rowsAhead, warm));
+        (comm->routing == EpComm::Routing::kOneLaunch || RouteRowsPays(n, numKeys, rowsAhead, warm || narrowCopies));
     const bool oneLaunchCompact = mayOneLaunch && !memoryRoute && p.expertCapacity <= 0 &&
         RouteCompactFits(p.expertIds, n, experts, maskMode) &&
         (comm->routing == EpComm::Routing::kOneLaunch || RouteCompactPays(n, experts));
@@ -260,23 +275,14 @@ int RunDispatchSingle(EpComm *comm, const EpDispatchParams &p, bool memoryRoute,
         }
     }
 
-    ScatterLaunch scatter {};
-    scatter.x = p.x;
     scatter.rowOf = rowOf;
     scatter.fusedPlace = (oneLaunch || separatePlace) ? nullptr : &place;
-    scatter.bs = p.bs;
-    scatter.h = p.h;
-    scatter.topK = p.topK;
-    scatter.quantMode = static_cast<int>(p.quantMode);
     // the MVP route's quantisers decode the input as fp16 whatever the caller's tensor holds
     // (reference: tilexr_ep_dispatch_helpers.h:121,167)
     scatter.inputBf16 = memoryRoute && p.dtype == TileXR::TILEXR_DATA_TYPE_BFP16;
     scatter.fp8E5m2 = p.expandXOutDtype == TileXR::TILEXR_DATA_TYPE_FP8E5M2;
     scatter.staticScale = static_cast<const float *>(p.scales);
-    scatter.out = p.expandXOut;
     scatter.scalesOut = p.dynamicScalesOut;
-    scatter.tileFlags = p.tileFlagsOut;
-    scatter.consumerBeside = p.metaReadyEvent != nullptr;
     // a tile never holds more rows than the dispatch can produce: larger values name the same single tile
     scatter.tileRows = std::min<int64_t>(p.tileRows, std::max<int64_t>(n, 1));
     scatter.epoch = flagEpoch;

@@ -54,6 +54,9 @@ constexpr int kAuxAgentScopeKept = 16;      // sc1 alone: for small tables a lat
                                             // the same table afterwards ran 10 us slower: 92 instead of 82 us)
 constexpr unsigned kRawBufferWord3 = 0x00020000u;
 
+// The cache between the L2s and memory, one for the device.
+constexpr int64_t kMemorySideCacheBytes = int64_t{256} << 20;
+
 // Workgroup b of a launch runs on XCD b % kXcdCount.  Units (token x part) placed by XCD: unit u belongs to token
 // (u / 8 / parts) * 8 + u % 8, part (u / 8) % parts, so that all parts of a token run on XCD token % 8; the tokens are
 // padded to a multiple of eight.

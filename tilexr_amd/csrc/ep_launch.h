@@ -167,6 +167,7 @@ struct ScatterLaunch {
     const int32_t *totalRowsPtr; // device word: rows kept by this dispatch (size of the last tile)
     bool consumerBeside;         // a consumer of the flags is expected to run beside this launch (the caller asked for a
                                  // metadata-ready event): keep the workgroups small enough to fit next to its waiting ones
+    bool combineTakesRows;       // what is written is read next by this library as it is: left in the memory-side cache
     const char **kernelNameOut;  // optional: receives the name of the kernel template that was launched
     hipStream_t stream;
 };
@@ -270,8 +271,10 @@ hipError_t LaunchRouteCount(const RouteCountLaunch &l);
 hipError_t LaunchRoutePlace(const RoutePlaceLaunch &l);
 hipError_t LaunchScatter(const ScatterLaunch &l);
 // Whether LaunchScatter copies rows with one workgroup per (route, slice), each reading its own copy of the token row
-// (plain payload, wide rows, 1024 tokens and more).  That kernel is the one that needs the token rows close by: it is
-// what RouteCountLaunch::warmRows is for.
+// (plain payload, wide rows, more of them than the memory-side cache holds).  That kernel is the one that needs the token
+// rows close by: it is what RouteCountLaunch::warmRows is for.  Looks at x, out, the sizes, tileFlags and consumerBeside;
+// the second form stands for a launch without the last two.
+bool ScatterCopiesPerRoute(const ScatterLaunch &l);
 bool ScatterCopiesPerRoute(const void *x, const void *out, int64_t bs, int64_t h, int64_t topK, int quantMode);
 hipError_t LaunchInvert(const InvertLaunch &l);
 // Empties a table of tagged words.  Such a table is otherwise never cleared: a word holds for the call whose epoch it

@@ -1,7 +1,7 @@
 // scatter: each token row is read once and written to the rows its routes were placed at (gfx950, wave64).
 //
 // HBM-bound byte movement, no MFMA.  Three kernels share the work:
-//   ep_scatter_route_kernel    plain copies of wide rows in batches of 1024 tokens and more: one workgroup per
+//   ep_scatter_route_kernel    plain copies of wide rows that the memory-side cache cannot hold: one workgroup per
 //                              (token, k, slice of 512 vectors; 1024 when readiness flags are published), two 16-byte
 //                              loads and two 16-byte stores per lane
 //   ep_scatter_vec_kernel      everything else that is 16-byte aligned (quantised payloads, narrow rows, small
@@ -9,9 +9,7 @@
 //                              for wide ones); a lane keeps V 16-byte vectors of the row in registers, so every load of
 //                              the row is in flight before the first store, then writes them to each destination row
 //   ep_scatter_generic_kernel  any width and alignment, element by element
-// Rows are written with non-temporal stores (they are not read again by this kernel; the input row is loaded with the
-// default policy so that the sibling workgroups of a token find it in L2), or with agent-scope write-through stores
-// when readiness flags are published.  Destination order (sorted or random rows) makes no difference.
+// How rows are stored decides where the next kernel finds them: see RowStores.
 //
 //   QMODE 0  byte copy             (reference: src/ep/kernels/tilexr_ep_dispatch_helpers.h:104-112)
 //   QMODE 1  static int8           (reference: tilexr_ep_dispatch_helpers.h:114-136)
@@ -71,26 +69,37 @@ __device__ __forceinline__ float GroupMax(float v, float *red, int lane)
     return v;
 }
 
-// Row stores of the register-resident kernels.  WT = false: non-temporal stores (the rows are not read again by this
-// kernel).  WT = true: agent-scope write-through stores, used when readiness flags are published: such a store is
-// complete for every XCD once the issuing wave's vmcnt is zero, so publishing needs no L2 write-back.
-template <bool WT>
+// Row stores of the register-resident kernels.  A streaming store goes past the L2 and past the 256 MiB memory-side cache:
+// whoever reads the row next (an expert stage, combine) fetches it from memory, row by row at unrelated places.  One that
+// is written through without the streaming hint leaves the row in that cache, and it is the cheaper store as well, since
+// what the cache takes need not reach memory within the launch.  Dispatch + combine, us, streaming and kept, six sets of
+// buffers in turn: 1000 x 7168 x top-8 52.4 -> 45.3, 600 tokens 34.9 -> 31.1, 3000 x 2048 48.3 -> 41.3; int8 8192 x 4096 x
+// top-6 108.4 -> 100.2 (its scatter 49.9 -> 42.5), 4096 x 7168 x top-8 127.0 -> 109.0; block fp8 16384 x 2048 under a
+// capacity 98.4 -> 92.0 (scatter 48.9 -> 39.0, reduce 40.7 -> 44.4: it waits for rows that leave the cache).  Ordinary
+// stores (dirty in the L2 until the launch ends) come in between: 46.0, 101.8, 93.1 for three of those.
+enum class RowStores {
+    kStream,        // non-temporal
+    kKeep,          // written through (sc1) and kept
+    kPublish,       // written through and streaming (sc1 nt)
+};
+
+template <RowStores S>
 __device__ __forceinline__ void RowStore(const u32x4 &v, char *rowBase, __amdgpu_buffer_rsrc_t rsrc, int byteOffset)
 {
-    if (WT) {
-        __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, byteOffset, 0, kAuxAgentScope);
-    } else {
+    if (S == RowStores::kStream) {
         __builtin_nontemporal_store(v, reinterpret_cast<u32x4 *>(rowBase + byteOffset));
+    } else {
+        __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, byteOffset, 0, S == RowStores::kKeep ? kAuxAgentScopeKept : kAuxAgentScope);
     }
 }
 
-template <bool WT>
+template <RowStores S>
 __device__ __forceinline__ void RowStore(const u32x2 &v, char *rowBase, __amdgpu_buffer_rsrc_t rsrc, int byteOffset)
 {
-    if (WT) {
-        __builtin_amdgcn_raw_buffer_store_b64(v, rsrc, byteOffset, 0, kAuxAgentScope);
-    } else {
+    if (S == RowStores::kStream) {
         __builtin_nontemporal_store(v, reinterpret_cast<u32x2 *>(rowBase + byteOffset));
+    } else {
+        __builtin_amdgcn_raw_buffer_store_b64(v, rsrc, byteOffset, 0, S == RowStores::kKeep ? kAuxAgentScopeKept : kAuxAgentScope);
     }
 }
 
@@ -118,7 +127,7 @@ __device__ __forceinline__ void PublishRow(const ScatterArgs &a, int row, int pa
 }
 
 // Publishes the rows of one token.  Each wave waits for its own stores and the barrier collects the waves.
-// WT = true: the rows were written through and are then complete.  WT = false: the rows may still sit dirty in this
+// WT = true: the rows were written through (kKeep, kPublish) and are then complete for every XCD, with no L2 write-back.  WT = false: the rows may still sit dirty in this
 // XCD's L2 and one release fence per publishing wave writes them back (slow under load; element-granular fallback only).
 template <bool WT>
 __device__ __forceinline__ void PublishRows(const ScatterArgs &a, const int *pos, int lane, int G)
@@ -146,7 +155,8 @@ __device__ __forceinline__ void PublishRows(const ScatterArgs &a, const int *pos
 // XCD's L2 the other topK - 1 times.  Two 16-byte loads then two 16-byte stores per lane is what this memory system
 // rewards, whatever the workgroup size: measured on 4096 x 7168 x top-8, 83-85 us with two vectors per lane (128 to
 // 448 lanes per workgroup), 92-95 us with three to fourteen, 105-130 us with one; 93 us for "one workgroup writes all
-// topK rows", and 132 us when the workgroups of a token are spread over the XCDs.
+// topK rows", and 132 us when the workgroups of a token are spread over the XCDs.  The rows must stream: kept ones push the
+// token rows out of the L2s (dispatch + combine 182 us, 234 us with kKeep).
 constexpr int kRouteVecs = 2;
 constexpr unsigned kRouteCapLdsBytes = 27 * 1024;    // 160 KiB of LDS per compute unit: five workgroups fit
 template <int THREADS, int V, bool WT>
@@ -187,7 +197,7 @@ __global__ __launch_bounds__(THREADS) void ep_scatter_route_kernel(ScatterArgs a
     for (int i = 0; i < V; ++i) {
         const int idx = colBase + i * THREADS + lane;
         if (idx < vecs) {
-            RowStore<WT>(v[i], dst, rsrc, idx * 16);
+            RowStore<WT ? RowStores::kPublish : RowStores::kStream>(v[i], dst, rsrc, idx * 16);
         }
     }
     if (WT && a.tileFlags != nullptr) {
@@ -328,7 +338,7 @@ __device__ __forceinline__ void QuantiseRow(const ScatterArgs &a, const u32x4 (&
 }
 
 // Writes the row (or its payload and scales) held by the group's lanes to row `row` of the outputs.
-template <int G, int V, int QMODE, bool WT>
+template <int G, int V, int QMODE, RowStores S, bool WT>
 __device__ __forceinline__ void StoreRow(const ScatterArgs &a, int row, const u32x4 (&v)[V], const QuantisedRow<V> &out, int lane)
 {
     const int vecs = a.h / 8;
@@ -339,7 +349,7 @@ __device__ __forceinline__ void StoreRow(const ScatterArgs &a, int row, const u3
         for (int j = 0; j < V; ++j) {
             const int idx = j * G + lane;
             if (idx < vecs) {
-                RowStore<WT>(v[j], dst, rsrc, idx * 16);
+                RowStore<S>(v[j], dst, rsrc, idx * 16);
             }
         }
         return;
@@ -353,7 +363,7 @@ __device__ __forceinline__ void StoreRow(const ScatterArgs &a, int row, const u3
     for (int j = 0; j < V; ++j) {
         const int idx = j * G + lane;
         if (idx < vecs) {
-            RowStore<WT>(out.q[j], dst, rsrc, idx * 8);
+            RowStore<S>(out.q[j], dst, rsrc, idx * 8);
             if (QMODE == TILEXR_EP_QUANT_MXFP8 && (idx & 3) == 0) {
                 uint8_t *sc = static_cast<uint8_t *>(a.scalesOut) + static_cast<int64_t>(row) * mxScales;
                 ScalarStore<WT>(sc + (idx >> 2), static_cast<uint8_t>(out.sharedExp[j] + 127));
@@ -373,7 +383,7 @@ __device__ __forceinline__ void StoreRow(const ScatterArgs &a, int row, const u3
 }
 
 // Publishing launches: one token per group, because a group stays until its own stores have landed.
-template <int G, int V, int QMODE, bool BF16, bool E5M2>
+template <int G, int V, int QMODE, bool BF16, bool E5M2, RowStores S>
 __device__ __forceinline__ void ScatterAndPublish(const ScatterArgs &a)
 {
     constexpr int kTokens = kThreads / G;
@@ -406,7 +416,7 @@ __device__ __forceinline__ void ScatterAndPublish(const ScatterArgs &a)
         // the lanes of a wave share one token, so the row is wave-uniform
         const int row = __builtin_amdgcn_readfirstlane(s_pos[tg][k]);
         if (row >= 0) {
-            StoreRow<G, V, QMODE, true>(a, row, v, out, lane);
+            StoreRow<G, V, QMODE, S, true>(a, row, v, out, lane);
         }
     }
     if (a.tileFlags != nullptr) {
@@ -417,9 +427,11 @@ __device__ __forceinline__ void ScatterAndPublish(const ScatterArgs &a)
 // Everything else.  Nothing is shared between the waves of a group but the int8 maximum: lane k of every wave works out the
 // row of route (token, k) for itself, so no wave waits at a barrier between its loads and its stores (16384 x 7168 bf16
 // x top-8 from HBM: 400 us = 5.3 TB/s, 426 us with the rows handed round through LDS).  Bound by memory: with token rows
-// that come from HBM the reads and the writes share it, and no kernel of this mix was measured above 5.4 TB/s here (all
-// cache policies of the loads and stores, one to four tokens in flight per group, a token read ahead of the stores).
-template <int G, int V, int QMODE, bool BF16, bool E5M2>
+// that come from HBM the reads and the writes share it.  (One to four tokens in flight per group, a token read ahead of the
+// stores, and quantised rows stored sixteen bytes a lane instead of eight made no difference; the token rows read once by
+// the routing launch, as for the per-route kernel, cost int8 8192 x 4096 as much as they saved while rows streamed, 108.4
+// and 109.0 us, and more since they are kept, 99.8 and 106.9: the read-ahead and the routing want the same memory.)
+template <int G, int V, int QMODE, bool BF16, bool E5M2, RowStores S>
 __device__ __forceinline__ void ScatterOnly(const ScatterArgs &a)
 {
     constexpr int kTokens = kThreads / G;
@@ -452,18 +464,18 @@ __device__ __forceinline__ void ScatterOnly(const ScatterArgs &a)
     for (int k = 0; k < a.topK; ++k) {
         const int rowOfK = __builtin_amdgcn_readlane(row, k);
         if (rowOfK >= 0) {
-            StoreRow<G, V, QMODE, false>(a, rowOfK, v, out, lane);
+            StoreRow<G, V, QMODE, S, false>(a, rowOfK, v, out, lane);
         }
     }
 }
 
-template <int G, int V, int QMODE, bool BF16, bool E5M2, bool WT>
+template <int G, int V, int QMODE, bool BF16, bool E5M2, bool WT, RowStores S>
 __global__ __launch_bounds__(kThreads) void ep_scatter_vec_kernel(ScatterArgs a)
 {
     if constexpr (WT) {
-        ScatterAndPublish<G, V, QMODE, BF16, E5M2>(a);
+        ScatterAndPublish<G, V, QMODE, BF16, E5M2, S>(a);
     } else {
-        ScatterOnly<G, V, QMODE, BF16, E5M2>(a);
+        ScatterOnly<G, V, QMODE, BF16, E5M2, S>(a);
     }
 }
 
@@ -562,26 +574,88 @@ inline bool WriteThrough(const ScatterArgs &a)
     return a.tileFlags != nullptr;
 }
 
-template <int G, int V, int QMODE, bool BF16, bool E5M2>
-void LaunchVec(const ScatterArgs &a, hipStream_t stream)
+// Unused dynamic LDS that holds the scatter kernels to so many workgroups per compute unit (160 KiB of LDS).
+constexpr unsigned CapLdsBytes(int workgroups)
+{
+    return workgroups == 3 ? 53u * 1024u : workgroups == 4 ? 40u * 1024u : workgroups == 5 ? kRouteCapLdsBytes : 0u;
+}
+
+// Workgroups per compute unit that the launch without flags is held to, 0 for as many as fit.  Eight workgroups that each
+// store a wide row topK times oversubscribe the memory system like those of the per-route kernel.
+//   quantised: five.  (8192 x 4096 int8 x top-6, microseconds at eight, six, five, four, three: 53.5, 50.1, 49.4, 49.9,
+//     50.8; 2048 x 7168 MXFP8 27.3, 27.0, 25.9, 25.6, 25.5.)  That takes rows that store enough: dispatch + combine at eight
+//     and at five, int8 or block fp8, 2048 x 7168 top-8 65.7 -> 62.3, 4096 x 7168 top-4 69.3 -> 67.1, 2048 x 8192 top-4 43.4
+//     -> 42.1, 8192 x 4096 top-6 107.9 -> 105.5; but 2048 x 4096 top-2 20.4 and 21.4, 8192 x 2304 top-2 42.3 and 44.6, 16384
+//     x 2304 top-8 181 and 201, 16384 x 3072 top-8 205 and 213, 16384 x 4096 top-5 181 and 187, 2048 x 12288 top-2 46.8 and
+//     48.6.  (Rows a wave holds: no difference.)
+//   copies, dispatch + combine at eight, four and three: 2200 x 7168 x top-8 95.8, 93.6, 91.5; 3000 x 5120 93.1, 92.3, 89.3;
+//     16384 x 7168 769.6, 764.6, 759.7; 16384 x 6144 x top-4 354, 350, 365 (token rows from memory, few stores each); up to
+//     512 vectors 16384 x 4096 x top-8 439, 428, 462; 6000 x 2560 95.9, 92.9, 93.5; 10000 x 2056 160, 167, 188.  1000 tokens
+//     and fewer: no difference.
+template <int G, int QMODE>
+int CapWorkgroups(const ScatterArgs &a)
+{
+    const int vecs = a.h / 8;
+    if (QMODE != TILEXR_EP_QUANT_NONE) {
+        return vecs >= 2 * kThreads && a.topK >= 4 && vecs * a.topK >= 12 * kThreads ? 5 : 0;
+    }
+    if (G < kThreads || vecs < 320) {
+        return 0;
+    }
+    const bool cachedTokens = static_cast<int64_t>(a.bs) * a.h * 2 <= kMemorySideCacheBytes / 2;
+    return vecs > 2 * kThreads && (cachedTokens || a.topK > 4) ? 3 : 4;
+}
+
+// Whether the rows are left in the memory-side cache.  They are where this library's combine can take them as they are; a
+// payload that only an expert stage decodes streams (dispatch + combine of other rows, streaming and kept: MXFP8 2048 x
+// 7168 88.9 and 91.2 us, 4096 x 7168 155 and 168, int8 on the MVP route 4000 x 2048 49.0 and 51.4).  Block fp8 rows beyond
+// twice that cache stream too (16384 x 7168 x top-6 378 and 388, 8192 x 8192 x top-8 274 -> 269), int8 and plain ones are
+// kept at any size (16384 x 7168 x top-8 int8 468.5 -> 466.2, plain 775.5 -> 770.3).  Rows that end within a 128-byte line
+// are two partial lines each and want a launch worth it: 1000 columns, 1501 tokens x top-6 19.1 and 19.6, 4000 x top-6 31.2
+// and 31.4, 4000 x top-8 39.4 -> 37.1.
+template <int QMODE>
+bool KeepsRows(const ScatterArgs &a)
+{
+    const int64_t rowBytes = QMODE == TILEXR_EP_QUANT_NONE ? int64_t{2} * a.h : a.h;
+    const int64_t bytes = static_cast<int64_t>(a.bs) * a.topK * rowBytes;
+    if (QMODE == TILEXR_EP_QUANT_FP8_BLOCK128 && bytes > 2 * kMemorySideCacheBytes) {
+        return false;
+    }
+    return WriteThrough(a) || rowBytes % 128 == 0 || bytes >= (int64_t{32} << 20);
+}
+
+template <int G, int V, int QMODE, bool BF16, bool E5M2, RowStores S>
+void LaunchVecStoring(const ScatterArgs &a, hipStream_t stream)
 {
     constexpr int kTokens = kThreads / G;
-    const int groups = (a.bs + kTokens - 1) / kTokens;
+    const dim3 groups((a.bs + kTokens - 1) / kTokens);
+    if constexpr (S != RowStores::kStream) {
+        if (WriteThrough(a)) {
+            hipLaunchKernelGGL((ep_scatter_vec_kernel<G, V, QMODE, BF16, E5M2, true, S>), groups, dim3(kThreads), 0, stream, a);
+            return;
+        }
+    }
+    if constexpr (S != RowStores::kPublish) {
+        hipLaunchKernelGGL((ep_scatter_vec_kernel<G, V, QMODE, BF16, E5M2, false, S>), groups, dim3(kThreads),
+            CapLdsBytes(CapWorkgroups<G, QMODE>(a)), stream, a);
+    }
+}
+
+template <int G, int V, int QMODE, bool BF16, bool E5M2>
+void LaunchVec(const ScatterLaunch &l, const ScatterArgs &a)
+{
+    constexpr bool kCombineTakes = QMODE == TILEXR_EP_QUANT_NONE || QMODE == TILEXR_EP_QUANT_TOKEN_INT8 ||
+        QMODE == TILEXR_EP_QUANT_FP8_BLOCK128;
+    if constexpr (kCombineTakes) {
+        if (l.combineTakesRows && KeepsRows<QMODE>(a)) {
+            LaunchVecStoring<G, V, QMODE, BF16, E5M2, RowStores::kKeep>(a, l.stream);
+            return;
+        }
+    }
     if (WriteThrough(a)) {
-        hipLaunchKernelGGL((ep_scatter_vec_kernel<G, V, QMODE, BF16, E5M2, true>), dim3(groups), dim3(kThreads), 0, stream, a);
+        LaunchVecStoring<G, V, QMODE, BF16, E5M2, RowStores::kPublish>(a, l.stream);
     } else {
-        // Eight workgroups per compute unit that each quantise a wide row and store it topK times oversubscribe the memory
-        // system like those of the per-route kernel; unused dynamic LDS caps them at five.  (8192 x 4096 int8 x top-6,
-        // microseconds at eight, six, five, four, three: 53.5, 50.1, 49.4, 49.9, 50.8; 2048 x 7168 MXFP8 27.3, 27.0, 25.9,
-        // 25.6, 25.5.  Copies, 16384 x 7168 x top-8: 402, 403, 417, 430, 436.)  That takes rows that store enough: dispatch +
-        // combine at eight and at five, int8 or block fp8, 2048 x 7168 top-8 65.7 -> 62.3, 4096 x 7168 top-4 69.3 -> 67.1,
-        // 2048 x 8192 top-4 43.4 -> 42.1, 8192 x 4096 top-6 107.9 -> 105.5; but 2048 x 4096 top-2 20.4 and 21.4, 8192 x
-        // 2304 top-2 42.3 and 44.6, 16384 x 2304 top-8 181 and 201, 16384 x 3072 top-8 205 and 213, 16384 x 4096 top-5 181
-        // and 187, 2048 x 12288 top-2 46.8 and 48.6.  (Rows a wave holds: no difference.)
-        const int vecs = a.h / 8;
-        const bool capped = QMODE != TILEXR_EP_QUANT_NONE && vecs >= 2 * kThreads && a.topK >= 4 && vecs * a.topK >= 12 * kThreads;
-        const unsigned capLds = capped ? kRouteCapLdsBytes : 0u;
-        hipLaunchKernelGGL((ep_scatter_vec_kernel<G, V, QMODE, BF16, E5M2, false>), dim3(groups), dim3(kThreads), capLds, stream, a);
+        LaunchVecStoring<G, V, QMODE, BF16, E5M2, RowStores::kStream>(a, l.stream);
     }
 }
 
@@ -590,8 +664,7 @@ void LaunchByMode(const ScatterLaunch &l, const ScatterArgs &a)
 {
     switch (l.quantMode) {
         case TILEXR_EP_QUANT_NONE:
-            // small batches are latency-bound and gain nothing from the extra workgroups
-            if (G == kThreads && ScatterCopiesPerRoute(l.x, l.out, l.bs, l.h, l.topK, l.quantMode)) {
+            if (G == kThreads && ScatterCopiesPerRoute(l)) {
                 const dim3 blocks(static_cast<unsigned>(8 * a.colSlices), static_cast<unsigned>(a.topK),
                     static_cast<unsigned>((a.bs + 7) / 8));
                 if (l.kernelNameOut != nullptr) {
@@ -624,39 +697,39 @@ void LaunchByMode(const ScatterLaunch &l, const ScatterArgs &a)
                         l.stream, a);
                 }
             } else {
-                LaunchVec<G, V, TILEXR_EP_QUANT_NONE, true, false>(a, l.stream);
+                LaunchVec<G, V, TILEXR_EP_QUANT_NONE, true, false>(l, a);
             }
             break;
         case TILEXR_EP_QUANT_STATIC_INT8:
-            LaunchVec<G, V, TILEXR_EP_QUANT_STATIC_INT8, false, false>(a, l.stream);
+            LaunchVec<G, V, TILEXR_EP_QUANT_STATIC_INT8, false, false>(l, a);
             break;
         case TILEXR_EP_QUANT_TOKEN_INT8:
             if (l.inputBf16) {
-                LaunchVec<G, V, TILEXR_EP_QUANT_TOKEN_INT8, true, false>(a, l.stream);
+                LaunchVec<G, V, TILEXR_EP_QUANT_TOKEN_INT8, true, false>(l, a);
             } else {
-                LaunchVec<G, V, TILEXR_EP_QUANT_TOKEN_INT8, false, false>(a, l.stream);
+                LaunchVec<G, V, TILEXR_EP_QUANT_TOKEN_INT8, false, false>(l, a);
             }
             break;
         case TILEXR_EP_QUANT_MXFP8:
             if (l.inputBf16) {
                 if (l.fp8E5m2) {
-                    LaunchVec<G, V, TILEXR_EP_QUANT_MXFP8, true, true>(a, l.stream);
+                    LaunchVec<G, V, TILEXR_EP_QUANT_MXFP8, true, true>(l, a);
                 } else {
-                    LaunchVec<G, V, TILEXR_EP_QUANT_MXFP8, true, false>(a, l.stream);
+                    LaunchVec<G, V, TILEXR_EP_QUANT_MXFP8, true, false>(l, a);
                 }
             } else {
                 if (l.fp8E5m2) {
-                    LaunchVec<G, V, TILEXR_EP_QUANT_MXFP8, false, true>(a, l.stream);
+                    LaunchVec<G, V, TILEXR_EP_QUANT_MXFP8, false, true>(l, a);
                 } else {
-                    LaunchVec<G, V, TILEXR_EP_QUANT_MXFP8, false, false>(a, l.stream);
+                    LaunchVec<G, V, TILEXR_EP_QUANT_MXFP8, false, false>(l, a);
                 }
             }
             break;
         default:
             if (l.inputBf16) {
-                LaunchVec<G, V, TILEXR_EP_QUANT_FP8_BLOCK128, true, false>(a, l.stream);
+                LaunchVec<G, V, TILEXR_EP_QUANT_FP8_BLOCK128, true, false>(l, a);
             } else {
-                LaunchVec<G, V, TILEXR_EP_QUANT_FP8_BLOCK128, false, false>(a, l.stream);
+                LaunchVec<G, V, TILEXR_EP_QUANT_FP8_BLOCK128, false, false>(l, a);
             }
             break;
     }
@@ -664,13 +737,36 @@ void LaunchByMode(const ScatterLaunch &l, const ScatterArgs &a)
 
 } // namespace
 
+// The per-route kernel's rows have to stream, the per-token kernel's are kept: dispatch + combine, per route and per token
+// (three or four workgroups to a compute unit), us: 235 MB of rows (2048 x 7168 x top-8) 93.9 and 85.0, 315 MB 128.1 and
+// 122.8, 367 MB 144.8 and 145.4, 470 MB 182.2 and 187.8, 688 MB 273.0 and 274.4; 4096 columns, 328 MB 132.1 and 128.3, 393 MB
+// 155.8 and 157.1, 786 MB 310.7 and 316.2.  So it takes what the memory-side cache cannot hold, and of that what has token
+// rows it can: beyond 104 MiB of them reading them ahead no longer pays (117 MB 379.8 and 375.6, 123 MB 405.6 and 392.4, 134
+// MB 470 and 428); publishing, where the per-token kernel waits for its stores topK at a time, beyond 128 MiB (117 MB 378.4
+// and 379.9, 123 MB 395.3 and 398.0).  Published rows wider than one of its workgroups (1024 vectors) are its own at any size:
+// callers and tests count on their parts being landed one by one (1024 x 12288 x top-4 52.8 us, 46.1 per token).  A consumer
+// that runs beside the launch is given rows as early as before.
+bool ScatterCopiesPerRoute(const ScatterLaunch &l)
+{
+    const int64_t vecs = l.h / 8;
+    const int64_t tokenBytes = l.bs * l.h * 2;
+    const bool publishes = l.tileFlags != nullptr;
+    const bool inParts = publishes && vecs > 4 * kThreads;
+    return l.quantMode == TILEXR_EP_QUANT_NONE && l.h % 8 == 0 && Aligned16(l.x) && Aligned16(l.out) && vecs > 4 * kWave &&
+        vecs <= 8 * kThreads && l.topK > 1 && l.bs >= 1024 && tokenBytes <= (publishes ? int64_t{128} << 20 : int64_t{104} << 20) &&
+        (l.consumerBeside || inParts || tokenBytes * l.topK > (int64_t{320} << 20)) && (l.bs + 7) / 8 <= 65535 && l.topK <= 65535;
+}
+
 bool ScatterCopiesPerRoute(const void *x, const void *out, int64_t bs, int64_t h, int64_t topK, int quantMode)
 {
-    const int64_t vecs = h / 8;
-    // token rows beyond half the memory-side cache (256 MiB) cannot be kept close by: the per-token kernel takes those
-    return quantMode == TILEXR_EP_QUANT_NONE && h % 8 == 0 && Aligned16(x) && Aligned16(out) && vecs > 4 * kWave &&
-        vecs <= 8 * kThreads && topK > 1 && bs >= 1024 && bs * h * 2 <= (int64_t{128} << 20) &&
-        (bs + 7) / 8 <= 65535 && topK <= 65535;
+    ScatterLaunch l {};
+    l.x = x;
+    l.out = const_cast<void *>(out);       // only its alignment is looked at
+    l.bs = bs;
+    l.h = h;
+    l.topK = topK;
+    l.quantMode = quantMode;
+    return ScatterCopiesPerRoute(l);
 }
 
 hipError_t LaunchScatter(const ScatterLaunch &l)
