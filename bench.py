@@ -164,8 +164,8 @@ def parse():
     p.add_argument("--stage-tile-ns", type=int, default=40000,
                    help="expert-stage leg: time the producer spends on a tile at least, in nanoseconds")
     p.add_argument("--moon-cached-row-bytes", type=int, default=None,
-                   help="M1: value for TileXRMoonEpSetCachedRowBytes (0 = always the scatter kernel that tolerates "
-                        "token rows that come from HBM)")
+                   help="M1: value for TileXRMoonEpSetCachedRowBytes (0 = always the scatter kernel that reads every "
+                        "token row once)")
     p.add_argument("--no-ceilings", action="store_true",
                    help="skip the memory-system yardsticks (probe kernels of the library) reported under `ceilings`")
     p.add_argument("--no-rotate-leg", action="store_true",

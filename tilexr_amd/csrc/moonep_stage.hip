@@ -10,6 +10,7 @@
 //                                src/moonep/combine/kernels/tilexr_moonep_combine_kernel.cpp:117-177, 285-366, 449-541,
 //                                568-606, 648-733
 #include <atomic>
+#include <type_traits>
 
 #include <hip/hip_runtime.h>
 
@@ -26,16 +27,21 @@ using TileXREp::kWave;
 
 constexpr int kXcds = 8;
 constexpr int kRowVecs = 2;     // 16-byte vectors per lane per row slice
+constexpr int kTokenVecs = 4 * kThreads;    // 16-byte vectors of a row slice of the per-token scatter
 
-std::atomic<int64_t> gCachedRowBytes {int64_t{256} << 20};     // TileXRMoonEpSetCachedRowBytes
+constexpr int64_t kDefaultCachedRowBytes = int64_t{256} << 20;   // with this setting the library goes by rows and token rows
+std::atomic<int64_t> gCachedRowBytes {kDefaultCachedRowBytes};  // TileXRMoonEpSetCachedRowBytes
 // Unused dynamic LDS of the copying workgroups: five of them fit a compute unit's 160 KiB.  Eight keep more stores in
 // flight than this memory system digests (4096 x 7168 x top-8, microseconds at eight, seven, six, five, four: 83, 79, 74,
 // 73, 81; five hold their time in both directions, built and saved plans).
 constexpr unsigned kScatterCapLdsBytes = 27 * 1024;
+constexpr unsigned kTokenCapLdsBytes = 53 * 1024;       // per-token scatter: three
 constexpr int kFusedPlanChunks = 1024;  // chunks of 2048 rows per rank up to which the scatter launch builds a fresh plan
 constexpr int64_t kFusedPlanRowBytes = int64_t{256} << 20;     // ... and bytes of rows the world's routes write
 constexpr int kSelfPlanChunks = 8;      // ... and up to which its plan workgroups add up the earlier chunks themselves
 constexpr int64_t kWarmRowBytes = int64_t{128} << 20;          // token rows of a world that are read ahead of the per-route scatter
+constexpr int64_t kKeptRowBytes = int64_t{360} << 20;          // rows of a world up to which the per-token scatter is the faster one,
+constexpr int64_t kPerRouteTokenBytes = int64_t{104} << 20;    // and token rows beyond which it is again (LaunchMoonDispatch)
 
 const char *gScatterName = "";
 const char *gReduceName = "";
@@ -302,6 +308,19 @@ template <bool SELF>
 __device__ __forceinline__ void DedupGroupsOfChunk(const DispatchWorld &a, int rank, int chunk, bool lastChunk,
     int (*s_part)[kThreads / kWave], int *s_base);
 
+// A plan workgroup of a scatter launch: chunk blockIdx.x of destination rank blockIdx.y.
+__device__ __forceinline__ void PlanWorkgroup(const DispatchWorld &a, int planChunks, int planSelf)
+{
+    __shared__ int s_part[2][kThreads / kWave];
+    __shared__ int s_base[2];
+    const int chunk = blockIdx.x;
+    if (chunk < planChunks && planSelf != 0) {
+        DedupGroupsOfChunk<true>(a, blockIdx.y, chunk, chunk == planChunks - 1, s_part, s_base);
+    } else if (chunk < planChunks) {
+        DedupGroupsOfChunk<false>(a, blockIdx.y, chunk, chunk == planChunks - 1, s_part, s_base);
+    }
+}
+
 // One workgroup per (token, route, slice of 512 vectors) of source rank blockIdx.y.  What the routes record was written
 // ahead, by moon_records_kernel or moon_agree_kernel.
 //
@@ -317,14 +336,7 @@ __global__ __launch_bounds__(kThreads) void moon_scatter_kernel(DispatchWorld a,
 {
     static_assert(FRESH || !PLAN, "only a Dispatch that builds its plan has plan workgroups");
     if (PLAN && blockIdx.x < planBlocks) {
-        __shared__ int s_part[2][kThreads / kWave];
-        __shared__ int s_base[2];
-        const int chunk = blockIdx.x;
-        if (chunk < planChunks && planSelf != 0) {
-            DedupGroupsOfChunk<true>(a, blockIdx.y, chunk, chunk == planChunks - 1, s_part, s_base);
-        } else if (chunk < planChunks) {
-            DedupGroupsOfChunk<false>(a, blockIdx.y, chunk, chunk == planChunks - 1, s_part, s_base);
-        }
+        PlanWorkgroup(a, planChunks, planSelf);
         return;
     }
     const unsigned block = blockIdx.x - (PLAN ? planBlocks : 0u);
@@ -368,60 +380,69 @@ __global__ __launch_bounds__(kThreads) void moon_scatter_kernel(DispatchWorld a,
     }
 }
 
-// One workgroup per (token, slice of kTokenThreads vectors) of source rank blockIdx.y: the slice is loaded once, one
-// 16-byte vector per lane, and stored once per route.  For worlds whose token rows do not all stay in the memory-side
-// cache from one call to the next (eight ranks of 4096 x 7168 on one device): a kernel whose every workgroup loads
-// before it stores keeps most of its speed when the rows come from HBM (127 us per rank against 150-160 us for the
-// workgroup-per-route kernel, which is the faster one, 104-107 against 113-116 us, while the rows are in that cache).
-constexpr int kTokenThreads = 512;
-template <bool FRESH>
-__global__ __launch_bounds__(kTokenThreads) void moon_scatter_token_kernel(DispatchWorld a, int colSlices)
+// G lanes per (token, slice of G x V vectors) of source rank blockIdx.y: the slice is loaded once and stored once per route.
+// What the routes record was written ahead, as for moon_scatter_kernel; PLAN as there.  Lane k of every wave works out the
+// row of route k for itself, so nothing is handed round and no wave waits between its loads and its stores.  The rows are
+// written through and kept in the memory-side cache for Combine (the per-route kernel's must stream, or they push the token
+// rows that its workgroups share out of the L2s).  Workgroup b runs on XCD b % 8 and takes tokens t with t % 8 == b % 8, as
+// the reduce of a small world does.
+template <bool FRESH, bool PLAN, int G, int V>
+__global__ __launch_bounds__(kThreads) void moon_scatter_token_kernel(DispatchWorld a, int colSlices, unsigned planBlocks,
+    int planChunks, int planSelf)
 {
-    __shared__ int32_t s_dst[kMaxTopK];
-    __shared__ Route s_route[kMaxTopK];
-    __shared__ uint32_t s_tag[kMaxTopK];        // row tag bits of the route; 0 = the source does not write the row
-    __shared__ char *s_row[kMaxTopK];           // destination row
+    static_assert(FRESH || !PLAN, "only a Dispatch that builds its plan has plan workgroups");
+    if (PLAN && blockIdx.x < planBlocks) {
+        PlanWorkgroup(a, planChunks, planSelf);
+        return;
+    }
+    constexpr int kTokens = kThreads / G;
+    const unsigned block = blockIdx.x - (PLAN ? planBlocks : 0u);
     const int src = blockIdx.y;
-    const int token = blockIdx.x / colSlices;
-    const int slice = blockIdx.x % colSlices;
-    const int lane = threadIdx.x;
+    const int j = static_cast<int>(block / kXcds);
+    const int slice = j % colSlices;
+    const int tg = threadIdx.x / G;
+    const int64_t token = (static_cast<int64_t>(j / colSlices) * kTokens + tg) * kXcds + block % kXcds;
+    if (token >= a.s) {
+        return;
+    }
+    const int lane = threadIdx.x % G;
+    const int waveLane = threadIdx.x % kWave;
     const int K = static_cast<int>(a.k);
     const int h = static_cast<int>(a.h);
     const int vecs = h / 8;
-    const int idx = slice * kTokenThreads + lane;
-    if (lane < K) {
-        // one lane per route decodes it (two 64-bit divisions) for the whole workgroup
-        const int64_t route = static_cast<int64_t>(token) * K + lane;
-        const int32_t word = a.dst[src][route];
-        const uint8_t direct = FRESH ? 0 : a.tables.direct[static_cast<int64_t>(src) * a.tables.stride + route];
-        const Route r = Decode(word, a.nvS, a.world);
-        uint32_t tagBits = 0;
-        const bool writes = r.ok && SourceWrites<FRESH>(r, direct, &tagBits);
-        s_dst[lane] = word;
-        s_route[lane] = r;
-        s_tag[lane] = r.ok ? tagBits : 0u;
-        s_row[lane] = writes ? static_cast<char *>(a.hiddenNvsh[r.peer]) + static_cast<int64_t>(r.row) * h * 2 : nullptr;
+    const int colBase = slice * (G * V);
+    int32_t word = 0;
+    uint8_t direct = 0;
+    if (waveLane < K) {
+        const int64_t route = token * K + waveLane;
+        word = a.dst[src][route];
+        direct = FRESH ? 0 : a.tables.direct[static_cast<int64_t>(src) * a.tables.stride + route];
     }
-    const u32x4 *srcRow = reinterpret_cast<const u32x4 *>(static_cast<const char *>(a.hiddenSh[src]) +
-        static_cast<int64_t>(token) * h * 2);
-    const u32x4 v = idx < vecs ? srcRow[idx] : u32x4{0u, 0u, 0u, 0u};
-    __syncthreads();
+    const u32x4 *srcRow = reinterpret_cast<const u32x4 *>(static_cast<const char *>(a.hiddenSh[src]) + token * h * 2);
+    u32x4 v[V];
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+        const int idx = colBase + i * G + lane;
+        v[i] = idx < vecs ? srcRow[idx] : u32x4{0u, 0u, 0u, 0u};
+    }
+    const Route r = Decode(word, a.nvS, a.world);
+    uint32_t tagBits = 0;
+    const bool writes = waveLane < K && r.ok && SourceWrites<FRESH>(r, direct, &tagBits);
+    const int row = writes ? r.row : -1;
     for (int k = 0; k < K; ++k) {
-        char *row = s_row[k];
-        if (row != nullptr && idx < vecs) {
-            __builtin_nontemporal_store(v, reinterpret_cast<u32x4 *>(row) + idx);
+        const int rowOfK = __builtin_amdgcn_readlane(row, k);
+        if (rowOfK < 0) {
+            continue;
         }
-    }
-    if (slice == 0 && lane < kWave) {
-        for (int k = 0; k < K; ++k) {
-            const Route r = s_route[k];
-            if (!r.ok) {
-                if (lane == 0) {
-                    RecordFailure(a.tables, src, a.epoch, kDispatchInvalidRoute);
-                }
-                continue;
+        const int peer = __builtin_amdgcn_readlane(r.peer, k);
+        const __amdgpu_buffer_rsrc_t dst = TileXREp::RowResource(
+            static_cast<const char *>(a.hiddenNvsh[peer]) + static_cast<int64_t>(rowOfK) * h * 2, vecs * 16);
+#pragma unroll
+        for (int i = 0; i < V; ++i) {
+            const int idx = colBase + i * G + lane;
+            if (idx < vecs) {
+                __builtin_amdgcn_raw_buffer_store_b128(v[i], dst, idx * 16, 0, TileXREp::kAuxAgentScopeKept);
             }
-            RouteRecords<FRESH>(a, src, token, k, r, s_tag[k], s_dst);
         }
     }
 }
@@ -1299,34 +1320,38 @@ hipError_t LaunchMoonDispatch(const DispatchWorld &w, hipStream_t stream, const 
     const int64_t vecs = w.h / 8;
     const int colSlices = static_cast<int>((vecs + kRowVecs * kThreads - 1) / (kRowVecs * kThreads));
     const int64_t blocks = (w.s + kXcds - 1) / kXcds * kXcds * w.k * colSlices;
-    const int tokenSlices = static_cast<int>((vecs + kTokenThreads - 1) / kTokenThreads);
-    // token rows that cannot all stay in the memory-side cache from one call to the next: the kernel that keeps its speed
-    // when they come from HBM
+    const int tokenSlices = static_cast<int>((vecs + kTokenVecs - 1) / kTokenVecs);
+    // Which scatter: one workgroup per (token, route, slice) for wide rows that the memory-side cache cannot keep for Combine
+    // but whose token rows can be read ahead, one per token slice everywhere else.  All four stages (fwd: the forward two),
+    // top-8, us per route and per token, one rank: 128 x 7168 67 and 66, 1024 x 7168 139.5 and 129.5, 3000 x 7168 309 and 299,
+    // 3500 x 7168 348 and 352, 4096 x 7168 398.2 and 405.7, 8192 x 4096 454 and 474, 8192 x 7168 778 and 772; narrow rows 3000
+    // x 1024 125 and 95, 4096 x 2048 fwd 89 and 77, 16384 x 2048 fwd 255 and 246; four ranks, 4096 x 7168 2098 and 1785, two
+    // ranks, top-6, fwd 386 and 374.
     const int64_t worldRowBytes = static_cast<int64_t>(w.world) * w.s * w.h * 2;
-    const bool uncachedRows = worldRowBytes > gCachedRowBytes.load();
+    const int64_t cachedRowBytes = gCachedRowBytes.load();
+    const bool wantsPerToken = cachedRowBytes != kDefaultCachedRowBytes ? worldRowBytes > cachedRowBytes :
+        vecs <= 4 * kWave || worldRowBytes * w.k <= kKeptRowBytes || worldRowBytes > kPerRouteTokenBytes;
     const int64_t rowVecs = w.s * vecs;
-    const bool perToken = vec && uncachedRows && w.s * tokenSlices <= 0x7fffffff;
+    const bool perToken = vec && wantsPerToken && (w.s + 4 * kXcds) * tokenSlices <= 0x7fffffff;
     const bool perRoute = vec && !perToken && blocks <= 0x7fffffff;
-    // up to half the memory-side cache of token rows: read them once so that the per-route kernel finds them there
+    const bool recordsAhead = perToken || perRoute;
+    // per-route copies of up to half the memory-side cache of token rows: read them once so that the kernel finds them there
     // (one rank's share of 4096 x 7168: 257 -> about 210 us per layer on rows that were not cached, a few us more
     // on rows that were)
     const bool warm = perRoute && worldRowBytes <= kWarmRowBytes;
     const unsigned warmBlocks = warm ? static_cast<unsigned>((rowVecs + kThreads * kWarmLoads - 1) / (kThreads * kWarmLoads)) : 0u;
     const unsigned routeBlocks = static_cast<unsigned>((w.s * w.k + kThreads - 1) / kThreads);
-    // A fresh plan of a world whose rows are copied per route and come to at most kFusedPlanRowBytes: what the routes
-    // record is written ahead of the scatter, by the launch that reads the token rows ahead, and the plan is built by
-    // extra workgroups of the scatter launch; only the finish kernel follows the scatter.  Three launches instead of five
-    // while a rank has at most kSelfPlanChunks chunks, four (the chunk totals need one) beyond: 128 tokens x 7168 x top-8
-    // 36.6 -> 34.2 us per layer, 384 tokens 47.8 -> 41.6, 1024 tokens 77.5 -> 71.8, 4096 tokens x 2048 99.8 -> 93.6.  The
-    // scatter kernel that holds the plan's code has 50 registers per lane instead of 16, and its short-lived workgroups
-    // then start more slowly: from about 256 MB of rows on that costs more than the launches saved (4096 tokens x 7168
-    // 201 -> 204 us, 8192 tokens 365 -> 386 us), so larger worlds keep the plain kernel and the launches after it.
+    // What the routes record is written ahead of the scatter, and a fresh plan is built by extra workgroups of the scatter
+    // launch; only the finish kernel follows.  Three launches instead of five while a rank has at most kSelfPlanChunks chunks,
+    // four (the chunk totals need one) beyond.  Per-route copies of more than kFusedPlanRowBytes keep the launches after the
+    // scatter: with the plan's code that kernel has 50 registers per lane instead of 16, and its short-lived workgroups then
+    // start more slowly, which costs more than the launches saved (4096 tokens x 7168 201 -> 204 us, 8192 tokens 365 -> 386).
     const int planChunks = static_cast<int>((w.nvS + kBuildRows - 1) / kBuildRows);
-    const bool planInScatter = w.fresh && perRoute && planChunks <= kFusedPlanChunks &&
-        static_cast<int64_t>(w.world) * w.s * w.k * w.h * 2 <= kFusedPlanRowBytes;
+    const bool planInScatter = w.fresh && planChunks <= kFusedPlanChunks &&
+        (perToken || (perRoute && static_cast<int64_t>(w.world) * w.s * w.k * w.h * 2 <= kFusedPlanRowBytes));
     const bool planSelf = planChunks <= kSelfPlanChunks;
     const unsigned planBlocks = planInScatter ? static_cast<unsigned>((planChunks + kXcds - 1) / kXcds * kXcds) : 0u;
-    if (w.fresh && perRoute) {
+    if (w.fresh && recordsAhead) {
         hipLaunchKernelGGL(moon_records_kernel, dim3(routeBlocks + warmBlocks, R), dim3(kThreads), 0, stream, w, routeBlocks,
             warm ? rowVecs : int64_t{0});
         MOON_LAUNCH_CHECK();
@@ -1338,7 +1363,7 @@ hipError_t LaunchMoonDispatch(const DispatchWorld &w, hipStream_t stream, const 
         hipLaunchKernelGGL(moon_group_walk_kernel, dim3(rowBlocks, R), dim3(kThreads), 0, stream, w);
         MOON_LAUNCH_CHECK();
         hipLaunchKernelGGL(moon_agree_kernel, dim3(routeBlocks + warmBlocks, R), dim3(kThreads), 0, stream, w, routeBlocks,
-            warm ? rowVecs : int64_t{0}, perRoute ? 1 : 0);
+            warm ? rowVecs : int64_t{0}, recordsAhead ? 1 : 0);
         MOON_LAUNCH_CHECK();
     }
     hipError_t err = RecordIf(timing.start, stream);
@@ -1347,11 +1372,35 @@ hipError_t LaunchMoonDispatch(const DispatchWorld &w, hipStream_t stream, const 
     }
     if (perToken) {
         gScatterName = "moon_scatter_token_kernel";
-        const dim3 grid(static_cast<unsigned>(w.s * tokenSlices), R);
-        if (w.fresh) {
-            hipLaunchKernelGGL(moon_scatter_token_kernel<true>, grid, dim3(kTokenThreads), 0, stream, w, tokenSlices);
+        // Three workgroups to a compute unit, or as many as fit where the rows come to a GiB and more; us at eight, four and
+        // three: 1024 x 7168 x top-8 132.6, 130.7, 129.5; four ranks x 2000 x 2048 490, 472, 447; four ranks x 4096 x 7168 (1.9
+        // GB) 1785, 1817, 1816, eight x 2500 x 7168 fwd 1137, 1161, 1161.
+        const unsigned capLds = worldRowBytes * w.k <= (int64_t{1} << 30) ? kTokenCapLdsBytes : 0u;
+        auto launch = [&](auto lanes, auto vecsPerLane) {
+            constexpr int G = decltype(lanes)::value;
+            constexpr int V = decltype(vecsPerLane)::value;
+            constexpr int64_t kTokens = kThreads / G * kXcds;       // tokens of eight neighbouring workgroups
+            const dim3 grid(static_cast<unsigned>((w.s + kTokens - 1) / kTokens * kXcds * tokenSlices) + planBlocks, R);
+            if (planInScatter) {
+                hipLaunchKernelGGL((moon_scatter_token_kernel<true, true, G, V>), grid, dim3(kThreads), capLds, stream, w, tokenSlices,
+                    planBlocks, planChunks, planSelf ? 1 : 0);
+            } else if (w.fresh) {
+                hipLaunchKernelGGL((moon_scatter_token_kernel<true, false, G, V>), grid, dim3(kThreads), capLds, stream, w, tokenSlices,
+                    0u, 0, 0);
+            } else {
+                hipLaunchKernelGGL((moon_scatter_token_kernel<false, false, G, V>), grid, dim3(kThreads), capLds, stream, w, tokenSlices,
+                    0u, 0, 0);
+            }
+        };
+        // narrow rows: a wave per token (four tokens per workgroup); wide ones: the workgroup
+        if (vecs <= 2 * kWave) {
+            launch(std::integral_constant<int, kWave>{}, std::integral_constant<int, 2>{});
+        } else if (vecs <= 4 * kWave) {
+            launch(std::integral_constant<int, kWave>{}, std::integral_constant<int, 4>{});
+        } else if (vecs <= 2 * kThreads) {
+            launch(std::integral_constant<int, kThreads>{}, std::integral_constant<int, 2>{});
         } else {
-            hipLaunchKernelGGL(moon_scatter_token_kernel<false>, grid, dim3(kTokenThreads), 0, stream, w, tokenSlices);
+            launch(std::integral_constant<int, kThreads>{}, std::integral_constant<int, kTokenVecs / kThreads>{});
         }
     } else if (perRoute) {
         gScatterName = "moon_scatter_kernel";
