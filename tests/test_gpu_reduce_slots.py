@@ -1,0 +1,68 @@
+"""Slots of a token that the lanes of a wave look up, and put in order, for themselves: counts of slots on both sides of what
+is read at once, up to one per lane; rows that are missing; rows whose order is not the slots'; one, two and four waves to a
+token; several tokens to a workgroup, the last one not full.  Bit for bit against the oracle."""
+import numpy as np
+import pytest
+import torch
+
+from gpu_harness import DEV, Session, bits16, to_dev
+from oracle import ep as O
+from tilexr_amd import ep
+from test_gpu_parity import ids_for, x_for
+
+pytestmark = pytest.mark.gpu
+
+
+def _lose(rng, d, bs, k):
+    keep = rng.random((bs, k)) < rng.random((bs, 1))
+    keep[0], keep[1], keep[2, :k - 1], keep[2, k - 1] = True, False, False, True
+    assist = d["assist"].copy()
+    assist[~keep[assist[:, 1], assist[:, 2]], 1] = -1
+    return assist
+
+
+@pytest.mark.parametrize("k", [1, 4, 5, 6, 7, 32])
+@pytest.mark.parametrize("h", [64, 1040, 2064, 4096, 4112])
+@pytest.mark.parametrize("quant", [ep.Q_TOKEN_INT8, ep.Q_FP8_BLOCK128])
+@pytest.mark.parametrize("dtype", [ep.DT_BF16, ep.DT_FP16])
+def test_quantised_rows_by_slots(k, h, quant, dtype):
+    bs, experts = 67, 40
+    rng = np.random.default_rng(k * 10000 + h + quant)
+    ids = ids_for(rng, bs, k, experts)
+    _, xb = x_for(rng, bs, h, dtype, scale=2.0)
+    d = O.mem_dispatch(O.Case(1, bs, h, k, experts, dtype=dtype, quant_mode=quant), 0, xb[None], ids[None])
+    assist = _lose(rng, d, bs, k)
+    w = (0.5 + rng.random((bs, k))).astype(np.float32)
+    tdt = torch.bfloat16 if dtype == ep.DT_BF16 else torch.float16
+    with Session() as s:
+        y = torch.full((bs, h), 7.0, dtype=tdt, device=DEV)
+        args = [to_dev(v) for v in (d["expand_x"], assist, d["send_counts"], d["dyn_scales"], w)]
+        torch.cuda.synchronize()
+        assert ep.combine_memory_ex(args[0], args[1], args[2], s.comm, bs, h, k, experts, y, dtype, s.stream,
+                                    expert_out_quant_mode=quant, expert_out_scales=args[3], expert_scales=args[4]) == 0
+        s.sync()
+        assert ep.last_kernel_name(s.comm, ep.K_REDUCE) == "ep_reduce_quant_kernel"
+        want = O.mem_combine(O.Case(1, bs, h, k, experts, dtype=dtype), 0, d["expand_x"][None], assist[None],
+                             d["send_counts"][None], expert_scales=w, in_quant=quant, in_scales=d["dyn_scales"])
+        assert np.array_equal(bits16(y), want)
+
+
+@pytest.mark.parametrize("bs,h,k", [(5, 64, 8), (700, 64, 5), (41, 1024, 64), (300, 1032, 8), (65, 4104, 33), (3, 16384, 2)])
+def test_sums_in_the_order_of_the_rows(bs, h, k):
+    """The MVP route adds rows in ascending row order; here the rows of a token stand in any order of its slots."""
+    experts = 64
+    rng = np.random.default_rng(bs + h + k)
+    ids = ids_for(rng, bs, k, experts)
+    _, xb = x_for(rng, bs, h, ep.DT_FP16, scale=2.0)
+    case = O.Case(1, bs, h, k, experts, dtype=O.DT_FP16)
+    d = O.mvp_dispatch(case, 0, xb[None], ids[None])
+    assist = _lose(rng, d, bs, k)[rng.permutation(bs * k)]
+    rows = xb[rng.integers(0, bs, bs * k)]
+    counts = np.array([bs * k], np.int32)
+    with Session() as s:
+        y = torch.full((bs, h), 7.0, dtype=torch.float16, device=DEV)
+        args = [to_dev(v) for v in (rows, assist, counts)]
+        torch.cuda.synchronize()
+        assert ep.combine_v2(args[0], args[1], args[2], s.comm, bs, h, k, experts, y, ep.DT_FP16, s.stream) == 0
+        s.sync()
+        assert np.array_equal(bits16(y), O.mvp_combine(case, 0, rows[None], assist[None], counts[None]))

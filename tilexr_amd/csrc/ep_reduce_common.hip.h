@@ -156,6 +156,24 @@ __device__ inline void SortRows(int *rows, int k, const uint64_t *orderKeys)
     }
 }
 
+// The same order for a wave that holds slot k's row in lane k (all 64 lanes active): every lane counts the slots ahead of its
+// own, then the rows change places in one exchange.  Slots with equal keys keep their order.
+__device__ __forceinline__ int SortedRowOfLane(int row, int slots, const uint64_t *orderKeys)
+{
+    const int lane = static_cast<int>(threadIdx.x) % kWave;
+    uint64_t key = ~0ull;
+    if (row >= 0) {
+        key = orderKeys != nullptr ? orderKeys[row] : static_cast<uint64_t>(row);
+    }
+    int ahead = lane < slots ? 0 : lane;
+    for (int k = 0; k < slots; ++k) {
+        const uint64_t other = static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(key >> 32), k))) << 32 |
+            static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(key), k));
+        ahead += lane < slots && (other < key || (other == key && k < lane)) ? 1 : 0;
+    }
+    return __builtin_amdgcn_ds_permute(ahead * 4, row);
+}
+
 // Row loads of the register-resident kernels.  FL = false: non-temporal loads.  FL = true (rows published through
 // readiness flags, possibly a moment ago by a workgroup on another XCD): agent-scope loads, served from memory, so
 // that no acquire fence (an invalidate of this XCD's whole L2) is needed per token.
@@ -256,153 +274,153 @@ __device__ __forceinline__ bool LoadRoutes(const ReduceArgs &a, int token, bool 
     return pending;
 }
 
-// Runs unit(group) for this workgroup's groups: blockIdx.x, blockIdx.x + gridDim.x, ...  `load(group, mode)`
-// fills the workgroup's route tables for a group and returns (per lane) whether a tile it needs is not published yet;
-// `tokenAt(group, t)` names the t-th of a group's `tokensPerGroup` tokens (-1 = none).
+// Launches that do not wait: lane k < slots of a wave that works on `token` looks slot k up for itself.  Nothing is handed
+// round through LDS, no wave waits for another one, and small launches are shorter by two LDS trips and a barrier.  us, with
+// the route tables in LDS and without: eight decode layers in a graph, 128 x 7168 100.8 -> 96.9, 1 x 4096 53.1 -> 50.8; 600 x
+// 7168 31.1 -> 30.6, block fp8 4096 x 7168 114.6 -> 113.9.
+__device__ __forceinline__ int RouteOfLane(const ReduceArgs &a, int token, bool tokOk, int waveLane, float *weight)
+{
+    *weight = 1.0f;
+    if (!tokOk || waveLane >= a.slots) {
+        return -1;
+    }
+    if (a.expertScales != nullptr && waveLane < a.topK) {
+        *weight = a.expertScales[static_cast<int64_t>(token) * a.topK + waveLane];
+    }
+    return LookupRow(a, static_cast<int64_t>(token) * a.slots + waveLane);
+}
+
+// Launches that may wait: runs unit(group) for the groups this workgroup claims.  `load(group, mode)` fills the workgroup's
+// route tables for a group and returns (per lane) whether a tile it needs is not published yet; `tokenAt(group, t)` names
+// the t-th of a group's `tokensPerGroup` tokens (-1 = none).
 //
-// Without readiness flags, or with flags that were all published before the launch began, that is a plain loop.  A
-// launch that may have to wait (WAITS, flags not settled) never sits on one group while others are ready: a token needs
-// the tiles of all its rows, which a producer that works tile by tile finishes at unrelated times, so tokens become
-// ready in no particular order.  A workgroup holds a few groups at a time.  Fresh ones are looked at once and reduced
-// if their tiles are there.  For what is left it goes in rounds: all lanes together look once at every tile the held
-// groups need (one round trip for the lot), the groups that have become complete are reduced, and a round without any
-// is followed by a sleep that grows to about 14 us.  When nothing it holds has become ready for the wait bound, or
-// another workgroup has reported an expired wait, the rest is given up: those tokens get rows of zeros and the launch's
-// status word is set.
-template <bool WAITS, typename TokenAt, typename Load, typename Unit>
+// Such a launch never sits on one group while others are ready: a token needs the tiles of all its rows, which a producer
+// that works tile by tile finishes at unrelated times, so tokens become ready in no particular order.  A workgroup holds a
+// few groups at a time.  Fresh ones are looked at once and reduced if their tiles are there.  For what is left it goes in
+// rounds: all lanes together look once at every tile the held groups need (one round trip for the lot), the groups that have
+// become complete are reduced, and a round without any is followed by a sleep that grows to about 14 us.  When nothing it
+// holds has become ready for the wait bound, or another workgroup has reported an expired wait, the rest is given up: those
+// tokens get rows of zeros and the launch's status word is set.
+template <typename TokenAt, typename Load, typename Unit>
 __device__ __forceinline__ void ForEachGroup(const ReduceArgs &a, int groups, int tokensPerGroup, TokenAt tokenAt,
     Load load, Unit unit)
 {
-    const bool plainLoop = !WAITS || a.flagsSettled != 0;
-    if (plainLoop) {
-        // no flags, or flags that were all published before this launch began: the route tables trust every tile, and
-        // the kernel looks at the words itself, beside the rows (SettledWordLoad)
-        for (int group = blockIdx.x; group < groups; group += gridDim.x) {
-            __syncthreads();        // the previous iteration's readers are done with the route tables
-            load(group, kRouteTrusted);
-            __syncthreads();
-            unit(group);
-        }
-        return;
-    }
-    if constexpr (WAITS) {
-        // the control flow is ClaimAndReduce of ep_token_claim.h (the host-side model of the protocol runs the same
-        // code); what follows are its operations for a workgroup: atomics, barriers, LDS
-        __shared__ uint32_t s_notReady;
-        __shared__ int s_group[kClaimHeld];
-        __shared__ int s_base;
-        struct WorkgroupEnv {
-            const ReduceArgs &a;
-            TokenAt &tokenAt;
-            Load &load;
-            Unit &unit;
-            uint32_t *notReady;
-            int *group;
-            int *base;
-            int perGroup;                   // (token, slot) pairs of a group
-            int tokensPerGroup;
-            int dealt;                      // next group by block index (launches without a claim counter)
-            uint64_t idleSince;
+    // the control flow is ClaimAndReduce of ep_token_claim.h (the host-side model of the protocol runs the same
+    // code); what follows are its operations for a workgroup: atomics, barriers, LDS
+    __shared__ uint32_t s_notReady;
+    __shared__ int s_group[kClaimHeld];
+    __shared__ int s_base;
+    struct WorkgroupEnv {
+        const ReduceArgs &a;
+        TokenAt &tokenAt;
+        Load &load;
+        Unit &unit;
+        uint32_t *notReady;
+        int *group;
+        int *base;
+        int perGroup;                   // (token, slot) pairs of a group
+        int tokensPerGroup;
+        int dealt;                      // next group by block index (launches without a claim counter)
+        uint64_t idleSince;
 
-            __device__ __forceinline__ int Claim(int want)
-            {
-                if (a.claim == nullptr) {
-                    return 0;
-                }
-                __syncthreads();            // readers of *base from the previous refill are done
-                if (threadIdx.x == 0) {
-                    *base = static_cast<int>(__hip_atomic_fetch_add(a.claim, static_cast<uint32_t>(want), __ATOMIC_RELAXED,
-                        __HIP_MEMORY_SCOPE_AGENT));
-                }
-                __syncthreads();
-                return *base;
+        __device__ __forceinline__ int Claim(int want)
+        {
+            if (a.claim == nullptr) {
+                return 0;
             }
-            __device__ __forceinline__ int NextGroup(int *next)
-            {
-                if (a.claim != nullptr) {
-                    return (*next)++;
+            __syncthreads();            // readers of *base from the previous refill are done
+            if (threadIdx.x == 0) {
+                *base = static_cast<int>(__hip_atomic_fetch_add(a.claim, static_cast<uint32_t>(want), __ATOMIC_RELAXED,
+                    __HIP_MEMORY_SCOPE_AGENT));
+            }
+            __syncthreads();
+            return *base;
+        }
+        __device__ __forceinline__ int NextGroup(int *next)
+        {
+            if (a.claim != nullptr) {
+                return (*next)++;
+            }
+            const int mine = dealt;
+            dealt += static_cast<int>(gridDim.x);
+            return mine;
+        }
+        __device__ __forceinline__ void Hold(int slot, int g)
+        {
+            if (threadIdx.x == 0) {
+                group[slot] = g;
+            }
+        }
+        __device__ __forceinline__ void HoldDone()
+        {
+            __syncthreads();
+        }
+        __device__ __forceinline__ bool Try(int slot, int mode)
+        {
+            const int g = group[slot];
+            __syncthreads();
+            const bool waiting = load(g, mode);
+            if (__syncthreads_or((mode == kRouteCheck && waiting) ? 1 : 0) != 0) {
+                return false;           // uniform: every lane gets the same answer
+            }
+            unit(g);
+            return true;
+        }
+        __device__ __forceinline__ uint32_t Scan(uint32_t pending)
+        {
+            // all lanes together look once at every tile the held groups need: one round trip for the lot
+            if (threadIdx.x == 0) {
+                *notReady = 0u;
+            }
+            __syncthreads();
+            for (int idx = threadIdx.x; idx < kClaimHeld * perGroup; idx += blockDim.x) {
+                const int i = idx / perGroup;
+                if (((pending >> i) & 1u) == 0u) {
+                    continue;
                 }
-                const int mine = dealt;
-                dealt += static_cast<int>(gridDim.x);
-                return mine;
-            }
-            __device__ __forceinline__ void Hold(int slot, int g)
-            {
-                if (threadIdx.x == 0) {
-                    group[slot] = g;
+                const int token = tokenAt(group[i], (idx % perGroup) / a.slots);
+                if (token < 0) {
+                    continue;
                 }
-            }
-            __device__ __forceinline__ void HoldDone()
-            {
-                __syncthreads();
-            }
-            __device__ __forceinline__ bool Try(int slot, int mode)
-            {
-                const int g = group[slot];
-                __syncthreads();
-                const bool waiting = load(g, mode);
-                if (__syncthreads_or((mode == kRouteCheck && waiting) ? 1 : 0) != 0) {
-                    return false;           // uniform: every lane gets the same answer
-                }
-                unit(g);
-                return true;
-            }
-            __device__ __forceinline__ uint32_t Scan(uint32_t pending)
-            {
-                // all lanes together look once at every tile the held groups need: one round trip for the lot
-                if (threadIdx.x == 0) {
-                    *notReady = 0u;
-                }
-                __syncthreads();
-                for (int idx = threadIdx.x; idx < kClaimHeld * perGroup; idx += blockDim.x) {
-                    const int i = idx / perGroup;
-                    if (((pending >> i) & 1u) == 0u) {
-                        continue;
-                    }
-                    const int token = tokenAt(group[i], (idx % perGroup) / a.slots);
-                    if (token < 0) {
-                        continue;
-                    }
-                    const int row = LookupRow(a, static_cast<int64_t>(token) * a.slots + idx % a.slots);
-                    if (row >= 0 && !TilePublished(a, row)) {
-                        atomicOr(notReady, 1u << i);
-                    }
-                }
-                __syncthreads();
-                return *notReady;
-            }
-            __device__ __forceinline__ bool GiveUpNow()
-            {
-                bool stop = false;
-                if (threadIdx.x == 0) {
-                    stop = static_cast<int64_t>(wall_clock64() - idleSince) > a.waitTimeoutTicks ||
-                        (a.deviceStatus != nullptr &&
-                         __hip_atomic_load(a.deviceStatus, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0);
-                }
-                return __syncthreads_or(stop ? 1 : 0) != 0;
-            }
-            __device__ __forceinline__ void Touch()
-            {
-                idleSince = wall_clock64();
-            }
-            __device__ __forceinline__ void Sleep(int level)
-            {
-                for (int r = 0; r < (1 << level); ++r) {
-                    __builtin_amdgcn_s_sleep(127);      // 127 x 64 clocks, about 3.5 us
+                const int row = LookupRow(a, static_cast<int64_t>(token) * a.slots + idx % a.slots);
+                if (row >= 0 && !TilePublished(a, row)) {
+                    atomicOr(notReady, 1u << i);
                 }
             }
-            __device__ __forceinline__ void Leave()
-            {
-                if (a.claim != nullptr && threadIdx.x == 0) {
-                    DeviceTileOps ops;
-                    LeaveClaimWords(ops, a.claim, gridDim.x);
-                }
+            __syncthreads();
+            return *notReady;
+        }
+        __device__ __forceinline__ bool GiveUpNow()
+        {
+            bool stop = false;
+            if (threadIdx.x == 0) {
+                stop = static_cast<int64_t>(wall_clock64() - idleSince) > a.waitTimeoutTicks ||
+                    (a.deviceStatus != nullptr &&
+                     __hip_atomic_load(a.deviceStatus, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0);
             }
-        };
-        WorkgroupEnv env {a, tokenAt, load, unit, &s_notReady, s_group, &s_base, tokensPerGroup * a.slots, tokensPerGroup,
-            static_cast<int>(blockIdx.x), 0};
-        ClaimAndReduce(env, groups);
-    }
+            return __syncthreads_or(stop ? 1 : 0) != 0;
+        }
+        __device__ __forceinline__ void Touch()
+        {
+            idleSince = wall_clock64();
+        }
+        __device__ __forceinline__ void Sleep(int level)
+        {
+            for (int r = 0; r < (1 << level); ++r) {
+                __builtin_amdgcn_s_sleep(127);      // 127 x 64 clocks, about 3.5 us
+            }
+        }
+        __device__ __forceinline__ void Leave()
+        {
+            if (a.claim != nullptr && threadIdx.x == 0) {
+                DeviceTileOps ops;
+                LeaveClaimWords(ops, a.claim, gridDim.x);
+            }
+        }
+    };
+    WorkgroupEnv env {a, tokenAt, load, unit, &s_notReady, s_group, &s_base, tokensPerGroup * a.slots, tokensPerGroup,
+        static_cast<int>(blockIdx.x), 0};
+    ClaimAndReduce(env, groups);
 }
 
 } // namespace

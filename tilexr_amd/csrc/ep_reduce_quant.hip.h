@@ -22,13 +22,19 @@ constexpr int kFlagsNone = 0;
 constexpr int kFlagsMayWait = 1;
 constexpr int kFlagsSettled = 2;
 
-template <int G, int V, int INQ, bool BF16, int FL>
-__global__ __launch_bounds__(kThreads, (V == 1 && BF16) ? ((FL == kFlagsMayWait && INQ == TILEXR_EP_QUANT_FP8_BLOCK128) ? 6 : 7) : 1) void ep_reduce_quant_kernel(ReduceArgs a)
+//
+// KB rows in flight per lane: four, or two of the widest rows.  Five or six slots to a token take six at once instead of four
+// and then the rest, at five waves per SIMD instead of seven (8192 x 4096 x top-6 int8, dispatch + combine 99.4 -> 97.5 us;
+// eight for eight slots is no such bargain: 16384 x 2048 int8 130.6 -> 129.8, but block fp8 that lost rows to a capacity, four
+// left of eight, 91.0 -> 93.0, and 8192 x 4096 x top-2 57.0 -> 59.4).
+template <int G, int V, int INQ, bool BF16, int FL, int KB>
+__global__ __launch_bounds__(kThreads, (V == 1 && BF16) ? (KB > 4 ? 5 : (FL == kFlagsMayWait && INQ == TILEXR_EP_QUANT_FP8_BLOCK128) ? 6 : 7) : 1) void ep_reduce_quant_kernel(ReduceArgs a)
 {
     constexpr int kTokens = kThreads / G;
-    constexpr int KB = V >= 4 ? 2 : 4;
-    __shared__ int s_row[kTokens][kMaxTopK];
-    __shared__ float s_w[kTokens][kMaxTopK];
+    constexpr bool kWaits = FL == kFlagsMayWait;
+    // route tables of launches that may wait
+    __shared__ int s_row[kWaits ? kTokens : 1][kMaxTopK];
+    __shared__ float s_w[kWaits ? kTokens : 1][kMaxTopK];
 
     const int tg = threadIdx.x / G;
     const int lane = threadIdx.x % G;
@@ -54,7 +60,9 @@ __global__ __launch_bounds__(kThreads, (V == 1 && BF16) ? ((FL == kFlagsMayWait 
         const int waveLane = threadIdx.x % kWave;
         int slotRow = -1;
         float myWeight = 0.0f;
-        if (waveLane < a.slots) {
+        if (!kWaits) {
+            slotRow = RouteOfLane(a, token, tokOk, waveLane, &myWeight);
+        } else if (waveLane < a.slots) {
             slotRow = s_row[tg][waveLane];
             myWeight = s_w[tg][waveLane];
         }
@@ -234,12 +242,16 @@ __global__ __launch_bounds__(kThreads, (V == 1 && BF16) ? ((FL == kFlagsMayWait 
             }
         }
     };
-    ForEachGroup<FL == kFlagsMayWait>(a, groups, kTokens, tokenAt, load, reduceUnit);
+    if constexpr (kWaits) {
+        ForEachGroup(a, groups, kTokens, tokenAt, load, reduceUnit);
+    } else {
+        reduceUnit(blockIdx.x);         // a workgroup for every group
+    }
 }
 
 
-template <int G, int V, bool BF16, int FL>
-void LaunchQuant(const ReduceLaunch &l, const ReduceArgs &a, int gridLimit)
+template <int G, int V, bool BF16, int FL, int KB>
+void LaunchQuantRows(const ReduceLaunch &l, const ReduceArgs &a, int gridLimit)
 {
     constexpr int kTokens = kThreads / G;
     int grid = (a.bs + kTokens - 1) / kTokens;
@@ -249,10 +261,22 @@ void LaunchQuant(const ReduceLaunch &l, const ReduceArgs &a, int gridLimit)
     const dim3 g(grid);
     const dim3 b(kThreads);
     if (l.inQuant == TILEXR_EP_QUANT_TOKEN_INT8) {
-        hipLaunchKernelGGL((ep_reduce_quant_kernel<G, V, TILEXR_EP_QUANT_TOKEN_INT8, BF16, FL>), g, b, 0, l.stream, a);
+        hipLaunchKernelGGL((ep_reduce_quant_kernel<G, V, TILEXR_EP_QUANT_TOKEN_INT8, BF16, FL, KB>), g, b, 0, l.stream, a);
     } else {
-        hipLaunchKernelGGL((ep_reduce_quant_kernel<G, V, TILEXR_EP_QUANT_FP8_BLOCK128, BF16, FL>), g, b, 0, l.stream, a);
+        hipLaunchKernelGGL((ep_reduce_quant_kernel<G, V, TILEXR_EP_QUANT_FP8_BLOCK128, BF16, FL, KB>), g, b, 0, l.stream, a);
     }
+}
+
+template <int G, int V, bool BF16, int FL>
+void LaunchQuant(const ReduceLaunch &l, const ReduceArgs &a, int gridLimit)
+{
+    if constexpr (V == 1 && FL != kFlagsMayWait) {
+        if (a.slots == 5 || a.slots == 6) {
+            LaunchQuantRows<G, V, BF16, FL, 6>(l, a, gridLimit);
+            return;
+        }
+    }
+    LaunchQuantRows<G, V, BF16, FL, V >= 4 ? 2 : 4>(l, a, gridLimit);
 }
 
 } // namespace

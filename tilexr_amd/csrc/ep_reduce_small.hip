@@ -99,18 +99,15 @@ __global__ __launch_bounds__(kSmallReduceThreads) void ep_reduce_small_kernel(Sm
         }
     }
     __syncthreads();
-    if (KIND == kReducePerAdd) {
-        if (tid == 0) {
-            SortRows(s_row, a.topK, nullptr);
-        }
-        __syncthreads();
-    }
     const int colBase = wave * (kWave * V);
     if (colBase >= vecs) {
         return;
     }
     // lane k keeps slot k's row and weight
-    const int myRow = (lane < a.topK && active) ? s_row[lane] : -1;
+    int myRow = (lane < a.topK && active) ? s_row[lane] : -1;
+    if (KIND == kReducePerAdd) {
+        myRow = SortedRowOfLane(myRow, a.topK, nullptr);
+    }
 
     float acc[V][8];
 #pragma unroll

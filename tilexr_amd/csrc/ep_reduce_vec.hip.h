@@ -23,6 +23,7 @@
 #endif
 
 #include <algorithm>
+#include <type_traits>
 
 #include "ep_reduce_common.hip.h"
 
@@ -57,8 +58,9 @@ __device__ __forceinline__ void ReduceVec(const ReduceArgs &a)
     constexpr int kTokens = kThreads / G;
     constexpr bool kMx = COMMQ != 0;
     constexpr bool kCommE5m2 = COMMQ == TILEXR_EP_QUANT_COMM_MXFP8_E5M2;
-    __shared__ int s_row[kTokens][kMaxTopK];
-    __shared__ float s_w[kTokens][kMaxTopK];
+    // route tables of launches that may wait
+    __shared__ int s_row[FL ? kTokens : 1][kMaxTopK];
+    __shared__ float s_w[FL ? kTokens : 1][kMaxTopK];
 
     const int tg = threadIdx.x / G;
     const int lane = threadIdx.x % G;
@@ -97,13 +99,15 @@ __device__ __forceinline__ void ReduceVec(const ReduceArgs &a)
         const int token = placeOf(group * unitsPerGroup + tg, &slice);
         return LoadRoutes<false>(a, token < 0 ? 0 : token, token >= 0, lane, G, s_row[tg], s_w[tg], mode);
     };
-    auto reduceUnit = [&](int group) {
+    // direct: every wave looks its token's slots up, no route tables
+    auto reduceUnit = [&](int group, auto direct) {
+        constexpr bool kDirect = decltype(direct)::value;
         int slice;
         const int placed = placeOf(group * unitsPerGroup + tg, &slice);
         const bool tokOk = placed >= 0;
         const int token = tokOk ? placed : 0;
         const int colBase = slice * (G * V);
-        if (KIND == kReducePerAdd) {
+        if (!kDirect && KIND == kReducePerAdd) {
             if (lane == 0) {
                 SortRows(s_row[tg], a.slots, a.orderKeys);
             }
@@ -116,7 +120,12 @@ __device__ __forceinline__ void ReduceVec(const ReduceArgs &a)
         const int waveLane = threadIdx.x % kWave;
         int slotRow = -1;
         float myWeight = 0.0f;
-        if (waveLane < a.slots) {
+        if (kDirect) {
+            slotRow = RouteOfLane(a, token, tokOk, waveLane, &myWeight);
+            if (KIND == kReducePerAdd) {
+                slotRow = SortedRowOfLane(slotRow, a.slots, a.orderKeys);
+            }
+        } else if (waveLane < a.slots) {
             slotRow = s_row[tg][waveLane];
             myWeight = s_w[tg][waveLane];
         }
@@ -292,7 +301,17 @@ __device__ __forceinline__ void ReduceVec(const ReduceArgs &a)
             }
         }
     };
-    ForEachGroup<FL>(a, groups, unitsPerGroup, tokenAt, load, reduceUnit);
+    if constexpr (!FL) {
+        reduceUnit(blockIdx.x, std::true_type {});      // a workgroup for every group
+    } else if (a.flagsSettled != 0) {
+        for (int group = blockIdx.x; group < groups; group += gridDim.x) {
+            reduceUnit(group, std::true_type {});
+        }
+    } else {
+        ForEachGroup(a, groups, unitsPerGroup, tokenAt, load, [&](int group) {
+            reduceUnit(group, std::false_type {});
+        });
+    }
 }
 
 
