@@ -21,13 +21,8 @@ __device__ inline int BlockExclusiveScan(int *vals, int m, int *part)
     for (int i = begin; i < begin + per && i < m; ++i) {
         local += vals[i];
     }
-    // inclusive scan of the per-thread sums inside each wave (shuffles), then across the four waves through LDS
-    int incl = local;
-#pragma unroll
-    for (int off = 1; off < kWave; off <<= 1) {
-        const int up = __shfl_up(incl, off);
-        incl += lane >= off ? up : 0;
-    }
+    // inclusive scan of the per-thread sums inside each wave, then across the four waves through LDS
+    const int incl = WaveInclusiveSum(local);
     if (lane == kWave - 1) {
         part[wave] = incl;
     }

@@ -48,9 +48,7 @@ __device__ __forceinline__ int ChunkLiveLimit(const ChunkRouteArgs &a, int *s_su
     for (int t = threadIdx.x; t < a.bs; t += kThreads) {
         local += a.mask[t] != 0 ? 1 : 0;
     }
-    for (int off = kWave / 2; off >= 1; off >>= 1) {
-        local += __shfl_xor(local, off);
-    }
+    local = WaveSum(local);
     if ((threadIdx.x & (kWave - 1)) == 0) {
         atomicAdd(s_sum, local);
     }

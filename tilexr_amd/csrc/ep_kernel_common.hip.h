@@ -66,6 +66,59 @@ __host__ __device__ inline int XcdPlacedUnits(int tokens, int parts)
     return (tokens + kXcdCount - 1) / kXcdCount * kXcdCount * parts;
 }
 
+// Sums, maxima and scans of a wave, all 64 lanes active, in the registers' own cross-lane moves: four moves within rows of
+// sixteen lanes, then four scalar reads, where shuffles are six dependent trips through LDS of about a hundred clocks each.
+constexpr int kDppQuadSwap1 = 0xb1;         // lanes 1 0 3 2 of a quad
+constexpr int kDppQuadSwap2 = 0x4e;         // lanes 2 3 0 1
+constexpr int kDppHalfRowMirror = 0x141;    // lane i of eight takes lane 7 - i
+constexpr int kDppRowMirror = 0x140;        // lane i of sixteen takes lane 15 - i
+constexpr int kDppRowShift = 0x110;         // + n: lane i of sixteen takes lane i - n, zero below
+constexpr int kDppRowBroadcast15 = 0x142;   // rows one and three take the last lane of the row before them
+constexpr int kDppRowBroadcast31 = 0x143;   // rows two and three take lane 31
+
+template <int CTRL, int ROWS = 0xf>
+__device__ __forceinline__ int DppMove(int v)
+{
+    return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xf, true);
+}
+
+__device__ __forceinline__ int WaveSum(int v)
+{
+    v += DppMove<kDppQuadSwap1>(v);
+    v += DppMove<kDppQuadSwap2>(v);
+    v += DppMove<kDppHalfRowMirror>(v);
+    v += DppMove<kDppRowMirror>(v);
+    return __builtin_amdgcn_readlane(v, 0) + __builtin_amdgcn_readlane(v, 16) + __builtin_amdgcn_readlane(v, 32) +
+        __builtin_amdgcn_readlane(v, 48);
+}
+
+// Largest of the lane's row of sixteen.
+__device__ __forceinline__ float RowMax(float v)
+{
+    v = fmaxf(v, __int_as_float(DppMove<kDppQuadSwap1>(__float_as_int(v))));
+    v = fmaxf(v, __int_as_float(DppMove<kDppQuadSwap2>(__float_as_int(v))));
+    v = fmaxf(v, __int_as_float(DppMove<kDppHalfRowMirror>(__float_as_int(v))));
+    return fmaxf(v, __int_as_float(DppMove<kDppRowMirror>(__float_as_int(v))));
+}
+
+__device__ __forceinline__ float WaveMax(float v)
+{
+    const int m = __float_as_int(RowMax(v));
+    return fmaxf(fmaxf(__int_as_float(__builtin_amdgcn_readlane(m, 0)), __int_as_float(__builtin_amdgcn_readlane(m, 16))),
+        fmaxf(__int_as_float(__builtin_amdgcn_readlane(m, 32)), __int_as_float(__builtin_amdgcn_readlane(m, 48))));
+}
+
+__device__ __forceinline__ int WaveInclusiveSum(int v)
+{
+    v += DppMove<kDppRowShift + 1>(v);
+    v += DppMove<kDppRowShift + 2>(v);
+    v += DppMove<kDppRowShift + 4>(v);
+    v += DppMove<kDppRowShift + 8>(v);
+    v += DppMove<kDppRowBroadcast15, 0xa>(v);
+    v += DppMove<kDppRowBroadcast31, 0xc>(v);
+    return v;
+}
+
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t RowResource(const void *row, int bytes)
 {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(row), 0, bytes, kRawBufferWord3);

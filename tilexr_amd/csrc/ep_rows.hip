@@ -67,15 +67,6 @@ struct RouteRowsArgs {
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 
 
-__device__ __forceinline__ int WaveSum(int v)
-{
-#pragma unroll
-    for (int off = kWave / 2; off >= 1; off >>= 1) {
-        v += __shfl_xor(v, off);
-    }
-    return v;
-}
-
 // Slots s0 .. s0 + kRowsBatch - 1 of the wave's sixteenth (those below `slots`), all requested before any is looked
 // at: slot s, lane l holds routes waveFirst + s * 256 + l * 4 ... + 3.  Elements beyond the table read as 0 (the buffer
 // bound sees to that), which names an expert: the kernel corrects its counts by their number, which it knows, instead

@@ -55,10 +55,7 @@ __device__ __forceinline__ int RowOfRoute(const ScatterArgs &a, int route)
 template <int G>
 __device__ __forceinline__ float GroupMax(float v, float *red, int lane)
 {
-#pragma unroll
-    for (int off = kWave / 2; off >= 1; off >>= 1) {
-        v = fmaxf(v, __shfl_xor(v, off));
-    }
+    v = WaveMax(v);
     if (G > kWave) {
         if ((lane & (kWave - 1)) == 0) {
             red[lane / kWave] = v;
@@ -283,11 +280,7 @@ __device__ __forceinline__ void QuantiseRow(const ScatterArgs &a, const u32x4 (&
             for (int e = 0; e < 8; ++e) {
                 amax = fmaxf(amax, fabsf(f[e]));
             }
-            // 128 columns = 16 neighbouring lanes
-#pragma unroll
-            for (int off = 1; off < 16; off <<= 1) {
-                amax = fmaxf(amax, __shfl_xor(amax, off));
-            }
+            amax = RowMax(amax);        // 128 columns = 16 neighbouring lanes
             const float sc = amax > 0.0f ? __fdiv_rn(amax, 448.0f) : 1.0f;
             out.blockScale[j] = sc;
             // eight quotients by one divisor: what depends on the divisor alone is done once (ep_numerics.hip.h)

@@ -301,13 +301,10 @@ __global__ __launch_bounds__(kThreads) void ep_dispatch_small_route_kernel(Small
         outCounts += (e[j] == expert ? 1 : 0) + (ok && e[j] <= expert ? 0x10000 : 0);
         valid += ok ? 1 : 0;
     }
-#pragma unroll
-    for (int off = kWave / 2; off >= 1; off >>= 1) {
-        rowCounts += __shfl_xor(rowCounts, off);
-        outCounts += __shfl_xor(outCounts, off);
-        if (WT) {
-            valid += __shfl_xor(valid, off);
-        }
+    rowCounts = WaveSum(rowCounts);
+    outCounts = WaveSum(outCounts);
+    if (WT) {
+        valid = WaveSum(valid);
     }
     if (lane == 0) {
         s_sum[wave][0] = rowCounts;

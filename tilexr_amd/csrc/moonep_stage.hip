@@ -543,15 +543,8 @@ __device__ __forceinline__ void ScanPair(int localOpen, int localSize, int (*s_p
 {
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = threadIdx.x / kWave;
-    int inclOpen = localOpen;
-    int inclSize = localSize;
-#pragma unroll
-    for (int off = 1; off < kWave; off <<= 1) {
-        const int upOpen = __shfl_up(inclOpen, off);
-        const int upSize = __shfl_up(inclSize, off);
-        inclOpen += lane >= off ? upOpen : 0;
-        inclSize += lane >= off ? upSize : 0;
-    }
+    const int inclOpen = TileXREp::WaveInclusiveSum(localOpen);
+    const int inclSize = TileXREp::WaveInclusiveSum(localSize);
     if (lane == kWave - 1) {
         s_part[0][wave] = inclOpen;
         s_part[1][wave] = inclSize;
@@ -1111,12 +1104,7 @@ __global__ __launch_bounds__(G) void moon_reduce_kernel(CombineWorld a, int colS
     const int slotQ = travels ? static_cast<int>(where / nvS) : 0;
     const int slotRow = travels ? static_cast<int>(where % nvS) : 0;
     const int slotItems = travels ? 1 + slotCount : 0;
-    int slotFirst = slotItems;                       // inclusive prefix over the K <= 32 slot lanes, then exclusive
-#pragma unroll
-    for (int off = 1; off < kMaxTopK; off <<= 1) {
-        const int below = __shfl_up(slotFirst, off);
-        slotFirst += lane >= off ? below : 0;
-    }
+    int slotFirst = TileXREp::WaveInclusiveSum(slotItems);     // over the K <= 32 slot lanes, then exclusive
     const int total = __builtin_amdgcn_readlane(slotFirst, kMaxTopK - 1);      // lanes from K on add nothing
     slotFirst -= slotItems;
     float sub[kRowVecs][8];                          // sum of the group that is open (groups may span windows)
