@@ -1,4 +1,5 @@
-"""ctypes binding of libtilexr-ep.so: the calls of include/tilexr_ep.h and include/tilexr_api.h for Python callers.
+"""Binding of libtilexr-ep.so: the calls of include/tilexr_ep.h and include/tilexr_api.h for Python callers, through ctypes
+and, for those a program makes per layer, a native module (csrc/py_calls.cpp).
 
 Device memory is passed as torch tensors (or None for optional arguments); `stream` is a torch.cuda.Stream or a stream
 handle (the C ABI rejects a null stream, as the reference does: the default stream is STREAM_LEGACY).  Every function
@@ -65,6 +66,15 @@ class CombineExOptions(C.Structure):
 
 _lib = None
 
+# Calls whose arguments the native module converts, in the order in which its bind() takes their entry points.  Once the
+# library is loaded the module's functions stand in this module's place of those below, which have the same signatures.
+# us a dispatch + combine of 8 tokens x 7168, called eagerly: 12.7 through ctypes, 8.6 this way, 8.0 from a C++ loop.
+_NATIVE = {
+    "dispatch_v2": "TileXRMoeEpDispatchV2", "dispatch_memory_v2": "TileXRMoeEpDispatchMemoryV2",
+    "combine_v2": "TileXRMoeEpCombineV2", "combine_memory_v2": "TileXRMoeEpCombineMemoryV2",
+    "dispatch_memory_ex": "TileXRMoeEpDispatchMemoryEx", "combine_memory_ex": "TileXRMoeEpCombineMemoryEx",
+}
+
 
 def lib():
     """Loads the library once.  Raises if it has not been built: there is no other implementation to fall back to."""
@@ -103,7 +113,24 @@ def lib():
             fn = getattr(_lib, name)
             if name not in ("TileXREpVersion", "TileXREpLastKernelName"):
                 fn.restype = C.c_int
+        try:
+            _bind(_lib)
+        except BaseException:
+            _lib = None
+            raise
     return _lib
+
+
+def _bind(loaded):
+    from .lib import _calls
+    _calls.bind(*(C.cast(getattr(loaded, name), C.c_void_p).value for name in _NATIVE.values()))
+    globals().update({name: getattr(_calls, name) for name in _NATIVE})
+    return _calls
+
+
+def _call(name):
+    """The native form of a call that was made before the library was loaded, or through a name taken before."""
+    return getattr(_bind(lib()), name)
 
 
 def version():
@@ -185,12 +212,11 @@ def dispatch_v2(x, expert_ids, comm, bs, h, top_k, experts, expand_x, assist, to
                 tp_rank_id=0, expert_shard_type=0, shared_expert_num=0, shared_expert_rank_num=0, quant_mode=0,
                 global_bs=0, token_nums_type=1, dynamic_scales=None, tp_recv_counts=None, expand_scales=None,
                 workspace=None):
-    return lib().TileXRMoeEpDispatchV2(
-        _ptr(x), _ptr(expert_ids), _ptr(scales), _ptr(active_mask), _ptr(expert_scales), _h(comm), bs, h, top_k,
-        experts, ep_world_size, ep_rank_id, tp_world_size, tp_rank_id, expert_shard_type, shared_expert_num,
-        shared_expert_rank_num, quant_mode, global_bs, token_nums_type, _ptr(expand_x), _ptr(dynamic_scales),
-        _ptr(assist), _ptr(token_nums), _ptr(recv_counts), _ptr(tp_recv_counts), _ptr(expand_scales),
-        _ptr(workspace), dtype, _stream(stream))
+    return _call("dispatch_v2")(x, expert_ids, comm, bs, h, top_k, experts, expand_x, assist, token_nums, recv_counts,
+                                dtype, stream, scales, active_mask, expert_scales, ep_world_size, ep_rank_id,
+                                tp_world_size, tp_rank_id, expert_shard_type, shared_expert_num,
+                                shared_expert_rank_num, quant_mode, global_bs, token_nums_type, dynamic_scales,
+                                tp_recv_counts, expand_scales, workspace)
 
 
 def dispatch_memory_v2(x, expert_ids, comm, bs, h, top_k, experts, expand_x, assist, token_nums, send_counts, dtype,
@@ -198,12 +224,12 @@ def dispatch_memory_v2(x, expert_ids, comm, bs, h, top_k, experts, expand_x, ass
                        ep_world_size=0, ep_rank_id=0, tp_world_size=1, tp_rank_id=0, expert_shard_type=0,
                        shared_expert_num=0, shared_expert_rank_num=0, quant_mode=0, global_bs=0, token_nums_type=1,
                        dynamic_scales=None, tp_recv_counts=None, expand_scales=None, expand_x_dtype=DT_RESERVED):
-    return lib().TileXRMoeEpDispatchMemoryV2(
-        _ptr(x), _ptr(expert_ids), _ptr(scales), _ptr(active_mask), active_mask_type, _ptr(expert_scales), _h(comm),
-        bs, h, top_k, experts, ep_world_size, ep_rank_id, tp_world_size, tp_rank_id, expert_shard_type,
-        shared_expert_num, shared_expert_rank_num, quant_mode, global_bs, token_nums_type, _ptr(expand_x),
-        _ptr(dynamic_scales), _ptr(assist), _ptr(token_nums), _ptr(send_counts), _ptr(tp_recv_counts),
-        _ptr(expand_scales), dtype, expand_x_dtype, _stream(stream))
+    return _call("dispatch_memory_v2")(x, expert_ids, comm, bs, h, top_k, experts, expand_x, assist, token_nums,
+                                       send_counts, dtype, stream, scales, active_mask, active_mask_type,
+                                       expert_scales, ep_world_size, ep_rank_id, tp_world_size, tp_rank_id,
+                                       expert_shard_type, shared_expert_num, shared_expert_rank_num, quant_mode,
+                                       global_bs, token_nums_type, dynamic_scales, tp_recv_counts, expand_scales,
+                                       expand_x_dtype)
 
 
 def combine(expert_out, assist, recv_counts, comm, bs, h, top_k, experts, y, dtype, stream):
@@ -212,8 +238,8 @@ def combine(expert_out, assist, recv_counts, comm, bs, h, top_k, experts, y, dty
 
 
 def combine_v2(expert_out, assist, recv_counts, comm, bs, h, top_k, experts, y, dtype, stream, workspace=None):
-    return lib().TileXRMoeEpCombineV2(_ptr(expert_out), _ptr(assist), _ptr(recv_counts), _h(comm), bs, h, top_k,
-                                      experts, _ptr(y), _ptr(workspace), dtype, _stream(stream))
+    return _call("combine_v2")(expert_out, assist, recv_counts, comm, bs, h, top_k, experts, y, dtype, stream,
+                               workspace)
 
 
 def combine_memory(expert_out, assist, send_counts, comm, bs, h, top_k, experts, y, dtype, stream):
@@ -225,11 +251,10 @@ def combine_memory_v2(expert_out, assist, send_counts, comm, bs, h, top_k, exper
                       expert_scales=None, active_mask=None, active_mask_type=MASK_NONE, shared_expert_x=None,
                       ep_world_size=0, ep_rank_id=0, tp_world_size=1, tp_rank_id=0, expert_shard_type=0,
                       shared_expert_num=0, shared_expert_rank_num=0, quant_mode=0, global_bs=0):
-    return lib().TileXRMoeEpCombineMemoryV2(
-        _ptr(expert_out), _ptr(assist), _ptr(send_counts), _ptr(expert_scales), _ptr(active_mask), active_mask_type,
-        _ptr(shared_expert_x), _h(comm), bs, h, top_k, experts, ep_world_size, ep_rank_id, tp_world_size, tp_rank_id,
-        expert_shard_type, shared_expert_num, shared_expert_rank_num, quant_mode, global_bs, _ptr(y), dtype,
-        _stream(stream))
+    return _call("combine_memory_v2")(expert_out, assist, send_counts, comm, bs, h, top_k, experts, y, dtype, stream,
+                                      expert_scales, active_mask, active_mask_type, shared_expert_x, ep_world_size,
+                                      ep_rank_id, tp_world_size, tp_rank_id, expert_shard_type, shared_expert_num,
+                                      shared_expert_rank_num, quant_mode, global_bs)
 
 
 # ---- additions -------------------------------------------------------------------------------------------
@@ -238,47 +263,20 @@ def dispatch_memory_ex(x, expert_ids, comm, bs, h, top_k, experts, expand_x, ass
                        active_mask_type=MASK_NONE, dynamic_scales=None, expand_x_dtype=None, row_index_map=None,
                        tile_flags=None, tile_rows=0, meta_ready_event=None):
     """Returns (status, epoch)."""
-    epoch = C.c_int64(0)
-    opt = DispatchExOptions()
-    opt.quantMode = quant_mode
-    opt.expertCapacity = expert_capacity
-    opt.expertTokenNumsType = token_nums_type
-    opt.activeMaskType = active_mask_type
-    opt.xActiveMask = _ptr(active_mask)
-    opt.rowIndexMapOut = _ptr(row_index_map)
-    opt.tileFlagsOut = _ptr(tile_flags)
-    opt.tileRows = tile_rows
-    opt.epochOut = C.pointer(epoch)
-    opt.metaReadyEvent = C.c_void_p(meta_ready_event) if meta_ready_event else None
-    if expand_x_dtype is None:
-        expand_x_dtype = {Q_NONE: dtype, Q_TOKEN_INT8: DT_INT8, Q_MXFP8: DT_FP8E4M3, Q_FP8_BLOCK128: DT_FP8E4M3}.get(
-            quant_mode, dtype)
-    ret = lib().TileXRMoeEpDispatchMemoryEx(_ptr(x), _ptr(expert_ids), _h(comm), bs, h, top_k, experts, C.byref(opt),
-                                            _ptr(expand_x), _ptr(dynamic_scales), _ptr(assist), _ptr(token_nums),
-                                            _ptr(send_counts), dtype, expand_x_dtype, _stream(stream))
-    return ret, epoch.value
+    return _call("dispatch_memory_ex")(x, expert_ids, comm, bs, h, top_k, experts, expand_x, assist, token_nums,
+                                       send_counts, dtype, stream, quant_mode, expert_capacity, token_nums_type,
+                                       active_mask, active_mask_type, dynamic_scales, expand_x_dtype, row_index_map,
+                                       tile_flags, tile_rows, meta_ready_event)
 
 
 def combine_memory_ex(expert_out, assist, send_counts, comm, bs, h, top_k, experts, y, dtype, stream,
                       comm_quant_mode=0, expert_out_quant_mode=0, expert_out_scales=None, expert_scales=None,
                       active_mask=None, active_mask_type=MASK_NONE, shared_expert_x=None, row_index_map=None,
                       tile_flags=None, tile_rows=0, flag_epoch=0, wait_timeout_us=0, device_status=None):
-    opt = CombineExOptions()
-    opt.commQuantMode = comm_quant_mode
-    opt.expertOutQuantMode = expert_out_quant_mode
-    opt.expertOutScales = _ptr(expert_out_scales)
-    opt.expertScales = _ptr(expert_scales)
-    opt.activeMaskType = active_mask_type
-    opt.xActiveMask = _ptr(active_mask)
-    opt.sharedExpertX = _ptr(shared_expert_x)
-    opt.rowIndexMap = _ptr(row_index_map)
-    opt.tileFlags = _ptr(tile_flags)
-    opt.tileRows = tile_rows
-    opt.flagEpoch = flag_epoch
-    opt.waitTimeoutUs = wait_timeout_us
-    opt.deviceStatusOut = _ptr(device_status)
-    return lib().TileXRMoeEpCombineMemoryEx(_ptr(expert_out), _ptr(assist), _ptr(send_counts), _h(comm), bs, h, top_k,
-                                            experts, C.byref(opt), _ptr(y), dtype, _stream(stream))
+    return _call("combine_memory_ex")(expert_out, assist, send_counts, comm, bs, h, top_k, experts, y, dtype, stream,
+                                      comm_quant_mode, expert_out_quant_mode, expert_out_scales, expert_scales,
+                                      active_mask, active_mask_type, shared_expert_x, row_index_map, tile_flags,
+                                      tile_rows, flag_epoch, wait_timeout_us, device_status)
 
 
 K_COUNT, K_PLACE, K_SCATTER, K_INVERT, K_REDUCE = range(5)
