@@ -70,6 +70,15 @@ __global__ __launch_bounds__(kSmallReduceThreads) void ep_reduce_small_kernel(Sm
     }
     const int held = a.counts[a.lastCount];
     const bool active = a.tokenMask == nullptr || a.tokenMask[token] != 0;
+    // ... and the shared expert's row, which the sum needs last (asked for there it was a trip to memory of its own)
+    const int colBase = wave * (kWave * V);
+    const __amdgpu_buffer_rsrc_t sharedRow = RowResource(static_cast<const char *>(a.sharedExpertX) +
+        (a.sharedExpertX != nullptr ? static_cast<int64_t>(token) * a.h * 2 : 0), a.sharedExpertX != nullptr ? vecs * 16 : 0);
+    u32x4 shared[V];
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+        shared[j] = __builtin_amdgcn_raw_buffer_load_b128(sharedRow, (colBase + j * kWave + lane) * 16, 0, 0);
+    }
     if (tid < kMaxTopK) {
         s_row[tid] = -1;
     }
@@ -99,7 +108,6 @@ __global__ __launch_bounds__(kSmallReduceThreads) void ep_reduce_small_kernel(Sm
         }
     }
     __syncthreads();
-    const int colBase = wave * (kWave * V);
     if (colBase >= vecs) {
         return;
     }
@@ -161,18 +169,12 @@ __global__ __launch_bounds__(kSmallReduceThreads) void ep_reduce_small_kernel(Sm
         }
     }
     if (a.sharedExpertX != nullptr && active) {
-        const u32x4 *sx = reinterpret_cast<const u32x4 *>(static_cast<const char *>(a.sharedExpertX) +
-            static_cast<int64_t>(token) * a.h * 2);
 #pragma unroll
         for (int j = 0; j < V; ++j) {
-            const int idx = colBase + j * kWave + lane;
-            if (idx < vecs) {
-                const u32x4 v = sx[idx];
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    acc[j][2 * q] = __fadd_rn(acc[j][2 * q], Decode16<BF16>(v[q] & 0xffffu));
-                    acc[j][2 * q + 1] = __fadd_rn(acc[j][2 * q + 1], Decode16<BF16>(v[q] >> 16));
-                }
+            for (int q = 0; q < 4; ++q) {
+                acc[j][2 * q] = __fadd_rn(acc[j][2 * q], Decode16<BF16>(shared[j][q] & 0xffffu));
+                acc[j][2 * q + 1] = __fadd_rn(acc[j][2 * q + 1], Decode16<BF16>(shared[j][q] >> 16));
             }
         }
     }
