@@ -205,6 +205,16 @@ int SlicesOf(const ReduceLaunch &l, int ranks)
     return few ? slices : 1;
 }
 
+// Whether a workgroup is one wave with one unit.  Sliced rows: many small workgroups reach the highest gather bandwidth here.
+// Narrow rows that a single-launch dispatch wrote, too: their tokens can then run on the XCD that wrote them (PlacesByXcd;
+// eight layers in a graph, 1024 columns, top-8, us: 4 tokens 54.5 -> 50.9, 100 tokens 64.3 -> 58.8, 250 tokens 81.1 -> 75.1).
+// Beyond, four neighbouring tokens to a workgroup follow the per-token scatter, which has them so (600 x 1024 11.2 us, 13.3
+// with a wave each).
+bool WaveUnits(const ReduceLaunch &l, int slices, int ranks)
+{
+    return slices > 1 || (l.tileFlags == nullptr && ranks == 1 && l.bs * (l.topK + l.sharedSlots) <= kSmallRoutes);
+}
+
 // 16-byte vectors per lane of a wave that takes one of `slices` slices.
 int VecsPerLane(int64_t vecs, int slices)
 {
@@ -233,6 +243,7 @@ hipError_t LaunchReduceWorld(const ReduceLaunch *ls, int ranks)
     for (int r = 0; r < ranks; ++r) {
         w.rank[r] = ArgsOf(ls[r]);
         w.rank[r].colSlices = slices;
+        w.rank[r].waveUnits = WaveUnits(ls[0], slices, ranks) ? 1 : 0;
         if (ls[r].kernelNameOut != nullptr) {
             *ls[r].kernelNameOut = "ep_reduce_vec_world_kernel";
         }
@@ -284,6 +295,7 @@ hipError_t LaunchReduce(const ReduceLaunch &l)
             }
         } else {
             a.colSlices = SlicesOf(l, 1);
+            a.waveUnits = WaveUnits(l, a.colSlices, 1) ? 1 : 0;
             LaunchVecKernels(kWave, VecsPerLane(vecs, a.colSlices), l, a, gridLimit, nullptr, 1);
         }
     } else {

@@ -35,6 +35,7 @@ struct ReduceArgs {
     int slots;                       // rows summed per token: topK routed ones, then the shared-expert slots
     void *y;
     int colSlices;                   // slices a row is cut into (vec kernel, wide rows), else 1
+    int waveUnits;                   // vec kernel: workgroups of one wave, one unit each
     const uint64_t *tileFlags;
     int tileRows;
     int tileShift;                   // log2(tileRows) where that is a whole number, else -1

@@ -34,7 +34,7 @@ namespace {
 // (decode): a wave that has a SIMD to itself gains nothing from small registers, and a token's rows arrive in one
 // round trip instead of two.
 //
-// Launches with sliced rows (single-wave workgroups) that do not wait place their units by XCD: workgroup b runs on
+// Launches of single-wave workgroups that do not wait place their units by XCD: workgroup b runs on
 // XCD b % 8 and takes a slice of a token t with t % 8 == b % 8, as the dispatch kernels do with a token's routes, so that
 // rows which still sit in the L2 of the XCD that wrote them are read there (the eight L2s are not one cache: rows
 // written on one XCD and read on another travel through memory).  128 tokens x 7168 x top-8, dispatch and combine in
@@ -43,12 +43,11 @@ namespace {
 template <bool FL>
 __host__ __device__ inline bool PlacesByXcd(const ReduceArgs &a, int lanesPerUnit)
 {
-    // sliced rows are launched with one wave per workgroup and one unit per wave; a launch that may wait has whole
-    // workgroups per token and claims them as they become ready.  Up to three times the L2s' 32 MB of rows: beyond that
+    // a launch that may wait has whole workgroups per token and claims them as they become ready.  Up to three times the L2s' 32 MB of rows: beyond that
     // nothing is left to find there, and consecutive workgroups that read consecutive slices of the same rows are the
     // better order for memory (4096 tokens x 7168 x top-8: 88.7 us against 90.3 us placed by XCD)
     constexpr int64_t kPlacedRowBytes = int64_t{96} << 20;
-    return lanesPerUnit == kWave && a.colSlices > 1 && (!FL || a.flagsSettled != 0) &&
+    return lanesPerUnit == kWave && a.waveUnits != 0 && (!FL || a.flagsSettled != 0) &&
         static_cast<int64_t>(a.bs) * a.slots * a.rowBytes <= kPlacedRowBytes;
 }
 
@@ -70,11 +69,11 @@ __device__ __forceinline__ void ReduceVec(const ReduceArgs &a)
     constexpr int KB = WIDE ? 8 : (G == kThreads ? 4 : (V <= 2 ? 4 : (V <= 4 ? 2 : 1)));
     const int vecs = a.h / 8;
     // a unit is one token, or -- for wide rows -- one slice of G * V vectors of a token
-    // A launch for sliced rows has single-wave workgroups, every other one kThreads lanes.  That is told from the slices and
-    // not from blockDim, which in a function that two kernels share is read from the implicit arguments: a scalar and then
+    // A launch for sliced rows, and a small one, has single-wave workgroups, every other one kThreads lanes.  That is told from
+    // the arguments and not from blockDim, which in a function that two kernels share is read from the implicit arguments: a scalar and then
     // a vector load that everything below waits for (eight decode layers of 128 x 7168 in a graph: 101.7 us that way,
     // 101.0 us this way).
-    const int unitsPerGroup = G == kThreads || a.colSlices > 1 ? 1 : kThreads / G;
+    const int unitsPerGroup = G == kThreads || a.waveUnits != 0 ? 1 : kThreads / G;
     const bool byXcd = PlacesByXcd<FL>(a, G);
     const int units = byXcd ? XcdPlacedUnits(a.bs, a.colSlices) : a.bs * a.colSlices;
     const int groups = (units + unitsPerGroup - 1) / unitsPerGroup;
@@ -340,8 +339,7 @@ void LaunchVec(const ReduceArgs &a, int gridLimit, const WorldReduceArgs *world,
         }
         hipLaunchKernelGGL((ep_reduce_vec_kernel<G, V, KIND, BF16, COMMQ, true>), dim3(grid), dim3(kThreads), 0, stream, a);
     } else {
-        // sliced rows: one wave per workgroup, so that no wave waits at a barrier for another slice's rows
-        const int threads = a.colSlices > 1 ? G : kThreads;
+        const int threads = a.waveUnits != 0 ? G : kThreads;
         const int perGroup = threads / G;
         int64_t units = static_cast<int64_t>(a.bs) * a.colSlices;
         bool wide = false;
