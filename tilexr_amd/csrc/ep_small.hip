@@ -46,16 +46,37 @@ struct SmallArgs {
     TilePublishArgs tiles;       // flags == nullptr: none (totalRows is filled in by the kernels)
 };
 
-// A row's vectors: streaming stores, or -- when readiness flags are published -- stores written through to memory, which
-// are complete for every XCD once the issuing wave's memory counter is zero.
-template <bool WT>
-__device__ __forceinline__ void SmallRowStore(const u32x4 &v, u32x4 *dst, __amdgpu_buffer_rsrc_t rsrc, int idx)
+// The lane's vectors of a row.  AUX, the cache policy: published rows are written through to memory (kAuxAgentScope) and are
+// complete for every XCD once the issuing wave's memory counter is zero.  Others stream (kAuxNonTemporal), or -- while token rows
+// and rows of the call together are few (LeavesRowsToL2) -- are left to the L2 (0), where the combine that runs on the same XCD
+// finds them.
+template <int V, int AUX>
+__device__ __forceinline__ void SmallRowStore(const SmallArgs &a, int row, const u32x4 (&v)[V])
 {
-    if (WT) {
-        __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, idx * 16, 0, kAuxAgentScope);
-    } else {
-        __builtin_nontemporal_store(v, dst + idx);
+    const int vecs = a.h / 8;
+    u32x4 *dst = reinterpret_cast<u32x4 *>(static_cast<char *>(a.out) + static_cast<int64_t>(row) * a.h * 2);
+    const __amdgpu_buffer_rsrc_t rsrc = RowResource(dst, vecs * 16);
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+        const int idx = j * kThreads + static_cast<int>(threadIdx.x);
+        if (idx >= vecs) {
+            continue;
+        }
+        if constexpr (AUX == kAuxNonTemporal) {
+            __builtin_nontemporal_store(v[j], dst + idx);
+        } else {
+            __builtin_amdgcn_raw_buffer_store_b128(v[j], rsrc, idx * 16, 0, AUX);
+        }
     }
+}
+
+// us for eight layers in a graph, streaming and left to the L2: 4 x 7168 x top-8 53.5 -> 52.4, 17 x 7168 (2.2 MB with the token
+// rows) 57.6 -> 56.6, 30 x 4096 56.5 -> 55.5, 60 x 4096 x top-2 (1.5 MB) 51.2 -> 49.8, top-4
+// (2.5 MB) 54.2 -> 53.4; but 60 x 8192 x top-2 (2.9 MB) 55.5 and
+// 57.6, 100 x 2048 (3.7 MB) 62.3 and 64.0, 100 x 7168 88.1 and 99.6.
+inline bool LeavesRowsToL2(const SmallDispatchLaunch &l)
+{
+    return l.bs * (l.topK + 1) * l.h * 2 <= (int64_t{10} << 18);
 }
 
 // Masked calls: first route that a token-prefix mask leaves out (n for a mask per route).  The mask is read beside the id
@@ -204,15 +225,7 @@ __global__ __launch_bounds__(kThreads) void ep_dispatch_small_kernel(SmallArgs a
         if (row < 0) {
             continue;
         }
-        u32x4 *dst = reinterpret_cast<u32x4 *>(static_cast<char *>(a.out) + static_cast<int64_t>(row) * a.h * 2);
-        const __amdgpu_buffer_rsrc_t rsrc = RowResource(dst, vecs * 16);
-#pragma unroll
-        for (int j = 0; j < V; ++j) {
-            const int idx = j * kThreads + tid;
-            if (idx < vecs) {
-                SmallRowStore<WT>(v[j], dst, rsrc, idx);
-            }
-        }
+        SmallRowStore<V, WT ? kAuxAgentScope : kAuxNonTemporal>(a, row, v);
     }
     if (WT) {
         // every wave waits for its own stores, the barrier collects the waves, then the rows are reported landed
@@ -242,9 +255,10 @@ __global__ __launch_bounds__(kThreads) void ep_dispatch_small_kernel(SmallArgs a
 // MASKED: the routes a mask leaves out are dropped from the counts like ids outside [0, E) (token-prefix mask: one more
 // LDS exchange, for the number of active tokens).  200 tokens x 7168 x top-8 of 256 with a token mask: 6.7 us, 13.3 us
 // for the count and scatter launches such calls took before.
-template <int V, bool WT, int IDS, bool MASKED>
+template <int V, int AUX, int IDS, bool MASKED>
 __global__ __launch_bounds__(kThreads) void ep_dispatch_small_route_kernel(SmallArgs a)
 {
+    constexpr bool WT = AUX == kAuxAgentScope;
     __shared__ int s_live[kWavesPerBlock];
     __shared__ int s_sum[kWavesPerBlock][3];     // per wave: smaller | earlier equal << 16, equal to blockIdx | not above << 16, valid
 
@@ -339,15 +353,7 @@ __global__ __launch_bounds__(kThreads) void ep_dispatch_small_route_kernel(Small
     if (row < 0) {
         return;
     }
-    u32x4 *dst = reinterpret_cast<u32x4 *>(static_cast<char *>(a.out) + static_cast<int64_t>(row) * a.h * 2);
-    const __amdgpu_buffer_rsrc_t rsrc = RowResource(dst, vecs * 16);
-#pragma unroll
-    for (int j = 0; j < V; ++j) {
-        const int idx = j * kThreads + tid;
-        if (idx < vecs) {
-            SmallRowStore<WT>(v[j], dst, rsrc, idx);
-        }
-    }
+    SmallRowStore<V, AUX>(a, row, v);
     if (WT) {
         WaitOwnStores();
         __syncthreads();        // uniform: a workgroup without a row has left as a whole
@@ -411,15 +417,24 @@ hipError_t LaunchSmallDispatch(const SmallDispatchLaunch &l)
         }
         const dim3 routes(static_cast<unsigned>(std::max<int64_t>(XcdPlacedUnits(static_cast<int>(l.bs), static_cast<int>(l.topK)), l.numExperts)));
         const bool few = l.bs * l.topK <= 4 * kThreads;
-        auto pickMasked = [&](auto vecsPerLane, auto masked) {
+        const bool plain = LeavesRowsToL2(l);
+        auto pickStores = [&](auto vecsPerLane, auto masked, auto ids) {
             constexpr int kV = decltype(vecsPerLane)::value;
+            constexpr int kIds = decltype(ids)::value;
             constexpr bool kMasked = decltype(masked)::value;
-            if (few) {
-                flags ? launch(ep_dispatch_small_route_kernel<kV, true, 4, kMasked>, routes) :
-                        launch(ep_dispatch_small_route_kernel<kV, false, 4, kMasked>, routes);
+            if (flags) {
+                launch(ep_dispatch_small_route_kernel<kV, kAuxAgentScope, kIds, kMasked>, routes);
+            } else if (plain) {
+                launch(ep_dispatch_small_route_kernel<kV, 0, kIds, kMasked>, routes);
             } else {
-                flags ? launch(ep_dispatch_small_route_kernel<kV, true, kIdsPerLane, kMasked>, routes) :
-                        launch(ep_dispatch_small_route_kernel<kV, false, kIdsPerLane, kMasked>, routes);
+                launch(ep_dispatch_small_route_kernel<kV, kAuxNonTemporal, kIds, kMasked>, routes);
+            }
+        };
+        auto pickMasked = [&](auto vecsPerLane, auto masked) {
+            if (few) {
+                pickStores(vecsPerLane, masked, std::integral_constant<int, 4> {});
+            } else {
+                pickStores(vecsPerLane, masked, std::integral_constant<int, kIdsPerLane> {});
             }
         };
         auto pick = [&](auto vecsPerLane) {
