@@ -2,8 +2,9 @@
 //
 // HBM-bound row movement, no MFMA.  A plan names the destination row of every route directly, so there is nothing to
 // count: dispatch is one read of each token row and one write per route; combine is one read per route and one write
-// per token.  Row copies use two 16-byte loads and two 16-byte stores per lane, and the workgroups of one token are
-// given block indices that land on one XCD (block b runs on XCD b % 8) so the token row is read from HBM once.
+// per token.  Rows are copied either per token, each row read once and stored once per route, or per route, where the
+// workgroups of one token are given block indices that land on one XCD (block b runs on XCD b % 8) so that the token row is
+// read from HBM once (LaunchMoonDispatch says which).
 // Every kernel is launched once for the whole world: blockIdx.y is the rank whose share the workgroup works on.
 //
 //   what is computed  reference: src/moonep/dispatch/kernels/tilexr_moonep_dispatch_kernel.cpp:108-147, 268-461
