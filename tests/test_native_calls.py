@@ -164,3 +164,98 @@ def test_what_is_refused(calls):
     assert module.combine_v2(*ok[:3], closed, *ok[4:]) == 5
     # integers are taken as the C types take them
     assert module.combine_v2(*ok[:4], -1, 1 << 64, *ok[6:]) == 5
+
+
+class Index:
+    def __index__(self):
+        return 6
+
+
+class Parameter:
+    def __init__(self, inner):
+        self._as_parameter_ = inner
+
+
+def _integers():
+    np, torch = pytest.importorskip("numpy"), pytest.importorskip("torch")
+    return [True, np.int64(3), np.int32(-4), np.uint64(2 ** 64 - 1), np.array(5), np.array([5]), np.float64(2.0), torch.tensor(7),
+            torch.tensor([8]), torch.tensor([1, 2]).max(), torch.tensor(9.0), torch.tensor([1, 2]), Index(), C.c_int64(11), C.c_int32(12),
+            C.c_uint64(13), C.c_int16(14), Parameter(15), Parameter(Index()), Parameter(C.c_int64(16)), Parameter(C.c_int32(17)),
+            Parameter(Parameter(18)), Parameter("text"), 1.5, "1", b"1", None, 1 << 70, -(1 << 63)]
+
+
+class Field(C.Structure):
+    _fields_ = [("v", C.c_int64)]
+
+
+def _as_ctypes_takes_it(value, name, param):
+    """What the ctypes binding of the entry point makes of an argument; a TypeError where it refuses it."""
+    if name.endswith("_ex") and param in ("quant_mode", "expert_capacity", "token_nums_type", "active_mask_type", "tile_rows", "comm_quant_mode",
+                                          "expert_out_quant_mode", "flag_epoch", "wait_timeout_us"):
+        f = Field()
+        f.v = value
+        return f.v
+    ctype = C.c_int32 if param in ("dtype", "expand_x_dtype") else C.c_int64
+    seen = []
+    keep = C.CFUNCTYPE(None, ctype)(seen.append)
+    raw = C.cast(keep, C.c_void_p).value
+    call = C.CFUNCTYPE(None, C.c_int64)(raw) if ctype is C.c_int64 else C.CFUNCTYPE(None, C.c_int32)(raw)
+    try:
+        call(value)
+    except C.ArgumentError as e:
+        raise TypeError(str(e))
+    return seen[0]
+
+
+@pytest.mark.parametrize("name", NAMES)
+def test_integers_are_those_that_ctypes_takes(name, calls):
+    """Every integer argument of every call, given as whatever a program may have a size in: taken, with the value, where ctypes
+    takes it, and refused where it is not."""
+    module, stub = calls
+    sig = inspect.signature(PYTHON_FORMS[name]).parameters
+    required = {p: 3 if p in ("bs", "h", "top_k", "experts", "dtype") else None for p, q in sig.items() if q.default is inspect._empty}
+    integers = [p for p, q in sig.items() if required.get(p) == 3 or (isinstance(q.default, int) and p != "meta_ready_event")]
+    if name.startswith("dispatch_memory"):
+        integers = sorted({*integers, "expand_x_dtype"})
+    assert len(integers) > 4
+    for param in integers:
+        for value in _integers():
+            if value is None and param == "expand_x_dtype":
+                continue            # None stands for the payload type of the mode there
+            try:
+                want = _as_ctypes_takes_it(value, name, param)
+            except TypeError:
+                with pytest.raises(TypeError):
+                    getattr(module, name)(**{**required, param: value})
+                continue
+            getattr(module, name)(**{**required, param: value})
+            got = _seen(stub)[ORDER[name].split().index(param)]
+            # the element types are an enumeration of 32 bits, whose sign is the compiler's choice
+            assert (got - want) % (1 << 32 if param in ("dtype", "expand_x_dtype") else 1 << 64) == 0, (param, value)
+
+
+def test_addresses_that_are_not_plain(calls):
+    module, stub = calls
+    ok = [None, None, None, None, 1, 2, 3, 4, None, 3, None]
+
+    class Null:
+        cuda_stream = None
+
+        def data_ptr(self):
+            return None
+
+    raw = Comm()
+    raw.handle = 0xC034
+    assert module.combine_v2(*ok[:3], raw, *ok[4:]) == 5
+    assert _seen(stub)[3] == 0xC034
+    assert module.combine_v2(Null(), *ok[1:-1], Null()) == 5
+    assert _seen(stub)[0] == 0 and _seen(stub)[-1] == 0
+    event = dict(zip("x expert_ids comm bs h top_k experts expand_x assist token_nums send_counts dtype stream".split(),
+                     [None, None, None, 1, 2, 3, 4, None, None, None, None, 3, None]))
+    at = ORDER["dispatch_memory_ex"].split().index("meta_ready_event")
+    for value, want in ((None, 0), (0, 0), (False, 0), ((), 0), (0xE7E, 0xE7E)):
+        module.dispatch_memory_ex(**event, meta_ready_event=value)
+        assert _seen(stub)[at] == want
+    for value in (1.5, "event", object()):
+        with pytest.raises(TypeError):
+            module.dispatch_memory_ex(**event, meta_ready_event=value)

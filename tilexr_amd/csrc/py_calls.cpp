@@ -14,12 +14,17 @@
 
 namespace {
 
+// What a parameter takes.  Integers are what ctypes takes for the C type: an int, an object with __index__ (numpy integers,
+// integer tensors of one element), an instance of that ctypes type, or an object whose _as_parameter_ is one of these.
 enum class Kind {
     kPointer,       // None, an address, or an object with data_ptr()
-    kInt,
-    kIntOrNone,
+    kInt64,
+    kInt32,
+    kField,         // a 64-bit integer that becomes a field of an options struct: no _as_parameter_
+    kInt32OrNone,
+    kEvent,         // an address, or anything false for none
     kStream,        // None, an address, or an object with cuda_stream
-    kComm,          // None, an address, or an object whose `handle` is None or has an integer `value`
+    kComm,          // None, an address, or an object whose `handle` is None, an address or has an integer `value`
 };
 
 struct Param {
@@ -29,7 +34,7 @@ struct Param {
 };
 
 constexpr int kMaxParams = 40;
-constexpr int64_t kNone = INT64_MIN;        // a kIntOrNone argument that is None
+constexpr int64_t kNone = INT64_MIN;        // a kInt32OrNone argument that is None
 
 struct Function {
     const char *name;
@@ -39,7 +44,8 @@ struct Function {
     PyObject *names[kMaxParams];            // interned
 };
 
-PyObject *gDataPtr, *gCudaStream, *gHandle, *gValue;
+PyObject *gDataPtr, *gCudaStream, *gHandle, *gValue, *gAsParameter;
+PyObject *gCInt64, *gCInt32;            // ctypes.c_int64, ctypes.c_int32
 
 struct Entries {
     decltype(&TileXRMoeEpDispatchV2) dispatchV2;
@@ -62,20 +68,59 @@ bool FromInt(PyObject *o, int64_t *out)
     return !PyErr_Occurred();
 }
 
+// What data_ptr(), cuda_stream or value gave (a new reference): an address, None for a null one.
 bool FromResult(PyObject *o, int64_t *out)
 {
-    const bool ok = o != nullptr && FromInt(o, out);
+    *out = 0;
+    const bool ok = o != nullptr && (o == Py_None || FromInt(o, out));
     Py_XDECREF(o);
     return ok;
 }
 
+bool FromInteger(PyObject *o, Kind kind, int64_t *out)
+{
+    if (PyLong_Check(o)) {
+        return FromInt(o, out);
+    }
+    if (PyIndex_Check(o)) {
+        PyObject *index = PyNumber_Index(o);
+        return index != nullptr && FromResult(index, out);
+    }
+    const int ofType = PyObject_IsInstance(o, kind == Kind::kInt64 || kind == Kind::kField ? gCInt64 : gCInt32);
+    if (ofType != 0) {
+        return ofType > 0 && FromResult(PyObject_GetAttr(o, gValue), out);
+    }
+    PyObject *inner = kind == Kind::kField ? nullptr : PyObject_GetAttr(o, gAsParameter);
+    if (inner != nullptr) {
+        bool ok = false;
+        if (Py_EnterRecursiveCall(" while taking _as_parameter_") == 0) {
+            ok = FromInteger(inner, kind, out);
+            Py_LeaveRecursiveCall();
+        }
+        Py_DECREF(inner);
+        return ok;
+    }
+    if (PyErr_Occurred() && !PyErr_ExceptionMatches(PyExc_AttributeError)) {
+        return false;
+    }
+    PyErr_Clear();
+    return FromInt(o, out);         // says what it is not
+}
+
 bool Convert(PyObject *o, Kind kind, int64_t *out)
 {
-    if (kind != Kind::kInt && o == Py_None) {
-        *out = kind == Kind::kIntOrNone ? kNone : 0;
+    if (kind == Kind::kInt64 || kind == Kind::kInt32 || kind == Kind::kField || (kind == Kind::kInt32OrNone && o != Py_None)) {
+        const bool ok = FromInteger(o, kind, out);
+        if (ok && kind != Kind::kInt64 && kind != Kind::kField) {
+            *out = static_cast<int32_t>(*out);      // kNone is no value of it
+        }
+        return ok;
+    }
+    if (o == Py_None) {
+        *out = kind == Kind::kInt32OrNone ? kNone : 0;
         return true;
     }
-    if (kind == Kind::kInt || kind == Kind::kIntOrNone || PyLong_Check(o)) {
+    if (PyLong_Check(o)) {
         return FromInt(o, out);
     }
     if (kind == Kind::kPointer) {
@@ -84,17 +129,17 @@ bool Convert(PyObject *o, Kind kind, int64_t *out)
     if (kind == Kind::kStream) {
         return FromResult(PyObject_GetAttr(o, gCudaStream), out);
     }
-    PyObject *handle = PyObject_GetAttr(o, gHandle);
-    if (handle == nullptr) {
-        return false;
-    }
-    PyObject *value = handle == Py_None ? Py_NewRef(Py_None) : PyObject_GetAttr(handle, gValue);
-    Py_DECREF(handle);
-    if (value == Py_None) {
-        Py_DECREF(value);
+    if (kind == Kind::kEvent) {
+        const int given = PyObject_IsTrue(o);
         *out = 0;
-        return true;
+        return given == 0 || (given > 0 && FromInt(o, out));
     }
+    PyObject *handle = PyObject_GetAttr(o, gHandle);
+    if (handle == nullptr || handle == Py_None || PyLong_Check(handle)) {
+        return FromResult(handle, out);
+    }
+    PyObject *value = PyObject_GetAttr(handle, gValue);
+    Py_DECREF(handle);
     return FromResult(value, out);
 }
 
@@ -200,13 +245,13 @@ using K = Kind;
 
 // ---- dispatch_v2 ---------------------------------------------------------------------------------------------------
 const Param kDispatchV2[] = {
-    {"x", K::kPointer, 0}, {"expert_ids", K::kPointer, 0}, {"comm", K::kComm, 0}, {"bs", K::kInt, 0}, {"h", K::kInt, 0},
-    {"top_k", K::kInt, 0}, {"experts", K::kInt, 0}, {"expand_x", K::kPointer, 0}, {"assist", K::kPointer, 0},
-    {"token_nums", K::kPointer, 0}, {"recv_counts", K::kPointer, 0}, {"dtype", K::kInt, 0}, {"stream", K::kStream, 0},
+    {"x", K::kPointer, 0}, {"expert_ids", K::kPointer, 0}, {"comm", K::kComm, 0}, {"bs", K::kInt64, 0}, {"h", K::kInt64, 0},
+    {"top_k", K::kInt64, 0}, {"experts", K::kInt64, 0}, {"expand_x", K::kPointer, 0}, {"assist", K::kPointer, 0},
+    {"token_nums", K::kPointer, 0}, {"recv_counts", K::kPointer, 0}, {"dtype", K::kInt32, 0}, {"stream", K::kStream, 0},
     {"scales", K::kPointer, 0}, {"active_mask", K::kPointer, 0}, {"expert_scales", K::kPointer, 0},
-    {"ep_world_size", K::kInt, 0}, {"ep_rank_id", K::kInt, 0}, {"tp_world_size", K::kInt, 0}, {"tp_rank_id", K::kInt, 0},
-    {"expert_shard_type", K::kInt, 0}, {"shared_expert_num", K::kInt, 0}, {"shared_expert_rank_num", K::kInt, 0},
-    {"quant_mode", K::kInt, 0}, {"global_bs", K::kInt, 0}, {"token_nums_type", K::kInt, 1},
+    {"ep_world_size", K::kInt64, 0}, {"ep_rank_id", K::kInt64, 0}, {"tp_world_size", K::kInt64, 0}, {"tp_rank_id", K::kInt64, 0},
+    {"expert_shard_type", K::kInt64, 0}, {"shared_expert_num", K::kInt64, 0}, {"shared_expert_rank_num", K::kInt64, 0},
+    {"quant_mode", K::kInt64, 0}, {"global_bs", K::kInt64, 0}, {"token_nums_type", K::kInt64, 1},
     {"dynamic_scales", K::kPointer, 0}, {"tp_recv_counts", K::kPointer, 0}, {"expand_scales", K::kPointer, 0},
     {"workspace", K::kPointer, 0},
 };
@@ -223,16 +268,16 @@ PyObject *DispatchV2(PyObject *, PyObject *const *args, Py_ssize_t nargs, PyObje
 
 // ---- dispatch_memory_v2 --------------------------------------------------------------------------------------------
 const Param kDispatchMemoryV2[] = {
-    {"x", K::kPointer, 0}, {"expert_ids", K::kPointer, 0}, {"comm", K::kComm, 0}, {"bs", K::kInt, 0}, {"h", K::kInt, 0},
-    {"top_k", K::kInt, 0}, {"experts", K::kInt, 0}, {"expand_x", K::kPointer, 0}, {"assist", K::kPointer, 0},
-    {"token_nums", K::kPointer, 0}, {"send_counts", K::kPointer, 0}, {"dtype", K::kInt, 0}, {"stream", K::kStream, 0},
-    {"scales", K::kPointer, 0}, {"active_mask", K::kPointer, 0}, {"active_mask_type", K::kInt, TileXREp::TILEXR_EP_ACTIVE_MASK_NONE},
-    {"expert_scales", K::kPointer, 0}, {"ep_world_size", K::kInt, 0}, {"ep_rank_id", K::kInt, 0},
-    {"tp_world_size", K::kInt, 1}, {"tp_rank_id", K::kInt, 0}, {"expert_shard_type", K::kInt, 0},
-    {"shared_expert_num", K::kInt, 0}, {"shared_expert_rank_num", K::kInt, 0}, {"quant_mode", K::kInt, 0},
-    {"global_bs", K::kInt, 0}, {"token_nums_type", K::kInt, 1}, {"dynamic_scales", K::kPointer, 0},
+    {"x", K::kPointer, 0}, {"expert_ids", K::kPointer, 0}, {"comm", K::kComm, 0}, {"bs", K::kInt64, 0}, {"h", K::kInt64, 0},
+    {"top_k", K::kInt64, 0}, {"experts", K::kInt64, 0}, {"expand_x", K::kPointer, 0}, {"assist", K::kPointer, 0},
+    {"token_nums", K::kPointer, 0}, {"send_counts", K::kPointer, 0}, {"dtype", K::kInt32, 0}, {"stream", K::kStream, 0},
+    {"scales", K::kPointer, 0}, {"active_mask", K::kPointer, 0}, {"active_mask_type", K::kInt64, TileXREp::TILEXR_EP_ACTIVE_MASK_NONE},
+    {"expert_scales", K::kPointer, 0}, {"ep_world_size", K::kInt64, 0}, {"ep_rank_id", K::kInt64, 0},
+    {"tp_world_size", K::kInt64, 1}, {"tp_rank_id", K::kInt64, 0}, {"expert_shard_type", K::kInt64, 0},
+    {"shared_expert_num", K::kInt64, 0}, {"shared_expert_rank_num", K::kInt64, 0}, {"quant_mode", K::kInt64, 0},
+    {"global_bs", K::kInt64, 0}, {"token_nums_type", K::kInt64, 1}, {"dynamic_scales", K::kPointer, 0},
     {"tp_recv_counts", K::kPointer, 0}, {"expand_scales", K::kPointer, 0},
-    {"expand_x_dtype", K::kInt, TileXR::TILEXR_DATA_TYPE_RESERVED},
+    {"expand_x_dtype", K::kInt32, TileXR::TILEXR_DATA_TYPE_RESERVED},
 };
 Function gDispatchMemoryV2 {"dispatch_memory_v2", kDispatchMemoryV2, 13, sizeof(kDispatchMemoryV2) / sizeof(Param), {}};
 
@@ -249,8 +294,8 @@ PyObject *DispatchMemoryV2(PyObject *, PyObject *const *args, Py_ssize_t nargs, 
 // ---- combine_v2 ----------------------------------------------------------------------------------------------------
 const Param kCombineV2[] = {
     {"expert_out", K::kPointer, 0}, {"assist", K::kPointer, 0}, {"recv_counts", K::kPointer, 0}, {"comm", K::kComm, 0},
-    {"bs", K::kInt, 0}, {"h", K::kInt, 0}, {"top_k", K::kInt, 0}, {"experts", K::kInt, 0}, {"y", K::kPointer, 0},
-    {"dtype", K::kInt, 0}, {"stream", K::kStream, 0}, {"workspace", K::kPointer, 0},
+    {"bs", K::kInt64, 0}, {"h", K::kInt64, 0}, {"top_k", K::kInt64, 0}, {"experts", K::kInt64, 0}, {"y", K::kPointer, 0},
+    {"dtype", K::kInt32, 0}, {"stream", K::kStream, 0}, {"workspace", K::kPointer, 0},
 };
 Function gCombineV2 {"combine_v2", kCombineV2, 11, sizeof(kCombineV2) / sizeof(Param), {}};
 
@@ -265,12 +310,12 @@ PyObject *CombineV2(PyObject *, PyObject *const *args, Py_ssize_t nargs, PyObjec
 // ---- combine_memory_v2 ---------------------------------------------------------------------------------------------
 const Param kCombineMemoryV2[] = {
     {"expert_out", K::kPointer, 0}, {"assist", K::kPointer, 0}, {"send_counts", K::kPointer, 0}, {"comm", K::kComm, 0},
-    {"bs", K::kInt, 0}, {"h", K::kInt, 0}, {"top_k", K::kInt, 0}, {"experts", K::kInt, 0}, {"y", K::kPointer, 0},
-    {"dtype", K::kInt, 0}, {"stream", K::kStream, 0}, {"expert_scales", K::kPointer, 0}, {"active_mask", K::kPointer, 0},
-    {"active_mask_type", K::kInt, TileXREp::TILEXR_EP_ACTIVE_MASK_NONE}, {"shared_expert_x", K::kPointer, 0},
-    {"ep_world_size", K::kInt, 0}, {"ep_rank_id", K::kInt, 0}, {"tp_world_size", K::kInt, 1}, {"tp_rank_id", K::kInt, 0},
-    {"expert_shard_type", K::kInt, 0}, {"shared_expert_num", K::kInt, 0}, {"shared_expert_rank_num", K::kInt, 0},
-    {"quant_mode", K::kInt, 0}, {"global_bs", K::kInt, 0},
+    {"bs", K::kInt64, 0}, {"h", K::kInt64, 0}, {"top_k", K::kInt64, 0}, {"experts", K::kInt64, 0}, {"y", K::kPointer, 0},
+    {"dtype", K::kInt32, 0}, {"stream", K::kStream, 0}, {"expert_scales", K::kPointer, 0}, {"active_mask", K::kPointer, 0},
+    {"active_mask_type", K::kInt64, TileXREp::TILEXR_EP_ACTIVE_MASK_NONE}, {"shared_expert_x", K::kPointer, 0},
+    {"ep_world_size", K::kInt64, 0}, {"ep_rank_id", K::kInt64, 0}, {"tp_world_size", K::kInt64, 1}, {"tp_rank_id", K::kInt64, 0},
+    {"expert_shard_type", K::kInt64, 0}, {"shared_expert_num", K::kInt64, 0}, {"shared_expert_rank_num", K::kInt64, 0},
+    {"quant_mode", K::kInt64, 0}, {"global_bs", K::kInt64, 0},
 };
 Function gCombineMemoryV2 {"combine_memory_v2", kCombineMemoryV2, 11, sizeof(kCombineMemoryV2) / sizeof(Param), {}};
 
@@ -285,13 +330,13 @@ PyObject *CombineMemoryV2(PyObject *, PyObject *const *args, Py_ssize_t nargs, P
 
 // ---- dispatch_memory_ex: (status, epoch) ---------------------------------------------------------------------------
 const Param kDispatchEx[] = {
-    {"x", K::kPointer, 0}, {"expert_ids", K::kPointer, 0}, {"comm", K::kComm, 0}, {"bs", K::kInt, 0}, {"h", K::kInt, 0},
-    {"top_k", K::kInt, 0}, {"experts", K::kInt, 0}, {"expand_x", K::kPointer, 0}, {"assist", K::kPointer, 0},
-    {"token_nums", K::kPointer, 0}, {"send_counts", K::kPointer, 0}, {"dtype", K::kInt, 0}, {"stream", K::kStream, 0},
-    {"quant_mode", K::kInt, 0}, {"expert_capacity", K::kInt, 0}, {"token_nums_type", K::kInt, 1},
-    {"active_mask", K::kPointer, 0}, {"active_mask_type", K::kInt, TileXREp::TILEXR_EP_ACTIVE_MASK_NONE},
-    {"dynamic_scales", K::kPointer, 0}, {"expand_x_dtype", K::kIntOrNone, kNone}, {"row_index_map", K::kPointer, 0},
-    {"tile_flags", K::kPointer, 0}, {"tile_rows", K::kInt, 0}, {"meta_ready_event", K::kIntOrNone, kNone},
+    {"x", K::kPointer, 0}, {"expert_ids", K::kPointer, 0}, {"comm", K::kComm, 0}, {"bs", K::kInt64, 0}, {"h", K::kInt64, 0},
+    {"top_k", K::kInt64, 0}, {"experts", K::kInt64, 0}, {"expand_x", K::kPointer, 0}, {"assist", K::kPointer, 0},
+    {"token_nums", K::kPointer, 0}, {"send_counts", K::kPointer, 0}, {"dtype", K::kInt32, 0}, {"stream", K::kStream, 0},
+    {"quant_mode", K::kField, 0}, {"expert_capacity", K::kField, 0}, {"token_nums_type", K::kField, 1},
+    {"active_mask", K::kPointer, 0}, {"active_mask_type", K::kField, TileXREp::TILEXR_EP_ACTIVE_MASK_NONE},
+    {"dynamic_scales", K::kPointer, 0}, {"expand_x_dtype", K::kInt32OrNone, kNone}, {"row_index_map", K::kPointer, 0},
+    {"tile_flags", K::kPointer, 0}, {"tile_rows", K::kField, 0}, {"meta_ready_event", K::kEvent, 0},
 };
 Function gDispatchEx {"dispatch_memory_ex", kDispatchEx, 13, sizeof(kDispatchEx) / sizeof(Param), {}};
 
@@ -309,7 +354,7 @@ PyObject *DispatchEx(PyObject *, PyObject *const *args, Py_ssize_t nargs, PyObje
     opt.tileFlagsOut = p(21);
     opt.tileRows = p(22);
     opt.epochOut = &epoch;
-    opt.metaReadyEvent = As<decltype(opt.metaReadyEvent)>(a[23] == kNone ? 0 : a[23]);
+    opt.metaReadyEvent = p(23);
     if (a[19] == kNone) {
         a[19] = a[13] == TileXREp::TILEXR_EP_QUANT_TOKEN_INT8 ? int64_t{TileXR::TILEXR_DATA_TYPE_INT8} :
             a[13] == TileXREp::TILEXR_EP_QUANT_MXFP8 || a[13] == TileXREp::TILEXR_EP_QUANT_FP8_BLOCK128 ? int64_t{TileXR::TILEXR_DATA_TYPE_FP8E4M3} :
@@ -325,12 +370,12 @@ PyObject *DispatchEx(PyObject *, PyObject *const *args, Py_ssize_t nargs, PyObje
 // ---- combine_memory_ex ---------------------------------------------------------------------------------------------
 const Param kCombineEx[] = {
     {"expert_out", K::kPointer, 0}, {"assist", K::kPointer, 0}, {"send_counts", K::kPointer, 0}, {"comm", K::kComm, 0},
-    {"bs", K::kInt, 0}, {"h", K::kInt, 0}, {"top_k", K::kInt, 0}, {"experts", K::kInt, 0}, {"y", K::kPointer, 0},
-    {"dtype", K::kInt, 0}, {"stream", K::kStream, 0}, {"comm_quant_mode", K::kInt, 0}, {"expert_out_quant_mode", K::kInt, 0},
+    {"bs", K::kInt64, 0}, {"h", K::kInt64, 0}, {"top_k", K::kInt64, 0}, {"experts", K::kInt64, 0}, {"y", K::kPointer, 0},
+    {"dtype", K::kInt32, 0}, {"stream", K::kStream, 0}, {"comm_quant_mode", K::kField, 0}, {"expert_out_quant_mode", K::kField, 0},
     {"expert_out_scales", K::kPointer, 0}, {"expert_scales", K::kPointer, 0}, {"active_mask", K::kPointer, 0},
-    {"active_mask_type", K::kInt, TileXREp::TILEXR_EP_ACTIVE_MASK_NONE}, {"shared_expert_x", K::kPointer, 0},
-    {"row_index_map", K::kPointer, 0}, {"tile_flags", K::kPointer, 0}, {"tile_rows", K::kInt, 0}, {"flag_epoch", K::kInt, 0},
-    {"wait_timeout_us", K::kInt, 0}, {"device_status", K::kPointer, 0},
+    {"active_mask_type", K::kField, TileXREp::TILEXR_EP_ACTIVE_MASK_NONE}, {"shared_expert_x", K::kPointer, 0},
+    {"row_index_map", K::kPointer, 0}, {"tile_flags", K::kPointer, 0}, {"tile_rows", K::kField, 0}, {"flag_epoch", K::kField, 0},
+    {"wait_timeout_us", K::kField, 0}, {"device_status", K::kPointer, 0},
 };
 Function gCombineEx {"combine_memory_ex", kCombineEx, 11, sizeof(kCombineEx) / sizeof(Param), {}};
 
@@ -428,6 +473,17 @@ PyMODINIT_FUNC PyInit__calls()
     gCudaStream = PyUnicode_InternFromString("cuda_stream");
     gHandle = PyUnicode_InternFromString("handle");
     gValue = PyUnicode_InternFromString("value");
+    gAsParameter = PyUnicode_InternFromString("_as_parameter_");
+    PyObject *ctypes = PyImport_ImportModule("ctypes");
+    if (ctypes == nullptr) {
+        return nullptr;
+    }
+    gCInt64 = PyObject_GetAttrString(ctypes, "c_int64");
+    gCInt32 = PyObject_GetAttrString(ctypes, "c_int32");
+    Py_DECREF(ctypes);
+    if (gCInt64 == nullptr || gCInt32 == nullptr) {
+        return nullptr;
+    }
     for (Function *f : {&gDispatchV2, &gDispatchMemoryV2, &gCombineV2, &gCombineMemoryV2, &gDispatchEx, &gCombineEx}) {
         for (int i = 0; i < f->total; ++i) {
             f->names[i] = PyUnicode_InternFromString(f->params[i].name);
