@@ -259,3 +259,28 @@ def test_addresses_that_are_not_plain(calls):
     for value in (1.5, "event", object()):
         with pytest.raises(TypeError):
             module.dispatch_memory_ex(**event, meta_ready_event=value)
+
+
+@pytest.mark.parametrize("name", NAMES)
+def test_a_name_taken_before_the_library_was_loaded_binds_nothing_again(name, monkeypatch):
+    """`from tilexr_amd.ep import combine_v2` at the top of a program: every call through that name goes straight to the bound
+    native module."""
+    from tilexr_amd.lib import _calls
+    ep._bind(ep.lib())
+    binds = []
+    monkeypatch.setattr(_calls, "bind", lambda *at: binds.append(at))
+    sig = inspect.signature(PYTHON_FORMS[name]).parameters
+    given = {p: 3 if p in ("bs", "h", "top_k", "experts", "dtype") else None for p, q in sig.items() if q.default is inspect._empty}
+    for _ in range(3):
+        ret = PYTHON_FORMS[name](**given)
+        assert (ret[0] if name == "dispatch_memory_ex" else ret) == ep.ERR_PARA_CHECK_FAIL
+    assert binds == []
+
+
+def test_a_library_that_cannot_be_bound_is_not_taken_for_loaded(monkeypatch):
+    monkeypatch.setattr(ep, "_lib", None)
+    monkeypatch.setattr(ep, "_bind", lambda loaded: 1 / 0)
+    for _ in range(2):
+        with pytest.raises(ZeroDivisionError):
+            ep.lib()
+    assert ep._lib is None

@@ -238,7 +238,8 @@ using K = Kind;
 
 #define PARSE_OR_RETURN(F, ENTRY)                                                                  \
     int64_t a[kMaxParams];                                                                         \
-    if (!Bound(gEntries.ENTRY) || !Parse(F, args, PyVectorcall_NARGS(nargs), keywords, a)) {      \
+    const auto entry = gEntries.ENTRY;          /* read with the lock held: bind() writes it so */  \
+    if (!Bound(entry) || !Parse(F, args, PyVectorcall_NARGS(nargs), keywords, a)) {                \
         return nullptr;                                                                            \
     }                                                                                              \
     auto p = [&a](int i) { return Value {a[i]}; }
@@ -261,7 +262,7 @@ PyObject *DispatchV2(PyObject *, PyObject *const *args, Py_ssize_t nargs, PyObje
 {
     PARSE_OR_RETURN(gDispatchV2, dispatchV2);
     return PyLong_FromLong(Unlocked([&] {
-        return gEntries.dispatchV2(p(0), p(1), p(13), p(14), p(15), p(2), p(3), p(4), p(5), p(6), p(16), p(17), p(18), p(19),
+        return entry(p(0), p(1), p(13), p(14), p(15), p(2), p(3), p(4), p(5), p(6), p(16), p(17), p(18), p(19),
             p(20), p(21), p(22), p(23), p(24), p(25), p(7), p(26), p(8), p(9), p(10), p(27), p(28), p(29), p(11), p(12));
     }));
 }
@@ -285,7 +286,7 @@ PyObject *DispatchMemoryV2(PyObject *, PyObject *const *args, Py_ssize_t nargs, 
 {
     PARSE_OR_RETURN(gDispatchMemoryV2, dispatchMemoryV2);
     return PyLong_FromLong(Unlocked([&] {
-        return gEntries.dispatchMemoryV2(p(0), p(1), p(13), p(14), p(15), p(16), p(2), p(3), p(4), p(5), p(6), p(17), p(18),
+        return entry(p(0), p(1), p(13), p(14), p(15), p(16), p(2), p(3), p(4), p(5), p(6), p(17), p(18),
             p(19), p(20), p(21), p(22), p(23), p(24), p(25), p(26), p(7), p(27), p(8), p(9), p(10), p(28), p(29), p(11), p(30),
             p(12));
     }));
@@ -303,7 +304,7 @@ PyObject *CombineV2(PyObject *, PyObject *const *args, Py_ssize_t nargs, PyObjec
 {
     PARSE_OR_RETURN(gCombineV2, combineV2);
     return PyLong_FromLong(Unlocked([&] {
-        return gEntries.combineV2(p(0), p(1), p(2), p(3), p(4), p(5), p(6), p(7), p(8), p(11), p(9), p(10));
+        return entry(p(0), p(1), p(2), p(3), p(4), p(5), p(6), p(7), p(8), p(11), p(9), p(10));
     }));
 }
 
@@ -323,7 +324,7 @@ PyObject *CombineMemoryV2(PyObject *, PyObject *const *args, Py_ssize_t nargs, P
 {
     PARSE_OR_RETURN(gCombineMemoryV2, combineMemoryV2);
     return PyLong_FromLong(Unlocked([&] {
-        return gEntries.combineMemoryV2(p(0), p(1), p(2), p(11), p(12), p(13), p(14), p(3), p(4), p(5), p(6), p(7), p(15),
+        return entry(p(0), p(1), p(2), p(11), p(12), p(13), p(14), p(3), p(4), p(5), p(6), p(7), p(15),
             p(16), p(17), p(18), p(19), p(20), p(21), p(22), p(23), p(8), p(9), p(10));
     }));
 }
@@ -361,7 +362,7 @@ PyObject *DispatchEx(PyObject *, PyObject *const *args, Py_ssize_t nargs, PyObje
             a[11];
     }
     const int status = Unlocked([&] {
-        return gEntries.dispatchMemoryEx(p(0), p(1), p(2), p(3), p(4), p(5), p(6), &opt, p(7), p(18), p(8), p(9), p(10), p(11),
+        return entry(p(0), p(1), p(2), p(3), p(4), p(5), p(6), &opt, p(7), p(18), p(8), p(9), p(10), p(11),
             p(19), p(12));
     });
     return Py_BuildValue("(iL)", status, static_cast<long long>(epoch));
@@ -397,7 +398,7 @@ PyObject *CombineEx(PyObject *, PyObject *const *args, Py_ssize_t nargs, PyObjec
     opt.waitTimeoutUs = p(22);
     opt.deviceStatusOut = p(23);
     return PyLong_FromLong(Unlocked([&] {
-        return gEntries.combineMemoryEx(p(0), p(1), p(2), p(3), p(4), p(5), p(6), p(7), &opt, p(8), p(9), p(10));
+        return entry(p(0), p(1), p(2), p(3), p(4), p(5), p(6), p(7), &opt, p(8), p(9), p(10));
     }));
 }
 

@@ -65,9 +65,11 @@ class CombineExOptions(C.Structure):
 
 
 _lib = None
+_native = None          # the native module, bound to the library's entry points
 
 # Calls whose arguments the native module converts, in the order in which its bind() takes their entry points.  Once the
-# library is loaded the module's functions stand in this module's place of those below, which have the same signatures.
+# library is loaded the module's functions stand in this module's place of those below, which have the same signatures; a name
+# taken before goes through those below to them (0.15 to 0.3 us a call more).
 # us a dispatch + combine of 8 tokens x 7168, called eagerly: 12.7 through ctypes, 8.6 this way, 8.0 from a C++ loop.
 _NATIVE = {
     "dispatch_v2": "TileXRMoeEpDispatchV2", "dispatch_memory_v2": "TileXRMoeEpDispatchMemoryV2",
@@ -83,54 +85,52 @@ def lib():
         if not os.path.exists(LIB_PATH):
             raise ImportError(f"{LIB_PATH} is missing: build it with `make -C tilexr_amd/csrc` "
                               "(or __graft_entry__.build())")
-        _lib = C.CDLL(LIB_PATH)
+        loaded = C.CDLL(LIB_PATH)
         i64, vp, i32 = C.c_int64, C.c_void_p, C.c_int
-        _lib.TileXREpVersion.restype = C.c_char_p
-        _lib.TileXREpLastKernelName.restype = C.c_char_p
-        _lib.TileXREpLastKernelName.argtypes = [C.c_void_p, C.c_int]
-        _lib.TileXRCommInitRankLocal.argtypes = [i32, i32, C.POINTER(vp)]
-        _lib.TileXRCommDestroy.argtypes = [vp]
-        _lib.TileXRCommNextMagic.argtypes = [vp, C.POINTER(i64)]
-        _lib.TileXRGetCommArgsHost.argtypes = [vp, C.POINTER(vp)]
-        _lib.TileXRGetCommArgsDev.argtypes = [vp, C.POINTER(vp)]
+        loaded.TileXREpVersion.restype = C.c_char_p
+        loaded.TileXREpLastKernelName.restype = C.c_char_p
+        loaded.TileXREpLastKernelName.argtypes = [C.c_void_p, C.c_int]
+        loaded.TileXRCommInitRankLocal.argtypes = [i32, i32, C.POINTER(vp)]
+        loaded.TileXRCommDestroy.argtypes = [vp]
+        loaded.TileXRCommNextMagic.argtypes = [vp, C.POINTER(i64)]
+        loaded.TileXRGetCommArgsHost.argtypes = [vp, C.POINTER(vp)]
+        loaded.TileXRGetCommArgsDev.argtypes = [vp, C.POINTER(vp)]
         simple_dispatch = [vp, vp, vp, i64, i64, i64, i64, vp, vp, vp, vp, i32, vp]
-        _lib.TileXRMoeEpDispatch.argtypes = simple_dispatch
-        _lib.TileXRMoeEpDispatchMemory.argtypes = simple_dispatch
-        _lib.TileXRMoeEpDispatchMemoryNoAlloc.argtypes = simple_dispatch
+        loaded.TileXRMoeEpDispatch.argtypes = simple_dispatch
+        loaded.TileXRMoeEpDispatchMemory.argtypes = simple_dispatch
+        loaded.TileXRMoeEpDispatchMemoryNoAlloc.argtypes = simple_dispatch
         simple_combine = [vp, vp, vp, vp, i64, i64, i64, i64, vp, i32, vp]
-        _lib.TileXRMoeEpCombine.argtypes = simple_combine
-        _lib.TileXRMoeEpCombineMemory.argtypes = simple_combine
-        _lib.TileXRMoeEpCombineV2.argtypes = [vp, vp, vp, vp, i64, i64, i64, i64, vp, vp, i32, vp]
-        _lib.TileXRMoeEpCombineMemoryV2.argtypes = ([vp] * 5 + [i64, vp, vp] + [i64] * 13 + [vp, i32, vp])
-        _lib.TileXRMoeEpDispatchV2.argtypes = ([vp] * 6 + [i64] * 14 + [vp] * 8 + [i32, vp])
-        _lib.TileXRMoeEpDispatchMemoryV2.argtypes = ([vp] * 4 + [i64, vp, vp] + [i64] * 14 + [vp] * 7 + [i32, i32, vp])
-        _lib.TileXRMoeEpDispatchMemoryEx.argtypes = [vp, vp, vp, i64, i64, i64, i64, C.POINTER(DispatchExOptions),
+        loaded.TileXRMoeEpCombine.argtypes = simple_combine
+        loaded.TileXRMoeEpCombineMemory.argtypes = simple_combine
+        loaded.TileXRMoeEpCombineV2.argtypes = [vp, vp, vp, vp, i64, i64, i64, i64, vp, vp, i32, vp]
+        loaded.TileXRMoeEpCombineMemoryV2.argtypes = ([vp] * 5 + [i64, vp, vp] + [i64] * 13 + [vp, i32, vp])
+        loaded.TileXRMoeEpDispatchV2.argtypes = ([vp] * 6 + [i64] * 14 + [vp] * 8 + [i32, vp])
+        loaded.TileXRMoeEpDispatchMemoryV2.argtypes = ([vp] * 4 + [i64, vp, vp] + [i64] * 14 + [vp] * 7 + [i32, i32, vp])
+        loaded.TileXRMoeEpDispatchMemoryEx.argtypes = [vp, vp, vp, i64, i64, i64, i64, C.POINTER(DispatchExOptions),
                                                       vp, vp, vp, vp, vp, i32, i32, vp]
-        _lib.TileXRMoeEpCombineMemoryEx.argtypes = [vp, vp, vp, vp, i64, i64, i64, i64, C.POINTER(CombineExOptions),
+        loaded.TileXRMoeEpCombineMemoryEx.argtypes = [vp, vp, vp, vp, i64, i64, i64, i64, C.POINTER(CombineExOptions),
                                                      vp, i32, vp]
-        _lib.TileXREpSetKernelTimingEvents.argtypes = [vp, i32, vp, vp]
+        loaded.TileXREpSetKernelTimingEvents.argtypes = [vp, i32, vp, vp]
         for name in EXPORTS:
-            fn = getattr(_lib, name)
+            fn = getattr(loaded, name)
             if name not in ("TileXREpVersion", "TileXREpLastKernelName"):
                 fn.restype = C.c_int
-        try:
-            _bind(_lib)
-        except BaseException:
-            _lib = None
-            raise
+        _bind(loaded)
+        _lib = loaded           # last: whoever finds it set, on whatever thread, finds it whole
     return _lib
 
 
 def _bind(loaded):
+    global _native
     from .lib import _calls
     _calls.bind(*(C.cast(getattr(loaded, name), C.c_void_p).value for name in _NATIVE.values()))
     globals().update({name: getattr(_calls, name) for name in _NATIVE})
-    return _calls
+    _native = _calls
 
 
-def _call(name):
-    """The native form of a call that was made before the library was loaded, or through a name taken before."""
-    return getattr(_bind(lib()), name)
+def _load():
+    lib()
+    return _native
 
 
 def version():
@@ -212,11 +212,11 @@ def dispatch_v2(x, expert_ids, comm, bs, h, top_k, experts, expand_x, assist, to
                 tp_rank_id=0, expert_shard_type=0, shared_expert_num=0, shared_expert_rank_num=0, quant_mode=0,
                 global_bs=0, token_nums_type=1, dynamic_scales=None, tp_recv_counts=None, expand_scales=None,
                 workspace=None):
-    return _call("dispatch_v2")(x, expert_ids, comm, bs, h, top_k, experts, expand_x, assist, token_nums, recv_counts,
-                                dtype, stream, scales, active_mask, expert_scales, ep_world_size, ep_rank_id,
-                                tp_world_size, tp_rank_id, expert_shard_type, shared_expert_num,
-                                shared_expert_rank_num, quant_mode, global_bs, token_nums_type, dynamic_scales,
-                                tp_recv_counts, expand_scales, workspace)
+    return (_native or _load()).dispatch_v2(x, expert_ids, comm, bs, h, top_k, experts, expand_x, assist, token_nums,
+                                            recv_counts, dtype, stream, scales, active_mask, expert_scales,
+                                            ep_world_size, ep_rank_id, tp_world_size, tp_rank_id, expert_shard_type,
+                                            shared_expert_num, shared_expert_rank_num, quant_mode, global_bs,
+                                            token_nums_type, dynamic_scales, tp_recv_counts, expand_scales, workspace)
 
 
 def dispatch_memory_v2(x, expert_ids, comm, bs, h, top_k, experts, expand_x, assist, token_nums, send_counts, dtype,
@@ -224,12 +224,12 @@ def dispatch_memory_v2(x, expert_ids, comm, bs, h, top_k, experts, expand_x, ass
                        ep_world_size=0, ep_rank_id=0, tp_world_size=1, tp_rank_id=0, expert_shard_type=0,
                        shared_expert_num=0, shared_expert_rank_num=0, quant_mode=0, global_bs=0, token_nums_type=1,
                        dynamic_scales=None, tp_recv_counts=None, expand_scales=None, expand_x_dtype=DT_RESERVED):
-    return _call("dispatch_memory_v2")(x, expert_ids, comm, bs, h, top_k, experts, expand_x, assist, token_nums,
-                                       send_counts, dtype, stream, scales, active_mask, active_mask_type,
-                                       expert_scales, ep_world_size, ep_rank_id, tp_world_size, tp_rank_id,
-                                       expert_shard_type, shared_expert_num, shared_expert_rank_num, quant_mode,
-                                       global_bs, token_nums_type, dynamic_scales, tp_recv_counts, expand_scales,
-                                       expand_x_dtype)
+    return (_native or _load()).dispatch_memory_v2(x, expert_ids, comm, bs, h, top_k, experts, expand_x, assist,
+                                                   token_nums, send_counts, dtype, stream, scales, active_mask,
+                                                   active_mask_type, expert_scales, ep_world_size, ep_rank_id,
+                                                   tp_world_size, tp_rank_id, expert_shard_type, shared_expert_num,
+                                                   shared_expert_rank_num, quant_mode, global_bs, token_nums_type,
+                                                   dynamic_scales, tp_recv_counts, expand_scales, expand_x_dtype)
 
 
 def combine(expert_out, assist, recv_counts, comm, bs, h, top_k, experts, y, dtype, stream):
@@ -238,8 +238,8 @@ def combine(expert_out, assist, recv_counts, comm, bs, h, top_k, experts, y, dty
 
 
 def combine_v2(expert_out, assist, recv_counts, comm, bs, h, top_k, experts, y, dtype, stream, workspace=None):
-    return _call("combine_v2")(expert_out, assist, recv_counts, comm, bs, h, top_k, experts, y, dtype, stream,
-                               workspace)
+    return (_native or _load()).combine_v2(expert_out, assist, recv_counts, comm, bs, h, top_k, experts, y, dtype,
+                                           stream, workspace)
 
 
 def combine_memory(expert_out, assist, send_counts, comm, bs, h, top_k, experts, y, dtype, stream):
@@ -251,10 +251,11 @@ def combine_memory_v2(expert_out, assist, send_counts, comm, bs, h, top_k, exper
                       expert_scales=None, active_mask=None, active_mask_type=MASK_NONE, shared_expert_x=None,
                       ep_world_size=0, ep_rank_id=0, tp_world_size=1, tp_rank_id=0, expert_shard_type=0,
                       shared_expert_num=0, shared_expert_rank_num=0, quant_mode=0, global_bs=0):
-    return _call("combine_memory_v2")(expert_out, assist, send_counts, comm, bs, h, top_k, experts, y, dtype, stream,
-                                      expert_scales, active_mask, active_mask_type, shared_expert_x, ep_world_size,
-                                      ep_rank_id, tp_world_size, tp_rank_id, expert_shard_type, shared_expert_num,
-                                      shared_expert_rank_num, quant_mode, global_bs)
+    return (_native or _load()).combine_memory_v2(expert_out, assist, send_counts, comm, bs, h, top_k, experts, y,
+                                                  dtype, stream, expert_scales, active_mask, active_mask_type,
+                                                  shared_expert_x, ep_world_size, ep_rank_id, tp_world_size,
+                                                  tp_rank_id, expert_shard_type, shared_expert_num,
+                                                  shared_expert_rank_num, quant_mode, global_bs)
 
 
 # ---- additions -------------------------------------------------------------------------------------------
@@ -263,20 +264,22 @@ def dispatch_memory_ex(x, expert_ids, comm, bs, h, top_k, experts, expand_x, ass
                        active_mask_type=MASK_NONE, dynamic_scales=None, expand_x_dtype=None, row_index_map=None,
                        tile_flags=None, tile_rows=0, meta_ready_event=None):
     """Returns (status, epoch)."""
-    return _call("dispatch_memory_ex")(x, expert_ids, comm, bs, h, top_k, experts, expand_x, assist, token_nums,
-                                       send_counts, dtype, stream, quant_mode, expert_capacity, token_nums_type,
-                                       active_mask, active_mask_type, dynamic_scales, expand_x_dtype, row_index_map,
-                                       tile_flags, tile_rows, meta_ready_event)
+    return (_native or _load()).dispatch_memory_ex(x, expert_ids, comm, bs, h, top_k, experts, expand_x, assist,
+                                                   token_nums, send_counts, dtype, stream, quant_mode, expert_capacity,
+                                                   token_nums_type, active_mask, active_mask_type, dynamic_scales,
+                                                   expand_x_dtype, row_index_map, tile_flags, tile_rows,
+                                                   meta_ready_event)
 
 
 def combine_memory_ex(expert_out, assist, send_counts, comm, bs, h, top_k, experts, y, dtype, stream,
                       comm_quant_mode=0, expert_out_quant_mode=0, expert_out_scales=None, expert_scales=None,
                       active_mask=None, active_mask_type=MASK_NONE, shared_expert_x=None, row_index_map=None,
                       tile_flags=None, tile_rows=0, flag_epoch=0, wait_timeout_us=0, device_status=None):
-    return _call("combine_memory_ex")(expert_out, assist, send_counts, comm, bs, h, top_k, experts, y, dtype, stream,
-                                      comm_quant_mode, expert_out_quant_mode, expert_out_scales, expert_scales,
-                                      active_mask, active_mask_type, shared_expert_x, row_index_map, tile_flags,
-                                      tile_rows, flag_epoch, wait_timeout_us, device_status)
+    return (_native or _load()).combine_memory_ex(expert_out, assist, send_counts, comm, bs, h, top_k, experts, y,
+                                                  dtype, stream, comm_quant_mode, expert_out_quant_mode,
+                                                  expert_out_scales, expert_scales, active_mask, active_mask_type,
+                                                  shared_expert_x, row_index_map, tile_flags, tile_rows, flag_epoch,
+                                                  wait_timeout_us, device_status)
 
 
 K_COUNT, K_PLACE, K_SCATTER, K_INVERT, K_REDUCE = range(5)
