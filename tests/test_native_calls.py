@@ -4,6 +4,8 @@ import ctypes as C
 import inspect
 import os
 import subprocess
+import sys
+import sysconfig
 
 import pytest
 
@@ -284,3 +286,29 @@ def test_a_library_that_cannot_be_bound_is_not_taken_for_loaded(monkeypatch):
         with pytest.raises(ZeroDivisionError):
             ep.lib()
     assert ep._lib is None
+
+
+def _make(*args):
+    return subprocess.run(["make", "-C", os.path.join(ROOT, "tilexr_amd", "csrc"), "-n", "-B", *args], capture_output=True, text=True)
+
+
+def test_the_module_is_for_the_interpreter_that_builds_it(monkeypatch):
+    """Its file carries the interpreter's tag (another minor version does not import it), and the build passes the interpreter it
+    runs in."""
+    from tilexr_amd.lib import _calls
+    suffix = sysconfig.get_config_var("EXT_SUFFIX")
+    assert os.path.basename(_calls.__file__) == "_calls" + suffix
+    built = _make("python", f"PYTHON={sys.executable}")
+    assert built.returncode == 0 and f"_calls{suffix}" in built.stdout and "libtilexr-ep" not in built.stdout
+    import __graft_entry__ as entry
+    ran = []
+    monkeypatch.setattr(entry.subprocess, "run", lambda cmd, **kw: ran.append(cmd))
+    entry.build()
+    assert any(f"PYTHON={sys.executable}" in cmd for cmd in ran)
+
+
+def test_the_library_builds_without_python_headers():
+    for target in ("all", "library"):
+        built = _make(target, "PYTHON=/nonexistent/python")
+        assert built.returncode == 0, built.stderr
+        assert "libtilexr-ep.so" in built.stdout and "py_calls" not in built.stdout

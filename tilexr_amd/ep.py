@@ -7,6 +7,7 @@ returns the library's status code; `check()` turns a non-zero code into an excep
 """
 import ctypes as C
 import os
+import sys
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libtilexr-ep.so")
@@ -122,7 +123,11 @@ def lib():
 
 def _bind(loaded):
     global _native
-    from .lib import _calls
+    try:
+        from .lib import _calls
+    except ImportError as e:
+        raise ImportError("the native module of the binding is not built for this interpreter: `make -C tilexr_amd/csrc python "
+                          f"PYTHON={sys.executable}` (needs Python's headers)") from e
     _calls.bind(*(C.cast(getattr(loaded, name), C.c_void_p).value for name in _NATIVE.values()))
     globals().update({name: getattr(_calls, name) for name in _NATIVE})
     _native = _calls
