@@ -229,6 +229,19 @@ __global__ __launch_bounds__(kThreads) void ep_drain_plan_kernel(DrainArgs a)
     DrainCounts(a, d, numSeg, s_cnt, s_off, s_tok, s_part);
 }
 
+// Said of an address that is the same for all lanes of a wave, which the compiler cannot see of a row that it gets from the
+// lane's index: without a word it wraps every store in a loop over the resources that the lanes might have.  (Drain and return
+// launches, us, with the loops and without: 4 x 128 x 1024 x top-2 6.2 and 4.2, 6.1 and 4.3; 4 x 512 x 4096 x top-8 46.4 and 13.3,
+// 45.7 and 13.1: they wait for memory either way.  The row's index made uniform instead, at its root, turns the tuple's loads
+// into scalar ones that the copy waits for: return 20.2.)
+__device__ __forceinline__ char *UniformPointer(char *p)
+{
+    const uint64_t at = reinterpret_cast<uintptr_t>(p);
+    const uint32_t low = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(at)));
+    const uint32_t high = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(at >> 32)));
+    return reinterpret_cast<char *>(static_cast<uintptr_t>(uint64_t{high} << 32 | low));
+}
+
 // A row is read here for the last time and read next by whoever it was copied for: it is loaded past the caches and left in the
 // memory-side cache.  dispatch + combine with ordinary loads and stores, and so, us: 4 ranks x 512 x 4096 x top-8 232 -> 217, 8
 // x 500 438 -> 417, 4 x 1000 x 7168 x top-4 355 -> 317, top-8 620 -> 587.  (Ordinary loads, kept stores 235; streaming loads,
@@ -239,7 +252,7 @@ __device__ __forceinline__ void CopyBytes(char *dst, const char *src, int64_t by
         const u32x4 *s = reinterpret_cast<const u32x4 *>(src);
         constexpr int kAhead = 4;       // vectors a lane has in flight
         const int vecs = static_cast<int>(bytes / 16);
-        const __amdgpu_buffer_rsrc_t rows = RowResource(dst, vecs * 16);
+        const __amdgpu_buffer_rsrc_t rows = RowResource(UniformPointer(dst), vecs * 16);
         for (int i = tid; i < vecs; i += kAhead * threads) {
             u32x4 v[kAhead];
 #pragma unroll
