@@ -54,6 +54,26 @@ constexpr int kAuxAgentScopeKept = 16;      // sc1 alone: for small tables a lat
                                             // the same table afterwards ran 10 us slower: 92 instead of 82 us)
 constexpr unsigned kRawBufferWord3 = 0x00020000u;
 
+// Unused dynamic LDS that holds a kernel to so many workgroups per compute unit, 0 for as many as fit.  A compute unit hands its
+// 160 KiB out in blocks of 1280 bytes (workgroups of a fixed wait, counted by the rounds a launch takes: 53 760 bytes three, one
+// block more two; 40 960 four, 40 bytes more three), so a size takes what the kernel's own tables come to into account.
+constexpr unsigned kLdsBlockBytes = 1280;
+constexpr unsigned kLdsBlocks = 128;
+constexpr unsigned kOwnLdsBytes = 1024;         // of the kernels that are capped, at most
+
+constexpr unsigned CapLdsBytes(int workgroups)
+{
+    return workgroups == 2 ? 56u * 1024u : workgroups == 4 ? 39u * 1024u : workgroups == 5 ? 27u * 1024u : 0u;
+}
+
+constexpr bool CapHolds(int workgroups)
+{
+    const unsigned least = (CapLdsBytes(workgroups) + kLdsBlockBytes - 1) / kLdsBlockBytes;
+    const unsigned most = (CapLdsBytes(workgroups) + kOwnLdsBytes + kLdsBlockBytes - 1) / kLdsBlockBytes;
+    return kLdsBlocks / least == static_cast<unsigned>(workgroups) && kLdsBlocks / most == static_cast<unsigned>(workgroups);
+}
+static_assert(CapHolds(2) && CapHolds(4) && CapHolds(5), "as many workgroups fit as the cap says");
+
 // The cache between the L2s and memory, one for the device.
 constexpr int64_t kMemorySideCacheBytes = int64_t{256} << 20;
 

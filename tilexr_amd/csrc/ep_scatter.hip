@@ -155,7 +155,7 @@ __device__ __forceinline__ void PublishRows(const ScatterArgs &a, const int *pos
 // topK rows", and 132 us when the workgroups of a token are spread over the XCDs.  The rows must stream: kept ones push the
 // token rows out of the L2s (dispatch + combine 182 us, 234 us with kKeep).
 constexpr int kRouteVecs = 2;
-constexpr unsigned kRouteCapLdsBytes = 27 * 1024;    // 160 KiB of LDS per compute unit: five workgroups fit
+constexpr int kRouteCapWorkgroups = 5;
 template <int THREADS, int V, bool WT>
 __global__ __launch_bounds__(THREADS) void ep_scatter_route_kernel(ScatterArgs a)
 {
@@ -567,24 +567,18 @@ inline bool WriteThrough(const ScatterArgs &a)
     return a.tileFlags != nullptr;
 }
 
-// Unused dynamic LDS that holds the scatter kernels to so many workgroups per compute unit (160 KiB of LDS).
-constexpr unsigned CapLdsBytes(int workgroups)
-{
-    return workgroups == 3 ? 53u * 1024u : workgroups == 4 ? 40u * 1024u : workgroups == 5 ? kRouteCapLdsBytes : 0u;
-}
-
 // Workgroups per compute unit that the launch without flags is held to, 0 for as many as fit.  Eight workgroups that each
 // store a wide row topK times oversubscribe the memory system like those of the per-route kernel.
-//   quantised: five.  (8192 x 4096 int8 x top-6, microseconds at eight, six, five, four, three: 53.5, 50.1, 49.4, 49.9,
-//     50.8; 2048 x 7168 MXFP8 27.3, 27.0, 25.9, 25.6, 25.5.)  That takes rows that store enough: dispatch + combine at eight
-//     and at five, int8 or block fp8, 2048 x 7168 top-8 65.7 -> 62.3, 4096 x 7168 top-4 69.3 -> 67.1, 2048 x 8192 top-4 43.4
+//   quantised: five.  (Dispatch + combine, us at eight, seven, six, five, four, three, two: 2048 x 7168 x top-8 block fp8 61.5,
+//     60.6, 59.9, 59.4, 60.1, 59.8, 61.2, MXFP8 83.4, 83.2, 82.7, 82.0, 81.5, 81.3, 81.5; 8192 x 4096 int8 x top-6 97.2, 96.9,
+//     97.3, 97.4, 97.3, 96.5, 104.8.)  That takes rows that store enough: at eight and at five, int8 or block fp8, 2048 x 7168 top-8 65.7 -> 62.3, 4096 x 7168 top-4 69.3 -> 67.1, 2048 x 8192 top-4 43.4
 //     -> 42.1, 8192 x 4096 top-6 107.9 -> 105.5; but 2048 x 4096 top-2 20.4 and 21.4, 8192 x 2304 top-2 42.3 and 44.6, 16384
 //     x 2304 top-8 181 and 201, 16384 x 3072 top-8 205 and 213, 16384 x 4096 top-5 181 and 187, 2048 x 12288 top-2 46.8 and
 //     48.6.  (Rows a wave holds: no difference.)
-//   copies, dispatch + combine at eight, four and three: 2200 x 7168 x top-8 95.8, 93.6, 91.5; 3000 x 5120 93.1, 92.3, 89.3;
-//     16384 x 7168 769.6, 764.6, 759.7; 16384 x 6144 x top-4 354, 350, 365 (token rows from memory, few stores each); up to
-//     512 vectors 16384 x 4096 x top-8 439, 428, 462; 6000 x 2560 95.9, 92.9, 93.5; 10000 x 2056 160, 167, 188.  1000 tokens
-//     and fewer: no difference.
+//   copies, dispatch + combine at eight, four, three and two: 2200 x 7168 x top-8 95.9, 93.4, 92.7, 91.2; 3000 x 5120 93.9, 92.2,
+//     90.6, 89.6; 16384 x 7168 768.5, 763.5, 768.9, 760.2; 16384 x 6144 x top-4 (token rows from memory, few stores each) 354.5,
+//     356.1, 355.5, 353.8; up to 512 vectors 16384 x 4096 x top-8 441.6, 431.4, 437.0, 466.7; 6000 x 2560 95.0, 91.5, 91.0, -;
+//     10000 x 2056 160, 167, -, 188.  1000 tokens and fewer: no difference.
 template <int G, int QMODE>
 int CapWorkgroups(const ScatterArgs &a)
 {
@@ -596,7 +590,7 @@ int CapWorkgroups(const ScatterArgs &a)
         return 0;
     }
     const bool cachedTokens = static_cast<int64_t>(a.bs) * a.h * 2 <= kMemorySideCacheBytes / 2;
-    return vecs > 2 * kThreads && (cachedTokens || a.topK > 4) ? 3 : 4;
+    return vecs > 2 * kThreads && (cachedTokens || a.topK > 4) ? 2 : 4;
 }
 
 // Whether the rows are left in the memory-side cache.  They are where this library's combine can take them as they are; a
@@ -682,10 +676,11 @@ void LaunchByMode(const ScatterLaunch &l, const ScatterArgs &a)
                         l.stream, a);
                 } else {
                     // Workgroups that only look their row up in the row map are short-lived, and eight of them per
-                    // compute unit keep more stores in flight than this memory system digests (4096 x 7168 x top-8:
-                    // 88.9 us; seven 86.5, five 81.7, four 85.3, three 98.2).  Unused dynamic LDS caps them at five.
+                    // compute unit keep more stores in flight than this memory system digests (dispatch + combine, us at
+                    // eight, seven, six, five, four, three, two: 1500 x 14336 x top-8 137.5, 136.0, 134.3, 132.9, 134.3,
+                    // 144.3, 168.6; 2000 x 12288 158.5, 157.8, 157.5, 156.4, 148.6, 153.4, 171.8).
                     // Workgroups that resolve their row themselves (three dependent loads) are slow enough as they are.
-                    const unsigned capLds = a.place.ids == nullptr ? kRouteCapLdsBytes : 0u;
+                    const unsigned capLds = a.place.ids == nullptr ? CapLdsBytes(kRouteCapWorkgroups) : 0u;
                     hipLaunchKernelGGL((ep_scatter_route_kernel<kThreads, kRouteVecs, false>), blocks, dim3(kThreads), capLds,
                         l.stream, a);
                 }
@@ -731,7 +726,7 @@ void LaunchByMode(const ScatterLaunch &l, const ScatterArgs &a)
 } // namespace
 
 // The per-route kernel's rows have to stream, the per-token kernel's are kept: dispatch + combine, per route and per token
-// (three or four workgroups to a compute unit), us: 235 MB of rows (2048 x 7168 x top-8) 93.9 and 85.0, 315 MB 128.1 and
+// (two or four workgroups to a compute unit), us: 235 MB of rows (2048 x 7168 x top-8) 93.9 and 85.0, 315 MB 128.1 and
 // 122.8, 367 MB 144.8 and 145.4, 470 MB 182.2 and 187.8, 688 MB 273.0 and 274.4; 4096 columns, 328 MB 132.1 and 128.3, 393 MB
 // 155.8 and 157.1, 786 MB 310.7 and 316.2.  So it takes what the memory-side cache cannot hold, and of that what has token
 // rows it can: beyond 104 MiB of them reading them ahead no longer pays (117 MB 379.8 and 375.6, 123 MB 405.6 and 392.4, 134

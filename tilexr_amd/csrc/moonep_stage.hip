@@ -32,11 +32,11 @@ constexpr int kTokenVecs = 4 * kThreads;    // 16-byte vectors of a row slice of
 
 constexpr int64_t kDefaultCachedRowBytes = int64_t{256} << 20;   // with this setting the library goes by rows and token rows
 std::atomic<int64_t> gCachedRowBytes {kDefaultCachedRowBytes};  // TileXRMoonEpSetCachedRowBytes
-// Unused dynamic LDS of the copying workgroups: five of them fit a compute unit's 160 KiB.  Eight keep more stores in
-// flight than this memory system digests (4096 x 7168 x top-8, microseconds at eight, seven, six, five, four: 83, 79, 74,
-// 73, 81; five hold their time in both directions, built and saved plans).
-constexpr unsigned kScatterCapLdsBytes = 27 * 1024;
-constexpr unsigned kTokenCapLdsBytes = 53 * 1024;       // per-token scatter: three
+// Workgroups per compute unit that the copying launches are held to.  Per route: eight keep more stores in flight than this
+// memory system digests (4096 x 7168 x top-8, four stages, us at eight, seven, six, five, four, three, two: 420, 415, 401, 397,
+// 410, 439, 512; 5800 x 4096, the forward two 170.3, 170.2, 170.1, 169.0, 169.2, 176.7, 200.5).
+constexpr unsigned kScatterCapLdsBytes = TileXREp::CapLdsBytes(5);
+constexpr unsigned kTokenCapLdsBytes = TileXREp::CapLdsBytes(2);        // per-token scatter (LaunchMoonDispatch)
 constexpr int kFusedPlanChunks = 1024;  // chunks of 2048 rows per rank up to which the scatter launch builds a fresh plan
 constexpr int64_t kFusedPlanRowBytes = int64_t{256} << 20;     // ... and bytes of rows the world's routes write
 constexpr int kSelfPlanChunks = 8;      // ... and up to which its plan workgroups add up the earlier chunks themselves
@@ -1361,9 +1361,9 @@ hipError_t LaunchMoonDispatch(const DispatchWorld &w, hipStream_t stream, const 
     }
     if (perToken) {
         gScatterName = "moon_scatter_token_kernel";
-        // Three workgroups to a compute unit, or as many as fit where the rows come to a GiB and more; us at eight, four and
-        // three: 1024 x 7168 x top-8 132.6, 130.7, 129.5; four ranks x 2000 x 2048 490, 472, 447; four ranks x 4096 x 7168 (1.9
-        // GB) 1785, 1817, 1816, eight x 2500 x 7168 fwd 1137, 1161, 1161.
+        // Two workgroups to a compute unit, or as many as fit where the rows come to a GiB and more; us at eight, four, three and
+        // two: 1024 x 7168 x top-8 132.7, 131.5, 130.1, 130.1; four ranks x 2000 x 2048 438, 416, 412, 407; four ranks x 4096 x
+        // 7168 (1.9 GB) 1785, 1817, -, 1816, eight x 2500 x 7168 fwd 1137, 1161, -, 1161.
         const unsigned capLds = worldRowBytes * w.k <= (int64_t{1} << 30) ? kTokenCapLdsBytes : 0u;
         auto launch = [&](auto lanes, auto vecsPerLane) {
             constexpr int G = decltype(lanes)::value;
