@@ -23,6 +23,12 @@ CASES = [
     (1000, 1048, 5, 16, "int8", "ep_scatter_vec_kernel"),
     (16384, 4096, 8, 64, "fp8", "ep_scatter_vec_kernel"),           # exactly 512 MiB
     (16385, 4096, 8, 64, "fp8", "ep_scatter_vec_kernel"),
+    # rows that the scatter resolves itself (too many routes x experts for the one-launch routing), on both sides of the vectors
+    # stored from which a cap of four and of two workgroups per compute unit pays
+    (2100, 3576, 8, 600, "none", "ep_scatter_vec_kernel"),
+    (2100, 3584, 8, 600, "none", "ep_scatter_vec_kernel"),
+    (2100, 4600, 8, 600, "none", "ep_scatter_vec_kernel"),
+    (2100, 4608, 8, 600, "none", "ep_scatter_vec_kernel"),
 ]
 QUANT = {"none": ep.Q_NONE, "int8": ep.Q_TOKEN_INT8, "fp8": ep.Q_FP8_BLOCK128}
 

@@ -571,14 +571,22 @@ inline bool WriteThrough(const ScatterArgs &a)
 // store a wide row topK times oversubscribe the memory system like those of the per-route kernel.
 //   quantised: five.  (Dispatch + combine, us at eight, seven, six, five, four, three, two: 2048 x 7168 x top-8 block fp8 61.5,
 //     60.6, 59.9, 59.4, 60.1, 59.8, 61.2, MXFP8 83.4, 83.2, 82.7, 82.0, 81.5, 81.3, 81.5; 8192 x 4096 int8 x top-6 97.2, 96.9,
-//     97.3, 97.4, 97.3, 96.5, 104.8.)  That takes rows that store enough: at eight and at five, int8 or block fp8, 2048 x 7168 top-8 65.7 -> 62.3, 4096 x 7168 top-4 69.3 -> 67.1, 2048 x 8192 top-4 43.4
-//     -> 42.1, 8192 x 4096 top-6 107.9 -> 105.5; but 2048 x 4096 top-2 20.4 and 21.4, 8192 x 2304 top-2 42.3 and 44.6, 16384
-//     x 2304 top-8 181 and 201, 16384 x 3072 top-8 205 and 213, 16384 x 4096 top-5 181 and 187, 2048 x 12288 top-2 46.8 and
-//     48.6.  (Rows a wave holds: no difference.)
+//     97.3, 97.4, 97.3, 96.5, 104.8.)  That takes rows that store enough: at eight and at five, int8 or block fp8, 2048 x 7168
+//     top-8 65.7 -> 62.3, 4096 x 7168 top-4 69.3 -> 67.1, 2048 x 8192 top-4 43.4 -> 42.1, 8192 x 4096 top-6 107.9 -> 105.5; but
+//     2048 x 4096 top-2 20.4 and 21.4, 8192 x 2304 top-2 42.3 and 44.6, 16384 x 2304 top-8 181 and 201, 16384 x 3072 top-8 205
+//     and 213, 16384 x 4096 top-5 181 and 187, 2048 x 12288 top-2 46.8 and 48.6.  (Rows a wave holds: no difference.)
 //   copies, dispatch + combine at eight, four, three and two: 2200 x 7168 x top-8 95.9, 93.4, 92.7, 91.2; 3000 x 5120 93.9, 92.2,
 //     90.6, 89.6; 16384 x 7168 768.5, 763.5, 768.9, 760.2; 16384 x 6144 x top-4 (token rows from memory, few stores each) 354.5,
 //     356.1, 355.5, 353.8; up to 512 vectors 16384 x 4096 x top-8 441.6, 431.4, 437.0, 466.7; 6000 x 2560 95.0, 91.5, 91.0, -;
 //     10000 x 2056 160, 167, -, 188.  1000 tokens and fewer: no difference.
+//     Workgroups that resolve their rows themselves (three dependent loads ahead of the first store) have to store enough to be
+//     worth fewer beside them.  Vectors stored, us at eight and four: 16384 x 2560 x top-3 960, 113.7 and 143.4; 24000 x 2560 x
+//     top-2 640, 135.8 and 179.0; 12000 x 3072 x top-4 1536, 127.6 and 137.2; 24000 x 3072 x top-5 1920, 318.7 and 344.2; 16384
+//     x 4096 x top-4 2048, 242.8 and 246.5; 6000 x 2560 x top-8 2560, 103.9 and 106.2; 24000 x 3072 x top-8 3072, 492.7 and
+//     499.4; 4500 x 3584 x top-8 3584, 110.3 and 106.5; 5000 x 4096 x top-8 4096, 137.1 and 132.3.  Wider rows at eight, four
+//     and two: 5558 x 5120 x top-3 1920, 79.4, 81.6, 94.8; 9000 x 4608 x top-4 2304, 148.2, 148.6, 162.7; 19884 x 5120 x top-5
+//     3200, 437.6, 431.4, 465.9; 24000 x 5120 x top-6 3840, 613.8, 606.6, 632.9; 4200 x 4608 x top-8 4608, 127.5, 123.4, 126.5;
+//     11304 x 5120 x top-8 5120, 387.2, 380.1, 384.9; 3000 x 7168 x top-6 5376, 110.6, 105.9, 105.4.
 template <int G, int QMODE>
 int CapWorkgroups(const ScatterArgs &a)
 {
@@ -589,8 +597,13 @@ int CapWorkgroups(const ScatterArgs &a)
     if (G < kThreads || vecs < 320) {
         return 0;
     }
+    const int stored = vecs * a.topK;
+    const bool resolves = a.place.ids != nullptr;
+    if (resolves && stored < 14 * kThreads) {
+        return 0;
+    }
     const bool cachedTokens = static_cast<int64_t>(a.bs) * a.h * 2 <= kMemorySideCacheBytes / 2;
-    return vecs > 2 * kThreads && (cachedTokens || a.topK > 4) ? 2 : 4;
+    return vecs > 2 * kThreads && (cachedTokens || a.topK > 4) && (!resolves || stored >= 18 * kThreads) ? 2 : 4;
 }
 
 // Whether the rows are left in the memory-side cache.  They are where this library's combine can take them as they are; a
