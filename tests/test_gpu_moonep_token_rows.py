@@ -25,6 +25,11 @@ CASES = [
     (1, 11, 2, 8200, 4),        # 1025: two, the second of one vector
     (1, 5, 32, 16384, 7),
     (2, 1100, 8, 64, 9000),     # more chunks than a plan workgroup adds up itself
+    (1, 17, 4, 4096, 1),        # 512 vectors held by a workgroup: four workgroups to a compute unit
+    (1, 17, 4, 4104, 1),        # 513: two
+    (2, 40, 4, 1024, 0),        # 512, of four tokens
+    (2, 40, 4, 1032, 0),        # 516
+    (2, 40, 3, 1032, 0),        # 516 stored three times: four
 ]
 
 
@@ -46,4 +51,27 @@ def test_token_rows_match_oracle(world, s, k, h, slack):
             res = w.dispatch(sh, plans, hidden, weights, flags=flags)
             w.sync()
             assert ep.last_kernel_name(w.comms[0], ep.K_SCATTER) == "moon_scatter_token_kernel"
+            check_dispatch(sh, res, plans, want, fresh=flags != 0)
+
+
+@pytest.mark.parametrize("s,k,kernel", [
+    (3291, 8, "moon_scatter_token_kernel"),     # 360 MiB of rows less 48 KiB: kept for Combine
+    (3292, 8, "moon_scatter_kernel"),           # more: token rows read ahead, a workgroup per route
+    (7606, 4, "moon_scatter_kernel"),           # 104 MiB of token rows less 12 KiB
+    (7607, 4, "moon_scatter_token_kernel"),     # more: not read ahead
+])
+def test_sizes_pick_the_scatter(s, k, kernel):
+    """The library's own choice, at the knob's default, on both sides of both of its lines; built and saved plans."""
+    rng = np.random.default_rng(s)
+    sh = M.Shape(1, s, k, 7168, s * k)
+    dst = MC.random_dst(sh, rng, duplicates=True)
+    hidden = random_rows(rng, (1, s, 7168))
+    weights = rng.standard_normal((1, s * k)).astype(np.float32)
+    want = M.dispatch_world(sh, dst, hidden, weights, flags=M.FLAG_BUILD_DEDUP)
+    with World(1) as w:
+        plans = w.plan_tensors(sh, dst)
+        for flags in (mp.FLAG_BUILD_DEDUP, 0):
+            res = w.dispatch(sh, plans, hidden, weights, flags=flags)
+            w.sync()
+            assert ep.last_kernel_name(w.comms[0], ep.K_SCATTER) == kernel
             check_dispatch(sh, res, plans, want, fresh=flags != 0)

@@ -36,7 +36,6 @@ std::atomic<int64_t> gCachedRowBytes {kDefaultCachedRowBytes};  // TileXRMoonEpS
 // memory system digests (4096 x 7168 x top-8, four stages, us at eight, seven, six, five, four, three, two: 420, 415, 401, 397,
 // 410, 439, 512; 5800 x 4096, the forward two 170.3, 170.2, 170.1, 169.0, 169.2, 176.7, 200.5).
 constexpr unsigned kScatterCapLdsBytes = TileXREp::CapLdsBytes(5);
-constexpr unsigned kTokenCapLdsBytes = TileXREp::CapLdsBytes(2);        // per-token scatter (LaunchMoonDispatch)
 constexpr int kFusedPlanChunks = 1024;  // chunks of 2048 rows per rank up to which the scatter launch builds a fresh plan
 constexpr int64_t kFusedPlanRowBytes = int64_t{256} << 20;     // ... and bytes of rows the world's routes write
 constexpr int kSelfPlanChunks = 8;      // ... and up to which its plan workgroups add up the earlier chunks themselves
@@ -1361,10 +1360,17 @@ hipError_t LaunchMoonDispatch(const DispatchWorld &w, hipStream_t stream, const 
     }
     if (perToken) {
         gScatterName = "moon_scatter_token_kernel";
-        // Two workgroups to a compute unit, or as many as fit where the rows come to a GiB and more; us at eight, four, three and
-        // two: 1024 x 7168 x top-8 132.7, 131.5, 130.1, 130.1; four ranks x 2000 x 2048 438, 416, 412, 407; four ranks x 4096 x
-        // 7168 (1.9 GB) 1785, 1817, -, 1816, eight x 2500 x 7168 fwd 1137, 1161, -, 1161.
-        const unsigned capLds = worldRowBytes * w.k <= (int64_t{1} << 30) ? kTokenCapLdsBytes : 0u;
+        // Two workgroups to a compute unit where each holds more than 512 vectors and stores them four times or more, four where it
+        // does not (fewer have too little in flight), as many as fit where the rows come to a GiB and more.  us at eight, four,
+        // three and two: 1024 x 7168 x top-8 132.7, 131.5, 130.1, 130.1; 1000 x 12288 205.8, 200.5, 199.5, 191.9; four ranks x 2000 x
+        // 2048 438, 416, 412, 407; 2500 x 5120 x top-4, fwd, 66.5, 66.2, 64.9, 64.2.  Held 384 or 512: two ranks x 4000 x 3072 x
+        // top-8 463, 455, 459, 470; 5064 x 3072 x top-4 155.8, 155.4, 160.5, 170.2; 8000 x 4096 x top-4 260.4, 257.5, 258.4, 268.4
+        // (2000 x 4096 x top-6 129.9, 128.1, 127.3, 126.6).  Stored once or twice: two ranks x 16333 x 4096 798, 794, 810, 872; 11308
+        // x 12288 x top-1, fwd, 263.3, 261.7, 268.2, 283.8; 3000 x 7168 x top-2 148.0, 147.2, 146.2, 149.8.  Four ranks x 4096 x 7168
+        // x top-8 (1.9 GB) 1785, 1817, -, 1816, eight x 2500 x 7168, fwd, 1137, 1161, -, 1161.
+        const int64_t heldVecs = vecs <= 4 * kWave ? vecs * (kThreads / kWave) : vecs;
+        const int capWorkgroups = heldVecs > 2 * kThreads && w.k >= 4 ? 2 : 4;
+        const unsigned capLds = worldRowBytes * w.k <= (int64_t{1} << 30) ? TileXREp::CapLdsBytes(capWorkgroups) : 0u;
         auto launch = [&](auto lanes, auto vecsPerLane) {
             constexpr int G = decltype(lanes)::value;
             constexpr int V = decltype(vecsPerLane)::value;
