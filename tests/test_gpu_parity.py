@@ -170,15 +170,18 @@ def test_one_launch_routing_on_random_tables(seed):
 def test_routing_kernels_are_picked_by_the_size_of_the_call():
     """Left to itself the library takes the one-launch routing where it was measured to be the faster one: small
     tables always; larger ones while routes x experts stays small, less far when the same launch also reads token rows
-    ahead of a scatter that copies per route (rows wider than 4 KiB, plain payload) and then only against count + place
-    (readiness flags ask for the rows ahead of the scatter)."""
+    ahead of a scatter that copies per route (plain rows of more than 320 MiB) and then only against count + place
+    (readiness flags ask for the rows ahead of the scatter).  Rows wider than 4 KiB that are copied per token are as others."""
     cases = [  # bs, K, E, h, flags, kernel
         (1024, 8, 256, 16, False, "ep_route_rows_kernel"), (2048, 8, 2048, 16, False, "ep_route_count_kernel"),
         (2048, 8, 2048, 16, True, "ep_route_rows_kernel"), (4096, 8, 256, 16, False, "ep_route_rows_kernel"),
         (4096, 8, 1024, 16, True, "ep_route_count_kernel"), (8192, 6, 64, 16, True, "ep_route_rows_kernel"),
         (8192, 8, 256, 16, True, "ep_route_count_kernel"), (16384, 8, 64, 16, False, "ep_route_count_kernel"),
-        (4096, 8, 256, 2056, False, "ep_route_count_kernel"), (4096, 8, 256, 2056, True, "ep_route_rows_kernel"),
-        (4096, 8, 512, 2056, True, "ep_route_count_kernel"), (6144, 8, 64, 2056, True, "ep_route_count_kernel"),
+        (4096, 8, 256, 5632, False, "ep_route_count_kernel"), (4096, 8, 256, 5632, True, "ep_route_rows_kernel"),
+        (4096, 8, 512, 5632, True, "ep_route_count_kernel"), (6144, 8, 64, 5632, True, "ep_route_count_kernel"),
+        (4096, 8, 256, 2056, False, "ep_route_rows_kernel"), (4096, 8, 256, 2056, True, "ep_route_rows_kernel"),
+        (4096, 8, 512, 2056, True, "ep_route_rows_kernel"), (6144, 8, 64, 2056, True, "ep_route_rows_kernel"),
+        (4096, 8, 1024, 2056, False, "ep_route_count_kernel"), (8192, 6, 256, 2552, False, "ep_route_count_kernel"),
     ]
     with Session() as s:
         for bs, K, E, h, with_flags, kernel in cases:

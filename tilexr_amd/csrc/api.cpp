@@ -128,13 +128,12 @@ int RunDispatchSingle(EpComm *comm, const EpDispatchParams &p, bool memoryRoute,
     // the scatter kernel that copies per route wants the token rows close by: the routing launch reads them ahead
     const bool warm = ScatterCopiesPerRoute(scatter);
     // Launches that read no token rows ahead resolve the rows in one launch further up (RouteRowsPays): dispatch + combine,
-    // count and one launch, 2200 x 7168 x top-8 95.9 -> 91.1 us, 4000 x 4096 101.2 -> 97.5, 8000 x 2560 138.7 -> 128.1.  Copies
-    // of 257 to 319 vectors stay where they were, on the count launch (tests name it for 2056 columns: 71.3 us, 69.5 in one).
-    const bool narrowCopies = p.quantMode == TILEXR_EP_QUANT_NONE && p.h > 2048 && p.h < 2560 && p.topK > 1 && p.bs >= 1024;
+    // count and one launch, 2200 x 7168 x top-8 95.9 -> 91.1 us, 4000 x 4096 101.2 -> 97.5, 8000 x 2560 138.7 -> 128.1, 8192 x
+    // 2304 x top-6 98.2 -> 91.5, 4096 x 2056 x top-8 70.2 -> 68.2.
     const bool mayOneLaunch = comm->routing != EpComm::Routing::kLegacy;
     const bool oneLaunchRows = mayOneLaunch && memoryRoute &&
         RouteRowsFits(p.expertIds, n, numKeys, maskMode, p.expertCapacity) &&
-        (comm->routing == EpComm::Routing::kOneLaunch || RouteRowsPays(n, numKeys, rowsAhead, warm || narrowCopies));
+        (comm->routing == EpComm::Routing::kOneLaunch || RouteRowsPays(n, numKeys, rowsAhead, warm));
     const bool oneLaunchCompact = mayOneLaunch && !memoryRoute && p.expertCapacity <= 0 &&
         RouteCompactFits(p.expertIds, n, experts, maskMode) &&
         (comm->routing == EpComm::Routing::kOneLaunch || RouteCompactPays(n, experts));
