@@ -154,10 +154,12 @@ def test_wide_quantised_rows_with_tile_flags(two_streams):
 
 @pytest.mark.parametrize("two_streams", [False, True], ids=["one_stream", "two_streams"])
 def test_rows_wider_than_one_publishing_workgroup(two_streams):
-    """Rows of 1536 vectors: the publishing per-route scatter cuts them into two workgroups of 512 lanes, each of which
-    reports its part of the row, so a row counts twice towards its tile (the headline rows fit one such workgroup)."""
+    """Rows of 1536 vectors: beside a consumer on another stream they are copied per route, and the publishing per-route scatter
+    cuts them into three workgroups of 256 lanes, each of which reports its part of the row, so a row counts three times towards
+    its tile.  On one stream a workgroup copies the token's rows and reports them whole."""
     wide = workloads.Workload("bf16@12288", 1, 1024, 12288, 4, 32, x_dist="normal", routing="zipf", zipf_s=1.0, seed=77)
-    run_and_check(layers_of(wide), 100, two_streams, expect_scatter="ep_scatter_route_kernel",
+    run_and_check(layers_of(wide), 100, two_streams,
+                  expect_scatter="ep_scatter_route_kernel" if two_streams else "ep_scatter_vec_kernel",
                   expect_reduce="ep_reduce_vec_kernel")
 
 

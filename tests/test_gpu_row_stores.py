@@ -20,6 +20,9 @@ CASES = [
     (687, 2560, 3, 16, "none", "ep_scatter_vec_kernel"),            # 320 vectors: the narrowest rows with a cap
     (411, 4104, 5, 16, "none", "ep_scatter_vec_kernel"),            # 513 vectors
     (1000, 16384, 3, 8, "none", "ep_scatter_vec_kernel"),           # the widest rows
+    (1400, 16384, 8, 64, "none", "ep_scatter_route_kernel"),        # ... published in two parts
+    (2600, 8200, 8, 64, "none", "ep_scatter_route_kernel"),         # a second part of one vector
+    (1100, 8200, 8, 64, "none", "ep_scatter_vec_kernel"),           # published whole
     (1000, 1048, 5, 16, "int8", "ep_scatter_vec_kernel"),
     (16384, 4096, 8, 64, "fp8", "ep_scatter_vec_kernel"),           # exactly 512 MiB
     (16385, 4096, 8, 64, "fp8", "ep_scatter_vec_kernel"),

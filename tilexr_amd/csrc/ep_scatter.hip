@@ -744,18 +744,17 @@ void LaunchByMode(const ScatterLaunch &l, const ScatterArgs &a)
 // 155.8 and 157.1, 786 MB 310.7 and 316.2.  So it takes what the memory-side cache cannot hold, and of that what has token
 // rows it can: beyond 104 MiB of them reading them ahead no longer pays (117 MB 379.8 and 375.6, 123 MB 405.6 and 392.4, 134
 // MB 470 and 428); publishing, where the per-token kernel waits for its stores topK at a time, beyond 128 MiB (117 MB 378.4
-// and 379.9, 123 MB 395.3 and 398.0).  Published rows wider than one of its workgroups (1024 vectors) are its own at any size:
-// callers and tests count on their parts being landed one by one (1024 x 12288 x top-4 52.8 us, 46.1 per token).  A consumer
-// that runs beside the launch is given rows as early as before.
+// and 379.9, 123 MB 395.3 and 398.0).  Rows wider than one of its publishing workgroups (1024 vectors) are no exception (published
+// on one stream, 1024 x 12288 x top-4 52.5 and 45.2, 1024 x 16384 x top-8 107.6 and 94.9, 4096 x 16384 x top-2 150.5 and 133.4).  A
+// consumer that runs beside the launch gets its rows one by one as they land, not a token's topK at a time.
 bool ScatterCopiesPerRoute(const ScatterLaunch &l)
 {
     const int64_t vecs = l.h / 8;
     const int64_t tokenBytes = l.bs * l.h * 2;
     const bool publishes = l.tileFlags != nullptr;
-    const bool inParts = publishes && vecs > 4 * kThreads;
     return l.quantMode == TILEXR_EP_QUANT_NONE && l.h % 8 == 0 && Aligned16(l.x) && Aligned16(l.out) && vecs > 4 * kWave &&
         vecs <= 8 * kThreads && l.topK > 1 && l.bs >= 1024 && tokenBytes <= (publishes ? int64_t{128} << 20 : int64_t{104} << 20) &&
-        (l.consumerBeside || inParts || tokenBytes * l.topK > (int64_t{320} << 20)) && (l.bs + 7) / 8 <= 65535 && l.topK <= 65535;
+        (l.consumerBeside || tokenBytes * l.topK > (int64_t{320} << 20)) && (l.bs + 7) / 8 <= 65535 && l.topK <= 65535;
 }
 
 bool ScatterCopiesPerRoute(const void *x, const void *out, int64_t bs, int64_t h, int64_t topK, int quantMode)
