@@ -44,14 +44,15 @@ __device__ __forceinline__ void LdsBarrier()
 // may hit a stale line until an acquire fence invalidates the reader's L2 (measured: 240 us instead of 90 us for the
 // reduce with one fence per token).  An agent-scope (sc1) store is written through to memory and is complete, for
 // every XCD, when the wave's vmcnt reaches zero; an agent-scope load is served from memory.  Rows published through
-// readiness flags therefore move with sc1 accesses and need no cache maintenance at all.  The streaming hint (nt)
-// stays on: without it the written-through rows are also allocated in L2 and push out the input rows the sibling
-// workgroups of a token share (measured: 132 us instead of 93 us for the scatter).
+// readiness flags therefore move with sc1 accesses and need no cache maintenance at all.  The streaming hint (nt) is
+// for rows whose token row several workgroups share: without it the written-through rows are also allocated in L2 and push
+// out the input rows those workgroups find there (measured: 132 us instead of 93 us for the per-route scatter).
 constexpr int kAuxAgentScope = 16 | 2;      // sc1 nt
 constexpr int kAuxNonTemporal = 2;          // nt
-constexpr int kAuxAgentScopeKept = 16;      // sc1 alone: for small tables a later kernel reads again (with nt on the
-                                            // loads of the count kernel's histograms the scatter that resolves rows from
-                                            // the same table afterwards ran 10 us slower: 92 instead of 82 us)
+constexpr int kAuxAgentScopeKept = 16;      // sc1 alone: for rows one workgroup copies to all their places (RowStores in
+                                            // ep_scatter.hip) and for small tables a later kernel reads again (with nt on
+                                            // the loads of the count kernel's histograms the scatter that resolves rows
+                                            // from the same table afterwards ran 10 us slower: 92 instead of 82 us)
 constexpr unsigned kRawBufferWord3 = 0x00020000u;
 
 // Unused dynamic LDS that holds a kernel to so many workgroups per compute unit, 0 for as many as fit.  A compute unit hands its

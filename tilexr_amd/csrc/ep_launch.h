@@ -167,7 +167,8 @@ struct ScatterLaunch {
     const int32_t *totalRowsPtr; // device word: rows kept by this dispatch (size of the last tile)
     bool consumerBeside;         // a consumer of the flags is expected to run beside this launch (the caller asked for a
                                  // metadata-ready event): keep the workgroups small enough to fit next to its waiting ones
-    bool combineTakesRows;       // what is written is read next by this library as it is: left in the memory-side cache
+    bool combineTakesRows;       // this library's combine or drain can take the rows as they are: plain, per-token int8 and block
+                                 // fp8 ones are then left in the memory-side cache (KeepsRows)
     const char **kernelNameOut;  // optional: receives the name of the kernel template that was launched
     hipStream_t stream;
 };

@@ -1,8 +1,9 @@
 // scatter: each token row is read once and written to the rows its routes were placed at (gfx950, wave64).
 //
 // HBM-bound byte movement, no MFMA.  Three kernels share the work:
-//   ep_scatter_route_kernel    plain copies of wide rows that the memory-side cache cannot hold: one workgroup per
-//                              (token, k, slice of 512 vectors; 1024 when readiness flags are published), two 16-byte
+//   ep_scatter_route_kernel    plain copies of wide rows, 1024 tokens and more, that the memory-side cache cannot hold or that
+//                              a consumer beside the launch waits for (ScatterCopiesPerRoute): one workgroup per (token, k,
+//                              slice of 512 vectors; 1024 when readiness flags are published for this stream), two 16-byte
 //                              loads and two 16-byte stores per lane
 //   ep_scatter_vec_kernel      everything else that is 16-byte aligned (quantised payloads, narrow rows, small
 //                              batches): G lanes cooperate on one token (a wave for narrow rows, the whole workgroup
@@ -67,9 +68,9 @@ __device__ __forceinline__ float GroupMax(float v, float *red, int lane)
 }
 
 // Row stores of the register-resident kernels.  A streaming store goes past the L2 and past the 256 MiB memory-side cache:
-// whoever reads the row next (an expert stage, combine) fetches it from memory, row by row at unrelated places.  One that
-// is written through without the streaming hint leaves the row in that cache, and it is the cheaper store as well, since
-// what the cache takes need not reach memory within the launch.  Dispatch + combine, us, streaming and kept, six sets of
+// whoever reads the row next fetches it from memory, row by row at unrelated places.  One that is written through without the
+// streaming hint leaves the row in that cache, and it is the cheaper store as well, since what the cache takes need not reach
+// memory within the launch.  Dispatch + combine of the rows as they are, us, streaming and kept, six sets of
 // buffers in turn: 1000 x 7168 x top-8 52.4 -> 45.3, 600 tokens 34.9 -> 31.1, 3000 x 2048 48.3 -> 41.3; int8 8192 x 4096 x
 // top-6 108.4 -> 100.2 (its scatter 49.9 -> 42.5), 4096 x 7168 x top-8 127.0 -> 109.0; block fp8 16384 x 2048 under a
 // capacity 98.4 -> 92.0 (scatter 48.9 -> 39.0, reduce 40.7 -> 44.4: it waits for rows that leave the cache).  Ordinary
@@ -124,8 +125,9 @@ __device__ __forceinline__ void PublishRow(const ScatterArgs &a, int row, int pa
 }
 
 // Publishes the rows of one token.  Each wave waits for its own stores and the barrier collects the waves.
-// WT = true: the rows were written through (kKeep, kPublish) and are then complete for every XCD, with no L2 write-back.  WT = false: the rows may still sit dirty in this
-// XCD's L2 and one release fence per publishing wave writes them back (slow under load; element-granular fallback only).
+// WT = true: the rows were written through (kKeep, kPublish) and are then complete for every XCD, with no L2 write-back.
+// WT = false: the rows may still sit dirty in this XCD's L2 and one release fence per publishing wave writes them back (slow
+// under load; element-granular fallback only).
 template <bool WT>
 __device__ __forceinline__ void PublishRows(const ScatterArgs &a, const int *pos, int lane, int G)
 {
@@ -561,8 +563,8 @@ __global__ __launch_bounds__(kThreads) void ep_scatter_generic_kernel(ScatterArg
     }
 }
 
-// Rows move with write-through stores when readiness flags are published (see RowStore).
-inline bool WriteThrough(const ScatterArgs &a)
+// Whether readiness flags are published: rows are then written through, streaming or kept, and reported once they have landed.
+inline bool Publishes(const ScatterArgs &a)
 {
     return a.tileFlags != nullptr;
 }
@@ -606,13 +608,22 @@ int CapWorkgroups(const ScatterArgs &a)
     return vecs > 2 * kThreads && (cachedTokens || a.topK > 4) && (!resolves || stored >= 18 * kThreads) ? 2 : 4;
 }
 
-// Whether the rows are left in the memory-side cache.  They are where this library's combine can take them as they are; a
-// payload that only an expert stage decodes streams (dispatch + combine of other rows, streaming and kept: MXFP8 2048 x
-// 7168 88.9 and 91.2 us, 4096 x 7168 155 and 168, int8 on the MVP route 4000 x 2048 49.0 and 51.4).  Block fp8 rows beyond
-// twice that cache stream too (16384 x 7168 x top-6 378 and 388, 8192 x 8192 x top-8 274 -> 269), int8 and plain ones are
-// kept at any size (16384 x 7168 x top-8 int8 468.5 -> 466.2, plain 775.5 -> 770.3).  Rows that end within a 128-byte line
-// are two partial lines each and want a launch worth it: 1000 columns, 1501 tokens x top-6 19.1 and 19.6, 4000 x top-6 31.2
-// and 31.4, 4000 x top-8 39.4 -> 37.1.
+// Whether the rows are left in the memory-side cache.  They are where this library's combine can take them as they are.  A
+// payload that only an expert stage decodes streams (dispatch + combine of other rows with nothing in between, streaming and
+// kept: MXFP8 2048 x 7168 88.9 and 91.2 us, 4096 x 7168 155 and 168, int8 on the MVP route 4000 x 2048 49.0 and 51.4).
+//   With an expert stage in between, dispatch + stage + combine in us, rows streamed (by the launches that suit that) and kept.
+// Two matrix products through 2048 columns into another buffer: 1000 x 7168 x top-8 437 -> 426, 1500 x 7168 689 -> 684, 2200
+// x 7168 1050 -> 1046, 16384 x 7168 6813 -> 6792, 4000 x 4096 950 -> 944, 16384 x 2048 2002 -> 1976; int8 1000 x 7168 533 ->
+// 492, 8192 x 4096 x top-6 1816 -> 1802, block fp8 16384 x 2048 2501 -> 2498.  One elementwise pass over the rows where they
+// are: 87.4 -> 78.2, 119.6 -> 114.1, 173.6 -> 163.9, 1392 and 1392, 179 -> 173, 398 -> 390.  A stage that is bound by memory
+// and writes elsewhere pays for the write-back of the kept rows itself: the same pass into another buffer 88.5 and 88.6,
+// 122.1 and 129.1, 182.2 and 189.0, 1379 and 1384, 187.6 and 196.6, 402 and 408; products through 256 columns 185.4 and
+// 184.2, 244 and 251, 312 and 323, 1984 and 1990, 294 and 305, 633 and 648.  Rows are kept all the same: what stands between
+// dispatch and combine at these sizes are products.
+//   Block fp8 rows beyond twice that cache stream too (16384 x 7168 x top-6 378 and 388, 8192 x 8192 x top-8 274 -> 269), int8
+// and plain ones are kept at any size (16384 x 7168 x top-8 int8 468.5 -> 466.2, plain 775.5 -> 770.3).  Rows that end within
+// a 128-byte line are two partial lines each and want a launch worth it: 1000 columns, 1501 tokens x top-6 19.1 and 19.6,
+// 4000 x top-6 31.2 and 31.4, 4000 x top-8 39.4 -> 37.1.
 template <int QMODE>
 bool KeepsRows(const ScatterArgs &a)
 {
@@ -621,7 +632,7 @@ bool KeepsRows(const ScatterArgs &a)
     if (QMODE == TILEXR_EP_QUANT_FP8_BLOCK128 && bytes > 2 * kMemorySideCacheBytes) {
         return false;
     }
-    return WriteThrough(a) || rowBytes % 128 == 0 || bytes >= (int64_t{32} << 20);
+    return Publishes(a) || rowBytes % 128 == 0 || bytes >= (int64_t{32} << 20);
 }
 
 template <int G, int V, int QMODE, bool BF16, bool E5M2, RowStores S>
@@ -630,7 +641,7 @@ void LaunchVecStoring(const ScatterArgs &a, hipStream_t stream)
     constexpr int kTokens = kThreads / G;
     const dim3 groups((a.bs + kTokens - 1) / kTokens);
     if constexpr (S != RowStores::kStream) {
-        if (WriteThrough(a)) {
+        if (Publishes(a)) {
             hipLaunchKernelGGL((ep_scatter_vec_kernel<G, V, QMODE, BF16, E5M2, true, S>), groups, dim3(kThreads), 0, stream, a);
             return;
         }
@@ -652,7 +663,7 @@ void LaunchVec(const ScatterLaunch &l, const ScatterArgs &a)
             return;
         }
     }
-    if (WriteThrough(a)) {
+    if (Publishes(a)) {
         LaunchVecStoring<G, V, QMODE, BF16, E5M2, RowStores::kPublish>(a, l.stream);
     } else {
         LaunchVecStoring<G, V, QMODE, BF16, E5M2, RowStores::kStream>(a, l.stream);
@@ -670,7 +681,7 @@ void LaunchByMode(const ScatterLaunch &l, const ScatterArgs &a)
                 if (l.kernelNameOut != nullptr) {
                     *l.kernelNameOut = "ep_scatter_route_kernel";
                 }
-                if (WriteThrough(a) && a.colSlices > 1 && !l.consumerBeside) {
+                if (Publishes(a) && a.colSlices > 1 && !l.consumerBeside) {
                     // A publishing workgroup stays until its stores have landed and then counts its part of the row
                     // towards the tile: worth doing once per row rather than once per half row, so rows wider than 512
                     // vectors get workgroups of 512 lanes (4096 x 7168 x top-8: 82.2 instead of 84.7 us; without
@@ -684,7 +695,7 @@ void LaunchByMode(const ScatterLaunch &l, const ScatterArgs &a)
                         static_cast<unsigned>((a.bs + 7) / 8));
                     hipLaunchKernelGGL((ep_scatter_route_kernel<kWide, kRouteVecs, true>), wideBlocks, dim3(kWide), 0,
                         l.stream, wide);
-                } else if (WriteThrough(a)) {
+                } else if (Publishes(a)) {
                     hipLaunchKernelGGL((ep_scatter_route_kernel<kThreads, kRouteVecs, true>), blocks, dim3(kThreads), 0,
                         l.stream, a);
                 } else {

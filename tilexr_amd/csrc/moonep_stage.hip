@@ -37,9 +37,10 @@ std::atomic<int64_t> gCachedRowBytes {kDefaultCachedRowBytes};  // TileXRMoonEpS
 // 410, 439, 512; 5800 x 4096, the forward two 170.3, 170.2, 170.1, 169.0, 169.2, 176.7, 200.5).
 constexpr unsigned kScatterCapLdsBytes = TileXREp::CapLdsBytes(5);
 constexpr int kFusedPlanChunks = 1024;  // chunks of 2048 rows per rank up to which the scatter launch builds a fresh plan
-constexpr int64_t kFusedPlanRowBytes = int64_t{256} << 20;     // ... and bytes of rows the world's routes write
+constexpr int64_t kFusedPlanRowBytes = int64_t{256} << 20;     // ... and, copied per route, bytes of rows the world's routes write
 constexpr int kSelfPlanChunks = 8;      // ... and up to which its plan workgroups add up the earlier chunks themselves
 constexpr int64_t kWarmRowBytes = int64_t{128} << 20;          // token rows of a world that are read ahead of the per-route scatter
+                                                               // (with SetCachedRowBytes at its default there are 104 MiB at most)
 constexpr int64_t kKeptRowBytes = int64_t{360} << 20;          // rows of a world up to which the per-token scatter is the faster one,
 constexpr int64_t kPerRouteTokenBytes = int64_t{104} << 20;    // and token rows beyond which it is again (LaunchMoonDispatch)
 
@@ -1334,6 +1335,8 @@ hipError_t LaunchMoonDispatch(const DispatchWorld &w, hipStream_t stream, const 
     // four (the chunk totals need one) beyond.  Per-route copies of more than kFusedPlanRowBytes keep the launches after the
     // scatter: with the plan's code that kernel has 50 registers per lane instead of 16, and its short-lived workgroups then
     // start more slowly, which costs more than the launches saved (4096 tokens x 7168 201 -> 204 us, 8192 tokens 365 -> 386).
+    // At the default of SetCachedRowBytes the per-route kernel gets more rows than that: moon_scatter_kernel<true, true> serves
+    // callers who have asked for per-route copies of less.
     const int planChunks = static_cast<int>((w.nvS + kBuildRows - 1) / kBuildRows);
     const bool planInScatter = w.fresh && planChunks <= kFusedPlanChunks &&
         (perToken || (perRoute && static_cast<int64_t>(w.world) * w.s * w.k * w.h * 2 <= kFusedPlanRowBytes));

@@ -312,7 +312,7 @@ int SendRoutes(EpComm *comm, const EpDispatchParams &p, bool memoryRoute, const 
     scatter.fp8E5m2 = p.expandXOutDtype == TileXR::TILEXR_DATA_TYPE_FP8E5M2;
     scatter.staticScale = static_cast<const float *>(p.scales);
     scatter.out = myRows;
-    scatter.combineTakesRows = true;        // the drain does
+    scatter.combineTakesRows = true;        // the drain does (MXFP8 and static int8 rows stream all the same)
     scatter.scalesOut = myAux + plan.layout.scalesOffset;
     scatter.stream = stream;
     return Timed(comm, kKernelScatter, stream, "scatter", [&] { return LaunchScatter(scatter); });
