@@ -148,6 +148,11 @@ __device__ __forceinline__ void ReduceVec(const ReduceArgs &a)
         int firstSlot = 0;
         bool odd = false;       // MXFP8: one of the lane's blocks holds an infinity or a NaN
         // control flow below is uniform across the lanes that share a token (the MXFP8 round trip looks across lanes)
+        // Loads checked by the row's resource instead of a branch per load.  Where the rows come out of the order's exchange the
+        // branches had the compiler wait, ahead of most loads, for the load before (registers of an address and of an earlier
+        // row in one): MVP route, expert rows in another buffer, dispatch + combine 286 x 2048 x top-8 23.1 -> 17.9 us (20.8 with
+        // the route tables in LDS), 700 x 2048 24.9 -> 18.6, 1500 x 2048 29.0 -> 24.9; rows as dispatch left them 286 x 2048 19.5 -> 16.3.
+        constexpr bool kChecked = WIDE || (!FL && KIND == kReducePerAdd);
         while (todo != 0) {
             u32x4 v16[KB][V];
             int rowOfK[KB];
@@ -163,14 +168,14 @@ __device__ __forceinline__ void ReduceVec(const ReduceArgs &a)
                 rowOfK[u] = row;
                 weightOfK[u] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(myWeight), k));
                 const char *base = static_cast<const char *>(a.expertOut) + static_cast<int64_t>(row < 0 ? 0 : row) * a.rowBytes;
-                // WIDE: a slot without a row gets a resource of no bytes, and a lane beyond the row's end is beyond the
+                // kChecked: a slot without a row gets a resource of no bytes, and a lane beyond the row's end is beyond the
                 // resource's: both read as zeros without a test per load (at this size the kernel is paid in
                 // instructions)
-                const __amdgpu_buffer_rsrc_t rsrc = RowResource(base, WIDE && row < 0 ? 0 : vecs * 16);
+                const __amdgpu_buffer_rsrc_t rsrc = RowResource(base, kChecked && row < 0 ? 0 : vecs * 16);
 #pragma unroll
                 for (int j = 0; j < V; ++j) {
                     const int idx = colBase + j * G + lane;
-                    if (WIDE) {
+                    if (kChecked) {
                         v16[u][j] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, idx * 16, 0, kAuxNonTemporal);
                     } else {
                         v16[u][j] = (row >= 0 && idx < vecs) ? RowLoad<FL>(base, rsrc, idx * 16) : u32x4{0u, 0u, 0u, 0u};
