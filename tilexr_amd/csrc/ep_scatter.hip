@@ -578,9 +578,11 @@ inline bool Publishes(const ScatterArgs &a)
 //     2048 x 4096 top-2 20.4 and 21.4, 8192 x 2304 top-2 42.3 and 44.6, 16384 x 2304 top-8 181 and 201, 16384 x 3072 top-8 205
 //     and 213, 16384 x 4096 top-5 181 and 187, 2048 x 12288 top-2 46.8 and 48.6.  (Rows a wave holds: no difference.)
 //   copies, dispatch + combine at eight, four, three and two: 2200 x 7168 x top-8 95.9, 93.4, 92.7, 91.2; 3000 x 5120 93.9, 92.2,
-//     90.6, 89.6; 16384 x 7168 768.5, 763.5, 768.9, 760.2; 16384 x 6144 x top-4 (token rows from memory, few stores each) 354.5,
-//     356.1, 355.5, 353.8; up to 512 vectors 16384 x 4096 x top-8 441.6, 431.4, 437.0, 466.7; 6000 x 2560 95.0, 91.5, 91.0, -;
-//     10000 x 2056 160, 167, -, 188.  1000 tokens and fewer: no difference.
+//     90.6, 89.6; 16384 x 7168 768.5, 763.5, 768.9, 760.2; up to 512 vectors 16384 x 4096 x top-8 441.6, 431.4, 437.0, 466.7; 6000
+//     x 2560 95.0, 91.5, 91.0, -; 10000 x 2056 160, 167, -, 188.  1000 tokens and fewer: no difference.
+//     Where the rows are known and the token rows come from memory, fewer workgroups have too few of those under way: MVP route
+//     30000 x 3072 x top-5 404, 438, 467, 503; 16384 x 7168 x top-8 740, 745, 752, 764; 24000 x 5120 x top-6 617, 607, 603, 639;
+//     10000 x 7168 x top-8 444, 446, 450, 454; memory route 16384 x 7168 x top-4 411, 413, 414, 413.
 //     Workgroups that resolve their rows themselves (three dependent loads ahead of the first store) have to store enough to be
 //     worth fewer beside them.  Vectors stored, us at eight and four: 16384 x 2560 x top-3 960, 113.7 and 143.4; 24000 x 2560 x
 //     top-2 640, 135.8 and 179.0; 12000 x 3072 x top-4 1536, 127.6 and 137.2; 24000 x 3072 x top-5 1920, 318.7 and 344.2; 16384
@@ -601,11 +603,11 @@ int CapWorkgroups(const ScatterArgs &a)
     }
     const int stored = vecs * a.topK;
     const bool resolves = a.place.ids != nullptr;
-    if (resolves && stored < 14 * kThreads) {
+    const bool cachedTokens = static_cast<int64_t>(a.bs) * a.h * 2 <= kMemorySideCacheBytes / 2;
+    if (resolves ? stored < 14 * kThreads : !cachedTokens) {
         return 0;
     }
-    const bool cachedTokens = static_cast<int64_t>(a.bs) * a.h * 2 <= kMemorySideCacheBytes / 2;
-    return vecs > 2 * kThreads && (cachedTokens || a.topK > 4) && (!resolves || stored >= 18 * kThreads) ? 2 : 4;
+    return vecs > 2 * kThreads && (!resolves || (stored >= 18 * kThreads && (cachedTokens || a.topK > 4))) ? 2 : 4;
 }
 
 // Whether the rows are left in the memory-side cache.  They are where this library's combine can take them as they are.  A
