@@ -29,7 +29,11 @@ CASES = [
     (1, 17, 4, 4104, 1),        # 513: two
     (2, 40, 4, 1024, 0),        # 512, of four tokens
     (2, 40, 4, 1032, 0),        # 516
-    (2, 40, 3, 1032, 0),        # 516 stored three times: four
+    (2, 40, 3, 1032, 0),        # 516 stored three times
+    (1, 50, 4, 1000, 3),        # rows that end within a 128-byte line, four and more to a token: ordinary stores
+    (2, 33, 3, 520, 1),         # ... fewer: streaming ones
+    (1, 21, 3, 4104, 2),
+    (1, 21, 1, 2008, 0),
 ]
 
 

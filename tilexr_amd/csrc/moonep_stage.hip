@@ -383,11 +383,18 @@ __global__ __launch_bounds__(kThreads) void moon_scatter_kernel(DispatchWorld a,
 
 // G lanes per (token, slice of G x V vectors) of source rank blockIdx.y: the slice is loaded once and stored once per route.
 // What the routes record was written ahead, as for moon_scatter_kernel; PLAN as there.  Lane k of every wave works out the
-// row of route k for itself, so nothing is handed round and no wave waits between its loads and its stores.  The rows are
-// written through and kept in the memory-side cache for Combine (the per-route kernel's must stream, or they push the token
-// rows that its workgroups share out of the L2s).  Workgroup b runs on XCD b % 8 and takes tokens t with t % 8 == b % 8, as
-// the reduce of a small world does.
-template <bool FRESH, bool PLAN, int G, int V>
+// row of route k for itself, so nothing is handed round and no wave waits between its loads and its stores.  Workgroup b runs on
+// XCD b % 8 and takes tokens t with t % 8 == b % 8, as the reduce of a small world does.
+//
+// AUX, the stores' cache policy.  Rows of whole 128-byte lines are written through and kept in the memory-side cache for Combine
+// (kAuxAgentScopeKept; the per-route kernel's must stream, or they push the token rows that its workgroups share out of the L2s).
+// Of other rows nearly every store of a wave begins and ends within a line, which written through are two trips for one line.
+// They are ordinary stores (0), which come together in the L2, where a token has four and more of them, and stream below, where
+// there is less for Combine to find.  Forward stages, us copied per route, kept and so: 2223 x 2008 x top-6 54.0, 56.8 and 56.1,
+// 4000 x 2008 x top-2 48.2, 51.1 and 47.5, 2223 x 5000 x top-6 83.9, 89.6 and 86.4, 4000 x 5000 x top-2 72.0, 76.2 and 69.8, 7000 x
+// 1000 x top-6 90.4, 71.6 and 68.6; all four 1501 x 7176 x top-8 205.7, 211.3 and 206.2, 4000 x 7176 x top-3 233.4, 244.7 and 242.3.
+// (Ordinary stores for three of them 2223 x 7176 76.6, streaming ones 72.0.)
+template <bool FRESH, bool PLAN, int G, int V, int AUX>
 __global__ __launch_bounds__(kThreads) void moon_scatter_token_kernel(DispatchWorld a, int colSlices, unsigned planBlocks,
     int planChunks, int planSelf)
 {
@@ -442,7 +449,7 @@ __global__ __launch_bounds__(kThreads) void moon_scatter_token_kernel(DispatchWo
         for (int i = 0; i < V; ++i) {
             const int idx = colBase + i * G + lane;
             if (idx < vecs) {
-                __builtin_amdgcn_raw_buffer_store_b128(v[i], dst, idx * 16, 0, TileXREp::kAuxAgentScopeKept);
+                __builtin_amdgcn_raw_buffer_store_b128(v[i], dst, idx * 16, 0, AUX);
             }
         }
     }
@@ -1371,34 +1378,48 @@ hipError_t LaunchMoonDispatch(const DispatchWorld &w, hipStream_t stream, const 
         // (2000 x 4096 x top-6 129.9, 128.1, 127.3, 126.6).  Stored once or twice: two ranks x 16333 x 4096 798, 794, 810, 872; 11308
         // x 12288 x top-1, fwd, 263.3, 261.7, 268.2, 283.8; 3000 x 7168 x top-2 148.0, 147.2, 146.2, 149.8.  Four ranks x 4096 x 7168
         // x top-8 (1.9 GB) 1785, 1817, -, 1816, eight x 2500 x 7168, fwd, 1137, 1161, -, 1161.
+        // Two for rows that end within a line, which are not written through; fwd, at eight, four and two: 4000 x 3000 x top-4 72.5,
+        // 70.7 and 69.3, 4000 x 2008 x top-2 49.6, 49.9 and 47.3, 2223 x 5000 x top-2 53.0, 51.5 and 49.8, 2223 x 7176 x top-6 121.9,
+        // 119.4 and 118.0.
         const int64_t heldVecs = vecs <= 4 * kWave ? vecs * (kThreads / kWave) : vecs;
-        const int capWorkgroups = heldVecs > 2 * kThreads && w.k >= 4 ? 2 : 4;
+        const bool wholeLines = vecs % 8 == 0;
+        const int capWorkgroups = !wholeLines || (heldVecs > 2 * kThreads && w.k >= 4) ? 2 : 4;
         const unsigned capLds = worldRowBytes * w.k <= (int64_t{1} << 30) ? TileXREp::CapLdsBytes(capWorkgroups) : 0u;
-        auto launch = [&](auto lanes, auto vecsPerLane) {
+        auto launch = [&](auto lanes, auto vecsPerLane, auto stores) {
             constexpr int G = decltype(lanes)::value;
             constexpr int V = decltype(vecsPerLane)::value;
+            constexpr int kAux = decltype(stores)::value;
             constexpr int64_t kTokens = kThreads / G * kXcds;       // tokens of eight neighbouring workgroups
             const dim3 grid(static_cast<unsigned>((w.s + kTokens - 1) / kTokens * kXcds * tokenSlices) + planBlocks, R);
             if (planInScatter) {
-                hipLaunchKernelGGL((moon_scatter_token_kernel<true, true, G, V>), grid, dim3(kThreads), capLds, stream, w, tokenSlices,
-                    planBlocks, planChunks, planSelf ? 1 : 0);
+                hipLaunchKernelGGL((moon_scatter_token_kernel<true, true, G, V, kAux>), grid, dim3(kThreads), capLds, stream, w,
+                    tokenSlices, planBlocks, planChunks, planSelf ? 1 : 0);
             } else if (w.fresh) {
-                hipLaunchKernelGGL((moon_scatter_token_kernel<true, false, G, V>), grid, dim3(kThreads), capLds, stream, w, tokenSlices,
-                    0u, 0, 0);
+                hipLaunchKernelGGL((moon_scatter_token_kernel<true, false, G, V, kAux>), grid, dim3(kThreads), capLds, stream, w,
+                    tokenSlices, 0u, 0, 0);
             } else {
-                hipLaunchKernelGGL((moon_scatter_token_kernel<false, false, G, V>), grid, dim3(kThreads), capLds, stream, w, tokenSlices,
-                    0u, 0, 0);
+                hipLaunchKernelGGL((moon_scatter_token_kernel<false, false, G, V, kAux>), grid, dim3(kThreads), capLds, stream, w,
+                    tokenSlices, 0u, 0, 0);
+            }
+        };
+        auto pickStores = [&](auto lanes, auto vecsPerLane) {
+            if (wholeLines) {
+                launch(lanes, vecsPerLane, std::integral_constant<int, TileXREp::kAuxAgentScopeKept>{});
+            } else if (w.k >= 4) {
+                launch(lanes, vecsPerLane, std::integral_constant<int, 0>{});
+            } else {
+                launch(lanes, vecsPerLane, std::integral_constant<int, TileXREp::kAuxNonTemporal>{});
             }
         };
         // narrow rows: a wave per token (four tokens per workgroup); wide ones: the workgroup
         if (vecs <= 2 * kWave) {
-            launch(std::integral_constant<int, kWave>{}, std::integral_constant<int, 2>{});
+            pickStores(std::integral_constant<int, kWave>{}, std::integral_constant<int, 2>{});
         } else if (vecs <= 4 * kWave) {
-            launch(std::integral_constant<int, kWave>{}, std::integral_constant<int, 4>{});
+            pickStores(std::integral_constant<int, kWave>{}, std::integral_constant<int, 4>{});
         } else if (vecs <= 2 * kThreads) {
-            launch(std::integral_constant<int, kThreads>{}, std::integral_constant<int, 2>{});
+            pickStores(std::integral_constant<int, kThreads>{}, std::integral_constant<int, 2>{});
         } else {
-            launch(std::integral_constant<int, kThreads>{}, std::integral_constant<int, kTokenVecs / kThreads>{});
+            pickStores(std::integral_constant<int, kThreads>{}, std::integral_constant<int, kTokenVecs / kThreads>{});
         }
     } else if (perRoute) {
         gScatterName = "moon_scatter_kernel";
