@@ -246,32 +246,44 @@ __device__ __forceinline__ char *UniformPointer(char *p)
 // memory-side cache.  dispatch + combine with ordinary loads and stores, and so, us: 4 ranks x 512 x 4096 x top-8 232 -> 217, 8
 // x 500 438 -> 417, 4 x 1000 x 7168 x top-4 355 -> 317, top-8 620 -> 587.  (Ordinary loads, kept stores 235; streaming loads,
 // ordinary stores 219; streaming both 234.)
-__device__ __forceinline__ void CopyBytes(char *dst, const char *src, int64_t bytes, int tid, int threads)
+// Rows that end within a 128-byte line are copied by ordinary loads and stores (KEPT = false): written through, the parts of a
+// line are trips of their own.  Before the rows were kept, kept and now: 4 x 1500 x 7176 x top-6 715, 797 and 723, 8 x 700 x 7176 x
+// top-8 945, 1038 and 938, 4 x 1500 x 5000 x top-6 525, 557 and 533, 2 x 4000 x 3000 x top-4 283, 308 and 287 (streaming loads,
+// ordinary stores 319).
+template <bool KEPT>
+__device__ __forceinline__ void CopyVectors(char *dst, const char *src, int vecs, int tid, int threads)
 {
-    if (((reinterpret_cast<uintptr_t>(dst) | reinterpret_cast<uintptr_t>(src) | static_cast<uintptr_t>(bytes)) & 15u) == 0) {
-        const u32x4 *s = reinterpret_cast<const u32x4 *>(src);
-        constexpr int kAhead = 4;       // vectors a lane has in flight
-        const int vecs = static_cast<int>(bytes / 16);
-        const __amdgpu_buffer_rsrc_t rows = RowResource(UniformPointer(dst), vecs * 16);
-        for (int i = tid; i < vecs; i += kAhead * threads) {
-            u32x4 v[kAhead];
+    const u32x4 *s = reinterpret_cast<const u32x4 *>(src);
+    constexpr int kAhead = 4;       // vectors a lane has in flight
+    const __amdgpu_buffer_rsrc_t rows = RowResource(UniformPointer(dst), vecs * 16);
+    for (int i = tid; i < vecs; i += kAhead * threads) {
+        u32x4 v[kAhead];
 #pragma unroll
-            for (int u = 0; u < kAhead; ++u) {
-                const int at = i + u * threads;
-                v[u] = __builtin_nontemporal_load(s + (at < vecs ? at : i));
-            }
+        for (int u = 0; u < kAhead; ++u) {
+            const int at = i + u * threads;
+            const u32x4 *from = s + (at < vecs ? at : i);
+            v[u] = KEPT ? __builtin_nontemporal_load(from) : *from;
+        }
 #pragma unroll
-            for (int u = 0; u < kAhead; ++u) {
-                const int at = i + u * threads;
-                if (at < vecs) {
-                    __builtin_amdgcn_raw_buffer_store_b128(v[u], rows, at * 16, 0, kAuxAgentScopeKept);
-                }
+        for (int u = 0; u < kAhead; ++u) {
+            const int at = i + u * threads;
+            if (at < vecs) {
+                __builtin_amdgcn_raw_buffer_store_b128(v[u], rows, at * 16, 0, KEPT ? kAuxAgentScopeKept : 0);
             }
         }
-    } else {
+    }
+}
+
+__device__ __forceinline__ void CopyBytes(char *dst, const char *src, int64_t bytes, int tid, int threads)
+{
+    if (((reinterpret_cast<uintptr_t>(dst) | reinterpret_cast<uintptr_t>(src) | static_cast<uintptr_t>(bytes)) & 15u) != 0) {
         for (int64_t i = tid; i < bytes; i += threads) {
             dst[i] = src[i];
         }
+    } else if (bytes % 128 == 0) {
+        CopyVectors<true>(dst, src, static_cast<int>(bytes / 16), tid, threads);
+    } else {
+        CopyVectors<false>(dst, src, static_cast<int>(bytes / 16), tid, threads);
     }
 }
 
