@@ -24,6 +24,8 @@ CASES = [
     (2600, 8200, 8, 64, "none", "ep_scatter_route_kernel"),         # a second part of one vector
     (1100, 8200, 8, 64, "none", "ep_scatter_vec_kernel"),           # published whole
     (1000, 1048, 5, 16, "int8", "ep_scatter_vec_kernel"),
+    (4100, 1040, 8, 16, "int8", "ep_scatter_vec_kernel"),           # ends within a line, 32 MiB and more: ordinary stores
+    (1200, 7176, 4, 16, "none", "ep_scatter_vec_kernel"),
     (16384, 4096, 8, 64, "fp8", "ep_scatter_vec_kernel"),           # exactly 512 MiB
     (16385, 4096, 8, 64, "fp8", "ep_scatter_vec_kernel"),
     # rows that the scatter resolves itself (too many routes x experts for the one-launch routing), on both sides of the vectors

@@ -75,11 +75,20 @@ __device__ __forceinline__ float GroupMax(float v, float *red, int lane)
 // top-6 108.4 -> 100.2 (its scatter 49.9 -> 42.5), 4096 x 7168 x top-8 127.0 -> 109.0; block fp8 16384 x 2048 under a
 // capacity 98.4 -> 92.0 (scatter 48.9 -> 39.0, reduce 40.7 -> 44.4: it waits for rows that leave the cache).  Ordinary
 // stores (dirty in the L2 until the launch ends) come in between: 46.0, 101.8, 93.1 for three of those.
+// Rows that end within a 128-byte line are the exception: nearly every store of a wave begins and ends within a line, and written
+// through each half is a trip of its own, where the L2 puts ordinary ones together.  Streaming (by the launches that suit that),
+// kept and ordinary: 9000 x 7176 x top-6 369, 382 and 354, under a capacity 366, 389 and 341, on the MVP route 332, 370 and 334;
+// 1200 x 7176 x top-8 67.6, 68.0 and 65.6; 4000 x 6408 x top-6 156.9, 146.4 and 141.3; 4500 x 2008 x top-8 79.2, 75.0 and 70.7; int8
+// 9000 x 2064 x top-6 91.9, 79.0 and 77.0; but 2500 x 7176 x top-4 73.7, 75.9 and 75.3.
 enum class RowStores {
     kStream,        // non-temporal
     kKeep,          // written through (sc1) and kept
     kPublish,       // written through and streaming (sc1 nt)
+    kOrdinary,      // dirty in the L2 until the launch ends
 };
+
+template <RowStores S>
+constexpr int kRowAux = S == RowStores::kKeep ? kAuxAgentScopeKept : S == RowStores::kPublish ? kAuxAgentScope : 0;
 
 template <RowStores S>
 __device__ __forceinline__ void RowStore(const u32x4 &v, char *rowBase, __amdgpu_buffer_rsrc_t rsrc, int byteOffset)
@@ -87,7 +96,7 @@ __device__ __forceinline__ void RowStore(const u32x4 &v, char *rowBase, __amdgpu
     if (S == RowStores::kStream) {
         __builtin_nontemporal_store(v, reinterpret_cast<u32x4 *>(rowBase + byteOffset));
     } else {
-        __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, byteOffset, 0, S == RowStores::kKeep ? kAuxAgentScopeKept : kAuxAgentScope);
+        __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, byteOffset, 0, kRowAux<S>);
     }
 }
 
@@ -97,7 +106,7 @@ __device__ __forceinline__ void RowStore(const u32x2 &v, char *rowBase, __amdgpu
     if (S == RowStores::kStream) {
         __builtin_nontemporal_store(v, reinterpret_cast<u32x2 *>(rowBase + byteOffset));
     } else {
-        __builtin_amdgcn_raw_buffer_store_b64(v, rsrc, byteOffset, 0, S == RowStores::kKeep ? kAuxAgentScopeKept : kAuxAgentScope);
+        __builtin_amdgcn_raw_buffer_store_b64(v, rsrc, byteOffset, 0, kRowAux<S>);
     }
 }
 
@@ -610,6 +619,12 @@ int CapWorkgroups(const ScatterArgs &a)
     return vecs > 2 * kThreads && (!resolves || (stored >= 18 * kThreads && (cachedTokens || a.topK > 4))) ? 2 : 4;
 }
 
+template <int QMODE>
+int64_t RowBytes(const ScatterArgs &a)
+{
+    return QMODE == TILEXR_EP_QUANT_NONE ? int64_t{2} * a.h : a.h;
+}
+
 // Whether the rows are left in the memory-side cache.  They are where this library's combine can take them as they are.  A
 // payload that only an expert stage decodes streams (dispatch + combine of other rows with nothing in between, streaming and
 // kept: MXFP8 2048 x 7168 88.9 and 91.2 us, 4096 x 7168 155 and 168, int8 on the MVP route 4000 x 2048 49.0 and 51.4).
@@ -624,12 +639,12 @@ int CapWorkgroups(const ScatterArgs &a)
 // dispatch and combine at these sizes are products.
 //   Block fp8 rows beyond twice that cache stream too (16384 x 7168 x top-6 378 and 388, 8192 x 8192 x top-8 274 -> 269), int8
 // and plain ones are kept at any size (16384 x 7168 x top-8 int8 468.5 -> 466.2, plain 775.5 -> 770.3).  Rows that end within
-// a 128-byte line are two partial lines each and want a launch worth it: 1000 columns, 1501 tokens x top-6 19.1 and 19.6,
-// 4000 x top-6 31.2 and 31.4, 4000 x top-8 39.4 -> 37.1.
+// a 128-byte line (ordinary stores unless they are published) want a launch worth it: 1000 columns, streaming and written through,
+// 1501 tokens x top-6 19.1 and 19.6, 4000 x top-6 31.2 and 31.4, 4000 x top-8 39.4 -> 37.1.
 template <int QMODE>
 bool KeepsRows(const ScatterArgs &a)
 {
-    const int64_t rowBytes = QMODE == TILEXR_EP_QUANT_NONE ? int64_t{2} * a.h : a.h;
+    const int64_t rowBytes = RowBytes<QMODE>(a);
     const int64_t bytes = static_cast<int64_t>(a.bs) * a.topK * rowBytes;
     if (QMODE == TILEXR_EP_QUANT_FP8_BLOCK128 && bytes > 2 * kMemorySideCacheBytes) {
         return false;
@@ -642,7 +657,7 @@ void LaunchVecStoring(const ScatterArgs &a, hipStream_t stream)
 {
     constexpr int kTokens = kThreads / G;
     const dim3 groups((a.bs + kTokens - 1) / kTokens);
-    if constexpr (S != RowStores::kStream) {
+    if constexpr (S == RowStores::kKeep || S == RowStores::kPublish) {
         if (Publishes(a)) {
             hipLaunchKernelGGL((ep_scatter_vec_kernel<G, V, QMODE, BF16, E5M2, true, S>), groups, dim3(kThreads), 0, stream, a);
             return;
@@ -661,7 +676,11 @@ void LaunchVec(const ScatterLaunch &l, const ScatterArgs &a)
         QMODE == TILEXR_EP_QUANT_FP8_BLOCK128;
     if constexpr (kCombineTakes) {
         if (l.combineTakesRows && KeepsRows<QMODE>(a)) {
-            LaunchVecStoring<G, V, QMODE, BF16, E5M2, RowStores::kKeep>(a, l.stream);
+            if (Publishes(a) || RowBytes<QMODE>(a) % 128 == 0) {
+                LaunchVecStoring<G, V, QMODE, BF16, E5M2, RowStores::kKeep>(a, l.stream);
+            } else {
+                LaunchVecStoring<G, V, QMODE, BF16, E5M2, RowStores::kOrdinary>(a, l.stream);
+            }
             return;
         }
     }
