@@ -157,10 +157,11 @@ bool PrepareTables(WorldState *st, int world, int64_t nvS, int64_t n, WorldTable
     const int64_t stride = (rows + kTableAlign - 1) / kTableAlign * kTableAlign;
     const int64_t groups = (rows + kChunkRows - 1) / kChunkRows;
     const int64_t perRank8 = stride * 8;
-    // six 8-byte tables and the per-rank words; two 4-byte tables, the chunks' totals and a table of bytes
-    st->taggedWords = world * (6 * stride + 1);
+    // six 8-byte tables, the per-rank words and the chunks' tags; three 4-byte tables, the chunks' totals and a table of bytes
+    st->taggedWords = world * (6 * stride + 1 + stride / kTableAlign);
     if (!st->tables.Reserve(static_cast<size_t>(st->taggedWords * 8), true) ||
-        !st->plainTables.Reserve(static_cast<size_t>(world * (2 * stride * 4 + groups * 8 + stride)), true)) {
+        !st->plainTables.Reserve(static_cast<size_t>(world * (3 * stride * 4 + groups * 8 + stride)), true) ||
+        !st->arrived.Reserve(sizeof(uint32_t), true)) {
         return false;
     }
     char *p = static_cast<char *>(st->tables.ptr);
@@ -176,11 +177,14 @@ bool PrepareTables(WorldState *st, int world, int64_t nvS, int64_t n, WorldTable
     out->slotDup = reinterpret_cast<uint64_t *>(take(world * perRank8));
     out->slotGroup = reinterpret_cast<uint64_t *>(take(world * perRank8));
     out->fail = reinterpret_cast<uint64_t *>(take(world * 8));
+    out->chunkTag = reinterpret_cast<uint64_t *>(take(world * (stride / kTableAlign) * 8));
     p = static_cast<char *>(st->plainTables.ptr);
     out->sibling = reinterpret_cast<uint32_t *>(take(world * stride * 4));
     out->slotCount = reinterpret_cast<int32_t *>(take(world * stride * 4));
     out->chunkTotals = reinterpret_cast<int32_t *>(take(world * groups * 8));
+    out->origin = reinterpret_cast<uint32_t *>(take(world * stride * 4));
     out->direct = reinterpret_cast<uint8_t *>(take(world * stride));
+    out->arrived = static_cast<uint32_t *>(st->arrived.ptr);
     out->stride = stride;
     out->groupStride = groups;
     return true;
@@ -434,6 +438,7 @@ void ReleaseWorldState(WorldState *st)
     }
     st->tables.Release();
     st->plainTables.Release();
+    st->arrived.Release();
     for (RankEvents &e : st->events) {
         if (e.arrived != nullptr) {
             (void)hipEventDestroy(e.arrived);

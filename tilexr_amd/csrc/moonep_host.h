@@ -42,6 +42,7 @@ struct WorldState {
     TileXREp::DeviceBuffer tables;      // nothing but words that carry their epoch
     int64_t taggedWords = 0;            // how many of them the tables of the last shape have
     TileXREp::DeviceBuffer plainTables; // the tables of other words
+    TileXREp::DeviceBuffer arrived;     // one word at the same place for every shape: it is zero between dispatches
     std::vector<StageCall> dispatch;    // calls waiting for the rest of the world, by rank
     std::vector<StageCall> combine;
     std::vector<RankEvents> events;

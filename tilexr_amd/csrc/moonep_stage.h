@@ -33,6 +33,7 @@ constexpr int kMaxWorld = 16;       // ranks of a world this library runs the st
 constexpr int kMaxTopK = 32;        // reference: src/moonep/common/moonep_stage_layout.h:78
 constexpr int kTableAlign = 256;    // per-rank table strides are a multiple of this many entries
 constexpr int kChunkRows = 2048;    // rows per workgroup of the duplicate-plan build
+constexpr uint8_t kNoRank = 0xff;
 
 // Device status values (reference: src/moonep/common/moonep_peer_window.h:36-43).
 constexpr int32_t kDispatchOk = 2000;
@@ -53,8 +54,13 @@ struct WorldTables {
     uint64_t *slotDup;       // combine: per origin slot, epoch << 32 | 1 when that row is a duplicate (it does not travel)
     uint64_t *slotGroup;     // combine: per origin slot, epoch << 32 | first dupLoffs index when that row has duplicates
     int32_t *slotCount;      // combine: per origin slot, number of those duplicates (valid with slotGroup)
-    uint8_t *direct;         // dispatch, saved plans: per source route, 1 when the source writes the duplicate's row itself
-                             //           (rewritten for every route by every saved-plan dispatch)
+    uint8_t *direct;         // dispatch, per source route, rewritten for every route by every dispatch that reads it.  Saved
+                             //           plans: 1 when the source writes the route's row itself.  Fresh plans: the
+                             //           duplicate's rank within its group, kNoRank where the route is in none
+    uint32_t *origin;        // dispatch: source rank * n + route that writes the row (saved plans, rows tagged as written) or
+                             //           that opens the row's group (fresh plans, duplicates with sibling rank 0)
+    uint64_t *chunkTag;      // dispatch, fresh plans: [world][stride / kTableAlign] epoch << 32 | totals of so many rows
+    uint32_t *arrived;       // dispatch, fresh plans: ranks whose plan is built; zero whenever no dispatch is in flight
     uint64_t *fail;          // [world] epoch << 32 | device status of the rank's own failure
     int32_t *chunkTotals;    // dispatch, fresh plans: [world][groupStride][2] group-opening rows and duplicates per chunk
     int64_t stride;          // >= nvS and >= n, a multiple of kTableAlign

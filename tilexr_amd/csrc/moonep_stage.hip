@@ -11,6 +11,7 @@
 //                                src/moonep/combine/kernels/tilexr_moonep_combine_kernel.cpp:117-177, 285-366, 449-541,
 //                                568-606, 648-733
 #include <atomic>
+#include <initializer_list>
 #include <type_traits>
 
 #include <hip/hip_runtime.h>
@@ -35,10 +36,10 @@ std::atomic<int64_t> gCachedRowBytes {kDefaultCachedRowBytes};  // TileXRMoonEpS
 // Workgroups per compute unit that the copying launches are held to.  Per route: eight keep more stores in flight than this
 // memory system digests (4096 x 7168 x top-8, four stages, us at eight, seven, six, five, four, three, two: 420, 415, 401, 397,
 // 410, 439, 512; 5800 x 4096, the forward two 170.3, 170.2, 170.1, 169.0, 169.2, 176.7, 200.5).
-constexpr unsigned kScatterCapLdsBytes = TileXREp::CapLdsBytes(5);
-constexpr int kFusedPlanChunks = 1024;  // chunks of 2048 rows per rank up to which the scatter launch builds a fresh plan
-constexpr int64_t kFusedPlanRowBytes = int64_t{256} << 20;     // ... and, copied per route, bytes of rows the world's routes write
-constexpr int kSelfPlanChunks = 8;      // ... and up to which its plan workgroups add up the earlier chunks themselves
+constexpr int kScatterCapWorkgroups = 5;
+constexpr int kFusedPlanChunks = 2048;  // chunks of 256 rows per rank up to which the scatter launch builds a fresh plan: each of
+                                        // its workgroups looks at the totals of all chunks before its own
+constexpr int64_t kMostCopyBlocks = 0x7fffffff - (1 << 26);     // a rank's share of a grid, less its other workgroups
 constexpr int64_t kWarmRowBytes = int64_t{128} << 20;          // token rows of a world that are read ahead of the per-route scatter
                                                                // (with SetCachedRowBytes at its default there are 104 MiB at most)
 constexpr int64_t kKeptRowBytes = int64_t{360} << 20;          // rows of a world up to which the per-token scatter is the faster one,
@@ -157,13 +158,13 @@ __device__ __forceinline__ void RouteRecords(const DispatchWorld &a, int src, in
     }
 }
 
-// Whether the source writes the row of this route, and the tag the row gets.
+// Whether the row of this route holds its token's row before any copy is made from a primary, and the tag the row gets.
 //   fresh plan   every route: the plan is being built from these very route words, so a duplicate row is by construction
 //                a copy of this token's row
 //   saved plan   non-duplicates; and a duplicate whose primary, according to the plan (parent records written by the walk
-//                kernel), is the row this token's own non-duplicate route to that rank writes -- the copy the finish
-//                kernel would make is a copy of this token's row (`direct`, worked out by the agree kernel).  Any other
-//                duplicate is left to the finish kernel.
+//                kernel), is the row this token's own non-duplicate route to that rank writes -- the copy that would be
+//                made of its primary is a copy of this token's row (`direct`, worked out by the agree kernel).  Any other
+//                duplicate is left to FinishRows.
 template <bool FRESH>
 __device__ __forceinline__ bool SourceWrites(const Route &r, uint8_t direct, uint32_t *tagBits)
 {
@@ -202,10 +203,12 @@ __device__ __forceinline__ void WarmRows(const DispatchWorld &a, int rank, int64
 
 // Saved plans, one thread per route of source rank blockIdx.y: whether the source may write a duplicate's row itself
 // (see SourceWrites).  Done ahead of the scatter so that its workgroups find the answer with the route word, in one
-// round trip, instead of looking up the parent record after decoding it.  Ahead of the per-route scatter (`records`) it
-// also writes what a route records, weight and row tag, and reports a route that names no rank.  The workgroups from
-// `routeBlocks` on read the token rows ahead (WarmRows) when warmVecs is not zero: this launch waits on a few small loads
-// and leaves the memory system idle, so the read costs a saved-plan Dispatch no launch of its own.
+// round trip, instead of looking up the parent record after decoding it.  Ahead of a scatter that only copies (`records`) it
+// also writes what a route records -- weight, row tag, the row's origin -- and reports a route that names no rank; `direct`
+// then answers for every route, and is 0 too for a non-duplicate whose row the plan lists as a duplicate: FinishRows fills
+// that row, in the scatter's own launch.  The workgroups from `routeBlocks` on read the token rows ahead (WarmRows) when
+// warmVecs is not zero: this launch waits on a few small loads and leaves the memory system idle, so the read costs a
+// saved-plan Dispatch no launch of its own.
 __global__ __launch_bounds__(kThreads) void moon_agree_kernel(DispatchWorld a, unsigned routeBlocks, int64_t warmVecs, int records)
 {
     if (blockIdx.x >= routeBlocks) {
@@ -224,20 +227,25 @@ __global__ __launch_bounds__(kThreads) void moon_agree_kernel(DispatchWorld a, u
     uint8_t direct = 0;
     const Route r = Decode(words[k], a.nvS, a.world);
     const int64_t at = static_cast<int64_t>(r.peer) * a.tables.stride + r.row;
+    const uint64_t p = r.ok ? a.tables.parentTag[at] : 0ull;
+    const bool listed = Tagged(p, a.epoch);
     if (r.ok && r.duplicate) {
-        const uint64_t p = a.tables.parentTag[at];
-        direct = Tagged(p, a.epoch) && static_cast<int>(p & 0xffffffffu) - 1 == OwnPrimaryRow(a, words, k, r.peer) ? 1 : 0;
+        direct = listed && static_cast<int>(p & 0xffffffffu) - 1 == OwnPrimaryRow(a, words, k, r.peer) ? 1 : 0;
     }
-    a.tables.direct[static_cast<int64_t>(src) * a.tables.stride + route] = direct;
+    const int64_t at0 = static_cast<int64_t>(src) * a.tables.stride + route;
     if (records == 0) {
+        a.tables.direct[at0] = direct;
         return;
     }
+    a.tables.direct[at0] = r.ok && !r.duplicate && !listed ? 1 : direct;
     if (!r.ok) {
         RecordFailure(a.tables, src, a.epoch, kDispatchInvalidRoute);
         return;
     }
     uint32_t tagBits = 0;
-    SourceWrites<false>(r, direct, &tagBits);
+    if (SourceWrites<false>(r, direct, &tagBits)) {
+        a.tables.origin[at] = static_cast<uint32_t>(src * a.s * a.k + route);
+    }
     if (a.weightsSk[src] != nullptr) {
         a.weightsNvs[r.peer][r.row] = weight;
     }
@@ -248,8 +256,7 @@ __global__ __launch_bounds__(kThreads) void moon_agree_kernel(DispatchWorld a, u
 // failure of a route that names no rank, ahead of the per-route scatter, whose workgroups then only copy: with the records
 // in them they asked for route words, weights and the token's other routes between the copies of everybody else, and a
 // scatter on tables that were not cached took 110 us instead of 76 (4096 x 7168 x top-8).  Nothing the plan is built from
-// is written by the scatter launch, so for smaller worlds extra workgroups of that launch build it (moon_scatter_kernel,
-// PLAN) instead of launches after it.
+// is written by the scatter launch, so extra workgroups of that launch build it (PlanChunk).
 // The workgroups from `routeBlocks` on read the token rows ahead, as in moon_agree_kernel.
 __global__ __launch_bounds__(kThreads) void moon_records_kernel(DispatchWorld a, unsigned routeBlocks, int64_t warmVecs)
 {
@@ -267,7 +274,9 @@ __global__ __launch_bounds__(kThreads) void moon_records_kernel(DispatchWorld a,
     const int32_t *words = a.dst[src] + route - k;
     const float weight = a.weightsSk[src] != nullptr ? a.weightsSk[src][route] : 0.0f;
     const Route r = Decode(words[k], a.nvS, a.world);
+    uint8_t *rankInGroup = a.tables.direct + static_cast<int64_t>(src) * a.tables.stride + route;
     if (!r.ok) {
+        *rankInGroup = kNoRank;
         RecordFailure(a.tables, src, a.epoch, kDispatchInvalidRoute);
         return;
     }
@@ -277,6 +286,7 @@ __global__ __launch_bounds__(kThreads) void moon_records_kernel(DispatchWorld a,
     }
     a.tables.rowTag[at] = Tag(a.epoch, kRowNamed | kRowWritten);
     if (!r.duplicate) {
+        *rankInGroup = kNoRank;
         return;
     }
     // the token's other routes to the same rank: the first non-duplicate before this one is the primary, the duplicates
@@ -297,161 +307,15 @@ __global__ __launch_bounds__(kThreads) void moon_records_kernel(DispatchWorld a,
         }
     }
     if (primaryRow < 0) {
+        *rankInGroup = kNoRank;
         RecordFailure(a.tables, src, a.epoch, kDispatchInvalidRoute);
         return;
     }
+    *rankInGroup = static_cast<uint8_t>(before);
     a.tables.parentTag[at] = Tag(a.epoch, static_cast<uint32_t>(primaryRow) + 1u);
     a.tables.sibling[at] = before | (siblings << 16);
-}
-
-// defined with the kernels that build the duplicate plan, below
-template <bool SELF>
-__device__ __forceinline__ void DedupGroupsOfChunk(const DispatchWorld &a, int rank, int chunk, bool lastChunk,
-    int (*s_part)[kThreads / kWave], int *s_base);
-
-// A plan workgroup of a scatter launch: chunk blockIdx.x of destination rank blockIdx.y.
-__device__ __forceinline__ void PlanWorkgroup(const DispatchWorld &a, int planChunks, int planSelf)
-{
-    __shared__ int s_part[2][kThreads / kWave];
-    __shared__ int s_base[2];
-    const int chunk = blockIdx.x;
-    if (chunk < planChunks && planSelf != 0) {
-        DedupGroupsOfChunk<true>(a, blockIdx.y, chunk, chunk == planChunks - 1, s_part, s_base);
-    } else if (chunk < planChunks) {
-        DedupGroupsOfChunk<false>(a, blockIdx.y, chunk, chunk == planChunks - 1, s_part, s_base);
-    }
-}
-
-// One workgroup per (token, route, slice of 512 vectors) of source rank blockIdx.y.  What the routes record was written
-// ahead, by moon_records_kernel or moon_agree_kernel.
-//
-// PLAN: a fresh plan is built here as well: the first `planBlocks` workgroups of the launch (a multiple of eight, so
-// that the rest keep their XCDs) take one chunk of destination rank blockIdx.y each.  They depend on nothing this launch
-// writes and are done long before the rows are.  The totals of the chunks before its own a workgroup adds up itself
-// while the chunks are few (planSelf), a trip to memory per chunk, and those trips are slow beside the scatter's traffic
-// (measured: 5 us each; 32 chunks took longer than the rows); otherwise a launch of moon_dedup_totals_kernel ahead of
-// this one has left them.
-template <bool FRESH, bool PLAN>
-__global__ __launch_bounds__(kThreads) void moon_scatter_kernel(DispatchWorld a, int colSlices, unsigned planBlocks, int planChunks,
-    int planSelf)
-{
-    static_assert(FRESH || !PLAN, "only a Dispatch that builds its plan has plan workgroups");
-    if (PLAN && blockIdx.x < planBlocks) {
-        PlanWorkgroup(a, planChunks, planSelf);
-        return;
-    }
-    const unsigned block = blockIdx.x - (PLAN ? planBlocks : 0u);
-    const int src = blockIdx.y;
-    const int xcd = block % kXcds;
-    const int j = block / kXcds;
-    const int K = static_cast<int>(a.k);
-    const int perToken = K * colSlices;
-    const int token = (j / perToken) * kXcds + xcd;
-    const int k = (j % perToken) / colSlices;
-    const int slice = (j % perToken) % colSlices;
-    if (token >= a.s) {
-        return;
-    }
-    const int lane = threadIdx.x;
-    const int h = static_cast<int>(a.h);
-    const int vecs = h / 8;
-    const int colBase = slice * (kRowVecs * kThreads);
-    const int64_t route = static_cast<int64_t>(token) * K + k;
-    const int32_t encoded = a.dst[src][route];
-    const uint8_t direct = FRESH ? 0 : a.tables.direct[static_cast<int64_t>(src) * a.tables.stride + route];
-    const u32x4 *srcRow = reinterpret_cast<const u32x4 *>(static_cast<const char *>(a.hiddenSh[src]) +
-        static_cast<int64_t>(token) * h * 2);
-    u32x4 v[kRowVecs];
-#pragma unroll
-    for (int i = 0; i < kRowVecs; ++i) {
-        const int idx = colBase + i * kThreads + lane;
-        v[i] = idx < vecs ? srcRow[idx] : u32x4{0u, 0u, 0u, 0u};
-    }
-    const Route r = Decode(encoded, a.nvS, a.world);
-    uint32_t tagBits = 0;
-    if (r.ok && SourceWrites<FRESH>(r, direct, &tagBits)) {
-        u32x4 *dstRow = reinterpret_cast<u32x4 *>(static_cast<char *>(a.hiddenNvsh[r.peer]) + static_cast<int64_t>(r.row) * h * 2);
-#pragma unroll
-        for (int i = 0; i < kRowVecs; ++i) {
-            const int idx = colBase + i * kThreads + lane;
-            if (idx < vecs) {
-                __builtin_nontemporal_store(v[i], dstRow + idx);
-            }
-        }
-    }
-}
-
-// G lanes per (token, slice of G x V vectors) of source rank blockIdx.y: the slice is loaded once and stored once per route.
-// What the routes record was written ahead, as for moon_scatter_kernel; PLAN as there.  Lane k of every wave works out the
-// row of route k for itself, so nothing is handed round and no wave waits between its loads and its stores.  Workgroup b runs on
-// XCD b % 8 and takes tokens t with t % 8 == b % 8, as the reduce of a small world does.
-//
-// AUX, the stores' cache policy.  Rows of whole 128-byte lines are written through and kept in the memory-side cache for Combine
-// (kAuxAgentScopeKept; the per-route kernel's must stream, or they push the token rows that its workgroups share out of the L2s).
-// Of other rows nearly every store of a wave begins and ends within a line, which written through are two trips for one line.
-// They are ordinary stores (0), which come together in the L2, where a token has four and more of them, and stream below, where
-// there is less for Combine to find.  Forward stages, us copied per route, kept and so: 2223 x 2008 x top-6 54.0, 56.8 and 56.1,
-// 4000 x 2008 x top-2 48.2, 51.1 and 47.5, 2223 x 5000 x top-6 83.9, 89.6 and 86.4, 4000 x 5000 x top-2 72.0, 76.2 and 69.8, 7000 x
-// 1000 x top-6 90.4, 71.6 and 68.6; all four 1501 x 7176 x top-8 205.7, 211.3 and 206.2, 4000 x 7176 x top-3 233.4, 244.7 and 242.3.
-// (Ordinary stores for three of them 2223 x 7176 76.6, streaming ones 72.0.)
-template <bool FRESH, bool PLAN, int G, int V, int AUX>
-__global__ __launch_bounds__(kThreads) void moon_scatter_token_kernel(DispatchWorld a, int colSlices, unsigned planBlocks,
-    int planChunks, int planSelf)
-{
-    static_assert(FRESH || !PLAN, "only a Dispatch that builds its plan has plan workgroups");
-    if (PLAN && blockIdx.x < planBlocks) {
-        PlanWorkgroup(a, planChunks, planSelf);
-        return;
-    }
-    constexpr int kTokens = kThreads / G;
-    const unsigned block = blockIdx.x - (PLAN ? planBlocks : 0u);
-    const int src = blockIdx.y;
-    const int j = static_cast<int>(block / kXcds);
-    const int slice = j % colSlices;
-    const int tg = threadIdx.x / G;
-    const int64_t token = (static_cast<int64_t>(j / colSlices) * kTokens + tg) * kXcds + block % kXcds;
-    if (token >= a.s) {
-        return;
-    }
-    const int lane = threadIdx.x % G;
-    const int waveLane = threadIdx.x % kWave;
-    const int K = static_cast<int>(a.k);
-    const int h = static_cast<int>(a.h);
-    const int vecs = h / 8;
-    const int colBase = slice * (G * V);
-    int32_t word = 0;
-    uint8_t direct = 0;
-    if (waveLane < K) {
-        const int64_t route = token * K + waveLane;
-        word = a.dst[src][route];
-        direct = FRESH ? 0 : a.tables.direct[static_cast<int64_t>(src) * a.tables.stride + route];
-    }
-    const u32x4 *srcRow = reinterpret_cast<const u32x4 *>(static_cast<const char *>(a.hiddenSh[src]) + token * h * 2);
-    u32x4 v[V];
-#pragma unroll
-    for (int i = 0; i < V; ++i) {
-        const int idx = colBase + i * G + lane;
-        v[i] = idx < vecs ? srcRow[idx] : u32x4{0u, 0u, 0u, 0u};
-    }
-    const Route r = Decode(word, a.nvS, a.world);
-    uint32_t tagBits = 0;
-    const bool writes = waveLane < K && r.ok && SourceWrites<FRESH>(r, direct, &tagBits);
-    const int row = writes ? r.row : -1;
-    for (int k = 0; k < K; ++k) {
-        const int rowOfK = __builtin_amdgcn_readlane(row, k);
-        if (rowOfK < 0) {
-            continue;
-        }
-        const int peer = __builtin_amdgcn_readlane(r.peer, k);
-        const __amdgpu_buffer_rsrc_t dst = TileXREp::RowResource(
-            static_cast<const char *>(a.hiddenNvsh[peer]) + static_cast<int64_t>(rowOfK) * h * 2, vecs * 16);
-#pragma unroll
-        for (int i = 0; i < V; ++i) {
-            const int idx = colBase + i * G + lane;
-            if (idx < vecs) {
-                __builtin_amdgcn_raw_buffer_store_b128(v[i], dst, idx * 16, 0, AUX);
-            }
-        }
+    if (before == 0) {
+        a.tables.origin[at] = static_cast<uint32_t>(src * a.s * a.k + route);
     }
 }
 
@@ -501,9 +365,10 @@ __global__ __launch_bounds__(kThreads) void moon_scatter_generic_kernel(Dispatch
 // primary, groups take their dupLoffs slices in that order, and each slice lists its duplicates in ascending row order
 // (dispatch kernel :330-424).  With the rank-within-group and group size recorded by the sources, both numberings are
 // exclusive prefix sums over the rows: group index = number of earlier group-opening rows, slice start = sum of their
-// group sizes.  A workgroup scans one chunk of 2048 rows after adding up the chunks before its own -- from the rows
-// themselves while the chunks are few, from the totals a first launch leaves otherwise.  The slices are filled by the
-// finish kernel, which visits every row anyway.
+// group sizes.  PlanChunk does that within the scatter launch; the kernels here follow a scatter that does nothing else
+// (moon_scatter_generic_kernel, plans of more than kFusedPlanChunks chunks).  A workgroup scans one chunk of 2048 rows after adding
+// up the chunks before its own -- from the rows themselves while the chunks are few, from the totals a first launch leaves
+// otherwise.  The slices are filled by the finish kernel, which visits every row anyway.
 constexpr int kBuildRows = kChunkRows;
 constexpr int kBuildPer = kBuildRows / kThreads;
 constexpr unsigned kSelfTotalChunks = 2;    // up to this many chunks a workgroup sums the earlier ones itself (one after
@@ -586,42 +451,32 @@ __global__ __launch_bounds__(kThreads) void moon_dedup_totals_kernel(DispatchWor
 }
 
 // What the thread's rows of the chunks before `chunks` add to their totals.  Both words of a row are asked for whatever
-// the first one says: one trip to memory per chunk, not two.  (One chunk at a time: the kernel that runs this beside a
-// scatter must stay small in registers, see LaunchMoonDispatch.)
-constexpr int kTotalsAhead = 1;
+// the first one says: one trip to memory per chunk, not two.
 __device__ __forceinline__ void AddEarlierChunks(const DispatchWorld &a, int rank, int chunks, int *open, int *size)
 {
     const uint64_t *parent = a.tables.parentTag + static_cast<int64_t>(rank) * a.tables.stride;
     const uint32_t *sibling = a.tables.sibling + static_cast<int64_t>(rank) * a.tables.stride;
-    for (int c0 = 0; c0 < chunks; c0 += kTotalsAhead) {
-        uint64_t p[kTotalsAhead][kBuildPer];
-        uint32_t sib[kTotalsAhead][kBuildPer];
+    for (int c = 0; c < chunks; ++c) {
+        uint64_t p[kBuildPer];
+        uint32_t sib[kBuildPer];
 #pragma unroll
-        for (int u = 0; u < kTotalsAhead; ++u) {
-#pragma unroll
-            for (int i = 0; i < kBuildPer; ++i) {
-                const int64_t row = static_cast<int64_t>(c0 + u) * kBuildRows + static_cast<int64_t>(threadIdx.x) * kBuildPer + i;
-                const bool in = c0 + u < chunks && row < a.nvS;
-                p[u][i] = in ? parent[row] : 0ull;          // the epoch is never zero: an untagged word
-                sib[u][i] = in ? sibling[row] : 0u;
-            }
+        for (int i = 0; i < kBuildPer; ++i) {
+            const int64_t row = static_cast<int64_t>(c) * kBuildRows + static_cast<int64_t>(threadIdx.x) * kBuildPer + i;
+            p[i] = row < a.nvS ? parent[row] : 0ull;            // the epoch is never zero: an untagged word
+            sib[i] = row < a.nvS ? sibling[row] : 0u;
         }
 #pragma unroll
-        for (int u = 0; u < kTotalsAhead; ++u) {
-#pragma unroll
-            for (int i = 0; i < kBuildPer; ++i) {
-                const bool opens = Tagged(p[u][i], a.epoch) && (sib[u][i] & 0xffffu) == 0;
-                *open += opens ? 1 : 0;
-                *size += opens ? static_cast<int>(sib[u][i] >> 16) : 0;
-            }
+        for (int i = 0; i < kBuildPer; ++i) {
+            const bool opens = Tagged(p[i], a.epoch) && (sib[i] & 0xffffu) == 0;
+            *open += opens ? 1 : 0;
+            *size += opens ? static_cast<int>(sib[i] >> 16) : 0;
         }
     }
 }
 
 // Groups and slice starts of one chunk of destination rank `rank` (see above).
-// SELF: the workgroup adds up the chunks before its own from the row records themselves -- when the chunks are few, and
-// when it runs as an extra workgroup of the scatter launch, where nothing waits for it; otherwise from the totals that a
-// launch of moon_dedup_totals_kernel left.
+// SELF: the workgroup adds up the chunks before its own from the row records themselves, when the chunks are few; otherwise
+// from the totals that a launch of moon_dedup_totals_kernel left.
 template <bool SELF>
 __device__ __forceinline__ void DedupGroupsOfChunk(const DispatchWorld &a, int rank, int chunk, bool lastChunk,
     int (*s_part)[kThreads / kWave], int *s_base)
@@ -805,49 +660,83 @@ __global__ __launch_bounds__(kThreads) void moon_group_walk_kernel(DispatchWorld
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// dispatch: rows nobody wrote
+// dispatch: rows nobody wrote, device status
 // ---------------------------------------------------------------------------------------------------------------
 
-// Work item of the finish kernel: row | kind << 30.
-constexpr int32_t kFillZero = 0;
-constexpr int32_t kFillCopy = 1;
 constexpr int kFinishRows = 64;     // rows one workgroup looks after
 
-// What is left to do once every source has scattered.  The first wave of a workgroup looks at 64 rows, one per lane:
-// nothing (a route wrote the row), zeros (no route wrote it: the reference clears the whole window first, dispatch kernel
-// :206-230), or -- saved plans -- a copy of its primary row (dispatch kernel :426-461); the weight of a row no route
-// names is zero for the same reason; the duplicates of a fresh plan take their places in dupLoffs.  Then the whole
-// workgroup writes the rows that need writing.  Workgroup 0 of every rank writes the rank's device status.
-template <bool VEC>
-__global__ __launch_bounds__(kThreads) void moon_finish_kernel(DispatchWorld a)
+struct FinishList {
+    int32_t row[kFinishRows];
+    uint32_t from[kFinishRows];     // 0: zeros; else what to copy, plus one (FinishRows)
+    int count;
+};
+
+// Own failure first, then the first failed peer walking upwards from this rank (dispatch kernel :559-574).
+__device__ __forceinline__ void WriteDispatchStatus(const DispatchWorld &a, int rank)
 {
-    __shared__ int32_t s_items[kFinishRows];
-    __shared__ int s_count;
-    const int rank = blockIdx.y;
+    int32_t status = kDispatchOk;
+    const uint64_t own = __hip_atomic_load(&a.tables.fail[rank], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (Tagged(own, a.epoch)) {
+        status = static_cast<int32_t>(own & 0xffffffffu);
+    } else {
+        for (int o = 1; o < a.world; ++o) {
+            const int peer = (rank + o) % a.world;
+            const uint64_t f = __hip_atomic_load(&a.tables.fail[peer], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (Tagged(f, a.epoch)) {
+                status = kDispatchRemoteFailureBase + peer;
+                break;
+            }
+        }
+    }
+    a.status[rank][0] = status;
+}
+
+// 64 rows of `rank` that no route's own copy fills.  The first wave of a workgroup looks at them, one per lane: nothing (a
+// route writes the row), zeros (no route writes it: the reference clears the whole window first, dispatch kernel :206-230),
+// or -- saved plans -- a copy of its primary row (dispatch kernel :426-461); the weight of a row no route names is zero for
+// the same reason.  Then the whole workgroup writes the rows that need writing.
+//
+// AHEAD: the workgroup belongs to the scatter launch itself, after a launch that left what every route records.  A row is
+// then either a copying workgroup's or this one's (moon_agree_kernel), and a primary row is not read where it is being
+// written: its values are those of the token row its origin names.  A launch of its own for this took 4 us a Dispatch, and
+// the two that built a fresh plan 10; together, us a pass before and now: forward 4096 x 1024 x top-5 50.3 and 41.9,
+// 4096 x 2048 x top-8 76.3 and 68.9, 128 x 4096 x top-4 35 and 31; two ranks x 2048 x 2048 x top-8 137 and 126; all four stages 4096 x
+// 7168 x top-8 398 and 386 (1.5 us of it are arguments asked for together, AskedTogether).
+// Otherwise the rows are copied where they lie, once every source has scattered, and the duplicates of a fresh plan take
+// their places in dupLoffs here.
+template <bool VEC, bool AHEAD>
+__device__ __forceinline__ void FinishRows(const DispatchWorld &a, int rank, int64_t block, FinishList *s)
+{
     const int tid = threadIdx.x;
     const int64_t base = static_cast<int64_t>(rank) * a.tables.stride;
     if (tid < kWave) {
-        const int64_t row = static_cast<int64_t>(blockIdx.x) * kFinishRows + tid;
-        int32_t item = -1;
+        const int64_t row = block * kFinishRows + tid;
+        bool fill = false;
+        uint32_t from = 0;
         if (row < a.nvS) {
             const uint64_t tag = a.tables.rowTag[base + row];
+            const uint64_t p = a.tables.parentTag[base + row];
+            const uint32_t sibling = !AHEAD && a.fresh ? a.tables.sibling[base + row] : 0u;
             const bool tagged = Tagged(tag, a.epoch);
             const bool named = tagged && (tag & kRowNamed) != 0;
             const bool written = tagged && (tag & kRowWritten) != 0;
             const bool direct = tagged && (tag & kRowDirect) != 0;
-            const uint64_t p = a.tables.parentTag[base + row];
-            const uint32_t sibling = a.fresh ? a.tables.sibling[base + row] : 0u;
+            const int64_t primary = static_cast<int64_t>(p & 0xffffffffu) - 1;
             if (!a.fresh && Tagged(p, a.epoch) && !direct) {
-                item = static_cast<int32_t>(row) | (kFillCopy << 30);
+                // a primary no route wrote is all zeros in the reference too (the window was cleared)
+                fill = true;
+                const uint64_t ptag = a.tables.rowTag[base + primary];
+                const uint32_t source = AHEAD ? a.tables.origin[base + primary] : static_cast<uint32_t>(primary);
+                from = Tagged(ptag, a.epoch) && (ptag & kRowWritten) != 0 ? source + 1u : 0u;
             } else if (!written) {
-                item = static_cast<int32_t>(row) | (kFillZero << 30);
+                fill = true;
             }
             if (!named && a.weightsNvs[rank] != nullptr) {
                 a.weightsNvs[rank][row] = 0.0f;
             }
-            if (a.fresh && Tagged(p, a.epoch)) {
+            if (!AHEAD && a.fresh && Tagged(p, a.epoch)) {
                 // slot of this duplicate in its group's slice (dispatch kernel :393-419)
-                const uint64_t gs = a.tables.groupStart[base + static_cast<int64_t>(p & 0xffffffffu) - 1];
+                const uint64_t gs = a.tables.groupStart[base + primary];
                 if (Tagged(gs, a.epoch)) {
                     const int64_t at = static_cast<int64_t>(gs & 0xffffffffu) + (sibling & 0xffffu);
                     if (at < a.nvS) {
@@ -858,60 +747,399 @@ __global__ __launch_bounds__(kThreads) void moon_finish_kernel(DispatchWorld a)
                 }
             }
         }
-        const uint64_t have = __ballot(item >= 0);
-        if (item >= 0) {
-            s_items[__popcll(have & ((1ull << tid) - 1ull))] = item;
+        const uint64_t have = __ballot(fill);
+        if (fill) {
+            const int at = __popcll(have & ((1ull << tid) - 1ull));
+            s->row[at] = static_cast<int32_t>(row);
+            s->from[at] = from;
         }
         if (tid == 0) {
-            s_count = __popcll(have);
+            s->count = __popcll(have);
         }
     }
-    if (blockIdx.x == 0 && tid == 0) {
-        // own failure first, then the first failed peer walking upwards from this rank (dispatch kernel :559-574)
-        int32_t status = kDispatchOk;
-        const uint64_t own = __hip_atomic_load(&a.tables.fail[rank], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (Tagged(own, a.epoch)) {
-            status = static_cast<int32_t>(own & 0xffffffffu);
-        } else {
-            for (int o = 1; o < a.world; ++o) {
-                const int peer = (rank + o) % a.world;
-                const uint64_t f = __hip_atomic_load(&a.tables.fail[peer], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (Tagged(f, a.epoch)) {
-                    status = kDispatchRemoteFailureBase + peer;
-                    break;
-                }
-            }
-        }
-        a.status[rank][0] = status;
-    }
-    __syncthreads();
-    const int count = s_count;
+    TileXREp::LdsBarrier();
+    const int count = s->count;
     const int h = static_cast<int>(a.h);
     char *tensor = static_cast<char *>(a.hiddenNvsh[rank]);
+#pragma unroll 1
     for (int i = 0; i < count; ++i) {
-        const int32_t item = s_items[i];
-        const int row = item & 0x3fffffff;
-        bool copy = (item >> 30) == kFillCopy;
-        int primary = 0;
-        if (copy) {
-            primary = static_cast<int>(a.tables.parentTag[base + row] & 0xffffffffu) - 1;
-            // a primary no route wrote is all zeros in the reference too (the window was cleared)
-            const uint64_t tag = a.tables.rowTag[base + primary];
-            copy = Tagged(tag, a.epoch) && (tag & kRowWritten) != 0;
+        const uint32_t from = s->from[i];
+        char *dst = tensor + static_cast<int64_t>(s->row[i]) * h * 2;
+        const char *src = tensor;
+        if (from != 0 && AHEAD) {
+            const uint32_t n = static_cast<uint32_t>(a.s * a.k);
+            const uint32_t rankOf = (from - 1u) / n;
+            src = static_cast<const char *>(a.hiddenSh[rankOf]) +
+                static_cast<int64_t>((from - 1u - rankOf * n) / static_cast<uint32_t>(a.k)) * h * 2;
+        } else if (from != 0) {
+            src = tensor + static_cast<int64_t>(from - 1u) * h * 2;
         }
         if (VEC) {
             const int vecs = h / 8;
-            u32x4 *dstRow = reinterpret_cast<u32x4 *>(tensor + static_cast<int64_t>(row) * h * 2);
-            const u32x4 *srcRow = reinterpret_cast<const u32x4 *>(tensor + static_cast<int64_t>(primary) * h * 2);
+            u32x4 *dstRow = reinterpret_cast<u32x4 *>(dst);
+            const u32x4 *srcRow = reinterpret_cast<const u32x4 *>(src);
+#pragma unroll 1
             for (int idx = tid; idx < vecs; idx += kThreads) {
-                const u32x4 v = copy ? srcRow[idx] : u32x4{0u, 0u, 0u, 0u};
+                const u32x4 v = from != 0 ? srcRow[idx] : u32x4{0u, 0u, 0u, 0u};
                 __builtin_nontemporal_store(v, dstRow + idx);
             }
         } else {
-            uint16_t *dstRow = reinterpret_cast<uint16_t *>(tensor) + static_cast<int64_t>(row) * h;
-            const uint16_t *srcRow = reinterpret_cast<const uint16_t *>(tensor) + static_cast<int64_t>(primary) * h;
+            uint16_t *dstRow = reinterpret_cast<uint16_t *>(dst);
+            const uint16_t *srcRow = reinterpret_cast<const uint16_t *>(src);
             for (int c = tid; c < h; c += kThreads) {
-                dstRow[c] = copy ? srcRow[c] : static_cast<uint16_t>(0);
+                dstRow[c] = from != 0 ? srcRow[c] : static_cast<uint16_t>(0);
+            }
+        }
+    }
+}
+
+// What is left to do once every source has scattered, where no scatter launch does it.  Workgroup 0 of every rank writes
+// the rank's device status.
+template <bool VEC>
+__global__ __launch_bounds__(kThreads) void moon_finish_kernel(DispatchWorld a)
+{
+    __shared__ FinishList s_list;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        WriteDispatchStatus(a, blockIdx.y);
+    }
+    FinishRows<VEC, false>(a, blockIdx.y, blockIdx.x, &s_list);
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// dispatch: the plan as workgroups of the scatter launch
+// ---------------------------------------------------------------------------------------------------------------
+
+constexpr int kPlanRows = kThreads;     // rows of a plan workgroup, one per thread
+static_assert(kTableAlign == kPlanRows, "a workgroup has a word, and all its rows are in the tables");
+constexpr int kTotalsPolls = 4096;      // looks at a chunk's word before a thread adds the chunk up itself
+constexpr int kWordsAtOnce = 8;
+
+// A chunk's totals in one word, so that whoever finds the word has both: group-opening rows and the sizes of their groups.
+constexpr int kSizeShift = 12;
+static_assert(kPlanRows < (1 << kSizeShift) && kPlanRows * kMaxTopK < (1 << (32 - kSizeShift)), "both totals fit a word");
+
+__device__ __forceinline__ uint32_t PackTotals(int open, int size)
+{
+    return static_cast<uint32_t>(open) | (static_cast<uint32_t>(size) << kSizeShift);
+}
+
+// Totals of chunk c, which another workgroup of the launch leaves; the records they are made of were there before the
+// launch, so a thread that has waited long enough adds them up and depends on nobody.
+__device__ __forceinline__ uint32_t TotalsOfChunk(const DispatchWorld &a, int rank, int c)
+{
+    const uint64_t *word = a.tables.chunkTag + (static_cast<int64_t>(rank) * a.tables.stride / kPlanRows + c);
+#pragma unroll 1
+    for (int polls = 0; polls < kTotalsPolls; ++polls) {
+        const uint64_t w = __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (Tagged(w, a.epoch)) {
+            return static_cast<uint32_t>(w);
+        }
+        __builtin_amdgcn_s_sleep(4);
+    }
+    const int64_t at = static_cast<int64_t>(rank) * a.tables.stride + static_cast<int64_t>(c) * kPlanRows;
+    int open = 0;
+    int size = 0;
+#pragma unroll 1
+    for (int i = 0; i < kPlanRows; ++i) {
+        const uint32_t sibling = a.tables.sibling[at + i];
+        const bool opens = Tagged(a.tables.parentTag[at + i], a.epoch) && (sibling & 0xffffu) == 0;
+        open += opens ? 1 : 0;
+        size += opens ? static_cast<int>(sibling >> 16) : 0;
+    }
+    return PackTotals(open, size);
+}
+
+// The duplicate plan of one chunk of 256 rows, by a workgroup of the scatter launch: groups are numbered and their slices
+// start as in DedupGroupsOfChunk, and a thread whose row opens a group fills the group's slice too, so that nothing is left to
+// a launch after the copies.  It needs only what the launch before left, besides the totals of the chunks before its own.
+// Those the workgroups hand one another: they stand at the front of the launch, each waits for workgroups ahead of it
+// alone, and none waits for ever (TotalsOfChunk).
+//
+// The workgroup of a rank's last chunk knows the plan's extent, hence whether it is one; the last of those among the ranks
+// writes every rank's device status.  (One arrival per rank: atomics on one word complete at three per microsecond.)
+//
+// Beside the copies a trip to memory takes 3 to 5 us and a launch of narrow rows is over in 10, so there are two of them:
+// the rows' records, then the route words of the tokens that open groups (their ranks beside them), which are on their way
+// while the other chunks' totals are looked for.  A row per thread: in chunks of 2048 rows, eight per thread, the same steps
+// took 8 us more, the loads of few compute units that each touch 64 lines at a time.
+__device__ __forceinline__ void PlanChunk(const DispatchWorld &a, int rank, int chunk, int chunks, int (*s_part)[kThreads / kWave])
+{
+    const int tid = threadIdx.x;
+    // rows from nvS up to the stride are never tagged with a running epoch
+    const int64_t at = static_cast<int64_t>(rank) * a.tables.stride + static_cast<int64_t>(chunk) * kPlanRows + tid;
+    const uint64_t parent = a.tables.parentTag[at];
+    const uint32_t sibling = a.tables.sibling[at];
+    const uint32_t origin = a.tables.origin[at];
+    const bool opens = Tagged(parent, a.epoch) && (sibling & 0xffffu) == 0;
+    const int size = opens ? static_cast<int>(sibling >> 16) : 0;
+    int exclOpen, exclSize, totalOpen, totalSize;
+    ScanPair(opens ? 1 : 0, size, s_part, &exclOpen, &exclSize, &totalOpen, &totalSize);
+    if (tid == 0) {
+        __hip_atomic_store(a.tables.chunkTag + (static_cast<int64_t>(rank) * a.tables.stride / kPlanRows + chunk),
+            Tag(a.epoch, PackTotals(totalOpen, totalSize)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    const int K = static_cast<int>(a.k);
+    const uint32_t n = static_cast<uint32_t>(a.s * a.k);
+    const uint32_t firstRow = static_cast<uint32_t>(rank) * static_cast<uint32_t>(a.nvS);
+    const uint32_t src = opens ? origin / n : 0u;
+    const int64_t route = opens ? static_cast<int64_t>((origin - src * n) / static_cast<uint32_t>(K)) * K : 0;
+    const int32_t *words = a.dst[src] + route;
+    const uint8_t *ranks = a.tables.direct + static_cast<int64_t>(src) * a.tables.stride + route;
+    // rows of the group's members by route, and their ranks within it; other routes have no rank, or another rank's row
+    uint32_t row[kWordsAtOnce];
+    int place[kWordsAtOnce];
+    auto load = [&](int k0) {
+#pragma unroll
+        for (int j = 0; j < kWordsAtOnce; ++j) {
+            const int k = k0 + j < K ? k0 + j : K - 1;
+            row[j] = opens ? static_cast<uint32_t>(~words[k]) - firstRow : 0u;
+            place[j] = opens && k0 + j < K ? ranks[k] : kNoRank;
+        }
+    };
+    load(0);
+    int baseOpen = 0;
+    int baseSize = 0;
+    if (chunk != 0) {
+        int beforeOpen = 0;
+        int beforeSize = 0;
+#pragma unroll 1
+        for (int c = tid; c < chunk; c += kThreads) {
+            const uint32_t totals = TotalsOfChunk(a, rank, c);
+            beforeOpen += static_cast<int>(totals & ((1u << kSizeShift) - 1u));
+            beforeSize += static_cast<int>(totals >> kSizeShift);
+        }
+        TileXREp::LdsBarrier();
+        int dropOpen, dropSize;
+        ScanPair(beforeOpen, beforeSize, s_part, &dropOpen, &dropSize, &baseOpen, &baseSize);
+    }
+    const int64_t group = static_cast<int64_t>(baseOpen) + exclOpen;
+    const int64_t start = static_cast<int64_t>(baseSize) + exclSize;
+    // a plan in which duplicates of one token name the same row can claim more slots than there are rows
+    if (opens && group < a.nvS && start + size <= a.nvS) {
+        int32_t *g = a.dupGroups[rank] + group * 3;
+        g[0] = static_cast<int32_t>(parent & 0xffffffffu) - 1;
+        g[1] = static_cast<int32_t>(start);
+        g[2] = size;
+        int32_t *slice = a.dupLoffs[rank] + start;
+#pragma unroll 1
+        for (int k0 = 0; k0 < K; k0 += kWordsAtOnce) {
+            if (k0 != 0) {
+                load(k0);
+            }
+#pragma unroll
+            for (int j = 0; j < kWordsAtOnce; ++j) {
+                if (place[j] < size && row[j] < static_cast<uint32_t>(a.nvS)) {
+                    slice[place[j]] = static_cast<int32_t>(row[j]);
+                }
+            }
+        }
+    }
+    if (chunk == chunks - 1 && tid == 0) {
+        a.dupCounts[rank][0] = baseOpen + totalOpen;
+        a.dupCounts[rank][1] = baseSize + totalSize;
+        if (static_cast<int64_t>(baseSize) + totalSize > a.nvS) {
+            RecordFailure(a.tables, rank, a.epoch, kDispatchInvalidRoute);
+        }
+        TileXREp::WaitOwnStores();
+        bool last = true;
+        if (a.world > 1) {
+            last = __hip_atomic_fetch_add(a.tables.arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u ==
+                static_cast<uint32_t>(a.world);
+        }
+        if (last) {
+            if (a.world > 1) {
+                __hip_atomic_store(a.tables.arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            for (int r = 0; r < a.world; ++r) {
+                WriteDispatchStatus(a, r);
+            }
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------------------------------------------
+// dispatch: scatter
+// ---------------------------------------------------------------------------------------------------------------
+
+// What a scatter launch does besides its copies.  A rank's first workgroups build the plan of a fresh Dispatch
+// (PlanChunk); they are a multiple of eight, so that the copies keep their XCDs.  The last ones fill the rows nobody copies
+// to (FinishRows); looking for such rows is a trip to memory, which at the front of the launch would hold the copies up.
+struct ScatterExtras {
+    unsigned planBlocks;
+    int planChunks;
+    unsigned copyBlocks;
+};
+
+// A workgroup whose copy block, counted from the end of the plan's workgroups and so wrapped round for those, names no token.
+// (Grids are within 2^31, so a wrapped block's token is beyond any.)  Copying workgroups come to it by the one test of
+// their token that they make in any case: a test of the block number ahead of it, on arguments of its own, cost them a
+// dependent scalar load each and the 4096 x 7168 x top-8 scatter 9 us on top of 73.
+template <bool FRESH>
+__device__ __forceinline__ void DoExtra(const DispatchWorld &a, const ScatterExtras &x, unsigned block)
+{
+    __shared__ FinishList s_list;
+    if constexpr (FRESH) {
+        if (blockIdx.x < x.planBlocks) {
+            if (static_cast<int>(blockIdx.x) < x.planChunks) {
+                __shared__ int s_part[2][kThreads / kWave];
+                PlanChunk(a, blockIdx.y, blockIdx.x, x.planChunks, s_part);
+            }
+            return;
+        }
+    }
+    if (block < x.copyBlocks) {
+        return;     // a token that only pads the grid
+    }
+    if (!FRESH && block == x.copyBlocks && threadIdx.x == 0) {
+        WriteDispatchStatus(a, blockIdx.y);     // of a saved plan: nothing can fail any more
+    }
+    FinishRows<true, true>(a, blockIdx.y, block - x.copyBlocks, &s_list);
+}
+
+// Has the arguments asked for together, ahead of the first branch that needs one of them: a copying workgroup lives for some
+// microseconds, and each further wait for a scalar load is a part of that (saved plan, 4096 x 7168 x top-8: 78.2 us with the
+// plan's rows, the rank count and the `direct` table asked for behind the branch, 72.2 so).
+template <typename... T>
+__device__ __forceinline__ void AskedTogether(T &...v)
+{
+    (void)std::initializer_list<int>{([&v] { asm volatile("" : "+s"(v)); }(), 0)...};
+}
+
+// Whether the source's own workgroups copy the row of this route: every route's of a fresh plan; what moon_agree_kernel
+// found for a saved one.
+template <bool FRESH>
+__device__ __forceinline__ bool SourceCopies(const Route &r, uint8_t direct)
+{
+    return r.ok && (FRESH || direct != 0);
+}
+
+// One workgroup per (token, route, slice of 512 vectors) of source rank blockIdx.y.  What the routes record was written
+// ahead, by moon_records_kernel or moon_agree_kernel.
+template <bool FRESH>
+__global__ __launch_bounds__(kThreads) void moon_scatter_kernel(DispatchWorld a, int colSlices, ScatterExtras extras)
+{
+    const int src = blockIdx.y;
+    const int32_t *words = a.dst[src];
+    const char *rows = static_cast<const char *>(a.hiddenSh[src]);
+    char *firstOut = static_cast<char *>(a.hiddenNvsh[0]);
+    const uint8_t *directs = a.tables.direct + static_cast<int64_t>(src) * a.tables.stride;
+    int64_t rowBytes = a.h * 2;
+    int64_t nvS = a.nvS;
+    int world = a.world;
+    AskedTogether(words, rows, firstOut, rowBytes, nvS, world);
+    if (!FRESH) {
+        AskedTogether(directs);
+    }
+    const unsigned block = blockIdx.x - (FRESH ? extras.planBlocks : 0u);
+    const unsigned j = block / kXcds;
+    const unsigned K = static_cast<unsigned>(a.k);
+    const unsigned perToken = K * static_cast<unsigned>(colSlices);
+    const int64_t token = static_cast<int64_t>(j / perToken) * kXcds + block % kXcds;
+    if (token >= a.s) {
+        DoExtra<FRESH>(a, extras, block);
+        return;
+    }
+    const unsigned k = (j % perToken) / static_cast<unsigned>(colSlices);
+    const unsigned slice = (j % perToken) % static_cast<unsigned>(colSlices);
+    const int lane = threadIdx.x;
+    const int vecs = static_cast<int>(rowBytes / 16);
+    const int colBase = static_cast<int>(slice) * (kRowVecs * kThreads);
+    const int64_t route = token * K + k;
+    const int32_t encoded = words[route];
+    const uint8_t direct = FRESH ? 0 : directs[route];
+    const u32x4 *srcRow = reinterpret_cast<const u32x4 *>(rows + token * rowBytes);
+    u32x4 v[kRowVecs];
+#pragma unroll
+    for (int i = 0; i < kRowVecs; ++i) {
+        const int idx = colBase + i * kThreads + lane;
+        v[i] = idx < vecs ? srcRow[idx] : u32x4{0u, 0u, 0u, 0u};
+    }
+    const Route r = Decode(encoded, nvS, world);
+    if (SourceCopies<FRESH>(r, direct)) {
+        char *out = world == 1 ? firstOut : static_cast<char *>(a.hiddenNvsh[r.peer]);
+        u32x4 *dstRow = reinterpret_cast<u32x4 *>(out + r.row * rowBytes);
+#pragma unroll
+        for (int i = 0; i < kRowVecs; ++i) {
+            const int idx = colBase + i * kThreads + lane;
+            if (idx < vecs) {
+                __builtin_nontemporal_store(v[i], dstRow + idx);
+            }
+        }
+    }
+}
+
+// G lanes per (token, slice of G x V vectors) of source rank blockIdx.y: the slice is loaded once and stored once per route.
+// What the routes record was written ahead, as for moon_scatter_kernel.  Lane k of every wave works out the
+// row of route k for itself, so nothing is handed round and no wave waits between its loads and its stores.  Workgroup b runs on
+// XCD b % 8 and takes tokens t with t % 8 == b % 8, as the reduce of a small world does.
+//
+// AUX, the stores' cache policy.  Rows of whole 128-byte lines are written through and kept in the memory-side cache for Combine
+// (kAuxAgentScopeKept; the per-route kernel's must stream, or they push the token rows that its workgroups share out of the L2s).
+// Of other rows nearly every store of a wave begins and ends within a line, which written through are two trips for one line.
+// They are ordinary stores (0), which come together in the L2, where a token has four and more of them, and stream below, where
+// there is less for Combine to find.  Forward stages, us copied per route, kept and so: 2223 x 2008 x top-6 54.0, 56.8 and 56.1,
+// 4000 x 2008 x top-2 48.2, 51.1 and 47.5, 2223 x 5000 x top-6 83.9, 89.6 and 86.4, 4000 x 5000 x top-2 72.0, 76.2 and 69.8, 7000 x
+// 1000 x top-6 90.4, 71.6 and 68.6; all four 1501 x 7176 x top-8 205.7, 211.3 and 206.2, 4000 x 7176 x top-3 233.4, 244.7 and 242.3.
+// (Ordinary stores for three of them 2223 x 7176 76.6, streaming ones 72.0.)
+template <bool FRESH, int G, int V, int AUX>
+__global__ __launch_bounds__(kThreads) void moon_scatter_token_kernel(DispatchWorld a, int colSlices, ScatterExtras extras)
+{
+    constexpr int kTokens = kThreads / G;
+    const int src = blockIdx.y;
+    const int32_t *words = a.dst[src];
+    const char *rows = static_cast<const char *>(a.hiddenSh[src]);
+    char *firstOut = static_cast<char *>(a.hiddenNvsh[0]);
+    const uint8_t *directs = a.tables.direct + static_cast<int64_t>(src) * a.tables.stride;
+    int64_t rowBytes = a.h * 2;
+    int64_t nvS = a.nvS;
+    int world = a.world;
+    AskedTogether(words, rows, firstOut, rowBytes, nvS, world);
+    if (!FRESH) {
+        AskedTogether(directs);
+    }
+    const unsigned block = blockIdx.x - (FRESH ? extras.planBlocks : 0u);
+    const unsigned j = block / kXcds;
+    const int slice = static_cast<int>(j % static_cast<unsigned>(colSlices));
+    const int tg = threadIdx.x / G;
+    const int64_t token = (static_cast<int64_t>(j / static_cast<unsigned>(colSlices)) * kTokens + tg) * kXcds + block % kXcds;
+    if (token >= a.s) {
+        DoExtra<FRESH>(a, extras, block);
+        return;
+    }
+    const int lane = threadIdx.x % G;
+    const int waveLane = threadIdx.x % kWave;
+    const int K = static_cast<int>(a.k);
+    const int vecs = static_cast<int>(rowBytes / 16);
+    const int colBase = slice * (G * V);
+    int32_t word = 0;
+    uint8_t direct = 0;
+    if (waveLane < K) {
+        const int64_t route = token * K + waveLane;
+        word = words[route];
+        direct = FRESH ? 0 : directs[route];
+    }
+    const u32x4 *srcRow = reinterpret_cast<const u32x4 *>(rows + token * rowBytes);
+    u32x4 v[V];
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+        const int idx = colBase + i * G + lane;
+        v[i] = idx < vecs ? srcRow[idx] : u32x4{0u, 0u, 0u, 0u};
+    }
+    const Route r = Decode(word, nvS, world);
+    const int row = waveLane < K && SourceCopies<FRESH>(r, direct) ? r.row : -1;
+    for (int k = 0; k < K; ++k) {
+        const int rowOfK = __builtin_amdgcn_readlane(row, k);
+        if (rowOfK < 0) {
+            continue;
+        }
+        const int peer = __builtin_amdgcn_readlane(r.peer, k);
+        const char *out = world == 1 ? firstOut : static_cast<const char *>(a.hiddenNvsh[peer]);
+        const __amdgpu_buffer_rsrc_t dst = TileXREp::RowResource(out + rowOfK * rowBytes, vecs * 16);
+#pragma unroll
+        for (int i = 0; i < V; ++i) {
+            const int idx = colBase + i * G + lane;
+            if (idx < vecs) {
+                __builtin_amdgcn_raw_buffer_store_b128(v[i], dst, idx * 16, 0, AUX);
             }
         }
     }
@@ -1281,11 +1509,12 @@ const char *MoonReduceKernelName()
     return gReduceName;
 }
 
-// What follows the routes' records: the duplicate plan of a fresh Dispatch, then the rows and weights no route wrote.
-hipError_t LaunchPlanAndFinish(const DispatchWorld &w, hipStream_t stream, bool vec, bool plan)
+// What follows copies whose launch does nothing else: the duplicate plan of a fresh Dispatch, then the rows and weights no
+// route wrote.
+hipError_t LaunchPlanAndFinish(const DispatchWorld &w, hipStream_t stream, bool vec)
 {
     const unsigned R = static_cast<unsigned>(w.world);
-    if (w.fresh && plan) {
+    if (w.fresh) {
         const unsigned chunks = static_cast<unsigned>((w.nvS + kBuildRows - 1) / kBuildRows);
         if (chunks <= kSelfTotalChunks) {
             hipLaunchKernelGGL(moon_dedup_groups_kernel<true>, dim3(chunks, R), dim3(kThreads), 0, stream, w);
@@ -1328,8 +1557,8 @@ hipError_t LaunchMoonDispatch(const DispatchWorld &w, hipStream_t stream, const 
     const bool wantsPerToken = cachedRowBytes != kDefaultCachedRowBytes ? worldRowBytes > cachedRowBytes :
         vecs <= 4 * kWave || worldRowBytes * w.k <= kKeptRowBytes || worldRowBytes > kPerRouteTokenBytes;
     const int64_t rowVecs = w.s * vecs;
-    const bool perToken = vec && wantsPerToken && (w.s + 4 * kXcds) * tokenSlices <= 0x7fffffff;
-    const bool perRoute = vec && !perToken && blocks <= 0x7fffffff;
+    const bool perToken = vec && wantsPerToken && (w.s + 4 * kXcds) * tokenSlices <= kMostCopyBlocks;
+    const bool perRoute = vec && !perToken && blocks <= kMostCopyBlocks;
     const bool recordsAhead = perToken || perRoute;
     // per-route copies of up to half the memory-side cache of token rows: read them once so that the kernel finds them there
     // (one rank's share of 4096 x 7168: 257 -> about 210 us per layer on rows that were not cached, a few us more
@@ -1337,26 +1566,19 @@ hipError_t LaunchMoonDispatch(const DispatchWorld &w, hipStream_t stream, const 
     const bool warm = perRoute && worldRowBytes <= kWarmRowBytes;
     const unsigned warmBlocks = warm ? static_cast<unsigned>((rowVecs + kThreads * kWarmLoads - 1) / (kThreads * kWarmLoads)) : 0u;
     const unsigned routeBlocks = static_cast<unsigned>((w.s * w.k + kThreads - 1) / kThreads);
-    // What the routes record is written ahead of the scatter, and a fresh plan is built by extra workgroups of the scatter
-    // launch; only the finish kernel follows.  Three launches instead of five while a rank has at most kSelfPlanChunks chunks,
-    // four (the chunk totals need one) beyond.  Per-route copies of more than kFusedPlanRowBytes keep the launches after the
-    // scatter: with the plan's code that kernel has 50 registers per lane instead of 16, and its short-lived workgroups then
-    // start more slowly, which costs more than the launches saved (4096 tokens x 7168 201 -> 204 us, 8192 tokens 365 -> 386).
-    // At the default of SetCachedRowBytes the per-route kernel gets more rows than that: moon_scatter_kernel<true, true> serves
-    // callers who have asked for per-route copies of less.
-    const int planChunks = static_cast<int>((w.nvS + kBuildRows - 1) / kBuildRows);
-    const bool planInScatter = w.fresh && planChunks <= kFusedPlanChunks &&
-        (perToken || (perRoute && static_cast<int64_t>(w.world) * w.s * w.k * w.h * 2 <= kFusedPlanRowBytes));
-    const bool planSelf = planChunks <= kSelfPlanChunks;
-    const unsigned planBlocks = planInScatter ? static_cast<unsigned>((planChunks + kXcds - 1) / kXcds * kXcds) : 0u;
+    // What the routes record is written ahead of the scatter; the scatter launch then holds everything else a Dispatch does,
+    // two launches for a fresh plan and three for a saved one.  A rank of more than kFusedPlanChunks chunks keeps launches
+    // behind the copies.
+    const int planChunks = static_cast<int>((w.nvS + kPlanRows - 1) / kPlanRows);
+    const bool allInScatter = recordsAhead && (!w.fresh || planChunks <= kFusedPlanChunks);
+    ScatterExtras extras {};
+    extras.planChunks = planChunks;
+    extras.planBlocks = w.fresh && allInScatter ? static_cast<unsigned>((planChunks + kXcds - 1) / kXcds * kXcds) : 0u;
+    const unsigned finishBlocks = allInScatter ? static_cast<unsigned>((w.nvS + kFinishRows - 1) / kFinishRows) : 0u;
     if (w.fresh && recordsAhead) {
         hipLaunchKernelGGL(moon_records_kernel, dim3(routeBlocks + warmBlocks, R), dim3(kThreads), 0, stream, w, routeBlocks,
             warm ? rowVecs : int64_t{0});
         MOON_LAUNCH_CHECK();
-        if (planInScatter && !planSelf) {
-            hipLaunchKernelGGL(moon_dedup_totals_kernel, dim3(static_cast<unsigned>(planChunks), R), dim3(kThreads), 0, stream, w);
-            MOON_LAUNCH_CHECK();
-        }
     } else if (!w.fresh) {
         hipLaunchKernelGGL(moon_group_walk_kernel, dim3(rowBlocks, R), dim3(kThreads), 0, stream, w);
         MOON_LAUNCH_CHECK();
@@ -1390,16 +1612,14 @@ hipError_t LaunchMoonDispatch(const DispatchWorld &w, hipStream_t stream, const 
             constexpr int V = decltype(vecsPerLane)::value;
             constexpr int kAux = decltype(stores)::value;
             constexpr int64_t kTokens = kThreads / G * kXcds;       // tokens of eight neighbouring workgroups
-            const dim3 grid(static_cast<unsigned>((w.s + kTokens - 1) / kTokens * kXcds * tokenSlices) + planBlocks, R);
-            if (planInScatter) {
-                hipLaunchKernelGGL((moon_scatter_token_kernel<true, true, G, V, kAux>), grid, dim3(kThreads), capLds, stream, w,
-                    tokenSlices, planBlocks, planChunks, planSelf ? 1 : 0);
-            } else if (w.fresh) {
-                hipLaunchKernelGGL((moon_scatter_token_kernel<true, false, G, V, kAux>), grid, dim3(kThreads), capLds, stream, w,
-                    tokenSlices, 0u, 0, 0);
+            extras.copyBlocks = static_cast<unsigned>((w.s + kTokens - 1) / kTokens * kXcds * tokenSlices);
+            const dim3 grid(extras.planBlocks + extras.copyBlocks + finishBlocks, R);
+            if (w.fresh) {
+                hipLaunchKernelGGL((moon_scatter_token_kernel<true, G, V, kAux>), grid, dim3(kThreads), capLds, stream, w, tokenSlices,
+                    extras);
             } else {
-                hipLaunchKernelGGL((moon_scatter_token_kernel<false, false, G, V, kAux>), grid, dim3(kThreads), capLds, stream, w,
-                    tokenSlices, 0u, 0, 0);
+                hipLaunchKernelGGL((moon_scatter_token_kernel<false, G, V, kAux>), grid, dim3(kThreads), capLds, stream, w, tokenSlices,
+                    extras);
             }
         };
         auto pickStores = [&](auto lanes, auto vecsPerLane) {
@@ -1424,18 +1644,14 @@ hipError_t LaunchMoonDispatch(const DispatchWorld &w, hipStream_t stream, const 
     } else if (perRoute) {
         gScatterName = "moon_scatter_kernel";
         // The cap takes workgroups with both of their lanes' loads to do (four stages, top-8, us without and with it: 4096 x
-        // 4096 265 and 262, 4096 x 7168 436 and 415; up to 4096 x 2304 no difference beyond the runs' own).  The launch that
-        // builds the plan as well keeps eight: at five its narrow rows lose what its wide ones gain (forward stages, top-8:
-        // 4096 x 1024 76.0 and 77.6, 4096 x 2304 93.5 and 97.1; 1024 x 4096 53.1 and 51.1, 1024 x 7168 72.8 and 72.0).
-        const unsigned capLds = vecs > kThreads ? kScatterCapLdsBytes : 0u;
-        const dim3 grid(static_cast<unsigned>(blocks) + planBlocks, R);
-        if (planInScatter) {
-            hipLaunchKernelGGL((moon_scatter_kernel<true, true>), grid, dim3(kThreads), 0, stream, w, colSlices, planBlocks,
-                planChunks, planSelf ? 1 : 0);
-        } else if (w.fresh) {
-            hipLaunchKernelGGL((moon_scatter_kernel<true, false>), grid, dim3(kThreads), capLds, stream, w, colSlices, 0u, 0, 0);
+        // 4096 265 and 262, 4096 x 7168 436 and 415; up to 4096 x 2304 no difference beyond the runs' own).
+        const unsigned capLds = vecs > kThreads ? TileXREp::CapLdsBytes(kScatterCapWorkgroups) : 0u;
+        extras.copyBlocks = static_cast<unsigned>(blocks);
+        const dim3 grid(extras.planBlocks + extras.copyBlocks + finishBlocks, R);
+        if (w.fresh) {
+            hipLaunchKernelGGL(moon_scatter_kernel<true>, grid, dim3(kThreads), capLds, stream, w, colSlices, extras);
         } else {
-            hipLaunchKernelGGL((moon_scatter_kernel<false, false>), grid, dim3(kThreads), capLds, stream, w, colSlices, 0u, 0, 0);
+            hipLaunchKernelGGL(moon_scatter_kernel<false>, grid, dim3(kThreads), capLds, stream, w, colSlices, extras);
         }
     } else {
         gScatterName = "moon_scatter_generic_kernel";
@@ -1451,7 +1667,7 @@ hipError_t LaunchMoonDispatch(const DispatchWorld &w, hipStream_t stream, const 
     if (err != hipSuccess) {
         return err;
     }
-    return LaunchPlanAndFinish(w, stream, vec, !planInScatter);
+    return allInScatter ? hipSuccess : LaunchPlanAndFinish(w, stream, vec);
 }
 
 hipError_t LaunchMoonCombine(const CombineWorld &w, hipStream_t stream, const LaunchTiming &timing)
