@@ -47,6 +47,43 @@ def test_quantised_rows_by_slots(k, h, quant, dtype):
         assert np.array_equal(bits16(y), want)
 
 
+@pytest.mark.parametrize("h", [64, 2048, 4112, 16384])
+@pytest.mark.parametrize("k", [2, 6])
+@pytest.mark.parametrize("quant,edge", [(ep.Q_TOKEN_INT8, 511.875), (ep.Q_FP8_BLOCK128, 146.25)])
+def test_fp16_rows_that_saturate(h, k, quant, edge):
+    """A row's largest magnitude (128 or 448 times its scale) on both sides of the 65520 from which rounding to fp16 has to
+    saturate, beside rows that stay far below; infinite and NaN scales; zero and negative ones."""
+    bs, experts = 48, 8
+    rng = np.random.default_rng(h + k + quant)
+    ids = ids_for(rng, bs, k, experts)
+    _, xb = x_for(rng, bs, h, ep.DT_FP16, scale=2.0)
+    d = O.mem_dispatch(O.Case(1, bs, h, k, experts, dtype=ep.DT_FP16, quant_mode=quant), 0, xb[None], ids[None])
+    payload = d["expand_x"].view(np.uint8).copy()
+    payload[:, ::5] = 0x80 if quant == ep.Q_TOKEN_INT8 else 0x7e        # -128, 448
+    payload[:, 1::5] = 0x7f if quant == ep.Q_TOKEN_INT8 else 0xfe       # 127, -448
+    edge = np.float32(edge)
+    some = np.array([1.0, 0.0, np.nextafter(edge, np.float32(0)), edge, np.nextafter(edge, np.float32(1e9)), -edge, 3e4, 1e-6,
+                     np.inf, -np.inf, np.nan], np.float32)
+    scales = np.ones_like(d["dyn_scales"])
+    odd = rng.random(scales.shape) < 0.3
+    scales[odd] = rng.choice(some, int(odd.sum()))
+    w = (0.5 + rng.random((bs, k))).astype(np.float32)
+    with Session() as s:
+        y = torch.full((bs, h), 7.0, dtype=torch.float16, device=DEV)
+        args = [to_dev(v) for v in (payload, d["assist"], d["send_counts"], scales, w)]
+        torch.cuda.synchronize()
+        assert ep.combine_memory_ex(args[0], args[1], args[2], s.comm, bs, h, k, experts, y, ep.DT_FP16, s.stream,
+                                    expert_out_quant_mode=quant, expert_out_scales=args[3], expert_scales=args[4]) == 0
+        s.sync()
+        want = O.mem_combine(O.Case(1, bs, h, k, experts, dtype=ep.DT_FP16), 0, payload[None], d["assist"][None],
+                             d["send_counts"][None], expert_scales=w, in_quant=quant, in_scales=scales)
+        got, want = bits16(y), want.view(np.uint16).reshape(bs, h)
+        nan = (want & 0x7fff) > 0x7c00
+        assert nan.any() and not nan.all() and ((want & 0x7fff) == 0x7bff).any()
+        assert np.array_equal((got & 0x7fff) > 0x7c00, nan)             # (a NaN's sign is the adder's choice of operand)
+        assert np.array_equal(got[~nan], want[~nan])
+
+
 @pytest.mark.parametrize("bs,h,k", [(5, 64, 8), (700, 64, 5), (41, 1024, 64), (300, 1032, 8), (65, 4104, 33), (3, 16384, 2)])
 def test_sums_in_the_order_of_the_rows(bs, h, k):
     """The MVP route adds rows in ascending row order; here the rows of a token stand in any order of its slots."""

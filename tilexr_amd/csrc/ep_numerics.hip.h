@@ -72,6 +72,17 @@ __device__ __forceinline__ uint32_t FloatToHalfRneSat(float v)
     return FloatToHalfRne(v);
 }
 
+// Two fp32 values that do not saturate (finite, below 65520) rounded to fp16 (same rounding), returned as fp32.  Three
+// instructions for the two, where FloatToHalfRneSat and a decode take eight each: one pair convert, two converts back.
+__device__ __forceinline__ void FloatPairRoundedToHalf(float lo, float hi, float *rlo, float *rhi)
+{
+    typedef _Float16 half2 __attribute__((ext_vector_type(2)));
+    const f32x2 f = {lo, hi};
+    const half2 h = __builtin_convertvector(f, half2);
+    *rlo = static_cast<float>(h[0]);
+    *rhi = static_cast<float>(h[1]);
+}
+
 template <bool BF16>
 __device__ __forceinline__ uint32_t Encode16Sat(float v)
 {

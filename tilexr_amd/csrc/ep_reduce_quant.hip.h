@@ -28,7 +28,7 @@ constexpr int kFlagsSettled = 2;
 // eight for eight slots is no such bargain: 16384 x 2048 int8 130.6 -> 129.8, but block fp8 that lost rows to a capacity, four
 // left of eight, 91.0 -> 93.0, and 8192 x 4096 x top-2 57.0 -> 59.4).
 template <int G, int V, int INQ, bool BF16, int FL, int KB>
-__global__ __launch_bounds__(kThreads, (V == 1 && BF16) ? (KB > 4 ? 5 : (FL == kFlagsMayWait && INQ == TILEXR_EP_QUANT_FP8_BLOCK128) ? 6 : 7) : 1) void ep_reduce_quant_kernel(ReduceArgs a)
+__global__ __launch_bounds__(kThreads, V == 1 ? (KB > 4 ? 5 : (FL == kFlagsMayWait && (!BF16 || INQ == TILEXR_EP_QUANT_FP8_BLOCK128)) ? 6 : 7) : 1) void ep_reduce_quant_kernel(ReduceArgs a)
 {
     constexpr int kTokens = kThreads / G;
     constexpr bool kWaits = FL == kFlagsMayWait;
@@ -74,12 +74,19 @@ __global__ __launch_bounds__(kThreads, (V == 1 && BF16) ? (KB > 4 ? 5 : (FL == k
         const uint32_t tileWord = checkWords ? SettledWordLoad(a, myRow) : 0u;
         const uint64_t live = __ballot(myRow >= 0);
 
+        // A row's largest magnitude is 128 (448) times its scale: below this scale none reaches the 65520 from which
+        // rounding to fp16 has to saturate.
+        constexpr float kScaleSaturates = INQ == TILEXR_EP_QUANT_TOKEN_INT8 ? 511.875f : 146.25f;
+        bool saturates = false;
         float acc[V][16];
         // The K loop.  fp8 rows are decoded by the hardware convert alone, which differs from the reference decode in
         // one respect only (the sign of the NaN it returns for code 0x7f); a NaN code always surfaces as a NaN in the
         // sum, so a wave that finds a NaN among its sums runs the loop once more with the exact decode.  That keeps a
         // test of every word (four instructions and a branch per four values) out of the loop that everything else
-        // shares.
+        // shares.  Rounding to fp16 likewise: the loop takes the plain converts and looks at the scales, once per row
+        // and lane; a wave that meets a scale whose row could saturate, or a NaN, runs the loop once more with the
+        // saturating ones (2756 x 8192 x top-8, dispatch + combine, fp16 before and now, and bf16: int8 106.4, 84.7 and 81.5
+        // us, block fp8 108.8, 87.9 and 84.1; 8192 x 2048 x top-6 int8 69.2 -> 58.4).
         // throughMemory: rows and scales are read past this XCD's L2, as they must be while their producer may still
         // be writing neighbours of theirs.  Once the producer has finished (flagsSettled) the L2 is as good as memory,
         // and the scales, which the lanes of a token share, are worth keeping there (4096 x int8 rows: 58 -> 49 us).
@@ -133,6 +140,9 @@ __global__ __launch_bounds__(kThreads, (V == 1 && BF16) ? (KB > 4 ? 5 : (FL == k
                     const float w = weightOfK[u];
 #pragma unroll
                     for (int j = 0; j < V; ++j) {
+                        if (!BF16 && !kExactDecode) {
+                            saturates |= !(fabsf(sc[u][j]) < kScaleSaturates);
+                        }
 #pragma unroll
                         for (int d = 0; d < 4; ++d) {
                             const uint32_t word = q[u][j][d];
@@ -156,6 +166,8 @@ __global__ __launch_bounds__(kThreads, (V == 1 && BF16) ? (KB > 4 ? 5 : (FL == k
                                 if (BF16) {
                                     r0 = FloatRoundedToBf16(d0);
                                     r1 = FloatRoundedToBf16(d1);
+                                } else if (!kExactDecode) {
+                                    FloatPairRoundedToHalf(d0, d1, &r0, &r1);
                                 } else {
                                     r0 = __half2float(__ushort_as_half(static_cast<unsigned short>(FloatToHalfRneSat(d0))));
                                     r1 = __half2float(__ushort_as_half(static_cast<unsigned short>(FloatToHalfRneSat(d1))));
@@ -174,16 +186,18 @@ __global__ __launch_bounds__(kThreads, (V == 1 && BF16) ? (KB > 4 ? 5 : (FL == k
         } else {
             accumulate(std::false_type {}, std::false_type {});
         }
-        if (INQ == TILEXR_EP_QUANT_FP8_BLOCK128) {
-            bool sawNan = false;
+        if (INQ == TILEXR_EP_QUANT_FP8_BLOCK128 || !BF16) {
+            bool again = saturates;
+            if (INQ == TILEXR_EP_QUANT_FP8_BLOCK128) {
 #pragma unroll
-            for (int j = 0; j < V; ++j) {
+                for (int j = 0; j < V; ++j) {
 #pragma unroll
-                for (int e = 0; e < 16; ++e) {
-                    sawNan |= acc[j][e] != acc[j][e];
+                    for (int e = 0; e < 16; ++e) {
+                        again |= acc[j][e] != acc[j][e];
+                    }
                 }
             }
-            if (__any(sawNan ? 1 : 0)) {
+            if (__any(again ? 1 : 0)) {
                 if (throughMemory) {
                     accumulate(std::true_type {}, std::true_type {});
                 } else {
