@@ -66,7 +66,8 @@ int RunDispatchSingle(EpComm *comm, const EpDispatchParams &p, bool memoryRoute,
     } else if (p.xActiveMask != nullptr) {
         maskMode = p.activeMaskType == TILEXR_EP_ACTIVE_MASK_EXPERT ? kMaskPerRoute : kMaskTokenPrefix;
     }
-    if (memoryRoute && p.quantMode == TILEXR_EP_QUANT_NONE && p.metaReadyEvent == nullptr) {
+    // (a quantised call that may not allocate asks for the static scratch, whether or not its size needs it)
+    if (memoryRoute && (p.quantMode == TILEXR_EP_QUANT_NONE || !p.noAlloc) && p.metaReadyEvent == nullptr) {
         // decode-sized calls: one launch instead of count + scatter (a consumer that is to run beside the dispatch needs
         // the row map ahead of the rows, which takes the separate launches)
         SmallDispatchLaunch small {};
@@ -87,6 +88,11 @@ int RunDispatchSingle(EpComm *comm, const EpDispatchParams &p, bool memoryRoute,
         small.sendCountsOut = p.epRecvCountsOut;
         small.expertTokenNumsOut = p.expertTokenNumsOut;
         small.tokenNumsType = static_cast<int>(p.expertTokenNumsType);
+        small.quantMode = static_cast<int>(p.quantMode);
+        small.inputBf16 = p.dtype == TileXR::TILEXR_DATA_TYPE_BFP16;
+        small.fp8E5m2 = p.expandXOutDtype == TileXR::TILEXR_DATA_TYPE_FP8E5M2;
+        small.scalesOut = p.dynamicScalesOut;
+        small.tileFlags = p.tileFlagsOut;
         small.stream = stream;
         if (SmallDispatchFits(small)) {
             if (p.tileFlagsOut != nullptr) {
@@ -95,7 +101,6 @@ int RunDispatchSingle(EpComm *comm, const EpDispatchParams &p, bool memoryRoute,
                 if (!comm->tileCounters.Reserve(static_cast<size_t>(TileCounterWords(n, small.tileRows)) * sizeof(uint32_t), true)) {
                     return TileXR::TILEXR_ERROR_INTERNAL;
                 }
-                small.tileFlags = p.tileFlagsOut;
                 small.tileCounters = static_cast<uint32_t *>(comm->tileCounters.ptr);
                 small.epoch = flagEpoch;
             }

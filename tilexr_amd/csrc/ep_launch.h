@@ -262,6 +262,10 @@ struct SmallDispatchLaunch {
     uint32_t *tileCounters;          // TileCounterWords(bs * topK, tileRows) zeroed words
     int64_t tileRows;
     uint64_t epoch;
+    int quantMode;                   // as LaunchScatter's; the row scales, where the mode has any
+    bool inputBf16;
+    bool fp8E5m2;
+    void *scalesOut;
     hipStream_t stream;
     const char **kernelNameOut = nullptr;   // optional: receives the name of the kernel template that was launched
 };

@@ -424,6 +424,42 @@ __device__ __forceinline__ void ForEachGroup(const ReduceArgs &a, int groups, in
     ClaimAndReduce(env, groups);
 }
 
+// MXFP8 round trip of the lane's eight elements (COMMQ 3/4), for a block whose elements are all finite: 24 instructions for
+// eight elements, about 350 with the software codec.  Returns whether the block is such a one.
+template <bool BF16, bool E5M2>
+__device__ __forceinline__ bool MxRoundTrip(const u32x4 &v, float (&f)[8])
+{
+    const MxScaling mx = MxScalingOf<BF16, E5M2>(MxBlockMaxBits(v));
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const f32x2 back = MxDecodePair<E5M2>(MxEncodePair<BF16, E5M2, false>(0u, v[q], mx), mx);
+        f[2 * q] = back[0];
+        f[2 * q + 1] = back[1];
+    }
+    return mx.plain;
+}
+
+// ... for any block, with the codec that defines what becomes of infinities and NaNs.
+template <bool BF16, bool E5M2>
+__device__ __forceinline__ void MxRoundTripAny(const u32x4 &v, float (&f)[8])
+{
+    float amax = 0.0f;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        f[2 * q] = Decode16<BF16>(v[q] & 0xffffu);
+        f[2 * q + 1] = Decode16<BF16>(v[q] >> 16);
+        amax = fmaxf(amax, fmaxf(fabsf(f[2 * q]), fabsf(f[2 * q + 1])));
+    }
+    amax = fmaxf(amax, __shfl_xor(amax, 1));
+    amax = fmaxf(amax, __shfl_xor(amax, 2));
+    const int se = MxSharedExponent<E5M2>(amax);
+    const float up = Exp2Int(se);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        f[e] = __fmul_rn(Fp8Decode<E5M2>(Fp8Encode<E5M2>(ldexpf(f[e], -se))), up);
+    }
+}
+
 } // namespace
 } // namespace TileXREp
 

@@ -13,6 +13,7 @@
 //   KIND fp32     sum = 0; for k = 0..K-1: sum = sum + (w_k * row_k) in fp32, then the shared-expert row, one rounding
 //                 (saturating for fp16); an inactive token (mask) gives zeros
 //                 (reference: src/ep/kernels/tilexr_ep_combine_memory_kernel.h:505-553, 555-571, 573-601, 632-662)
+//   COMMQ 3/4     every row first takes the MXFP8 e5m2 / e4m3 round trip, as in ep_reduce_vec_kernel
 //   KIND per-add  rows in ascending row index; y = T(float(y) + float(row)) after every add
 //                 (reference: src/ep/kernels/tilexr_ep_combine_kernel.cpp:15-26, 54-101)
 // Two tuples that name the same (token, k) -- only a corrupted table has them -- leave the higher row, as the
@@ -50,11 +51,12 @@ struct SmallReduceArgs {
     int n;                          // bs * topK
 };
 
-template <int KIND, bool BF16>
+template <int KIND, bool BF16, int COMMQ>
 __global__ __launch_bounds__(kSmallReduceThreads) void ep_reduce_small_kernel(SmallReduceArgs a)
 {
     constexpr int V = kSmallReduceVecs;
     constexpr int KB = kSmallReduceRows;
+    constexpr bool kCommE5m2 = COMMQ == TILEXR_EP_QUANT_COMM_MXFP8_E5M2;
     __shared__ int s_row[kMaxTopK];
 
     const int token = blockIdx.x;
@@ -125,6 +127,7 @@ __global__ __launch_bounds__(kSmallReduceThreads) void ep_reduce_small_kernel(Sm
             acc[j][e] = 0.0f;
         }
     }
+    bool odd = false;       // MXFP8: one of the lane's blocks holds an infinity or a NaN
     for (int firstSlot = 0; firstSlot < a.topK; firstSlot += KB) {
         u32x4 v16[KB][V];
         int rowOfK[KB];
@@ -153,16 +156,48 @@ __global__ __launch_bounds__(kSmallReduceThreads) void ep_reduce_small_kernel(Sm
             const float w = weightOfK[u];
 #pragma unroll
             for (int j = 0; j < V; ++j) {
+                float f[8];
+                if constexpr (COMMQ != 0) {
+                    odd |= !MxRoundTrip<BF16, kCommE5m2>(v16[u][j], f);
+                } else {
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const float lo = Decode16<BF16>(v16[u][j][q] & 0xffffu);
-                    const float hi = Decode16<BF16>(v16[u][j][q] >> 16);
-                    if (KIND == kReducePerAdd) {
-                        acc[j][2 * q] = RoundTo16<BF16>(__fadd_rn(acc[j][2 * q], lo));
-                        acc[j][2 * q + 1] = RoundTo16<BF16>(__fadd_rn(acc[j][2 * q + 1], hi));
-                    } else {
-                        acc[j][2 * q] = __fadd_rn(acc[j][2 * q], __fmul_rn(lo, w));
-                        acc[j][2 * q + 1] = __fadd_rn(acc[j][2 * q + 1], __fmul_rn(hi, w));
+                    for (int q = 0; q < 4; ++q) {
+                        f[2 * q] = Decode16<BF16>(v16[u][j][q] & 0xffffu);
+                        f[2 * q + 1] = Decode16<BF16>(v16[u][j][q] >> 16);
+                    }
+                }
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    acc[j][e] = KIND == kReducePerAdd ? RoundTo16<BF16>(__fadd_rn(acc[j][e], f[e])) :
+                        __fadd_rn(acc[j][e], __fmul_rn(f[e], w));
+                }
+            }
+        }
+    }
+    if constexpr (COMMQ != 0) {
+        if (__any(odd ? 1 : 0)) {
+            // the same sums once more, one row at a time, with the codec for rows that are not finite somewhere
+#pragma unroll
+            for (int j = 0; j < V; ++j) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    acc[j][e] = 0.0f;
+                }
+            }
+#pragma unroll 1
+            for (uint64_t left = __ballot(myRow >= 0); left != 0; left &= left - 1) {
+                const int k = __builtin_ctzll(left);
+                const int row = __builtin_amdgcn_readlane(myRow, k);
+                const float w = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(myWeight), k));
+                const __amdgpu_buffer_rsrc_t rsrc = RowResource(static_cast<const char *>(a.expertOut) + static_cast<int64_t>(row) * a.h * 2, vecs * 16);
+#pragma unroll
+                for (int j = 0; j < V; ++j) {
+                    const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (colBase + j * kWave + lane) * 16, 0, 0);
+                    float f[8];
+                    MxRoundTripAny<BF16, kCommE5m2>(v, f);
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        acc[j][e] = __fadd_rn(acc[j][e], __fmul_rn(f[e], w));
                     }
                 }
             }
@@ -193,13 +228,13 @@ __global__ __launch_bounds__(kSmallReduceThreads) void ep_reduce_small_kernel(Sm
     }
 }
 
-template <int KIND>
+template <int KIND, int COMMQ>
 void LaunchByType(bool bf16, int grid, int threads, hipStream_t stream, const SmallReduceArgs &a)
 {
     if (bf16) {
-        hipLaunchKernelGGL((ep_reduce_small_kernel<KIND, true>), dim3(grid), dim3(threads), 0, stream, a);
+        hipLaunchKernelGGL((ep_reduce_small_kernel<KIND, true, COMMQ>), dim3(grid), dim3(threads), 0, stream, a);
     } else {
-        hipLaunchKernelGGL((ep_reduce_small_kernel<KIND, false>), dim3(grid), dim3(threads), 0, stream, a);
+        hipLaunchKernelGGL((ep_reduce_small_kernel<KIND, false, COMMQ>), dim3(grid), dim3(threads), 0, stream, a);
     }
 }
 
@@ -211,7 +246,7 @@ bool SmallReduceFits(const ReduceLaunch &l)
     const int64_t vecs = l.h / 8;
     return l.assistTable != nullptr && l.rowIndexMap == nullptr && l.inverseTagged == nullptr && l.orderKeys == nullptr &&
         l.bs > 0 && n <= kSmallRoutes && l.bs * n <= kSmallScanTuples && l.topK <= kMaxTopK && l.sharedSlots == 0 && l.tileFlags == nullptr &&
-        l.inQuant == 0 && l.commQuant == 0 && l.h % 8 == 0 && l.rowBytes == l.h * 2 &&
+        l.inQuant == 0 && (l.commQuant == 0 || (l.reduceKind == kReduceFp32 && l.h % 32 == 0)) && l.h % 8 == 0 && l.rowBytes == l.h * 2 &&
         vecs <= static_cast<int64_t>(kSmallReduceThreads / kWave) * kWave * kSmallReduceVecs &&
         l.assistTable->maxRows == n && l.assistTable->maxCountPerEntry == n && l.assistTable->bs == l.bs &&
         l.assistTable->topK == l.topK && (l.assistTable->countsArePrefix || l.assistTable->numCounts == 1) &&
@@ -244,10 +279,15 @@ hipError_t LaunchSmallReduce(const ReduceLaunch &l)
     if (l.kernelNameOut != nullptr) {
         *l.kernelNameOut = "ep_reduce_small_kernel";
     }
+    const int grid = static_cast<int>(l.bs);
     if (l.reduceKind == kReducePerAdd) {
-        LaunchByType<kReducePerAdd>(l.bf16, static_cast<int>(l.bs), threads, l.stream, a);
+        LaunchByType<kReducePerAdd, 0>(l.bf16, grid, threads, l.stream, a);
+    } else if (l.commQuant == TILEXR_EP_QUANT_COMM_MXFP8_E5M2) {
+        LaunchByType<kReduceFp32, TILEXR_EP_QUANT_COMM_MXFP8_E5M2>(l.bf16, grid, threads, l.stream, a);
+    } else if (l.commQuant == TILEXR_EP_QUANT_MXFP8) {
+        LaunchByType<kReduceFp32, TILEXR_EP_QUANT_MXFP8>(l.bf16, grid, threads, l.stream, a);
     } else {
-        LaunchByType<kReduceFp32>(l.bf16, static_cast<int>(l.bs), threads, l.stream, a);
+        LaunchByType<kReduceFp32, 0>(l.bf16, grid, threads, l.stream, a);
     }
     return hipGetLastError();
 }

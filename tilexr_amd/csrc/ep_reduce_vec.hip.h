@@ -192,18 +192,8 @@ __device__ __forceinline__ void ReduceVec(const ReduceArgs &a)
                 for (int j = 0; j < V; ++j) {
                     float f[8];
                     if constexpr (kMx) {
-                        // the round trip of a block whose elements are all finite: 24 instructions for eight elements
-                        // (about 350 with the software codec: the kernel was bound by them, 2048 x 7168 x top-8
-                        // 123 us then, 48.6 us = 5.5 TB/s now)
-                        const MxScaling mx = MxScalingOf<BF16, kCommE5m2>(MxBlockMaxBits(v16[u][j]));
-                        odd |= !mx.plain;
-#pragma unroll
-                        for (int q = 0; q < 4; ++q) {
-                            const f32x2 back = MxDecodePair<kCommE5m2>(
-                                MxEncodePair<BF16, kCommE5m2, false>(0u, v16[u][j][q], mx), mx);
-                            f[2 * q] = back[0];
-                            f[2 * q + 1] = back[1];
-                        }
+                        // (with the software codec the kernel was bound by it: 2048 x 7168 x top-8 123 us, 48.6 us = 5.5 TB/s now)
+                        odd |= !MxRoundTrip<BF16, kCommE5m2>(v16[u][j], f);
                     } else {
 #pragma unroll
                         for (int q = 0; q < 4; ++q) {
@@ -252,21 +242,10 @@ __device__ __forceinline__ void ReduceVec(const ReduceArgs &a)
                         const int idx = colBase + j * G + lane;
                         const u32x4 v = idx < vecs ? RowLoad<FL>(base, rsrc, idx * 16) : u32x4{0u, 0u, 0u, 0u};
                         float f[8];
-                        float amax = 0.0f;
-#pragma unroll
-                        for (int q = 0; q < 4; ++q) {
-                            f[2 * q] = Decode16<BF16>(v[q] & 0xffffu);
-                            f[2 * q + 1] = Decode16<BF16>(v[q] >> 16);
-                            amax = fmaxf(amax, fmaxf(fabsf(f[2 * q]), fabsf(f[2 * q + 1])));
-                        }
-                        amax = fmaxf(amax, __shfl_xor(amax, 1));
-                        amax = fmaxf(amax, __shfl_xor(amax, 2));
-                        const int se = MxSharedExponent<kCommE5m2>(amax);
-                        const float up = Exp2Int(se);
+                        MxRoundTripAny<BF16, kCommE5m2>(v, f);
 #pragma unroll
                         for (int e = 0; e < 8; ++e) {
-                            const float back = Fp8Decode<kCommE5m2>(Fp8Encode<kCommE5m2>(ldexpf(f[e], -se)));
-                            acc[j][e] = __fadd_rn(acc[j][e], __fmul_rn(__fmul_rn(back, up), w));
+                            acc[j][e] = __fadd_rn(acc[j][e], __fmul_rn(f[e], w));
                         }
                     }
                 }
