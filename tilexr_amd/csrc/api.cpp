@@ -89,7 +89,7 @@ int RunDispatchSingle(EpComm *comm, const EpDispatchParams &p, bool memoryRoute,
         small.expertTokenNumsOut = p.expertTokenNumsOut;
         small.tokenNumsType = static_cast<int>(p.expertTokenNumsType);
         small.quantMode = static_cast<int>(p.quantMode);
-        small.inputBf16 = p.dtype == TileXR::TILEXR_DATA_TYPE_BFP16;
+        small.inputBf16 = memoryRoute && p.dtype == TileXR::TILEXR_DATA_TYPE_BFP16;
         small.fp8E5m2 = p.expandXOutDtype == TileXR::TILEXR_DATA_TYPE_FP8E5M2;
         small.scalesOut = p.dynamicScalesOut;
         small.tileFlags = p.tileFlagsOut;
@@ -138,7 +138,7 @@ int RunDispatchSingle(EpComm *comm, const EpDispatchParams &p, bool memoryRoute,
     const bool mayOneLaunch = comm->routing != EpComm::Routing::kLegacy;
     const bool oneLaunchRows = mayOneLaunch && memoryRoute &&
         RouteRowsFits(p.expertIds, n, numKeys, maskMode, p.expertCapacity) &&
-        (comm->routing == EpComm::Routing::kOneLaunch || RouteRowsPays(n, numKeys, rowsAhead, warm));
+        (comm->routing == EpComm::Routing::kOneLaunch || RouteRowsPays(n, numKeys, rowsAhead, warm, maskMode == kMaskNone ? 0 : p.bs, p.expertCapacity));
     const bool oneLaunchCompact = mayOneLaunch && !memoryRoute && p.expertCapacity <= 0 &&
         RouteCompactFits(p.expertIds, n, experts, maskMode) &&
         (comm->routing == EpComm::Routing::kOneLaunch || RouteCompactPays(n, experts));
@@ -206,6 +206,8 @@ int RunDispatchSingle(EpComm *comm, const EpDispatchParams &p, bool memoryRoute,
         rows.tokenNumsType = static_cast<int>(p.expertTokenNumsType);
         rows.warmRows = warm ? p.x : nullptr;
         rows.warmBytes = p.bs * p.h * 2;
+        rows.mask = reinterpret_cast<const uint8_t *>(p.xActiveMask);
+        rows.capacity = std::max<int64_t>(p.expertCapacity, 0);
         rows.stream = stream;
         comm->lastKernel[kKernelCount] = "ep_route_rows_kernel";
         ret = Timed(comm, kKernelCount, stream, "route rows", [&] { return LaunchRouteRows(rows); });

@@ -72,8 +72,8 @@ struct RouteCountLaunch {
     hipStream_t stream;
 };
 
-// Memory route, one rank, keys = experts, no mask, no capacity limit: rows and assist tuples of all routes in one launch
-// (ep_rows.hip), for id tables small enough that every workgroup reads the whole table itself.
+// Memory route, one rank, keys = experts: rows and assist tuples of all routes in one launch (ep_rows.hip), for id tables
+// small enough that every workgroup reads the whole table itself.  A token-prefix mask or a capacity limit, not both.
 constexpr int kRowsTableRoutes = 262144;
 struct RouteRowsLaunch {
     const int32_t *ids;
@@ -91,9 +91,12 @@ struct RouteRowsLaunch {
     int tokenNumsType;
     const void *warmRows;        // as RouteCountLaunch
     int64_t warmBytes;
+    const uint8_t *mask;         // optional [bs]: the first sum(mask) tokens are dispatched
+    int64_t capacity;            // rows an expert keeps, 0 = all
     hipStream_t stream;
 };
-bool RouteRowsPays(int64_t routes, int64_t numKeys, bool rowsAhead, bool readsRowsAhead);
+// maskedTokens: tokens of the prefix mask, 0 without one
+bool RouteRowsPays(int64_t routes, int64_t numKeys, bool rowsAhead, bool readsRowsAhead, int64_t maskedTokens, int64_t capacity);
 bool RouteRowsFits(const int32_t *ids, int64_t routes, int64_t numKeys, int maskMode, int64_t capacity);
 hipError_t LaunchRouteRows(const RouteRowsLaunch &l);
 

@@ -1,5 +1,5 @@
 // rows: destination row and assist tuple of every route in ONE launch (gfx950, wave64; memory route, one rank, keys =
-// experts, no mask, no capacity limit, up to kRowsTableRoutes routes).  Replaces the count launch's ticket and
+// experts, up to kRowsTableRoutes routes).  Replaces the count launch's ticket and
 // last-workgroup scan and the separate place launch.
 //
 // What such a kernel costs on this part, measured: a hand-over between launches or workgroups is a round trip through
@@ -20,9 +20,16 @@
 // ranks its slots one after the other), so when the keys are few a key gets several workgroups: each counts the whole
 // table and ranks one part of every wave's sixteenth.
 //
+// A token-prefix mask makes the table shorter: every workgroup adds the mask up first, one more round trip.  A capacity
+// limit makes "valid ids below k" the sum of the smaller keys' counts, each cut at the limit, so those are counted in an
+// LDS histogram after all (RouteRowsPays: tables where that is cheaper than the hand-over); routes beyond a key's limit
+// get row -1 from the workgroup that ranks them.
+//
 // Same definitions as the count + place pair (reference: src/ep/kernels/tilexr_ep_dispatch_memory_kernel.h:791-818
 // rank within expert, :820-1089 count exchange and inclusive cumulative sum, :1142-1168 count outputs, :1240-1258
 // assist tuple).
+#include <algorithm>
+
 #include <hip/hip_runtime.h>
 
 #include "ep_chunk_rank.hip.h"
@@ -62,7 +69,14 @@ struct RouteRowsArgs {
     int tokenNumsType;
     const u32x4 *warmRows;
     int64_t warmVecs;
+    const uint8_t *mask;         // kRowsPrefix: [bs]
+    int bs;
+    int capacity;                // kRowsCapped: rows a key keeps
 };
+
+// Which routes have rows: those whose id names a key; of these, those of the first sum(mask) tokens; or the first
+// `capacity` of every key.
+enum RowsLimit { kRowsAll, kRowsPrefix, kRowsCapped };
 
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 
@@ -82,6 +96,30 @@ __device__ __forceinline__ void LoadSlots(const __amdgpu_buffer_rsrc_t &table, i
     }
 }
 
+// Tokens that a prefix mask leaves active, four bytes of it in flight per lane.  All lanes of the workgroup call it.
+__device__ __forceinline__ int TokensInPrefix(const uint8_t *mask, int tokens, int wave, int lane, int *s_part)
+{
+    constexpr int kBatch = 4;
+    const __amdgpu_buffer_rsrc_t bytes = RowResource(mask, tokens);     // those beyond the end read as zero
+    int live = 0;
+    for (int first = 0; first < tokens; first += kBatch * kRowsThreads) {
+        uint8_t m[kBatch];
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u) {
+            m[u] = __builtin_amdgcn_raw_buffer_load_b8(bytes, first + u * kRowsThreads + wave * kWave + lane, 0, 0);
+        }
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u) {
+            live += __popcll(__ballot(m[u] != 0));
+        }
+    }
+    if (lane == 0) {
+        s_part[wave] = live;
+    }
+    __syncthreads();
+    return WaveSum(lane < kRowsWaves ? s_part[lane] : 0);
+}
+
 // The kernel stays within 64 registers per lane whatever the table's size (ids are streamed, eight loads a lane at a
 // time, and only one bit per id is kept), so that two workgroups of 1024 lanes fit a compute unit: the workgroups that
 // read token rows start beside the routing ones instead of behind them (58.7 MB read in 15.6 us when they had to wait,
@@ -89,11 +127,14 @@ __device__ __forceinline__ void LoadSlots(const __amdgpu_buffer_rsrc_t &table, i
 //
 // SPLIT: a key has several workgroups (a.parts > 1).  The common case of one per key is compiled without the tests
 // that tell a workgroup's own slots from the rest.
-template <bool SPLIT>
+template <bool SPLIT, int LIMIT>
 __global__ __launch_bounds__(kRowsThreads, 8) void ep_route_rows_kernel(RouteRowsArgs a)
 {
+    constexpr bool kPrefix = LIMIT == kRowsPrefix;
+    constexpr bool kCapped = LIMIT == kRowsCapped;
     __shared__ int s_less[kRowsWaves];
     __shared__ int s_same[kRowsWaves];
+    __shared__ int s_hist[kCapped ? kMaxKeys : 1];      // routes of the keys below this workgroup's
 
     const int tid = threadIdx.x;
     const int wave = tid / kWave;
@@ -107,10 +148,16 @@ __global__ __launch_bounds__(kRowsThreads, 8) void ep_route_rows_kernel(RouteRow
         return;
     }
     const int waveFirst = wave * a.slots * kRowsSlotRoutes;
-    const __amdgpu_buffer_rsrc_t table = RowResource(a.ids, a.n * 4);
+    int n = a.n;                // routes that may have a row: the first n
+    if (kPrefix) {
+        n = TokensInPrefix(a.mask, a.bs, wave, lane, s_less) * a.topK;
+        __syncthreads();        // s_less is used again below
+    }
+    const __amdgpu_buffer_rsrc_t table = RowResource(a.ids, (block == keyBlocks ? a.n : n) * 4);
 
     if (block == keyBlocks) {
-        // ids outside [0, E) are skipped, not errors: their routes have no row, and this workgroup says so
+        // ids outside [0, E) are skipped, not errors: their routes have no row, nor have those behind the mask's prefix, and
+        // this workgroup says so
         const unsigned keys = static_cast<unsigned>(a.numKeys);
 #pragma unroll 1
         for (int s0 = 0; s0 < a.slots; s0 += kRowsBatch) {
@@ -119,13 +166,13 @@ __global__ __launch_bounds__(kRowsThreads, 8) void ep_route_rows_kernel(RouteRow
 #pragma unroll
             for (int u = 0; u < kRowsBatch; ++u) {
                 if (s0 + u < a.slots) {
-                    const bool none = static_cast<unsigned>(id[u][0]) >= keys || static_cast<unsigned>(id[u][1]) >= keys ||
+                    const int route = waveFirst + (s0 + u) * kRowsSlotRoutes + lane * 4;
+                    const bool none = (kPrefix && route + 3 >= n) || static_cast<unsigned>(id[u][0]) >= keys || static_cast<unsigned>(id[u][1]) >= keys ||
                         static_cast<unsigned>(id[u][2]) >= keys || static_cast<unsigned>(id[u][3]) >= keys;
                     if (__ballot(none) != 0ull) {
-                        const int route = waveFirst + (s0 + u) * kRowsSlotRoutes + lane * 4;
 #pragma unroll 1
                         for (int e = 0; e < 4; ++e) {
-                            if (route + e < a.n && static_cast<unsigned>(id[u][e]) >= keys) {
+                            if (route + e < a.n && ((kPrefix && route + e >= n) || static_cast<unsigned>(id[u][e]) >= keys)) {
                                 a.rowOf[route + e] = -1;
                             }
                         }
@@ -143,6 +190,12 @@ __global__ __launch_bounds__(kRowsThreads, 8) void ep_route_rows_kernel(RouteRow
     // pass 1, over the wave's whole sixteenth: per lane, ids below the key (unsigned compare: negative ids are above
     // every key) and ids equal to it, those ahead of the workgroup's own slots counted apart; which elements of its own
     // slots are equal is kept, four bits per slot, so that pass 2 needs no id any more
+    if (kCapped) {
+        for (int j = tid; j < key; j += kRowsThreads) {
+            s_hist[j] = 0;
+        }
+        __syncthreads();
+    }
     int less = 0;
     int same = 0;
     int sameAhead = 0;
@@ -156,9 +209,15 @@ __global__ __launch_bounds__(kRowsThreads, 8) void ep_route_rows_kernel(RouteRow
             const int s = s0 + u;
             if (s < a.slots) {
                 uint32_t mine = 0u;
+                const int inTable = kCapped ? n - (waveFirst + s * kRowsSlotRoutes + lane * 4) : 4;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    less += static_cast<unsigned>(id[u][e]) < static_cast<unsigned>(key) ? 1 : 0;
+                    const bool below = static_cast<unsigned>(id[u][e]) < static_cast<unsigned>(key);
+                    if (!kCapped) {
+                        less += below ? 1 : 0;
+                    } else if (below && e < inTable) {
+                        atomicAdd(&s_hist[id[u][e]], 1);
+                    }
                     mine |= id[u][e] == key ? 1u << e : 0u;
                 }
                 const int hits = __popc(mine);
@@ -172,19 +231,26 @@ __global__ __launch_bounds__(kRowsThreads, 8) void ep_route_rows_kernel(RouteRow
             }
         }
     }
-    less = WaveSum(less);
+    less = kCapped ? 0 : WaveSum(less);
     same = WaveSum(same);
     if (lane == 0) {
         s_less[wave] = less;
         s_same[wave] = same;
     }
     __syncthreads();
+    int capped = 0;             // rows of the keys below
+    if (kCapped) {
+        for (int j = lane; j < key; j += kWave) {
+            capped += min(s_hist[j], a.capacity);
+        }
+        capped = WaveSum(capped);
+    }
     // elements beyond the table read as id 0: below every other key, equal to key 0
-    const int beyond = kRowsWaves * a.slots * kRowsSlotRoutes - a.n;
+    const int beyond = kRowsWaves * a.slots * kRowsSlotRoutes - n;
     // lane w of every wave takes wave w's two counts; sums over the lanes (few registers: this kernel has 64)
     const int lessOf = lane < kRowsWaves ? s_less[lane] : 0;
     const int sameOf = lane < kRowsWaves ? s_same[lane] : 0;
-    const int lessTotal = WaveSum(lessOf) - (key > 0 ? beyond : 0);
+    const int lessTotal = kCapped ? capped : WaveSum(lessOf) - (key > 0 ? beyond : 0);
     const int total = WaveSum(sameOf) - (key == 0 ? beyond : 0);
 
     // pass 2: slot by slot, the lanes that hold the key are ranked (flat route order within a slot: lane, then element)
@@ -213,8 +279,12 @@ __global__ __launch_bounds__(kRowsThreads, 8) void ep_route_rows_kernel(RouteRow
                 const int route = first + s * kRowsSlotRoutes;
                 for (uint32_t left = mine; left != 0u; left &= left - 1u) {
                     const int e = __builtin_ctz(left);
-                    if (route + e >= a.n) {
+                    if (route + e >= n) {
                         break;              // beyond the table (key 0 only): nothing real follows in this lane
+                    }
+                    if (kCapped && row - lessTotal >= a.capacity) {
+                        a.rowOf[route + e] = -1;
+                        continue;           // so are the key's routes that follow
                     }
                     int kOf = k + e;
                     int tokenOf = token;
@@ -246,12 +316,13 @@ __global__ __launch_bounds__(kRowsThreads, 8) void ep_route_rows_kernel(RouteRow
     }
     if (tid == 0 && part == 0) {
         // ids up to this key = the inclusive cumulative sum the counts output holds
-        const int incl = lessTotal + total;
+        const int kept = kCapped ? min(total, a.capacity) : total;
+        const int incl = lessTotal + kept;
         if (a.sendCountsOut != nullptr) {
             a.sendCountsOut[key] = incl;
         }
         if (a.expertTokenNumsOut != nullptr) {
-            a.expertTokenNumsOut[key] = a.tokenNumsType == 0 ? incl : total;
+            a.expertTokenNumsOut[key] = a.tokenNumsType == 0 ? incl : kept;
         }
         if (key == a.numKeys - 1) {
             *a.totalRowsOut = incl;
@@ -398,8 +469,8 @@ __global__ __launch_bounds__(kRowsThreads, 8) void ep_route_compact_kernel(Route
 
 bool RouteRowsFits(const int32_t *ids, int64_t routes, int64_t numKeys, int maskMode, int64_t capacity)
 {
-    return routes > 0 && routes <= kRowsTableRoutes && numKeys > 0 && numKeys <= kMaxKeys && maskMode == kMaskNone &&
-        capacity <= 0 && Aligned16(ids);
+    return routes > 0 && routes <= kRowsTableRoutes && numKeys > 0 && numKeys <= kMaxKeys && Aligned16(ids) &&
+        (maskMode == kMaskNone || (maskMode == kMaskTokenPrefix && capacity <= 0));
 }
 
 // Where the one-launch routing is the faster choice.  Every key's workgroups read and count the whole table, so the
@@ -415,8 +486,16 @@ bool RouteRowsFits(const int32_t *ids, int64_t routes, int64_t numKeys, int mask
 //     32 768 routes                  1-4 us faster up to 512 experts
 //     65 536 routes                  1-4 us faster up to 64 experts, level up to 256, slower beyond
 //     131 072 routes and more        slower from 64 experts on (3-14 us at 128-256 experts, 200 us at 262 144 x 1024)
-bool RouteRowsPays(int64_t routes, int64_t numKeys, bool rowsAhead, bool readsRowsAhead)
+// Token-prefix masks, count and one launch: 400 x 2048 x top-8 of 64 20.0 -> 16.3 us, 1024 x 2048 of 256 24.2 -> 20.3, 2048 x
+// 2048 34.6 -> 30.5, 8192 x 2048 x top-4 of 64 65.5 -> 60.0; up to 8192 tokens (the mask is added up eight bytes a lane).
+// Capacity limits, whose histogram grows with the routes: 518 x 2048 x top-8 of 64 18.4 -> 14.2, with flags (no place launch)
+// 22.1 -> 17.2; 1729 x top-5 of 128 24.3 -> 20.8; 16 384 routes of 64 33.1 -> 30.0, of 512 35.0 -> 33.1, block fp8 23.0 and 22.9;
+// 32 768 routes of 128 55.1 and 54.9, block fp8 29.7 and 31.3, of 512 56.4 and 58.4; 65 536 routes 102.4 and 104.0, 53.2 and 58.0.
+bool RouteRowsPays(int64_t routes, int64_t numKeys, bool rowsAhead, bool readsRowsAhead, int64_t maskedTokens, int64_t capacity)
 {
+    if (maskedTokens > 8192 || (capacity > 0 && (routes > 16384 || numKeys > 512))) {
+        return false;
+    }
     if (routes <= 16384) {
         return rowsAhead || numKeys <= 1024;
     }
@@ -429,7 +508,7 @@ bool RouteRowsPays(int64_t routes, int64_t numKeys, bool rowsAhead, bool readsRo
 hipError_t LaunchRouteRows(const RouteRowsLaunch &l)
 {
     const int64_t n = l.bs * l.topK;
-    if (!RouteRowsFits(l.ids, n, l.numKeys, kMaskNone, 0)) {
+    if (!RouteRowsFits(l.ids, n, l.numKeys, l.mask != nullptr ? kMaskTokenPrefix : kMaskNone, l.capacity)) {
         return hipErrorInvalidValue;
     }
     RouteRowsArgs a {};
@@ -460,6 +539,9 @@ hipError_t LaunchRouteRows(const RouteRowsLaunch &l)
     a.firstOffsetOut = l.firstOffsetOut;
     a.expertTokenNumsOut = l.expertTokenNumsOut;
     a.tokenNumsType = l.tokenNumsType;
+    a.mask = l.mask;
+    a.bs = static_cast<int>(l.bs);
+    a.capacity = static_cast<int>(std::min<int64_t>(l.capacity, n));
     // the keys' workgroups, one for the routes without an expert, then those that read token rows
     unsigned blocks = static_cast<unsigned>(l.numKeys) * static_cast<unsigned>(a.parts) + 1u;
     if (l.warmRows != nullptr && l.warmBytes >= 16 && Aligned16(l.warmRows)) {
@@ -467,10 +549,13 @@ hipError_t LaunchRouteRows(const RouteRowsLaunch &l)
         a.warmVecs = l.warmBytes / 16;
         blocks += WarmWorkgroups(a.warmVecs, kRowsThreads, kRowsWarmLoads);
     }
-    if (a.parts > 1) {
-        hipLaunchKernelGGL(ep_route_rows_kernel<true>, dim3(blocks), dim3(kRowsThreads), 0, l.stream, a);
+    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kRowsThreads), 0, l.stream, a); };
+    if (l.capacity > 0) {
+        a.parts > 1 ? launch(ep_route_rows_kernel<true, kRowsCapped>) : launch(ep_route_rows_kernel<false, kRowsCapped>);
+    } else if (l.mask != nullptr) {
+        a.parts > 1 ? launch(ep_route_rows_kernel<true, kRowsPrefix>) : launch(ep_route_rows_kernel<false, kRowsPrefix>);
     } else {
-        hipLaunchKernelGGL(ep_route_rows_kernel<false>, dim3(blocks), dim3(kRowsThreads), 0, l.stream, a);
+        a.parts > 1 ? launch(ep_route_rows_kernel<true, kRowsAll>) : launch(ep_route_rows_kernel<false, kRowsAll>);
     }
     return hipGetLastError();
 }

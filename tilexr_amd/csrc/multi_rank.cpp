@@ -243,7 +243,7 @@ int SendRoutes(EpComm *comm, const EpDispatchParams &p, bool memoryRoute, const 
     const bool warm = ScatterCopiesPerRoute(p.x, myRows, p.bs, p.h, plan.perToken, static_cast<int>(p.quantMode));
     const bool oneLaunch = memoryRoute && shared == 0 && comm->routing != EpComm::Routing::kLegacy &&
         RouteRowsFits(routeIds, n, plan.numKeys, maskMode, 0) &&
-        (comm->routing == EpComm::Routing::kOneLaunch || RouteRowsPays(n, plan.numKeys, false, warm));
+        (comm->routing == EpComm::Routing::kOneLaunch || RouteRowsPays(n, plan.numKeys, false, warm, maskMode == kMaskNone ? 0 : p.bs, 0));
     int ret = kOk;
     RoutePlaceLaunch place {};
     if (oneLaunch) {
@@ -262,6 +262,7 @@ int SendRoutes(EpComm *comm, const EpDispatchParams &p, bool memoryRoute, const 
         rows.tokenNumsType = static_cast<int>(p.expertTokenNumsType);
         rows.warmRows = warm ? p.x : nullptr;
         rows.warmBytes = p.bs * p.h * 2;
+        rows.mask = routeMask;
         rows.stream = stream;
         comm->lastKernel[kKernelCount] = "ep_route_rows_kernel";
         ret = Timed(comm, kKernelCount, stream, "route rows", [&] { return LaunchRouteRows(rows); });
