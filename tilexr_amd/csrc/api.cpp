@@ -67,7 +67,8 @@ int RunDispatchSingle(EpComm *comm, const EpDispatchParams &p, bool memoryRoute,
         maskMode = p.activeMaskType == TILEXR_EP_ACTIVE_MASK_EXPERT ? kMaskPerRoute : kMaskTokenPrefix;
     }
     // (a quantised call that may not allocate asks for the static scratch, whether or not its size needs it)
-    if (memoryRoute && (p.quantMode == TILEXR_EP_QUANT_NONE || !p.noAlloc) && p.metaReadyEvent == nullptr) {
+    const bool mvpMayBeSmall = comm->routing == EpComm::Routing::kAuto && p.tpRecvCountsOut == nullptr;
+    if ((memoryRoute || mvpMayBeSmall) && (p.quantMode == TILEXR_EP_QUANT_NONE || !p.noAlloc) && p.metaReadyEvent == nullptr) {
         // decode-sized calls: one launch instead of count + scatter (a consumer that is to run beside the dispatch needs
         // the row map ahead of the rows, which takes the separate launches)
         SmallDispatchLaunch small {};
@@ -85,6 +86,7 @@ int RunDispatchSingle(EpComm *comm, const EpDispatchParams &p, bool memoryRoute,
         small.out = p.expandXOut;
         small.assist = p.assistInfoForCombineOut;
         small.rowOf = p.rowIndexMapOut;
+        small.mvp = !memoryRoute;
         small.sendCountsOut = p.epRecvCountsOut;
         small.expertTokenNumsOut = p.expertTokenNumsOut;
         small.tokenNumsType = static_cast<int>(p.expertTokenNumsType);

@@ -257,7 +257,8 @@ struct SmallDispatchLaunch {
     void *out;
     int32_t *assist;
     int32_t *rowOf;                  // optional
-    int32_t *sendCountsOut;
+    bool mvp;                        // MVP route: rows in route order whatever the expert
+    int32_t *sendCountsOut;          // MVP route: the one count of all rows, optional
     int32_t *firstOffsetOut;         // optional: set to zero (the word ahead of sendCountsOut, where the caller wants exclusive offsets)
     int64_t *expertTokenNumsOut;
     int tokenNumsType;

@@ -100,7 +100,7 @@ __device__ __forceinline__ void QuantiseRow(const Args &a, const u32x4 (&v)[V], 
     out.rowScale = 1.0f;
     // per-row / per-block scale, then 8 output bytes per input vector
     float rowScaleInv = 1.0f;
-    if (QMODE == TILEXR_EP_QUANT_STATIC_INT8) {
+    if constexpr (QMODE == TILEXR_EP_QUANT_STATIC_INT8) {
         rowScaleInv = a.staticScale[0];
     }
     if (QMODE == TILEXR_EP_QUANT_TOKEN_INT8) {

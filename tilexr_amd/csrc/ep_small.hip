@@ -157,6 +157,8 @@ __global__ __launch_bounds__(kThreads) void ep_dispatch_small_kernel(SmallArgs a
 
 } // namespace
 
+constexpr int64_t kSmallMvpExperts = 512;
+
 // Quantised rows: no capacity limit, and at most four vectors to a lane.  Dispatch + combine, routing and scatter launch before
 // and the one launch now, us: int8 512 x 2048 x top-4 12.4 -> 10.2, 2048 x 4096 x top-1 16.5 -> 15.4, 1000 x 7168 x top-2 16.9
 // and 16.8, 512 x 8192 x top-4 15.6 and 16.0 (each route's workgroup quantises the token's row again), block fp8 12.4 -> 10.7,
@@ -172,9 +174,19 @@ static bool SmallQuantFits(const SmallDispatchLaunch &l)
         (copesWithAny || l.bs * l.topK * l.h <= (int64_t{12} << 20));
 }
 
+// MVP route: no mask, no capacity limit, no flags.  Every expert wants a workgroup for its count.  Dispatch + combine, us, routing
+// and scatter launch before and the one launch now: 64 x 1024 x top-2 12.0 -> 8.1, 200 x 7168 x top-5 12.7 -> 10.4, 256 x 4096 x
+// top-8 13.6 -> 11.6, 2000 x 1024 x top-1 14.9 -> 11.7, 300 x 7168 x top-6 18.3 -> 16.7; int8 68 x 2048 x top-8 12.3 -> 8.8, 2000 x
+// 1024 x top-1 15.2 -> 12.6, 400 x 2048 x top-5 (4.1 M elements) 12.4 and 12.4, 256 x 4096 x top-8 (8.4 M) 12.9 and 13.8.
+static bool SmallMvpFits(const SmallDispatchLaunch &l)
+{
+    return l.numExperts <= kSmallMvpExperts && l.maskMode == kMaskNone && l.capacity <= 0 && l.tileFlags == nullptr &&
+        (l.quantMode == TILEXR_EP_QUANT_NONE || (l.quantMode == TILEXR_EP_QUANT_TOKEN_INT8 && !l.inputBf16 && l.bs * l.topK * l.h <= (int64_t{3} << 20)));
+}
+
 bool SmallDispatchFits(const SmallDispatchLaunch &l)
 {
-    return l.bs * l.topK <= kSmallRoutes && l.numExperts <= kMaxKeys && l.topK <= kMaxTopK && l.h % 8 == 0 &&
+    return (!l.mvp || SmallMvpFits(l)) && l.bs * l.topK <= kSmallRoutes && l.numExperts <= kMaxKeys && l.topK <= kMaxTopK && l.h % 8 == 0 &&
         l.h / 8 <= 8 * kThreads && Aligned16(l.x) &&
         (l.quantMode == TILEXR_EP_QUANT_NONE ? Aligned16(l.out) : SmallQuantFits(l)) &&
         (l.maskMode == kMaskNone || (l.mask != nullptr && (l.maskMode == kMaskPerRoute || l.maskMode == kMaskTokenPrefix)));
@@ -224,6 +236,19 @@ hipError_t LaunchSmallDispatch(const SmallDispatchLaunch &l)
         const dim3 routes(static_cast<unsigned>(std::max<int64_t>(XcdPlacedUnits(static_cast<int>(l.bs), static_cast<int>(l.topK)), l.numExperts)));
         if (l.quantMode != TILEXR_EP_QUANT_NONE) {
             return LaunchSmallQuantRoutes(l, a, routes.x);
+        }
+        if (l.mvp) {
+            auto pickMvp = [&](auto vecsPerLane) {
+                constexpr int kV = decltype(vecsPerLane)::value;
+                if (LeavesRowsToL2(l)) {
+                    launch(ep_dispatch_small_route_kernel<kV, 0, kIdsPerLane, false, TILEXR_EP_QUANT_NONE, true, false, true>, routes);
+                } else {
+                    launch(ep_dispatch_small_route_kernel<kV, kAuxNonTemporal, kIdsPerLane, false, TILEXR_EP_QUANT_NONE, true, false, true>, routes);
+                }
+            };
+            v == 2 ? pickMvp(std::integral_constant<int, 2> {}) : v == 4 ? pickMvp(std::integral_constant<int, 4> {}) :
+                pickMvp(std::integral_constant<int, 8> {});
+            return hipGetLastError();
         }
         const bool few = l.bs * l.topK <= 4 * kThreads;
         const bool plain = LeavesRowsToL2(l);

@@ -51,7 +51,15 @@ void LaunchByMode(const SmallDispatchLaunch &l, const SmallArgs &a, unsigned wor
 
 hipError_t LaunchSmallQuantRoutes(const SmallDispatchLaunch &l, const SmallArgs &a, unsigned workgroups)
 {
-    if (l.inputBf16) {
+    if (l.mvp) {
+        // MVP route: int8 rows, decoded as fp16, no flags, no mask
+        auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(workgroups), dim3(kThreads), 0, l.stream, a); };
+        if (l.h / 8 <= 2 * kThreads) {
+            launch(ep_dispatch_small_route_kernel<2, kAuxAgentScopeKept, kIdsPerLane, false, TILEXR_EP_QUANT_TOKEN_INT8, false, false, true>);
+        } else {
+            launch(ep_dispatch_small_route_kernel<4, kAuxAgentScopeKept, kIdsPerLane, false, TILEXR_EP_QUANT_TOKEN_INT8, false, false, true>);
+        }
+    } else if (l.inputBf16) {
         LaunchByMode<true>(l, a, workgroups);
     } else {
         LaunchByMode<false>(l, a, workgroups);

@@ -28,13 +28,12 @@ struct SmallArgs {
     void *out;
     int32_t *assist;
     int32_t *rowOf;              // optional [bs, topK]
-    int32_t *sendCountsOut;
+    int32_t *sendCountsOut;      // MVP route: one count of all rows, optional
     int32_t *firstOffsetOut;     // optional
     int64_t *expertTokenNumsOut;
     int tokenNumsType;
-    const float *staticScale;    // none: modes with scales of their own only
-    void *scalesOut;             // quantised payloads
     TilePublishArgs tiles;       // flags == nullptr: none (totalRows is filled in by the kernels)
+    void *scalesOut;             // quantised payloads
 };
 
 // ep_small_quant.hip: the launch for quantised rows of at most 4 * kThreads vectors.
@@ -122,7 +121,9 @@ __device__ __forceinline__ bool SmallRouteLive(const SmallArgs &a, int route, in
 //
 // QMODE: quantised payloads.  Every route's workgroup quantises the token's row for itself, K times the arithmetic of the scatter
 // kernel, which at this size costs less than the launch it saves.
-template <int V, int AUX, int IDS, bool MASKED, int QMODE = TILEXR_EP_QUANT_NONE, bool BF16 = true, bool E5M2 = false>
+//
+// MVP: rows in route order, whatever the expert: row = (earlier valid routes), and one count of all rows.
+template <int V, int AUX, int IDS, bool MASKED, int QMODE = TILEXR_EP_QUANT_NONE, bool BF16 = true, bool E5M2 = false, bool MVP = false>
 __global__ __launch_bounds__(kThreads) void ep_dispatch_small_route_kernel(SmallArgs a)
 {
     constexpr bool WT = AUX == kAuxAgentScope;
@@ -178,13 +179,13 @@ __global__ __launch_bounds__(kThreads) void ep_dispatch_small_route_kernel(Small
         const int i = j * kThreads + tid;
         const unsigned id = static_cast<unsigned>(e[j]);
         const bool ok = id < experts;
-        rowCounts += (ok && e[j] < key ? 1 : 0) + (e[j] == key && i < route ? 0x10000 : 0);
+        rowCounts += MVP ? (ok && i < route ? 1 : 0) : (ok && e[j] < key ? 1 : 0) + (e[j] == key && i < route ? 0x10000 : 0);
         outCounts += (e[j] == expert ? 1 : 0) + (ok && e[j] <= expert ? 0x10000 : 0);
         valid += ok ? 1 : 0;
     }
     rowCounts = WaveSum(rowCounts);
     outCounts = WaveSum(outCounts);
-    if (WT) {
+    if (WT || MVP) {
         valid = WaveSum(valid);
     }
     if (lane == 0) {
@@ -211,7 +212,11 @@ __global__ __launch_bounds__(kThreads) void ep_dispatch_small_route_kernel(Small
         }
         if (expert < a.numExperts) {
             const int outSum = s_sum[0][1] + s_sum[1][1] + s_sum[2][1] + s_sum[3][1];
-            a.sendCountsOut[expert] = outSum >> 16;
+            if (!MVP) {
+                a.sendCountsOut[expert] = outSum >> 16;
+            } else if (expert == 0 && a.sendCountsOut != nullptr) {
+                *a.sendCountsOut = s_sum[0][2] + s_sum[1][2] + s_sum[2][2] + s_sum[3][2];
+            }
             if (a.expertTokenNumsOut != nullptr) {
                 a.expertTokenNumsOut[expert] = a.tokenNumsType == 0 ? outSum >> 16 : outSum & 0xffff;
             }
