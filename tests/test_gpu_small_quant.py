@@ -105,3 +105,38 @@ def test_mx_exchange(bs, h, k, kernel, dtype, comm, infinite):
             want = O.mem_combine(O.Case(1, bs, h, k, e, dtype=dtype, mask_type=ep.MASK_TOKEN), 0, eo[None], d["assist"][None],
                                  d["send_counts"][None], expert_scales=w, token_mask=mask, shared_expert_x=shared, comm_quant=comm)
         assert np.array_equal(values(bits16(y), dtype), values(want, dtype))
+
+
+@pytest.mark.parametrize("bs,kernel", [(40, SMALL), (1100, GENERAL)])
+@pytest.mark.parametrize("dtype", [ep.DT_BF16, ep.DT_FP16])
+def test_int8_of_numbers_that_are_not_finite(bs, kernel, dtype):
+    """A NaN does not take part in its row's maximum and becomes -128; in a row with an infinity, whose scale is infinite, so does
+    the infinity, and what is finite becomes 0.  (The oracle takes finite rows.)"""
+    h, k, e = 136, 2, 8
+    rng = np.random.default_rng(bs)
+    ids = ids_for(rng, bs, k, e)
+    xt, _ = x_for(rng, bs, h, dtype, scale=2.0)
+    plain = xt.clone()
+    xt[::3, 5], xt[::3, h - 1] = float("nan"), -float("nan")
+    xt[1::3, 7] = float("inf")
+    plain[::3, 5] = plain[::3, h - 1] = 0.0
+    with Session() as s:
+        got = []
+        for x in (xt, plain):
+            out = alloc_dispatch_outputs(bs, h, k, e, quant=ep.Q_TOKEN_INT8)
+            counts = torch.zeros((e,), dtype=torch.int32, device=DEV)
+            assert ep.dispatch_memory_ex(x, to_dev(ids), s.comm, bs, h, k, e, out["expand_x"], out["assist"], out["token_nums"],
+                                         counts, dtype, s.stream, quant_mode=ep.Q_TOKEN_INT8, dynamic_scales=out["scales"],
+                                         row_index_map=out["row_map"])[0] == 0
+            s.sync()
+            assert ep.last_kernel_name(s.comm, ep.K_SCATTER) == kernel
+            got.append(fetch(out, "send_counts", counts))
+    token = got[0]["assist"][:, 1]
+    want, scales = got[1]["expand_x"].view(np.int8).copy(), got[1]["scales"].copy()
+    nan, inf = token % 3 == 0, token % 3 == 1
+    want[nan, 5] = want[nan, h - 1] = -128
+    want[inf] = 0
+    want[inf, 7] = -128
+    scales[inf] = np.inf
+    assert np.array_equal(got[0]["expand_x"].view(np.int8), want)
+    assert np.array_equal(got[0]["scales"], scales)

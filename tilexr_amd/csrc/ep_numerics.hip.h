@@ -103,15 +103,12 @@ __device__ __forceinline__ float RoundTo16(float v)
     return BF16 ? __uint_as_float(FloatToBf16Rne(v) << 16) : __half2float(__float2half_rn(v));
 }
 
-// add +-0.5, truncate toward zero, clamp to [-128, 127]
+// add +-0.5, truncate toward zero, clamp to [-128, 127] (ahead of the truncation, which comes to the same); NaN -> -128, which
+// is what the median of three makes of it
 __device__ __forceinline__ int ClampInt8(float v)
 {
-    float r = v >= 0.0f ? __fadd_rn(v, 0.5f) : __fadd_rn(v, -0.5f);
-    r = fminf(fmaxf(r, -129.0f), 128.0f);
-    int i = static_cast<int>(r);
-    i = i > 127 ? 127 : i;
-    i = i < -128 ? -128 : i;
-    return i;
+    const float r = __fadd_rn(v, __builtin_copysignf(0.5f, v));
+    return static_cast<int>(__builtin_amdgcn_fmed3f(r, -128.0f, 127.0f));
 }
 
 // Saturating round-to-nearest-even fp32 -> fp8 code (OCP e4m3fn / e5m2), by bit manipulation.

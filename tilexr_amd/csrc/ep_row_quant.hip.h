@@ -85,6 +85,14 @@ __device__ __forceinline__ void ScalarStore(T *p, T v)
     }
 }
 
+// The low bytes of four words, first one lowest.
+__device__ __forceinline__ uint32_t PackBytes(uint32_t a, uint32_t b, uint32_t c, uint32_t d)
+{
+    constexpr uint32_t kLowBytes = 0x0c0c0400u;         // bytes 0 of the second and of the first operand, zeros
+    constexpr uint32_t kLowHalves = 0x05040100u;
+    return __builtin_amdgcn_perm(__builtin_amdgcn_perm(d, c, kLowBytes), __builtin_amdgcn_perm(b, a, kLowBytes), kLowHalves);
+}
+
 // A row's payload and scales, as the lanes of its group hold them: eight bytes per 16-byte vector.
 template <int V>
 struct QuantisedRow {
@@ -196,15 +204,15 @@ __device__ __forceinline__ void QuantiseRow(const Args &a, const u32x4 (&v)[V], 
         } else {
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                bytes[e] = static_cast<uint32_t>(ClampInt8(__fmul_rn(f[e], rowScaleInv))) & 0xffu;
+                bytes[e] = static_cast<uint32_t>(ClampInt8(__fmul_rn(f[e], rowScaleInv)));
             }
         }
         if (QMODE == TILEXR_EP_QUANT_MXFP8 || QMODE == TILEXR_EP_QUANT_FP8_BLOCK128) {
             out.q[j][0] = fp8Words[0];
             out.q[j][1] = fp8Words[1];
         } else {
-            out.q[j][0] = bytes[0] | (bytes[1] << 8) | (bytes[2] << 16) | (bytes[3] << 24);
-            out.q[j][1] = bytes[4] | (bytes[5] << 8) | (bytes[6] << 16) | (bytes[7] << 24);
+            out.q[j][0] = PackBytes(bytes[0], bytes[1], bytes[2], bytes[3]);
+            out.q[j][1] = PackBytes(bytes[4], bytes[5], bytes[6], bytes[7]);
         }
     }
 }
