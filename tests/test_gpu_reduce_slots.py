@@ -103,3 +103,44 @@ def test_sums_in_the_order_of_the_rows(bs, h, k):
         assert ep.combine_v2(args[0], args[1], args[2], s.comm, bs, h, k, experts, y, ep.DT_FP16, s.stream) == 0
         s.sync()
         assert np.array_equal(bits16(y), O.mvp_combine(case, 0, rows[None], assist[None], counts[None]))
+
+
+@pytest.mark.parametrize("bs,h,k", [(2950, 8016, 1), (12007, 2064, 2), (23611, 1008, 1), (5801, 4096, 2)])
+@pytest.mark.parametrize("quant", [ep.Q_TOKEN_INT8, ep.Q_FP8_BLOCK128])
+@pytest.mark.parametrize("dtype", [ep.DT_BF16, ep.DT_FP16])
+def test_several_tokens_to_a_wave(bs, h, k, quant, dtype):
+    """One or two slots and outputs of 47 MB and more: slices that end within a row, tokens that do not fill the last wave,
+    lost rows, masked tokens, a shared expert; in places scales whose rows saturate in fp16, and NaN codes."""
+    experts = 16
+    rng = np.random.default_rng(bs + h + quant)
+    ids = ids_for(rng, bs, k, experts)
+    d = O.mem_dispatch(O.Case(1, bs, 16, k, experts), 0, np.zeros((1, bs, 16), np.uint16), ids[None])
+    assist = _lose(rng, d, bs, k)
+    n = bs * k
+    payload = rng.integers(0, 256, (n, h), dtype=np.uint8)
+    if quant == ep.Q_FP8_BLOCK128:
+        payload[(payload & 0x7f) == 0x7f] = 0x30
+        payload[rng.integers(0, n, 50), rng.integers(0, h, 50)] = rng.choice([0x7f, 0xff], 50)
+    scales = rng.random((n, 1 if quant == ep.Q_TOKEN_INT8 else (h + 127) // 128)).astype(np.float32)
+    scales[rng.integers(0, n, 60), rng.integers(0, scales.shape[1], 60)] = rng.choice(np.array([140, 147, 500, 512, 1e5], np.float32), 60)
+    w = (0.5 + rng.random((bs, k))).astype(np.float32)
+    mask = (rng.random(bs) < 0.9).astype(np.uint8)
+    _, shared = x_for(rng, bs, h, dtype)
+    with Session() as s:
+        y = torch.full((bs, h), 7.0, dtype=torch.bfloat16 if dtype == ep.DT_BF16 else torch.float16, device=DEV)
+        args = [to_dev(v) for v in (payload, assist, d["send_counts"], scales, w, mask, shared.view(np.int16))]
+        torch.cuda.synchronize()
+        assert ep.combine_memory_ex(args[0], args[1], args[2], s.comm, bs, h, k, experts, y, dtype, s.stream,
+                                    expert_out_quant_mode=quant, expert_out_scales=args[3], expert_scales=args[4],
+                                    active_mask=args[5], active_mask_type=ep.MASK_TOKEN, shared_expert_x=args[6]) == 0
+        s.sync()
+        assert ep.last_kernel_name(s.comm, ep.K_REDUCE) == "ep_reduce_quant_few_kernel"
+        got = bits16(y)
+    want = O.mem_combine(O.Case(1, bs, h, k, experts, dtype=dtype, mask_type=ep.MASK_TOKEN), 0, payload[None], assist[None],
+                         d["send_counts"][None], expert_scales=w, token_mask=mask, shared_expert_x=shared, in_quant=quant,
+                         in_scales=scales).view(np.uint16).reshape(bs, h)
+    infinity = 0x7f80 if dtype == ep.DT_BF16 else 0x7c00
+    nan = (want & 0x7fff) > infinity
+    assert nan.any() == (quant == ep.Q_FP8_BLOCK128)
+    assert np.array_equal((got & 0x7fff) > infinity, nan)       # (a NaN's sign is the adder's choice of operand)
+    assert np.array_equal(got[~nan], want[~nan])

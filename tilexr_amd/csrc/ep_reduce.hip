@@ -215,6 +215,23 @@ bool WaveUnits(const ReduceLaunch &l, int slices, int ranks)
     return slices > 1 || (l.tileFlags == nullptr && ranks == 1 && l.bs * (l.topK + l.sharedSlots) <= kSmallRoutes);
 }
 
+// Quantised rows, one or two to a token: several tokens to a wave (ep_reduce_quant_few_kernel) where the launch is long enough
+// to be bound by what its waves have under way, and its outputs and rows do not outgrow the memory-side cache.  Dispatch +
+// combine, us, a token to a wave and several, int8 and block fp8:
+//   top-1, outputs of 33 MB 16384 x 1024 25.1 and 25.6, 26.2 and 27.0; 49 MB 12000 x 2048 35.7 -> 34.6, 36.3 -> 35.6; 67 MB
+//     16384 x 2048 48.6 -> 44.3, 50.2 -> 46.2; 86 MB 6000 x 7168 59.8 -> 55.7, 63.2 -> 56.9; 164 MB 10000 x 8192 103.3 ->
+//     96.8, 108.9 -> 98.1; 235 MB 16384 x 7168 163.8 -> 160.7, 169.0 -> 159.7; 268 MB 16384 x 8192 174.3 and 175.9, 178.6 ->
+//     174.9
+//   top-2, 41 MB 5000 x 4096 36.3 and 36.8, 36.9 and 37.6; 67 MB 16384 x 2048 59.7 -> 56.1, 61.1 -> 58.4; 98 MB 6000 x 8192
+//     75.5 -> 74.0, 80.4 -> 75.7; 134 MB 16384 x 4096 103.6 -> 100.3, 104.4 -> 100.9; 164 MB 10000 x 8192 121.5 and 123.4,
+//     127.9 -> 125.8; 221 MB 13500 x 8192 179.1 and 181.7, 178.8 and 183.6
+bool QuantTakesFew(const ReduceLaunch &l)
+{
+    const int64_t outBytes = l.bs * l.h * 2;
+    return l.tileFlags == nullptr && l.topK <= 2 && l.sharedSlots == 0 && outBytes >= (int64_t{45} << 20) &&
+        outBytes <= (l.topK == 1 ? int64_t{224} << 20 : int64_t{128} << 20);
+}
+
 // 16-byte vectors per lane of a wave that takes one of `slices` slices.
 int VecsPerLane(int64_t vecs, int slices)
 {
@@ -271,7 +288,13 @@ hipError_t LaunchReduce(const ReduceLaunch &l)
         *l.kernelNameOut = quant ? "ep_reduce_quant_kernel" : (plain ? "ep_reduce_vec_kernel" : "ep_reduce_generic_kernel");
     }
     if (quant) {
-        if (qvecs <= kWave) {
+        if (QuantTakesFew(l)) {
+            a.colSlices = static_cast<int>((qvecs + kWave - 1) / kWave);
+            if (l.kernelNameOut != nullptr) {
+                *l.kernelNameOut = "ep_reduce_quant_few_kernel";
+            }
+            LaunchQuantKernels(kWave, kQuantFewSlots, l, a, 0);
+        } else if (qvecs <= kWave) {
             LaunchQuantKernels(kWave, 1, l, a, gridLimit);
         } else if (qvecs <= 2 * kWave) {
             LaunchQuantKernels(2 * kWave, 1, l, a, gridLimit);

@@ -55,6 +55,10 @@ struct WorldReduceArgs {
     ReduceArgs rank[kReduceRanks];
 };
 
+// As vectors per lane of the quantised launchers without flags: a slice of 64 vectors of several tokens to a wave, for tokens
+// of one or two slots.
+constexpr int kQuantFewSlots = 0;
+
 // Launchers of the register-resident kernels, one translation unit per (element type, with / without readiness flags).
 // g, v: lanes per token (or per slice of a token's row) and 16-byte vectors per lane; a combination that a unit does
 // not hold is a programming error and launches nothing.  world (units without flags only): one launch for `ranks` ranks,

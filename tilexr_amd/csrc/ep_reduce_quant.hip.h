@@ -18,6 +18,51 @@ namespace {
 // columns.  Each value is dequantised, rounded to the output element type, then accumulated exactly like an ordinary
 // row (fp32, k order, separate multiply and add).  Rows are a quarter the bytes of bf16 rows, so a lane owns 16
 // consecutive columns per vector (one 16-byte load) and KB rows are kept in flight at once.
+// A row's largest magnitude is 128 (448) times its scale: below this scale none reaches the 65520 from which rounding to fp16
+// has to saturate.
+template <int INQ>
+constexpr float kScaleSaturates = INQ == TILEXR_EP_QUANT_TOKEN_INT8 ? 511.875f : 146.25f;
+
+// Sixteen columns of a row: dequantised, rounded to the element type, weighted, added.  EXACT: the reference decode of NaN
+// codes and, for fp16, the saturating rounding.
+template <int INQ, bool BF16, bool EXACT>
+__device__ __forceinline__ void AddQuantRow(const u32x4 &q, float scale, float w, float (&acc)[16])
+{
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+        const uint32_t word = q[d];
+        float f[4];
+        if (INQ == TILEXR_EP_QUANT_TOKEN_INT8) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                f[e] = static_cast<float>(static_cast<int>(static_cast<int8_t>((word >> (8 * e)) & 0xffu)));
+            }
+        } else if (EXACT) {
+            Fp8E4m3DecodeWord(word, f);
+        } else {
+            Fp8E4m3DecodeWordFast(word, f);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; e += 2) {
+            const float d0 = __fmul_rn(f[e], scale);
+            const float d1 = __fmul_rn(f[e + 1], scale);
+            float r0;
+            float r1;
+            if (BF16) {
+                r0 = FloatRoundedToBf16(d0);
+                r1 = FloatRoundedToBf16(d1);
+            } else if (!EXACT) {
+                FloatPairRoundedToHalf(d0, d1, &r0, &r1);
+            } else {
+                r0 = __half2float(__ushort_as_half(static_cast<unsigned short>(FloatToHalfRneSat(d0))));
+                r1 = __half2float(__ushort_as_half(static_cast<unsigned short>(FloatToHalfRneSat(d1))));
+            }
+            acc[4 * d + e] = __fadd_rn(acc[4 * d + e], __fmul_rn(r0, w));
+            acc[4 * d + e + 1] = __fadd_rn(acc[4 * d + e + 1], __fmul_rn(r1, w));
+        }
+    }
+}
+
 constexpr int kFlagsNone = 0;
 constexpr int kFlagsMayWait = 1;
 constexpr int kFlagsSettled = 2;
@@ -74,9 +119,6 @@ __global__ __launch_bounds__(kThreads, V == 1 ? (KB > 4 ? 5 : (FL == kFlagsMayWa
         const uint32_t tileWord = checkWords ? SettledWordLoad(a, myRow) : 0u;
         const uint64_t live = __ballot(myRow >= 0);
 
-        // A row's largest magnitude is 128 (448) times its scale: below this scale none reaches the 65520 from which
-        // rounding to fp16 has to saturate.
-        constexpr float kScaleSaturates = INQ == TILEXR_EP_QUANT_TOKEN_INT8 ? 511.875f : 146.25f;
         bool saturates = false;
         float acc[V][16];
         // The K loop.  fp8 rows are decoded by the hardware convert alone, which differs from the reference decode in
@@ -141,7 +183,7 @@ __global__ __launch_bounds__(kThreads, V == 1 ? (KB > 4 ? 5 : (FL == kFlagsMayWa
 #pragma unroll
                     for (int j = 0; j < V; ++j) {
                         if (!BF16 && !kExactDecode) {
-                            saturates |= !(fabsf(sc[u][j]) < kScaleSaturates);
+                            saturates |= !(fabsf(sc[u][j]) < kScaleSaturates<INQ>);
                         }
 #pragma unroll
                         for (int d = 0; d < 4; ++d) {
@@ -264,6 +306,131 @@ __global__ __launch_bounds__(kThreads, V == 1 ? (KB > 4 ? 5 : (FL == kFlagsMayWa
 }
 
 
+// Tokens of one or two slots, launches without flags (QuantTakesFew).  A wave of the kernel above has one row or two in flight then and is
+// done with them before its look-up, its rows and its stores, one after the other, have cost it three trips to memory: the
+// waves a compute unit holds are too few for that.  Here a wave takes a slice of 64 vectors of ROWS / SLOTS neighbouring
+// tokens: their look-ups together, their ROWS rows together, then token by token the sum and the store.
+constexpr int kQuantFewRows = 4;
+
+template <int SLOTS, int INQ, bool BF16>
+__global__ __launch_bounds__(kThreads) void ep_reduce_quant_few_kernel(ReduceArgs a)
+{
+    constexpr int ROWS = kQuantFewRows;
+    constexpr int kTokens = ROWS / SLOTS;
+    constexpr bool perRow = INQ == TILEXR_EP_QUANT_TOKEN_INT8;
+    const int lane = threadIdx.x % kWave;
+    const int vecs = a.h / 16;
+    const int b128 = (a.h + 127) / 128;
+    const int unit = static_cast<int>(blockIdx.x) * kWavesPerBlock + static_cast<int>(threadIdx.x) / kWave;
+    const int group = unit / a.colSlices;
+    const int idx = (unit - group * a.colSlices) * kWave + lane;
+    const int firstToken = __builtin_amdgcn_readfirstlane(group * kTokens);
+
+    // lane l < ROWS: slot l % SLOTS of token firstToken + l / SLOTS
+    int myRow = -1;
+    float myWeight = 1.0f;
+    bool myActive = false;
+    const int myToken = firstToken + lane / SLOTS;
+    if (lane < ROWS && myToken < a.bs) {
+        const int64_t route = static_cast<int64_t>(firstToken) * SLOTS + lane;
+        if (a.expertScales != nullptr) {
+            myWeight = a.expertScales[route];
+        }
+        myActive = a.tokenMask == nullptr || a.tokenMask[myToken] != 0;
+        myRow = LookupRow(a, route);
+        myRow = myActive ? myRow : -1;
+    }
+    const uint64_t active = __ballot(myActive);
+    u32x4 q[ROWS];
+    float sc[ROWS];
+#pragma unroll
+    for (int u = 0; u < ROWS; ++u) {
+        const int row = __builtin_amdgcn_readlane(myRow, u);
+        const int64_t rowAt = row < 0 ? 0 : row;
+        // an absent row gets resources of zero bytes (as above)
+        const __amdgpu_buffer_rsrc_t rsrc = RowResource(static_cast<const char *>(a.expertOut) + rowAt * a.rowBytes, row < 0 ? 0 : vecs * 16);
+        const __amdgpu_buffer_rsrc_t scales = RowResource(a.inScales + (perRow ? rowAt : rowAt * b128), row < 0 ? 0 : (perRow ? 4 : b128 * 4));
+        q[u] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, idx * 16, 0, kAuxNonTemporal);
+        sc[u] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(scales, perRow ? 0 : (idx >> 3) * 4, 0, 0));
+    }
+#pragma unroll
+    for (int t = 0; t < kTokens; ++t) {
+        const int token = firstToken + t;
+        if (token >= a.bs) {
+            return;
+        }
+        float acc[16];
+        auto accumulate = [&](auto exact) {
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                acc[e] = 0.0f;
+            }
+#pragma unroll
+            for (int s = 0; s < SLOTS; ++s) {
+                const int u = t * SLOTS + s;
+                if (__builtin_amdgcn_readlane(myRow, u) >= 0) {
+                    AddQuantRow<INQ, BF16, decltype(exact)::value>(q[u], sc[u], __int_as_float(__builtin_amdgcn_readlane(__float_as_int(myWeight), u)), acc);
+                }
+            }
+        };
+        accumulate(std::false_type {});
+        if (INQ == TILEXR_EP_QUANT_FP8_BLOCK128 || !BF16) {
+            bool again = false;
+#pragma unroll
+            for (int s = 0; s < SLOTS; ++s) {
+                again |= !BF16 && !(fabsf(sc[t * SLOTS + s]) < kScaleSaturates<INQ>);
+            }
+            if (INQ == TILEXR_EP_QUANT_FP8_BLOCK128) {
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    again |= acc[e] != acc[e];
+                }
+            }
+            if (__any(again ? 1 : 0)) {
+                accumulate(std::true_type {});
+            }
+        }
+        if (idx >= vecs) {
+            continue;
+        }
+        if (a.sharedExpertX != nullptr && ((active >> (t * SLOTS)) & 1ull) != 0ull) {
+            const u32x4 *sx = reinterpret_cast<const u32x4 *>(static_cast<const char *>(a.sharedExpertX) + static_cast<int64_t>(token) * a.h * 2);
+#pragma unroll
+            for (int half = 0; half < 2; ++half) {
+                const u32x4 v = sx[idx * 2 + half];
+#pragma unroll
+                for (int q2 = 0; q2 < 4; ++q2) {
+                    acc[half * 8 + 2 * q2] = __fadd_rn(acc[half * 8 + 2 * q2], Decode16<BF16>(v[q2] & 0xffffu));
+                    acc[half * 8 + 2 * q2 + 1] = __fadd_rn(acc[half * 8 + 2 * q2 + 1], Decode16<BF16>(v[q2] >> 16));
+                }
+            }
+        }
+        // (a token without active rows has sums of zero)
+        u32x4 *dst = reinterpret_cast<u32x4 *>(static_cast<char *>(a.y) + static_cast<int64_t>(token) * a.h * 2);
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+            u32x4 o;
+#pragma unroll
+            for (int q2 = 0; q2 < 4; ++q2) {
+                o[q2] = EncodePair16Sat<BF16>(acc[half * 8 + 2 * q2], acc[half * 8 + 2 * q2 + 1]);
+            }
+            dst[idx * 2 + half] = o;
+        }
+    }
+}
+
+template <int SLOTS, bool BF16>
+void LaunchQuantFew(const ReduceLaunch &l, const ReduceArgs &a)
+{
+    constexpr int kTokens = kQuantFewRows / SLOTS;
+    const dim3 g(static_cast<unsigned>(((a.bs + kTokens - 1) / kTokens * a.colSlices + kWavesPerBlock - 1) / kWavesPerBlock));
+    if (l.inQuant == TILEXR_EP_QUANT_TOKEN_INT8) {
+        hipLaunchKernelGGL((ep_reduce_quant_few_kernel<SLOTS, TILEXR_EP_QUANT_TOKEN_INT8, BF16>), g, dim3(kThreads), 0, l.stream, a);
+    } else {
+        hipLaunchKernelGGL((ep_reduce_quant_few_kernel<SLOTS, TILEXR_EP_QUANT_FP8_BLOCK128, BF16>), g, dim3(kThreads), 0, l.stream, a);
+    }
+}
+
 template <int G, int V, bool BF16, int FL, int KB>
 void LaunchQuantRows(const ReduceLaunch &l, const ReduceArgs &a, int gridLimit)
 {
@@ -299,6 +466,12 @@ void TILEXR_REDUCE_ENTRY(int g, int v, const ReduceLaunch &l, const ReduceArgs &
 {
     constexpr bool kBf16 = TILEXR_REDUCE_BF16;
     constexpr int kFlags = TILEXR_REDUCE_FLAGS;
+    if constexpr (kFlags == kFlagsNone) {
+        if (v == kQuantFewSlots) {
+            a.slots == 1 ? LaunchQuantFew<1, kBf16>(l, a) : LaunchQuantFew<2, kBf16>(l, a);
+            return;
+        }
+    }
     if (g == kWave && v == 1) {
         LaunchQuant<kWave, 1, kBf16, kFlags>(l, a, gridLimit);
     } else if (g == 2 * kWave && v == 1) {
