@@ -140,7 +140,8 @@ int RunDispatchSingle(EpComm *comm, const EpDispatchParams &p, bool memoryRoute,
     const bool mayOneLaunch = comm->routing != EpComm::Routing::kLegacy;
     const bool oneLaunchRows = mayOneLaunch && memoryRoute &&
         RouteRowsFits(p.expertIds, n, numKeys, maskMode, p.expertCapacity) &&
-        (comm->routing == EpComm::Routing::kOneLaunch || RouteRowsPays(n, numKeys, rowsAhead, warm, maskMode == kMaskNone ? 0 : p.bs, p.expertCapacity));
+        (comm->routing == EpComm::Routing::kOneLaunch || (RouteRowsPays(n, numKeys, rowsAhead, warm) &&
+            (maskMode == kMaskNone || p.bs <= kRowsMaskedTokens) && RouteRowsLimitPays(n, numKeys, p.expertCapacity)));
     const bool oneLaunchCompact = mayOneLaunch && !memoryRoute && p.expertCapacity <= 0 &&
         RouteCompactFits(p.expertIds, n, experts, maskMode) &&
         (comm->routing == EpComm::Routing::kOneLaunch || RouteCompactPays(n, experts));

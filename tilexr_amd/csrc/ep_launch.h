@@ -95,8 +95,9 @@ struct RouteRowsLaunch {
     int64_t capacity;            // rows an expert keeps, 0 = all
     hipStream_t stream;
 };
-// maskedTokens: tokens of the prefix mask, 0 without one
-bool RouteRowsPays(int64_t routes, int64_t numKeys, bool rowsAhead, bool readsRowsAhead, int64_t maskedTokens, int64_t capacity);
+bool RouteRowsPays(int64_t routes, int64_t numKeys, bool rowsAhead, bool readsRowsAhead);
+constexpr int64_t kRowsMaskedTokens = 8192;     // largest call whose prefix mask the launch adds up where it is free not to
+bool RouteRowsLimitPays(int64_t routes, int64_t numKeys, int64_t capacity);
 bool RouteRowsFits(const int32_t *ids, int64_t routes, int64_t numKeys, int maskMode, int64_t capacity);
 hipError_t LaunchRouteRows(const RouteRowsLaunch &l);
 

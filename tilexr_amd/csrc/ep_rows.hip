@@ -22,7 +22,7 @@
 //
 // A token-prefix mask makes the table shorter: every workgroup adds the mask up first, one more round trip.  A capacity
 // limit makes "valid ids below k" the sum of the smaller keys' counts, each cut at the limit, so those are counted in an
-// LDS histogram after all (RouteRowsPays: tables where that is cheaper than the hand-over); routes beyond a key's limit
+// LDS histogram after all (RouteRowsLimitPays: tables where that is cheaper than the hand-over); routes beyond a key's limit
 // get row -1 from the workgroup that ranks them.
 //
 // Same definitions as the count + place pair (reference: src/ep/kernels/tilexr_ep_dispatch_memory_kernel.h:791-818
@@ -486,16 +486,8 @@ bool RouteRowsFits(const int32_t *ids, int64_t routes, int64_t numKeys, int mask
 //     32 768 routes                  1-4 us faster up to 512 experts
 //     65 536 routes                  1-4 us faster up to 64 experts, level up to 256, slower beyond
 //     131 072 routes and more        slower from 64 experts on (3-14 us at 128-256 experts, 200 us at 262 144 x 1024)
-// Token-prefix masks, count and one launch: 400 x 2048 x top-8 of 64 20.0 -> 16.3 us, 1024 x 2048 of 256 24.2 -> 20.3, 2048 x
-// 2048 34.6 -> 30.5, 8192 x 2048 x top-4 of 64 65.5 -> 60.0; up to 8192 tokens (the mask is added up eight bytes a lane).
-// Capacity limits, whose histogram grows with the routes: 518 x 2048 x top-8 of 64 18.4 -> 14.2, with flags (no place launch)
-// 22.1 -> 17.2; 1729 x top-5 of 128 24.3 -> 20.8; 16 384 routes of 64 33.1 -> 30.0, of 512 35.0 -> 33.1, block fp8 23.0 and 22.9;
-// 32 768 routes of 128 55.1 and 54.9, block fp8 29.7 and 31.3, of 512 56.4 and 58.4; 65 536 routes 102.4 and 104.0, 53.2 and 58.0.
-bool RouteRowsPays(int64_t routes, int64_t numKeys, bool rowsAhead, bool readsRowsAhead, int64_t maskedTokens, int64_t capacity)
+bool RouteRowsPays(int64_t routes, int64_t numKeys, bool rowsAhead, bool readsRowsAhead)
 {
-    if (maskedTokens > 8192 || (capacity > 0 && (routes > 16384 || numKeys > 512))) {
-        return false;
-    }
     if (routes <= 16384) {
         return rowsAhead || numKeys <= 1024;
     }
@@ -503,6 +495,17 @@ bool RouteRowsPays(int64_t routes, int64_t numKeys, bool rowsAhead, bool readsRo
         return rowsAhead && routes <= 32768 && numKeys <= 256;
     }
     return routes <= 32768 ? numKeys <= 512 : (routes <= 65536 && numKeys <= 64);
+}
+
+// ... and of a call whose routes are limited, where the other would be.  Token-prefix masks, count and one launch: 400 x 2048 x
+// top-8 of 64 20.0 -> 16.3 us, 1024 x 2048 of 256 24.2 -> 20.3, 2048 x 2048 34.6 -> 30.5, 8192 x 2048 x top-4 of 64 65.5 -> 60.0;
+// up to kRowsMaskedTokens (the mask is added up eight bytes a lane).
+// Capacity limits, whose histogram grows with the routes: 518 x 2048 x top-8 of 64 18.4 -> 14.2, with flags (no place launch)
+// 22.1 -> 17.2; 1729 x top-5 of 128 24.3 -> 20.8; 16 384 routes of 64 33.1 -> 30.0, of 512 35.0 -> 33.1, block fp8 23.0 and 22.9;
+// 32 768 routes of 128 55.1 and 54.9, block fp8 29.7 and 31.3, of 512 56.4 and 58.4; 65 536 routes 102.4 and 104.0, 53.2 and 58.0.
+bool RouteRowsLimitPays(int64_t routes, int64_t numKeys, int64_t capacity)
+{
+    return capacity <= 0 || (routes <= 16384 && numKeys <= 512);
 }
 
 hipError_t LaunchRouteRows(const RouteRowsLaunch &l)

@@ -243,7 +243,8 @@ int SendRoutes(EpComm *comm, const EpDispatchParams &p, bool memoryRoute, const 
     const bool warm = ScatterCopiesPerRoute(p.x, myRows, p.bs, p.h, plan.perToken, static_cast<int>(p.quantMode));
     const bool oneLaunch = memoryRoute && shared == 0 && comm->routing != EpComm::Routing::kLegacy &&
         RouteRowsFits(routeIds, n, plan.numKeys, maskMode, 0) &&
-        (comm->routing == EpComm::Routing::kOneLaunch || RouteRowsPays(n, plan.numKeys, false, warm, maskMode == kMaskNone ? 0 : p.bs, 0));
+        (comm->routing == EpComm::Routing::kOneLaunch || (RouteRowsPays(n, plan.numKeys, false, warm) &&
+            (maskMode == kMaskNone || p.bs <= kRowsMaskedTokens)));
     int ret = kOk;
     RoutePlaceLaunch place {};
     if (oneLaunch) {
