@@ -998,11 +998,32 @@ __device__ __forceinline__ void DoExtra(const DispatchWorld &a, const ScatterExt
 
 // Has the arguments asked for together, ahead of the first branch that needs one of them: a copying workgroup lives for some
 // microseconds, and each further wait for a scalar load is a part of that (saved plan, 4096 x 7168 x top-8: 78.2 us with the
-// plan's rows, the rank count and the `direct` table asked for behind the branch, 72.2 so).
+// plan's rows, the rank count and the `direct` table asked for behind the branch, 72.2 so).  Addresses go through as integers
+// and are pointers again behind it (Global): what a pointer that comes out of an asm points to is not known, and an access
+// through it is a flat one, by lanes, that is waited for with everything else.
 template <typename... T>
 __device__ __forceinline__ void AskedTogether(T &...v)
 {
     (void)std::initializer_list<int>{([&v] { asm volatile("" : "+s"(v)); }(), 0)...};
+}
+
+template <typename T>
+__device__ __forceinline__ T *Global(uintptr_t address)
+{
+    return (T *)(__attribute__((address_space(1))) T *)address;
+}
+
+// A value at an address that is the same for the whole workgroup, of memory that this launch does not write: through the scalar
+// unit (the compiler finds the address uniform but sees the stores of DoExtra ahead of the load), or by every lane.
+template <bool SCALAR, typename T>
+__device__ __forceinline__ T UniformLoad(uintptr_t address, int64_t index)
+{
+    if (SCALAR) {
+        return ((const __attribute__((address_space(4))) T *)address)[index];
+    }
+    int zero = 0;
+    asm volatile("" : "+v"(zero));
+    return Global<const T>(address)[index + zero];
 }
 
 // Whether the source's own workgroups copy the row of this route: every route's of a fresh plan; what moon_agree_kernel
@@ -1015,21 +1036,29 @@ __device__ __forceinline__ bool SourceCopies(const Route &r, uint8_t direct)
 
 // One workgroup per (token, route, slice of 512 vectors) of source rank blockIdx.y.  What the routes record was written
 // ahead, by moon_records_kernel or moon_agree_kernel.
-template <bool FRESH>
+//
+// SCALAR: the route word is taken apart by the scalar unit while the row is on its way, and with several ranks the receive
+// tensor's address is there too before the row is (by lanes it is a further trip behind the row's).  Four stages, us, by lanes
+// and so: two ranks x 2048 x 7168 x top-8 491 and 482, four x 1024 x 7168 591 and 575, one 3600 x 8192 x top-8 402 and 395, 5000 x
+// 8192 x top-5 378 and 374, 5800 x 4096 x top-8 321 and 317; but where one rank's rows end within a slice 4096 x 7168 382 and
+// 386, 4000 x 7168 x top-7 334 and 337, 4096 x 6144 341 and 346, 4096 x 5120 280 and 280: those keep the word by lanes.
+template <bool FRESH, bool SCALAR>
 __global__ __launch_bounds__(kThreads) void moon_scatter_kernel(DispatchWorld a, int colSlices, ScatterExtras extras)
 {
     const int src = blockIdx.y;
-    const int32_t *words = a.dst[src];
-    const char *rows = static_cast<const char *>(a.hiddenSh[src]);
-    char *firstOut = static_cast<char *>(a.hiddenNvsh[0]);
-    const uint8_t *directs = a.tables.direct + static_cast<int64_t>(src) * a.tables.stride;
+    uintptr_t wordsAt = reinterpret_cast<uintptr_t>(a.dst[src]);
+    uintptr_t rowsAt = reinterpret_cast<uintptr_t>(a.hiddenSh[src]);
+    uintptr_t firstOutAt = reinterpret_cast<uintptr_t>(a.hiddenNvsh[0]);
+    uintptr_t directsAt = reinterpret_cast<uintptr_t>(a.tables.direct + static_cast<int64_t>(src) * a.tables.stride);
     int64_t rowBytes = a.h * 2;
     int64_t nvS = a.nvS;
     int world = a.world;
-    AskedTogether(words, rows, firstOut, rowBytes, nvS, world);
+    AskedTogether(wordsAt, rowsAt, firstOutAt, rowBytes, nvS, world);
     if (!FRESH) {
-        AskedTogether(directs);
+        AskedTogether(directsAt);
     }
+    const char *rows = Global<const char>(rowsAt);
+    char *firstOut = Global<char>(firstOutAt);
     const unsigned block = blockIdx.x - (FRESH ? extras.planBlocks : 0u);
     const unsigned j = block / kXcds;
     const unsigned K = static_cast<unsigned>(a.k);
@@ -1045,8 +1074,9 @@ __global__ __launch_bounds__(kThreads) void moon_scatter_kernel(DispatchWorld a,
     const int vecs = static_cast<int>(rowBytes / 16);
     const int colBase = static_cast<int>(slice) * (kRowVecs * kThreads);
     const int64_t route = token * K + k;
-    const int32_t encoded = words[route];
-    const uint8_t direct = FRESH ? 0 : directs[route];
+    const int32_t encoded = UniformLoad<SCALAR, int32_t>(wordsAt, route);
+    // (a byte, out of the four that a scalar load takes; a rank's share of the table is a multiple of them)
+    const uint32_t directWord = FRESH ? 0u : UniformLoad<SCALAR, uint32_t>(directsAt, route / 4);
     const u32x4 *srcRow = reinterpret_cast<const u32x4 *>(rows + token * rowBytes);
     u32x4 v[kRowVecs];
 #pragma unroll
@@ -1055,8 +1085,8 @@ __global__ __launch_bounds__(kThreads) void moon_scatter_kernel(DispatchWorld a,
         v[i] = idx < vecs ? srcRow[idx] : u32x4{0u, 0u, 0u, 0u};
     }
     const Route r = Decode(encoded, nvS, world);
-    if (SourceCopies<FRESH>(r, direct)) {
-        char *out = world == 1 ? firstOut : static_cast<char *>(a.hiddenNvsh[r.peer]);
+    if (SourceCopies<FRESH>(r, static_cast<uint8_t>(directWord >> (route % 4 * 8)))) {
+        char *out = !SCALAR || world == 1 ? firstOut : static_cast<char *>(a.hiddenNvsh[r.peer]);
         u32x4 *dstRow = reinterpret_cast<u32x4 *>(out + r.row * rowBytes);
 #pragma unroll
         for (int i = 0; i < kRowVecs; ++i) {
@@ -1086,17 +1116,21 @@ __global__ __launch_bounds__(kThreads) void moon_scatter_token_kernel(DispatchWo
 {
     constexpr int kTokens = kThreads / G;
     const int src = blockIdx.y;
-    const int32_t *words = a.dst[src];
-    const char *rows = static_cast<const char *>(a.hiddenSh[src]);
-    char *firstOut = static_cast<char *>(a.hiddenNvsh[0]);
-    const uint8_t *directs = a.tables.direct + static_cast<int64_t>(src) * a.tables.stride;
+    uintptr_t wordsAt = reinterpret_cast<uintptr_t>(a.dst[src]);
+    uintptr_t rowsAt = reinterpret_cast<uintptr_t>(a.hiddenSh[src]);
+    uintptr_t firstOutAt = reinterpret_cast<uintptr_t>(a.hiddenNvsh[0]);
+    uintptr_t directsAt = reinterpret_cast<uintptr_t>(a.tables.direct + static_cast<int64_t>(src) * a.tables.stride);
     int64_t rowBytes = a.h * 2;
     int64_t nvS = a.nvS;
     int world = a.world;
-    AskedTogether(words, rows, firstOut, rowBytes, nvS, world);
+    AskedTogether(wordsAt, rowsAt, firstOutAt, rowBytes, nvS, world);
     if (!FRESH) {
-        AskedTogether(directs);
+        AskedTogether(directsAt);
     }
+    const int32_t *words = Global<const int32_t>(wordsAt);
+    const char *rows = Global<const char>(rowsAt);
+    char *firstOut = Global<char>(firstOutAt);
+    const uint8_t *directs = Global<const uint8_t>(directsAt);
     const unsigned block = blockIdx.x - (FRESH ? extras.planBlocks : 0u);
     const unsigned j = block / kXcds;
     const int slice = static_cast<int>(j % static_cast<unsigned>(colSlices));
@@ -1648,10 +1682,12 @@ hipError_t LaunchMoonDispatch(const DispatchWorld &w, hipStream_t stream, const 
         const unsigned capLds = vecs > kThreads ? TileXREp::CapLdsBytes(kScatterCapWorkgroups) : 0u;
         extras.copyBlocks = static_cast<unsigned>(blocks);
         const dim3 grid(extras.planBlocks + extras.copyBlocks + finishBlocks, R);
+        const bool scalar = w.world > 1 || vecs % (kRowVecs * kThreads) == 0;
+        auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kThreads), capLds, stream, w, colSlices, extras); };
         if (w.fresh) {
-            hipLaunchKernelGGL(moon_scatter_kernel<true>, grid, dim3(kThreads), capLds, stream, w, colSlices, extras);
+            scalar ? launch(moon_scatter_kernel<true, true>) : launch(moon_scatter_kernel<true, false>);
         } else {
-            hipLaunchKernelGGL(moon_scatter_kernel<false>, grid, dim3(kThreads), capLds, stream, w, colSlices, extras);
+            scalar ? launch(moon_scatter_kernel<false, true>) : launch(moon_scatter_kernel<false, false>);
         }
     } else {
         gScatterName = "moon_scatter_generic_kernel";
