@@ -1,0 +1,41 @@
+"""Launches of the plan-driven Dispatch by the sizes of a call: tests/cxx/plan_launches_check.cpp runs the library's own host side
+against a runtime that only notes them."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(ROOT, "tilexr_amd", "csrc")
+pytestmark = pytest.mark.skipif(shutil.which("hipcc") is None, reason="no compiler")
+
+
+@pytest.fixture(scope="module")
+def launches(tmp_path_factory):
+    tmp = tmp_path_factory.mktemp("plan_launches")
+    include = ["-I", os.path.join(ROOT, "include"), "-I", CSRC, "-I", os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include")]
+    subprocess.run(["hipcc", "-std=c++17", "-O1", "--offload-arch=gfx950", "--cuda-host-only", "-fPIC", *include, "-c",
+                    os.path.join(CSRC, "moonep_stage.hip"), "-o", str(tmp / "stage.o")], check=True, capture_output=True)
+    # (the kernels' code object is the one symbol that is left out)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__", *include,
+                    os.path.join(ROOT, "tests", "cxx", "plan_launches_check.cpp"), str(tmp / "stage.o"),
+                    "-Wl,--unresolved-symbols=ignore-all", "-o", str(tmp / "check")], check=True)
+
+    def run(ranks, tokens, k, h, rows, fresh):
+        out = subprocess.run([str(tmp / "check"), *(str(int(v)) for v in (ranks, tokens, k, h, rows, fresh))], check=True,
+                             capture_output=True, text=True, timeout=60).stdout
+        return [(name, int(x), int(y)) for name, x, y in (line.split() for line in out.splitlines())]
+
+    return run
+
+
+@pytest.mark.parametrize("fresh", [True, False])
+@pytest.mark.parametrize("ranks,tokens,k,h,rows", [
+    (2, 512, 8, 2048, 512 * 8 + 1), (4, 509, 8, 2048, 4200), (3, 100, 3, 1000, 321), (2, 2048, 8, 7168, 2048 * 8 + 70), (16, 9, 1, 64, 65)])
+def test_every_rank_copies_on_the_xcds_of_its_tokens(launches, ranks, tokens, k, h, rows, fresh):
+    """Workgroup b runs on XCD b % 8 counting through all ranks' shares of a launch: a share is a multiple of eight."""
+    copies = [(name, x, y) for name, x, y in launches(ranks, tokens, k, h, rows, fresh) if "moon_scatter" in name]
+    assert len(copies) == 1
+    name, x, y = copies[0]
+    assert "generic" not in name and y == ranks and x % 8 == 0

@@ -962,8 +962,8 @@ __device__ __forceinline__ void PlanChunk(const DispatchWorld &a, int rank, int 
 // ---------------------------------------------------------------------------------------------------------------
 
 // What a scatter launch does besides its copies.  A rank's first workgroups build the plan of a fresh Dispatch
-// (PlanChunk); they are a multiple of eight, so that the copies keep their XCDs.  The last ones fill the rows nobody copies
-// to (FinishRows); looking for such rows is a trip to memory, which at the front of the launch would hold the copies up.
+// (PlanChunk).  The last ones fill the rows nobody copies to (FinishRows); looking for such rows is a trip to memory, which at
+// the front of the launch would hold the copies up.  Both are a multiple of eight, so that every rank's copies keep their XCDs.
 struct ScatterExtras {
     unsigned planBlocks;
     int planChunks;
@@ -1608,7 +1608,8 @@ hipError_t LaunchMoonDispatch(const DispatchWorld &w, hipStream_t stream, const 
     ScatterExtras extras {};
     extras.planChunks = planChunks;
     extras.planBlocks = w.fresh && allInScatter ? static_cast<unsigned>((planChunks + kXcds - 1) / kXcds * kXcds) : 0u;
-    const unsigned finishBlocks = allInScatter ? static_cast<unsigned>((w.nvS + kFinishRows - 1) / kFinishRows) : 0u;
+    // (a multiple of eight, as the others are: the next rank's share of the launch begins on the XCD that its tokens count from)
+    const unsigned finishBlocks = allInScatter ? static_cast<unsigned>((w.nvS + kFinishRows - 1) / kFinishRows + kXcds - 1) / kXcds * kXcds : 0u;
     if (w.fresh && recordsAhead) {
         hipLaunchKernelGGL(moon_records_kernel, dim3(routeBlocks + warmBlocks, R), dim3(kThreads), 0, stream, w, routeBlocks,
             warm ? rowVecs : int64_t{0});
