@@ -19,6 +19,8 @@ CASES = [
     (2, 64, 8, 1032, 1),        # 513, two ranks: the last plan to be built writes both statuses
     (3, 40, 9, 64, 600),        # nine routes per token, read eight at a time; most rows unnamed
     (4, 30, 32, 64, 3),
+    (1, 100, 3, 520, 1748),     # 2048 rows, runs of 16 of them to a wave; most unnamed, in pieces of one pass and more
+    (2, 100, 3, 520, 1749),     # 2049
     (1, 8192, 8, 8, 7),         # 257 workgroups: a thread looks at two totals
     (1, 65536, 8, 8, 0),        # 2048 workgroups: the most
     (1, 65536, 8, 8, 1),        # one more: launches behind the copies

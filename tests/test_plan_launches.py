@@ -39,3 +39,10 @@ def test_every_rank_copies_on_the_xcds_of_its_tokens(launches, ranks, tokens, k,
     assert len(copies) == 1
     name, x, y = copies[0]
     assert "generic" not in name and y == ranks and x % 8 == 0
+
+
+@pytest.mark.parametrize("tokens,k,rows", [(32, 8, 256), (32, 8, 2048), (32, 8, 2049), (4096, 8, 32768), (4096, 8, 40000)])
+def test_a_workgroup_looks_after_as_many_rows_as_it_has_threads(launches, tokens, k, rows):
+    """The workgroups that look for rows nobody copies to: beside capped copies each is a trip to memory of few at a time."""
+    (_, x, _), = [launch for launch in launches(1, tokens, k, 1000, rows, False) if "moon_scatter" in launch[0]]
+    assert x == (tokens + 31) // 32 * 8 + (rows + 2047) // 2048 * 8

@@ -663,13 +663,8 @@ __global__ __launch_bounds__(kThreads) void moon_group_walk_kernel(DispatchWorld
 // dispatch: rows nobody wrote, device status
 // ---------------------------------------------------------------------------------------------------------------
 
-constexpr int kFinishRows = 64;     // rows one workgroup looks after
-
-struct FinishList {
-    int32_t row[kFinishRows];
-    uint32_t from[kFinishRows];     // 0: zeros; else what to copy, plus one (FinishRows)
-    int count;
-};
+constexpr int kFinishRows = kThreads;   // rows one workgroup looks after, one per thread
+constexpr int kFinishRun = 16;          // ... so many neighbours at a time: their tags are a line of memory
 
 // Own failure first, then the first failed peer walking upwards from this rank (dispatch kernel :559-574).
 __device__ __forceinline__ void WriteDispatchStatus(const DispatchWorld &a, int rank)
@@ -691,103 +686,109 @@ __device__ __forceinline__ void WriteDispatchStatus(const DispatchWorld &a, int 
     a.status[rank][0] = status;
 }
 
-// 64 rows of `rank` that no route's own copy fills.  The first wave of a workgroup looks at them, one per lane: nothing (a
-// route writes the row), zeros (no route writes it: the reference clears the whole window first, dispatch kernel :206-230),
+// Rows of `rank` that no route's own copy fills, workgroup `block` of `blocks`.  A wave looks at 64 rows, one per lane: nothing
+// (a route writes the row), zeros (no route writes it: the reference clears the whole window first, dispatch kernel :206-230),
 // or -- saved plans -- a copy of its primary row (dispatch kernel :426-461); the weight of a row no route names is zero for
-// the same reason.  Then the whole workgroup writes the rows that need writing.
+// the same reason.  Then the wave writes the rows that need writing.  Such rows lie together, at the end of a rank's rows for
+// instance: a workgroup's are 16 runs of neighbours from all over the rank, so that each has about as many to write.  (64
+// neighbours to a workgroup, looked at by its first wave, us a pass before and now: four ranks x 1000 x 7168 x top-4 229 and 210, x
+// 600 x top-2 all four stages 344 and 303, x 3000 x 4096 x top-8 434 and 422; 60000 x 1000 x top-8 498.6 and 488.8, 20000 167.0 and 165.0,
+// 16000 x 2560 x top-6 all four 451.8 and 444.5.)
 //
 // AHEAD: the workgroup belongs to the scatter launch itself, after a launch that left what every route records.  A row is
 // then either a copying workgroup's or this one's (moon_agree_kernel), and a primary row is not read where it is being
 // written: its values are those of the token row its origin names.  A launch of its own for this took 4 us a Dispatch, and
 // the two that built a fresh plan 10; together, us a pass before and now: forward 4096 x 1024 x top-5 50.3 and 41.9,
 // 4096 x 2048 x top-8 76.3 and 68.9, 128 x 4096 x top-4 35 and 31; two ranks x 2048 x 2048 x top-8 137 and 126; all four stages 4096 x
-// 7168 x top-8 398 and 386 (1.5 us of it are arguments asked for together, AskedTogether).
+// 7168 x top-8 400 and 382 (1.5 us of it are arguments asked for together, AskedTogether).
 // Otherwise the rows are copied where they lie, once every source has scattered, and the duplicates of a fresh plan take
 // their places in dupLoffs here.
 template <bool VEC, bool AHEAD>
-__device__ __forceinline__ void FinishRows(const DispatchWorld &a, int rank, int64_t block, FinishList *s)
+__device__ __forceinline__ void FinishRows(const DispatchWorld &a, int rank, int64_t block, int64_t blocks)
 {
     const int tid = threadIdx.x;
     const int64_t base = static_cast<int64_t>(rank) * a.tables.stride;
-    if (tid < kWave) {
-        const int64_t row = block * kFinishRows + tid;
-        bool fill = false;
-        uint32_t from = 0;
-        if (row < a.nvS) {
-            const uint64_t tag = a.tables.rowTag[base + row];
-            const uint64_t p = a.tables.parentTag[base + row];
-            const uint32_t sibling = !AHEAD && a.fresh ? a.tables.sibling[base + row] : 0u;
-            const bool tagged = Tagged(tag, a.epoch);
-            const bool named = tagged && (tag & kRowNamed) != 0;
-            const bool written = tagged && (tag & kRowWritten) != 0;
-            const bool direct = tagged && (tag & kRowDirect) != 0;
-            const int64_t primary = static_cast<int64_t>(p & 0xffffffffu) - 1;
-            if (!a.fresh && Tagged(p, a.epoch) && !direct) {
-                // a primary no route wrote is all zeros in the reference too (the window was cleared)
-                fill = true;
-                const uint64_t ptag = a.tables.rowTag[base + primary];
-                const uint32_t source = AHEAD ? a.tables.origin[base + primary] : static_cast<uint32_t>(primary);
-                from = Tagged(ptag, a.epoch) && (ptag & kRowWritten) != 0 ? source + 1u : 0u;
-            } else if (!written) {
-                fill = true;
-            }
-            if (!named && a.weightsNvs[rank] != nullptr) {
-                a.weightsNvs[rank][row] = 0.0f;
-            }
-            if (!AHEAD && a.fresh && Tagged(p, a.epoch)) {
-                // slot of this duplicate in its group's slice (dispatch kernel :393-419)
-                const uint64_t gs = a.tables.groupStart[base + primary];
-                if (Tagged(gs, a.epoch)) {
-                    const int64_t at = static_cast<int64_t>(gs & 0xffffffffu) + (sibling & 0xffffu);
-                    if (at < a.nvS) {
-                        a.dupLoffs[rank][at] = static_cast<int32_t>(row);
-                    } else {
-                        RecordFailure(a.tables, rank, a.epoch, kDispatchInvalidRoute);
-                    }
+    const int64_t row = (tid / kFinishRun * blocks + block) * kFinishRun + tid % kFinishRun;
+    bool fill = false;
+    uint32_t from = 0;          // 0: zeros; else what to copy, plus one
+    if (row < a.nvS) {
+        const uint64_t tag = a.tables.rowTag[base + row];
+        const uint64_t p = a.tables.parentTag[base + row];
+        const uint32_t sibling = !AHEAD && a.fresh ? a.tables.sibling[base + row] : 0u;
+        const bool tagged = Tagged(tag, a.epoch);
+        const bool named = tagged && (tag & kRowNamed) != 0;
+        const bool written = tagged && (tag & kRowWritten) != 0;
+        const bool direct = tagged && (tag & kRowDirect) != 0;
+        const int64_t primary = static_cast<int64_t>(p & 0xffffffffu) - 1;
+        if (!a.fresh && Tagged(p, a.epoch) && !direct) {
+            // a primary no route wrote is all zeros in the reference too (the window was cleared)
+            fill = true;
+            const uint64_t ptag = a.tables.rowTag[base + primary];
+            const uint32_t source = AHEAD ? a.tables.origin[base + primary] : static_cast<uint32_t>(primary);
+            from = Tagged(ptag, a.epoch) && (ptag & kRowWritten) != 0 ? source + 1u : 0u;
+        } else if (!written) {
+            fill = true;
+        }
+        if (!named && a.weightsNvs[rank] != nullptr) {
+            a.weightsNvs[rank][row] = 0.0f;
+        }
+        if (!AHEAD && a.fresh && Tagged(p, a.epoch)) {
+            // slot of this duplicate in its group's slice (dispatch kernel :393-419)
+            const uint64_t gs = a.tables.groupStart[base + primary];
+            if (Tagged(gs, a.epoch)) {
+                const int64_t at = static_cast<int64_t>(gs & 0xffffffffu) + (sibling & 0xffffu);
+                if (at < a.nvS) {
+                    a.dupLoffs[rank][at] = static_cast<int32_t>(row);
+                } else {
+                    RecordFailure(a.tables, rank, a.epoch, kDispatchInvalidRoute);
                 }
             }
         }
-        const uint64_t have = __ballot(fill);
-        if (fill) {
-            const int at = __popcll(have & ((1ull << tid) - 1ull));
-            s->row[at] = static_cast<int32_t>(row);
-            s->from[at] = from;
-        }
-        if (tid == 0) {
-            s->count = __popcll(have);
-        }
     }
-    TileXREp::LdsBarrier();
-    const int count = s->count;
     const int h = static_cast<int>(a.h);
+    const int lane = tid % kWave;
     char *tensor = static_cast<char *>(a.hiddenNvsh[rank]);
 #pragma unroll 1
-    for (int i = 0; i < count; ++i) {
-        const uint32_t from = s->from[i];
-        char *dst = tensor + static_cast<int64_t>(s->row[i]) * h * 2;
+    for (uint64_t left = __ballot(fill); left != 0; left &= left - 1) {
+        const int at = __builtin_ctzll(left);
+        const uint32_t origin = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(from), at));
+        // (rows are counted in 31 bits)
+        char *dst = tensor + static_cast<int64_t>(__builtin_amdgcn_readlane(static_cast<int>(row), at)) * h * 2;
         const char *src = tensor;
-        if (from != 0 && AHEAD) {
+        if (origin != 0 && AHEAD) {
             const uint32_t n = static_cast<uint32_t>(a.s * a.k);
-            const uint32_t rankOf = (from - 1u) / n;
+            const uint32_t rankOf = (origin - 1u) / n;
             src = static_cast<const char *>(a.hiddenSh[rankOf]) +
-                static_cast<int64_t>((from - 1u - rankOf * n) / static_cast<uint32_t>(a.k)) * h * 2;
-        } else if (from != 0) {
-            src = tensor + static_cast<int64_t>(from - 1u) * h * 2;
+                static_cast<int64_t>((origin - 1u - rankOf * n) / static_cast<uint32_t>(a.k)) * h * 2;
+        } else if (origin != 0) {
+            src = tensor + static_cast<int64_t>(origin - 1u) * h * 2;
         }
         if (VEC) {
             const int vecs = h / 8;
             u32x4 *dstRow = reinterpret_cast<u32x4 *>(dst);
             const u32x4 *srcRow = reinterpret_cast<const u32x4 *>(src);
+            constexpr int kAtOnce = 4;
 #pragma unroll 1
-            for (int idx = tid; idx < vecs; idx += kThreads) {
-                const u32x4 v = from != 0 ? srcRow[idx] : u32x4{0u, 0u, 0u, 0u};
-                __builtin_nontemporal_store(v, dstRow + idx);
+            for (int first = lane; first < vecs; first += kAtOnce * kWave) {
+                u32x4 v[kAtOnce];
+#pragma unroll
+                for (int j = 0; j < kAtOnce; ++j) {
+                    const int idx = first + j * kWave;
+                    v[j] = origin != 0 && idx < vecs ? srcRow[idx] : u32x4{0u, 0u, 0u, 0u};
+                }
+#pragma unroll
+                for (int j = 0; j < kAtOnce; ++j) {
+                    const int idx = first + j * kWave;
+                    if (idx < vecs) {
+                        __builtin_nontemporal_store(v[j], dstRow + idx);
+                    }
+                }
             }
         } else {
             uint16_t *dstRow = reinterpret_cast<uint16_t *>(dst);
             const uint16_t *srcRow = reinterpret_cast<const uint16_t *>(src);
-            for (int c = tid; c < h; c += kThreads) {
-                dstRow[c] = from != 0 ? srcRow[c] : static_cast<uint16_t>(0);
+            for (int c = lane; c < h; c += kWave) {
+                dstRow[c] = origin != 0 ? srcRow[c] : static_cast<uint16_t>(0);
             }
         }
     }
@@ -798,11 +799,10 @@ __device__ __forceinline__ void FinishRows(const DispatchWorld &a, int rank, int
 template <bool VEC>
 __global__ __launch_bounds__(kThreads) void moon_finish_kernel(DispatchWorld a)
 {
-    __shared__ FinishList s_list;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         WriteDispatchStatus(a, blockIdx.y);
     }
-    FinishRows<VEC, false>(a, blockIdx.y, blockIdx.x, &s_list);
+    FinishRows<VEC, false>(a, blockIdx.y, blockIdx.x, gridDim.x);
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -968,6 +968,7 @@ struct ScatterExtras {
     unsigned planBlocks;
     int planChunks;
     unsigned copyBlocks;
+    unsigned finishBlocks;
 };
 
 // A workgroup whose copy block, counted from the end of the plan's workgroups and so wrapped round for those, names no token.
@@ -977,7 +978,6 @@ struct ScatterExtras {
 template <bool FRESH>
 __device__ __forceinline__ void DoExtra(const DispatchWorld &a, const ScatterExtras &x, unsigned block)
 {
-    __shared__ FinishList s_list;
     if constexpr (FRESH) {
         if (blockIdx.x < x.planBlocks) {
             if (static_cast<int>(blockIdx.x) < x.planChunks) {
@@ -993,7 +993,7 @@ __device__ __forceinline__ void DoExtra(const DispatchWorld &a, const ScatterExt
     if (!FRESH && block == x.copyBlocks && threadIdx.x == 0) {
         WriteDispatchStatus(a, blockIdx.y);     // of a saved plan: nothing can fail any more
     }
-    FinishRows<true, true>(a, blockIdx.y, block - x.copyBlocks, &s_list);
+    FinishRows<true, true>(a, blockIdx.y, block - x.copyBlocks, x.finishBlocks);
 }
 
 // Has the arguments asked for together, ahead of the first branch that needs one of them: a copying workgroup lives for some
@@ -1609,7 +1609,7 @@ hipError_t LaunchMoonDispatch(const DispatchWorld &w, hipStream_t stream, const 
     extras.planChunks = planChunks;
     extras.planBlocks = w.fresh && allInScatter ? static_cast<unsigned>((planChunks + kXcds - 1) / kXcds * kXcds) : 0u;
     // (a multiple of eight, as the others are: the next rank's share of the launch begins on the XCD that its tokens count from)
-    const unsigned finishBlocks = allInScatter ? static_cast<unsigned>((w.nvS + kFinishRows - 1) / kFinishRows + kXcds - 1) / kXcds * kXcds : 0u;
+    extras.finishBlocks = allInScatter ? static_cast<unsigned>((w.nvS + kFinishRows - 1) / kFinishRows + kXcds - 1) / kXcds * kXcds : 0u;
     if (w.fresh && recordsAhead) {
         hipLaunchKernelGGL(moon_records_kernel, dim3(routeBlocks + warmBlocks, R), dim3(kThreads), 0, stream, w, routeBlocks,
             warm ? rowVecs : int64_t{0});
@@ -1648,7 +1648,7 @@ hipError_t LaunchMoonDispatch(const DispatchWorld &w, hipStream_t stream, const 
             constexpr int kAux = decltype(stores)::value;
             constexpr int64_t kTokens = kThreads / G * kXcds;       // tokens of eight neighbouring workgroups
             extras.copyBlocks = static_cast<unsigned>((w.s + kTokens - 1) / kTokens * kXcds * tokenSlices);
-            const dim3 grid(extras.planBlocks + extras.copyBlocks + finishBlocks, R);
+            const dim3 grid(extras.planBlocks + extras.copyBlocks + extras.finishBlocks, R);
             if (w.fresh) {
                 hipLaunchKernelGGL((moon_scatter_token_kernel<true, G, V, kAux>), grid, dim3(kThreads), capLds, stream, w, tokenSlices,
                     extras);
@@ -1682,7 +1682,7 @@ hipError_t LaunchMoonDispatch(const DispatchWorld &w, hipStream_t stream, const 
         // 4096 265 and 262, 4096 x 7168 436 and 415; up to 4096 x 2304 no difference beyond the runs' own).
         const unsigned capLds = vecs > kThreads ? TileXREp::CapLdsBytes(kScatterCapWorkgroups) : 0u;
         extras.copyBlocks = static_cast<unsigned>(blocks);
-        const dim3 grid(extras.planBlocks + extras.copyBlocks + finishBlocks, R);
+        const dim3 grid(extras.planBlocks + extras.copyBlocks + extras.finishBlocks, R);
         const bool scalar = w.world > 1 || vecs % (kRowVecs * kThreads) == 0;
         auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kThreads), capLds, stream, w, colSlices, extras); };
         if (w.fresh) {
