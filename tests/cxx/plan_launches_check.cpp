@@ -1,7 +1,7 @@
 // The launches of a plan-driven Dispatch: tilexr_amd/csrc/moonep_stage.hip's host side, linked against a runtime that only
 // notes what is launched.  Built and run by tests/test_plan_launches.py on the CPU.
 //
-//   plan_launches_check <ranks> <tokens> <top-k> <hidden> <rows per rank> <fresh>      a line per launch: kernel, grid x and y
+//   plan_launches_check <ranks> <tokens> <top-k> <hidden> <rows per rank> <fresh>      a line per launch: kernel, grid x and y, dynamic LDS
 #include <cstdio>
 #include <cstdlib>
 #include <map>
@@ -15,6 +15,7 @@ namespace {
 
 std::map<const void *, std::string> gKernels;
 dim3 gGrid, gBlock;
+size_t gLds;
 
 } // namespace
 
@@ -33,8 +34,9 @@ void __hipRegisterFunction(void **, const void *host, char *, const char *name, 
     gKernels[host] = name;
 }
 
-hipError_t __hipPushCallConfiguration(dim3 grid, dim3 block, size_t, hipStream_t)
+hipError_t __hipPushCallConfiguration(dim3 grid, dim3 block, size_t lds, hipStream_t)
 {
+    gLds = lds;
     gGrid = grid;
     gBlock = block;
     return hipSuccess;
@@ -44,14 +46,14 @@ hipError_t __hipPopCallConfiguration(dim3 *grid, dim3 *block, size_t *lds, hipSt
 {
     *grid = gGrid;
     *block = gBlock;
-    *lds = 0;
+    *lds = gLds;
     *stream = nullptr;
     return hipSuccess;
 }
 
-hipError_t hipLaunchKernel(const void *host, dim3 grid, dim3, void **, size_t, hipStream_t)
+hipError_t hipLaunchKernel(const void *host, dim3 grid, dim3, void **, size_t lds, hipStream_t)
 {
-    std::printf("%s %u %u\n", gKernels[host].c_str(), grid.x, grid.y);
+    std::printf("%s %u %u %zu\n", gKernels[host].c_str(), grid.x, grid.y, lds);
     return hipSuccess;
 }
 

@@ -25,7 +25,7 @@ def launches(tmp_path_factory):
     def run(ranks, tokens, k, h, rows, fresh):
         out = subprocess.run([str(tmp / "check"), *(str(int(v)) for v in (ranks, tokens, k, h, rows, fresh))], check=True,
                              capture_output=True, text=True, timeout=60).stdout
-        return [(name, int(x), int(y)) for name, x, y in (line.split() for line in out.splitlines())]
+        return [(name, int(x), int(y), int(lds)) for name, x, y, lds in (line.split() for line in out.splitlines())]
 
     return run
 
@@ -35,14 +35,20 @@ def launches(tmp_path_factory):
     (2, 512, 8, 2048, 512 * 8 + 1), (4, 509, 8, 2048, 4200), (3, 100, 3, 1000, 321), (2, 2048, 8, 7168, 2048 * 8 + 70), (16, 9, 1, 64, 65)])
 def test_every_rank_copies_on_the_xcds_of_its_tokens(launches, ranks, tokens, k, h, rows, fresh):
     """Workgroup b runs on XCD b % 8 counting through all ranks' shares of a launch: a share is a multiple of eight."""
-    copies = [(name, x, y) for name, x, y in launches(ranks, tokens, k, h, rows, fresh) if "moon_scatter" in name]
-    assert len(copies) == 1
-    name, x, y = copies[0]
+    (name, x, y, _), = [launch for launch in launches(ranks, tokens, k, h, rows, fresh) if "moon_scatter" in launch[0]]
     assert "generic" not in name and y == ranks and x % 8 == 0
 
 
 @pytest.mark.parametrize("tokens,k,rows", [(32, 8, 256), (32, 8, 2048), (32, 8, 2049), (4096, 8, 32768), (4096, 8, 40000)])
 def test_a_workgroup_looks_after_as_many_rows_as_it_has_threads(launches, tokens, k, rows):
     """The workgroups that look for rows nobody copies to: beside capped copies each is a trip to memory of few at a time."""
-    (_, x, _), = [launch for launch in launches(1, tokens, k, 1000, rows, False) if "moon_scatter" in launch[0]]
+    (_, x, _, _), = [launch for launch in launches(1, tokens, k, 1000, rows, False) if "moon_scatter" in launch[0]]
     assert x == (tokens + 31) // 32 * 8 + (rows + 2047) // 2048 * 8
+
+
+@pytest.mark.parametrize("tokens,rows,fresh,lds", [
+    (16384, 131072, True, 56 * 1024), (16385, 131080, True, 0), (16385, 131080, False, 56 * 1024), (60000, 480000, True, 0)])
+def test_two_to_a_compute_unit_only_while_they_hold_the_plan(launches, tokens, rows, fresh, lds):
+    """Rows that end within a line: the plan's workgroups, one per 256 rows, are ahead of the copies and under their cap."""
+    (_, _, _, got), = [launch for launch in launches(1, tokens, 8, 1000, rows, fresh) if "moon_scatter" in launch[0]]
+    assert got == lds

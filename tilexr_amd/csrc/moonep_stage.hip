@@ -28,6 +28,7 @@ using TileXREp::kThreads;
 using TileXREp::kWave;
 
 constexpr int kXcds = 8;
+constexpr int kComputeUnits = 256;
 constexpr int kRowVecs = 2;     // 16-byte vectors per lane per row slice
 constexpr int kTokenVecs = 4 * kThreads;    // 16-byte vectors of a row slice of the per-token scatter
 
@@ -1638,10 +1639,16 @@ hipError_t LaunchMoonDispatch(const DispatchWorld &w, hipStream_t stream, const 
         // Two for rows that end within a line, which are not written through; fwd, at eight, four and two: 4000 x 3000 x top-4 72.5,
         // 70.7 and 69.3, 4000 x 2008 x top-2 49.6, 49.9 and 47.3, 2223 x 5000 x top-2 53.0, 51.5 and 49.8, 2223 x 7176 x top-6 121.9,
         // 119.4 and 118.0.
+        // No cap of two where the plan's workgroups are more than such a launch holds at once: they go ahead of the copies, and
+        // it took them in rounds.  Fwd, top-8, two and as many as fit: 17000 x 1000 142.4 and 140.2, 20000 x 504 103.5 and 100.8, 40000
+        // x 1000 323 and 315, 60000 x 1000 488 and 468, 66000 x 520 (launches behind the copies 328) 322 and 301, two ranks x 20000 x
+        // 1000 368 and 366; but with fewer of them 4096 x 1000 51.1 and 53.0.  Four to a unit hold more than they lose: 60000 x 1024
+        // 409.2 and 411.7.
         const int64_t heldVecs = vecs <= 4 * kWave ? vecs * (kThreads / kWave) : vecs;
         const bool wholeLines = vecs % 8 == 0;
         const int capWorkgroups = !wholeLines || (heldVecs > 2 * kThreads && w.k >= 4) ? 2 : 4;
-        const unsigned capLds = worldRowBytes * w.k <= (int64_t{1} << 30) ? TileXREp::CapLdsBytes(capWorkgroups) : 0u;
+        const bool capped = worldRowBytes * w.k <= (int64_t{1} << 30) && (capWorkgroups != 2 || extras.planBlocks <= 2 * kComputeUnits);
+        const unsigned capLds = capped ? TileXREp::CapLdsBytes(capWorkgroups) : 0u;
         auto launch = [&](auto lanes, auto vecsPerLane, auto stores) {
             constexpr int G = decltype(lanes)::value;
             constexpr int V = decltype(vecsPerLane)::value;
