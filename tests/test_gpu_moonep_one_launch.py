@@ -22,8 +22,10 @@ CASES = [
     (1, 100, 3, 520, 1748),     # 2048 rows, runs of 16 of them to a wave; most unnamed, in pieces of one pass and more
     (2, 100, 3, 520, 1749),     # 2049
     (1, 8192, 8, 8, 7),         # 257 workgroups: a thread looks at two totals
-    (1, 65536, 8, 8, 0),        # 2048 workgroups: the most
-    (1, 65536, 8, 8, 1),        # one more: launches behind the copies
+    (1, 65536, 8, 8, 0),        # 2048 workgroups
+    (1, 65536, 8, 8, 1),        # 2049
+    (1, 131072, 8, 8, 0),       # 4096: the most of rows this narrow
+    (1, 131072, 8, 8, 1),       # one more: launches behind the copies
 ]
 
 
@@ -71,3 +73,19 @@ def test_saved_plans_that_disagree_with_the_routes(world, s, k, h, row_cache):  
         res = w.dispatch(sh, plans, hidden, flags=0)
         w.sync()
         check_dispatch(sh, res, plans, want, fresh=False)
+
+
+def test_largest_plan_of_wide_rows():
+    """8192 workgroups: a thread looks at 32 totals.  The plan does not depend on the rows' width, nor do the rows matter here."""
+    s, k, h = 262144, 8, 512
+    dst = MC.random_dst(M.Shape(1, s, k, 8, s * k), np.random.default_rng(s), duplicates=True)
+    want = M.dispatch_world(M.Shape(1, s, k, 8, s * k), dst, np.zeros((1, s, 8), np.uint16), flags=M.FLAG_BUILD_DEDUP)[3]
+    sh = M.Shape(1, s, k, h, s * k)
+    with World(1) as w:
+        plans = w.plan_tensors(sh, dst)
+        w.dispatch(sh, plans, np.zeros((1, s, h), np.uint16), flags=mp.FLAG_BUILD_DEDUP)
+        w.sync()
+        groups, places = (int(c) for c in plans[0]["counts"].cpu())
+        assert [groups, places] == want.counts[0].tolist() and int(plans[0]["status"][0]) == 2000
+        np.testing.assert_array_equal(plans[0]["groups"].cpu().numpy()[:groups], want.groups[0, :groups])
+        np.testing.assert_array_equal(plans[0]["loffs"].cpu().numpy()[:places], want.loffs[0, :places])

@@ -52,3 +52,17 @@ def test_two_to_a_compute_unit_only_while_they_hold_the_plan(launches, tokens, r
     """Rows that end within a line: the plan's workgroups, one per 256 rows, are ahead of the copies and under their cap."""
     (_, _, _, got), = [launch for launch in launches(1, tokens, 8, 1000, rows, fresh) if "moon_scatter" in launch[0]]
     assert got == lds
+
+
+@pytest.mark.parametrize("rows,h,fused", [
+    (64, 8, True), (524288, 64, True), (524289, 1024, True), (1048576, 504, True), (1048577, 504, False), (1048577, 512, True),
+    (2097152, 1024, True), (2097153, 1024, False)])
+@pytest.mark.parametrize("ranks", [1, 4])
+def test_plans_that_the_scatter_launch_builds(launches, ranks, rows, h, fused):
+    """Two launches where the scatter builds a fresh plan, launches of the plan and of the rest behind the copies where not."""
+    names = [name for name, *_ in launches(ranks, rows // 8, 8, h, rows, True)]
+    assert sum("moon_scatter" in name for name in names) == 1
+    if fused:
+        assert len(names) == 2 and "moon_records" in names[0] and "moon_scatter" in names[1]
+    else:
+        assert "moon_dedup_groups" in names[-2] and "moon_finish" in names[-1]

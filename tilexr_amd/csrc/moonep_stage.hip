@@ -38,8 +38,14 @@ std::atomic<int64_t> gCachedRowBytes {kDefaultCachedRowBytes};  // TileXRMoonEpS
 // memory system digests (4096 x 7168 x top-8, four stages, us at eight, seven, six, five, four, three, two: 420, 415, 401, 397,
 // 410, 439, 512; 5800 x 4096, the forward two 170.3, 170.2, 170.1, 169.0, 169.2, 176.7, 200.5).
 constexpr int kScatterCapWorkgroups = 5;
-constexpr int kFusedPlanChunks = 2048;  // chunks of 256 rows per rank up to which the scatter launch builds a fresh plan: each of
-                                        // its workgroups looks at the totals of all chunks before its own
+// Chunks of 256 rows per rank up to which the scatter launch builds a fresh plan.  Each of its workgroups looks at the totals of
+// all chunks before its own, which wide rows' copies hide and narrow ones' do not.  Forward stages, top-8, us, launches
+// behind the copies and one launch: 528 000 rows x 512 277.5 and 263.3, x 520 328 and 301; 786 000 x 64 221 and 213.5, x 256 305.7 and
+// 298.8; 1 048 576 x 64 304 and 300, x 256 397 and 393.5, x 512 510 and 503.5, x 1024 908 and 892; 1 600 000 x 256 608 and 613; 2 097 152 x 256 777 and 793, x
+// 512 1024 and 1019, x 1024 1835 and 1826.
+constexpr int kFusedPlanChunks = 8192;
+constexpr int kFusedNarrowPlanChunks = 4096;
+constexpr int64_t kFusedWideRow = 512;      // elements
 constexpr int64_t kMostCopyBlocks = 0x7fffffff - (1 << 26);     // a rank's share of a grid, less its other workgroups
 constexpr int64_t kWarmRowBytes = int64_t{128} << 20;          // token rows of a world that are read ahead of the per-route scatter
                                                                // (with SetCachedRowBytes at its default there are 104 MiB at most)
@@ -1602,10 +1608,10 @@ hipError_t LaunchMoonDispatch(const DispatchWorld &w, hipStream_t stream, const 
     const unsigned warmBlocks = warm ? static_cast<unsigned>((rowVecs + kThreads * kWarmLoads - 1) / (kThreads * kWarmLoads)) : 0u;
     const unsigned routeBlocks = static_cast<unsigned>((w.s * w.k + kThreads - 1) / kThreads);
     // What the routes record is written ahead of the scatter; the scatter launch then holds everything else a Dispatch does,
-    // two launches for a fresh plan and three for a saved one.  A rank of more than kFusedPlanChunks chunks keeps launches
-    // behind the copies.
+    // two launches for a fresh plan and three for a saved one.  A rank of more than kFusedPlanChunks chunks (narrow rows:
+    // kFusedNarrowPlanChunks) keeps launches behind the copies.
     const int planChunks = static_cast<int>((w.nvS + kPlanRows - 1) / kPlanRows);
-    const bool allInScatter = recordsAhead && (!w.fresh || planChunks <= kFusedPlanChunks);
+    const bool allInScatter = recordsAhead && (!w.fresh || planChunks <= (w.h >= kFusedWideRow ? kFusedPlanChunks : kFusedNarrowPlanChunks));
     ScatterExtras extras {};
     extras.planChunks = planChunks;
     extras.planBlocks = w.fresh && allInScatter ? static_cast<unsigned>((planChunks + kXcds - 1) / kXcds * kXcds) : 0u;
