@@ -49,6 +49,23 @@ def test_built_and_saved_plans(world, s, k, h, slack, row_cache):  # noqa: F811
             check_dispatch(sh, res, plans, want, fresh=flags != 0)
 
 
+@pytest.mark.parametrize("world,s,k,slack", [(1, 51, 5, 0), (2, 64, 8, 1), (3, 100, 9, 600), (1, 8192, 8, 7)])
+def test_a_chunk_whose_totals_do_not_come(world, s, k, slack, row_cache, monkeypatch):  # noqa: F811
+    """No look at another workgroup's word: every thread adds up the chunks before its own from their rows' records, as it would
+    after so many looks."""
+    monkeypatch.setenv("TILEXR_MOONEP_PLAN_POLLS", "0")
+    rng = np.random.default_rng(world + s + k)
+    sh = M.Shape(world, s, k, 64, s * k + slack)
+    dst = MC.random_dst(sh, rng, duplicates=True)
+    hidden = random_rows(rng, (world, s, sh.h))
+    want = M.dispatch_world(sh, dst, hidden, flags=M.FLAG_BUILD_DEDUP)
+    with World(world) as w:
+        plans = w.plan_tensors(sh, dst)
+        res = w.dispatch(sh, plans, hidden, flags=mp.FLAG_BUILD_DEDUP)
+        w.sync()
+        check_dispatch(sh, res, plans, want, fresh=True)
+
+
 @pytest.mark.parametrize("world,s,k,h", [(1, 40, 4, 64), (2, 33, 3, 4104)])
 def test_saved_plans_that_disagree_with_the_routes(world, s, k, h, row_cache):  # noqa: F811
     """A plan is data: it may list a row that a route of its own names, an unnamed row, or another token's row as the primary.

@@ -9,6 +9,7 @@
 // therefore complete once every rank has made the call and the rank's stream has been synchronised.  A world of one
 // rank runs directly on the caller's stream.
 #include <cstddef>
+#include <cstdlib>
 #include <limits>
 #include <mutex>
 #include <vector>
@@ -211,6 +212,9 @@ WorldState *StateOf(EpWorld *world)
 {
     if (world->moon == nullptr) {
         WorldState *st = new WorldState();
+        if (const char *polls = std::getenv("TILEXR_MOONEP_PLAN_POLLS")) {
+            st->totalsPolls = std::atoi(polls);
+        }
         st->dispatch.resize(static_cast<size_t>(world->rankSize));
         st->combine.resize(static_cast<size_t>(world->rankSize));
         st->events.resize(static_cast<size_t>(world->rankSize));
@@ -314,6 +318,7 @@ int LaunchDispatchWorld(EpWorld *world, WorldState *st)
     w.h = shape.h;
     w.nvS = shape.nvS;
     w.fresh = (shape.flags & TILEXR_MOONEP_FLAG_BUILD_DEDUP) != 0;
+    w.totalsPolls = st->totalsPolls;
     for (int r = 0; r < R; ++r) {
         const StageCall &c = calls[static_cast<size_t>(r)];
         w.dst[r] = c.dst;

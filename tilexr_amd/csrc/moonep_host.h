@@ -8,6 +8,7 @@
 #include <hip/hip_runtime_api.h>
 
 #include "ep_context.h"
+#include "moonep_stage.h"
 
 namespace TileXRMoon {
 
@@ -43,6 +44,7 @@ struct WorldState {
     int64_t taggedWords = 0;            // how many of them the tables of the last shape have
     TileXREp::DeviceBuffer plainTables; // the tables of other words
     TileXREp::DeviceBuffer arrived;     // one word at the same place for every shape: it is zero between dispatches
+    int totalsPolls = kTotalsPolls;     // TILEXR_MOONEP_PLAN_POLLS at the world's first call (a switch for tests)
     std::vector<StageCall> dispatch;    // calls waiting for the rest of the world, by rank
     std::vector<StageCall> combine;
     std::vector<RankEvents> events;

@@ -34,6 +34,7 @@ constexpr int kMaxTopK = 32;        // reference: src/moonep/common/moonep_stage
 constexpr int kTableAlign = 256;    // per-rank table strides are a multiple of this many entries
 constexpr int kChunkRows = 2048;    // rows per workgroup of the duplicate-plan build
 constexpr uint8_t kNoRank = 0xff;
+constexpr int kTotalsPolls = 4096;  // looks at a chunk's word of totals before a thread adds the chunk up itself
 
 // Device status values (reference: src/moonep/common/moonep_peer_window.h:36-43).
 constexpr int32_t kDispatchOk = 2000;
@@ -83,6 +84,7 @@ struct DispatchWorld {
     int32_t *dupLoffs[kMaxWorld];              // [nvS]
     int32_t *dupCounts[kMaxWorld];             // [2]
     int32_t *status[kMaxWorld];
+    int totalsPolls;                           // kTotalsPolls, or what a test asks for
 };
 
 // One Combine of every rank of a world.

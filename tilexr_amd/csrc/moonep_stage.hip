@@ -818,7 +818,6 @@ __global__ __launch_bounds__(kThreads) void moon_finish_kernel(DispatchWorld a)
 
 constexpr int kPlanRows = kThreads;     // rows of a plan workgroup, one per thread
 static_assert(kTableAlign == kPlanRows, "a workgroup has a word, and all its rows are in the tables");
-constexpr int kTotalsPolls = 4096;      // looks at a chunk's word before a thread adds the chunk up itself
 constexpr int kWordsAtOnce = 8;
 
 // A chunk's totals in one word, so that whoever finds the word has both: group-opening rows and the sizes of their groups.
@@ -836,7 +835,7 @@ __device__ __forceinline__ uint32_t TotalsOfChunk(const DispatchWorld &a, int ra
 {
     const uint64_t *word = a.tables.chunkTag + (static_cast<int64_t>(rank) * a.tables.stride / kPlanRows + c);
 #pragma unroll 1
-    for (int polls = 0; polls < kTotalsPolls; ++polls) {
+    for (int polls = 0; polls < a.totalsPolls; ++polls) {
         const uint64_t w = __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (Tagged(w, a.epoch)) {
             return static_cast<uint32_t>(w);
@@ -859,8 +858,8 @@ __device__ __forceinline__ uint32_t TotalsOfChunk(const DispatchWorld &a, int ra
 // The duplicate plan of one chunk of 256 rows, by a workgroup of the scatter launch: groups are numbered and their slices
 // start as in DedupGroupsOfChunk, and a thread whose row opens a group fills the group's slice too, so that nothing is left to
 // a launch after the copies.  It needs only what the launch before left, besides the totals of the chunks before its own.
-// Those the workgroups hand one another: they stand at the front of the launch, each waits for workgroups ahead of it
-// alone, and none waits for ever (TotalsOfChunk).
+// Those the workgroups hand one another: they stand at the front of their rank's share of the launch, each waits for
+// workgroups ahead of it alone, and none waits for ever (TotalsOfChunk).
 //
 // The workgroup of a rank's last chunk knows the plan's extent, hence whether it is one; the last of those among the ranks
 // writes every rank's device status.  (One arrival per rank: atomics on one word complete at three per microsecond.)
