@@ -29,18 +29,7 @@ Range RangeOf(T *first, int64_t count)
     return {reinterpret_cast<const char *>(first), reinterpret_cast<const char *>(first + count)};
 }
 
-void NoteTables(int world, const TileXRMoon::WorldTables &t)
-{
-    const int64_t n = world * t.stride;
-    for (uint64_t *words : {t.rowTag, t.parentTag, t.groupStart, t.slotSrc, t.slotDup, t.slotGroup}) {
-        gTagged.push_back(RangeOf(words, n));
-    }
-    gTagged.push_back(RangeOf(t.fail, world));
-    gOther.push_back(RangeOf(t.sibling, n));
-    gOther.push_back(RangeOf(t.slotCount, n));
-    gOther.push_back(RangeOf(t.chunkTotals, world * t.groupStride * 2));
-    gOther.push_back(RangeOf(t.direct, n));
-}
+constexpr size_t kTagged = 8, kOther = 6;     // tables of a call
 
 bool Overlap(const Range &a, const Range &b)
 {
@@ -53,6 +42,25 @@ void Expect(bool ok, const char *what)
         std::printf("FAIL: %s\n", what);
         ++gFailures;
     }
+}
+
+void NoteTables(int world, const TileXRMoon::WorldTables &t)
+{
+    const int64_t n = world * t.stride;
+    for (uint64_t *words : {t.rowTag, t.parentTag, t.groupStart, t.slotSrc, t.slotDup, t.slotGroup}) {
+        gTagged.push_back(RangeOf(words, n));
+    }
+    gTagged.push_back(RangeOf(t.fail, world));
+    gTagged.push_back(RangeOf(t.chunkTag, n / TileXRMoon::kTableAlign));
+    gOther.push_back(RangeOf(t.sibling, n));
+    gOther.push_back(RangeOf(t.slotCount, n));
+    gOther.push_back(RangeOf(t.chunkTotals, world * t.groupStride * 2));
+    gOther.push_back(RangeOf(t.direct, n));
+    gOther.push_back(RangeOf(t.origin, n));
+    // (zero between dispatches, of whatever sizes: neither another table's place nor one that moves with the sizes)
+    gOther.push_back(RangeOf(t.arrived, 1));
+    static const uint32_t *const arrived = t.arrived;
+    Expect(t.arrived == arrived, "the count of built plans is at another place");
 }
 
 TileXRMoonEpTensorV1 Tensor(uint32_t dtype, int64_t rows, int64_t columns)
@@ -202,7 +210,7 @@ int main(int argc, char **argv)
     Exchange(ranks, 16, 8, 128);
     Exchange(ranks, 300, 2, 5000);
     Exchange(ranks, 1, 1, 1);
-    Expect(gTagged.size() == 4 * 3 * 7, "tables of every exchange");
+    Expect(gTagged.size() == 4 * 3 * kTagged, "tables of every exchange");
     bool apart = true;
     for (const Range &t : gTagged) {
         for (const Range &o : gOther) {
@@ -211,9 +219,9 @@ int main(int argc, char **argv)
     }
     Expect(apart, "one size's untagged words lie where another looks for tagged ones");
     // within a call no two tables share a word
-    for (size_t call = 0; call < gTagged.size() / 7; ++call) {
-        std::vector<Range> all(gTagged.begin() + static_cast<long>(call * 7), gTagged.begin() + static_cast<long>(call * 7 + 7));
-        all.insert(all.end(), gOther.begin() + static_cast<long>(call * 4), gOther.begin() + static_cast<long>(call * 4 + 4));
+    for (size_t call = 0; call < gTagged.size() / kTagged; ++call) {
+        std::vector<Range> all(gTagged.begin() + static_cast<long>(call * kTagged), gTagged.begin() + static_cast<long>((call + 1) * kTagged));
+        all.insert(all.end(), gOther.begin() + static_cast<long>(call * kOther), gOther.begin() + static_cast<long>((call + 1) * kOther));
         for (size_t i = 0; i < all.size(); ++i) {
             for (size_t j = 0; j < i; ++j) {
                 Expect(!Overlap(all[i], all[j]), "two tables of a call overlap");

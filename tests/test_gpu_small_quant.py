@@ -1,6 +1,6 @@
 """Decode-sized calls of quantised rows, a dispatch and a combine of one launch each: both sides of the largest table and
-width they take, rows narrower than a workgroup, more experts than routes, masks, readiness flags, MXFP8 exchange with
-and without infinities.  Bit for bit against the oracle."""
+width they take, rows narrower than a workgroup, more experts than routes, masks, readiness flags of every payload, MXFP8
+exchange with and without infinities.  Bit for bit against the oracle."""
 import numpy as np
 import pytest
 import torch
@@ -34,11 +34,11 @@ def test_dispatch(bs, h, k, e, kernel, dtype, quant, fp8, mask_type):
     with Session() as s:
         out = alloc_dispatch_outputs(bs, h, k, e, quant=quant)
         counts = torch.zeros((e,), dtype=torch.int32, device=DEV)
-        flags = torch.zeros(((bs * k + 63) // 64,), dtype=torch.int64, device=DEV) if quant != ep.Q_MXFP8 else None
+        flags = torch.zeros(((bs * k + 63) // 64,), dtype=torch.int64, device=DEV)
         st, epoch = ep.dispatch_memory_ex(
             xt, to_dev(ids), s.comm, bs, h, k, e, out["expand_x"], out["assist"], out["token_nums"], counts, dtype, s.stream,
             quant_mode=quant, dynamic_scales=out["scales"], expand_x_dtype=fp8, row_index_map=out["row_map"],
-            active_mask=to_dev(mask), active_mask_type=mask_type, tile_flags=flags, tile_rows=64 if flags is not None else 0)
+            active_mask=to_dev(mask), active_mask_type=mask_type, tile_flags=flags, tile_rows=64)
         assert st == 0
         s.sync()
         assert ep.last_kernel_name(s.comm, ep.K_SCATTER) == kernel
@@ -48,11 +48,13 @@ def test_dispatch(bs, h, k, e, kernel, dtype, quant, fp8, mask_type):
         n = want["rows"]
         assert np.array_equal(got["send_counts"], want["send_counts"])
         assert np.array_equal(got["scales"][:n], want["dyn_scales"][:n])
-        if flags is not None and h % 16 == 0:
+        tiles = [min(64, n - t) for t in range(0, n, 64)]
+        assert flags.cpu().tolist() == [(epoch << 32) | t for t in tiles] + [0] * (len(flags) - len(tiles))
+        if quant != ep.Q_MXFP8 and h % 16 == 0:
             # every row reported landed: the combine on the same stream finds all words and reads what is there
             w = (0.5 + rng.random((bs, k))).astype(np.float32)
             y = torch.full((bs, h), 7.0, dtype=xt.dtype, device=DEV)
-            status = torch.full((1,), -1, dtype=torch.int32, device=DEV)
+            status = torch.zeros((1,), dtype=torch.int32, device=DEV)
             assert ep.combine_memory_ex(
                 out["expand_x"], out["assist"], counts, s.comm, bs, h, k, e, y, dtype, s.stream, expert_out_quant_mode=quant,
                 expert_out_scales=out["scales"], expert_scales=to_dev(w), row_index_map=out["row_map"], tile_flags=flags,
@@ -60,7 +62,7 @@ def test_dispatch(bs, h, k, e, kernel, dtype, quant, fp8, mask_type):
             s.sync()
             wy = O.mem_combine(O.Case(1, bs, h, k, e, dtype=dtype), 0, want["expand_x"][None], want["assist"][None],
                                want["send_counts"][None], expert_scales=w, in_quant=quant, in_scales=want["dyn_scales"])
-            assert np.array_equal(bits16(y), wy)
+            assert int(status) == 0 and np.array_equal(bits16(y), wy)
 
 
 @pytest.mark.parametrize("bs,h,k,kernel", [
