@@ -96,7 +96,7 @@ struct RouteRowsLaunch {
     hipStream_t stream;
 };
 bool RouteRowsPays(int64_t routes, int64_t numKeys, bool rowsAhead, bool readsRowsAhead);
-constexpr int64_t kRowsMaskedTokens = 8192;     // largest call whose prefix mask the launch adds up where it is free not to
+constexpr int64_t kRowsMaskedTokens = 8192;     // largest call whose prefix mask the launch adds up unasked (RouteRowsLimitPays)
 bool RouteRowsLimitPays(int64_t routes, int64_t numKeys, int64_t capacity);
 bool RouteRowsFits(const int32_t *ids, int64_t routes, int64_t numKeys, int maskMode, int64_t capacity);
 hipError_t LaunchRouteRows(const RouteRowsLaunch &l);

@@ -216,8 +216,8 @@ bool WaveUnits(const ReduceLaunch &l, int slices, int ranks)
 }
 
 // Quantised rows, one or two to a token: several tokens to a wave (ep_reduce_quant_few_kernel) where the launch is long enough
-// to be bound by what its waves have under way, and its outputs and rows do not outgrow the memory-side cache.  Dispatch +
-// combine, us, a token to a wave and several, int8 and block fp8:
+// to be bound by what its waves have under way, up to the largest outputs that both payloads were measured to gain at; at the
+// next sizes int8 loses and block fp8 gains or loses.  Dispatch + combine, us, a token to a wave and several, int8 and block fp8:
 //   top-1, outputs of 33 MB 16384 x 1024 25.1 and 25.6, 26.2 and 27.0; 49 MB 12000 x 2048 35.7 -> 34.6, 36.3 -> 35.6; 67 MB
 //     16384 x 2048 48.6 -> 44.3, 50.2 -> 46.2; 86 MB 6000 x 7168 59.8 -> 55.7, 63.2 -> 56.9; 164 MB 10000 x 8192 103.3 ->
 //     96.8, 108.9 -> 98.1; 235 MB 16384 x 7168 163.8 -> 160.7, 169.0 -> 159.7; 268 MB 16384 x 8192 174.3 and 175.9, 178.6 ->

@@ -14,17 +14,16 @@
 namespace TileXREp {
 namespace {
 
-// Quantised expert output: int8 rows with one fp32 scale per row, or fp8 e4m3 rows with one fp32 scale per 128
-// columns.  Each value is dequantised, rounded to the output element type, then accumulated exactly like an ordinary
-// row (fp32, k order, separate multiply and add).  Rows are a quarter the bytes of bf16 rows, so a lane owns 16
-// consecutive columns per vector (one 16-byte load) and KB rows are kept in flight at once.
 // A row's largest magnitude is 128 (448) times its scale: below this scale none reaches the 65520 from which rounding to fp16
 // has to saturate.
 template <int INQ>
 constexpr float kScaleSaturates = INQ == TILEXR_EP_QUANT_TOKEN_INT8 ? 511.875f : 146.25f;
 
 // Sixteen columns of a row: dequantised, rounded to the element type, weighted, added.  EXACT: the reference decode of NaN
-// codes and, for fp16, the saturating rounding.
+// codes and, for fp16, the saturating rounding.  For ep_reduce_quant_few_kernel.  The K loop of ep_reduce_quant_kernel has
+// the same steps in place and has to change with them: called there, this costs it up to 26 vector registers (block fp8, four
+// rows 60 and 70; int8 to fp16, six rows 66 and 92), and eight of the twelve narrower instances that may wait for flags spill two to
+// eleven; those without flags take the same time either way (int8 8192 x 4096 x top-6 96.6 us, block fp8 16384 x 2048 x top-8 133.5).
 template <int INQ, bool BF16, bool EXACT>
 __device__ __forceinline__ void AddQuantRow(const u32x4 &q, float scale, float w, float (&acc)[16])
 {
@@ -67,6 +66,10 @@ constexpr int kFlagsNone = 0;
 constexpr int kFlagsMayWait = 1;
 constexpr int kFlagsSettled = 2;
 
+// Quantised expert output: int8 rows with one fp32 scale per row, or fp8 e4m3 rows with one fp32 scale per 128
+// columns.  Each value is dequantised, rounded to the output element type, then accumulated exactly like an ordinary
+// row (fp32, k order, separate multiply and add).  Rows are a quarter the bytes of bf16 rows, so a lane owns 16
+// consecutive columns per vector (one 16-byte load) and KB rows are kept in flight at once.
 //
 // KB rows in flight per lane: four, or two of the widest rows.  Five or six slots to a token take six at once instead of four
 // and then the rest, at five waves per SIMD instead of seven (8192 x 4096 x top-6 int8, dispatch + combine 99.4 -> 97.5 us;
@@ -185,6 +188,7 @@ __global__ __launch_bounds__(kThreads, V == 1 ? (KB > 4 ? 5 : (FL == kFlagsMayWa
                         if (!BF16 && !kExactDecode) {
                             saturates |= !(fabsf(sc[u][j]) < kScaleSaturates<INQ>);
                         }
+                        // AddQuantRow's steps
 #pragma unroll
                         for (int d = 0; d < 4; ++d) {
                             const uint32_t word = q[u][j][d];
@@ -305,11 +309,10 @@ __global__ __launch_bounds__(kThreads, V == 1 ? (KB > 4 ? 5 : (FL == kFlagsMayWa
     }
 }
 
-
-// Tokens of one or two slots, launches without flags (QuantTakesFew).  A wave of the kernel above has one row or two in flight then and is
-// done with them before its look-up, its rows and its stores, one after the other, have cost it three trips to memory: the
-// waves a compute unit holds are too few for that.  Here a wave takes a slice of 64 vectors of ROWS / SLOTS neighbouring
-// tokens: their look-ups together, their ROWS rows together, then token by token the sum and the store.
+// Tokens of one or two slots, launches without flags (QuantTakesFew).  A wave of the kernel above has one row or two in flight
+// then and is done with them before its look-up, its rows and its stores, one after the other, have cost it three trips to
+// memory: the waves a compute unit holds are too few for that.  Here a wave takes a slice of 64 vectors of ROWS / SLOTS
+// neighbouring tokens: their look-ups together, their ROWS rows together, then token by token the sum and the store.
 constexpr int kQuantFewRows = 4;
 
 template <int SLOTS, int INQ, bool BF16>

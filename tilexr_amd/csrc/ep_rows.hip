@@ -499,7 +499,8 @@ bool RouteRowsPays(int64_t routes, int64_t numKeys, bool rowsAhead, bool readsRo
 
 // ... and of a call whose routes are limited, where the other would be.  Token-prefix masks, count and one launch: 400 x 2048 x
 // top-8 of 64 20.0 -> 16.3 us, 1024 x 2048 of 256 24.2 -> 20.3, 2048 x 2048 34.6 -> 30.5, 8192 x 2048 x top-4 of 64 65.5 -> 60.0;
-// up to kRowsMaskedTokens (the mask is added up eight bytes a lane).
+// up to kRowsMaskedTokens.  That line is where the first measurements ended, not where the gain does: 9000 x 2048 x top-2 of 64
+// 50.7 and 39.9, 16384 x 1024 x top-4 72.7 and 65.4, 32768 x 1024 x top-1 82.7 and 54.6, 60000 x 512 122.6 and 68.9.
 // Capacity limits, whose histogram grows with the routes: 518 x 2048 x top-8 of 64 18.4 -> 14.2, with flags (no place launch)
 // 22.1 -> 17.2; 1729 x top-5 of 128 24.3 -> 20.8; 16 384 routes of 64 33.1 -> 30.0, of 512 35.0 -> 33.1, block fp8 23.0 and 22.9;
 // 32 768 routes of 128 55.1 and 54.9, block fp8 29.7 and 31.3, of 512 56.4 and 58.4; 65 536 routes 102.4 and 104.0, 53.2 and 58.0.

@@ -373,7 +373,7 @@ __global__ __launch_bounds__(kThreads) void moon_scatter_generic_kernel(Dispatch
 // (dispatch kernel :330-424).  With the rank-within-group and group size recorded by the sources, both numberings are
 // exclusive prefix sums over the rows: group index = number of earlier group-opening rows, slice start = sum of their
 // group sizes.  PlanChunk does that within the scatter launch; the kernels here follow a scatter that does nothing else
-// (moon_scatter_generic_kernel, plans of more than kFusedPlanChunks chunks).  A workgroup scans one chunk of 2048 rows after adding
+// (moon_scatter_generic_kernel, plans beyond kFusedPlanChunks).  A workgroup scans one chunk of 2048 rows after adding
 // up the chunks before its own -- from the rows themselves while the chunks are few, from the totals a first launch leaves
 // otherwise.  The slices are filled by the finish kernel, which visits every row anyway.
 constexpr int kBuildRows = kChunkRows;
