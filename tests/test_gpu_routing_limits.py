@@ -60,6 +60,19 @@ def test_capacity(bs, k, e, invalid, limit, legacy):
         _run(legacy, xt, xb, ids, e, 1, capacity=capacity, quant=ep.Q_TOKEN_INT8)
 
 
+@pytest.mark.parametrize("bs,k,e", [(16384, 1, 64), (2048, 8, 64), (2100, 5, 7), (2500, 1, 1024), (2500, 1, 1025), (1024, 16, 2048)])
+@pytest.mark.parametrize("first", ["low", "high"])
+def test_capacity_when_every_token_goes_the_same_way(bs, k, e, first):
+    """All lanes count the same expert at once; both layouts of the counters, up to their last key."""
+    rng = np.random.default_rng(bs + k + e)
+    start = 0 if first == "low" else e - k - 1 if e > k else 0
+    ids = np.tile(np.arange(start, start + k, dtype=np.int32), (bs, 1))
+    ids[rng.integers(0, bs, 20), rng.integers(0, k, 20)] = e - 1
+    xt, xb = x_for(rng, bs, 16, ep.DT_BF16)
+    for capacity in (1, bs // 3, bs * k):
+        _run(False, xt, xb, ids, e, 1, capacity=capacity)
+
+
 @pytest.mark.parametrize("bs,k,e,invalid", SHAPES)
 @pytest.mark.parametrize("active", ["none", "one", "some", "all"])
 @pytest.mark.parametrize("legacy", [False, True])

@@ -22,8 +22,9 @@
 //
 // A token-prefix mask makes the table shorter: every workgroup adds the mask up first, one more round trip.  A capacity
 // limit makes "valid ids below k" the sum of the smaller keys' counts, each cut at the limit, so those are counted in an
-// LDS histogram after all (RouteRowsLimitPays: tables where that is cheaper than the hand-over); routes beyond a key's limit
-// get row -1 from the workgroup that ranks them.
+// LDS histogram after all (RouteRowsLimitPays: tables where that is cheaper than the hand-over), in eight counters a key
+// taken by the lanes in turn: adds to one counter go one after the other, and a wave may hold one expert's ids only.  Routes
+// beyond a key's limit get row -1 from the workgroup that ranks them.
 //
 // Same definitions as the count + place pair (reference: src/ep/kernels/tilexr_ep_dispatch_memory_kernel.h:791-818
 // rank within expert, :820-1089 count exchange and inclusive cumulative sum, :1142-1168 count outputs, :1240-1258
@@ -77,6 +78,14 @@ struct RouteRowsArgs {
 // Which routes have rows: those whose id names a key; of these, those of the first sum(mask) tokens; or the first
 // `capacity` of every key.
 enum RowsLimit { kRowsAll, kRowsPrefix, kRowsCapped };
+
+// Counters of a workgroup under a capacity limit: eight for each of half the most keys, four for more; a key's own are an odd
+// multiple of four words apart, so in LDS banks of their own.
+constexpr int kRowsFewKeys = kMaxKeys / 2;
+constexpr int kRowsFewKeysStride = kRowsFewKeys + 4;
+constexpr int kRowsManyKeysStride = kMaxKeys + 4;
+constexpr int kRowsCounters = 8 * kRowsFewKeysStride;
+static_assert(4 * kRowsManyKeysStride <= kRowsCounters, "both fit");
 
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 
@@ -134,7 +143,9 @@ __global__ __launch_bounds__(kRowsThreads, 8) void ep_route_rows_kernel(RouteRow
     constexpr bool kCapped = LIMIT == kRowsCapped;
     __shared__ int s_less[kRowsWaves];
     __shared__ int s_same[kRowsWaves];
-    __shared__ int s_hist[kCapped ? kMaxKeys : 1];      // routes of the keys below this workgroup's
+    // routes of the keys below this workgroup's, counted apart by lane
+    __shared__ int s_hist[kCapped ? kRowsCounters : 1];
+    __shared__ int s_capped[kCapped ? kRowsWaves : 1];
 
     const int tid = threadIdx.x;
     const int wave = tid / kWave;
@@ -187,12 +198,22 @@ __global__ __launch_bounds__(kRowsThreads, 8) void ep_route_rows_kernel(RouteRow
     const int mineFirst = SPLIT ? part * a.partSlots : 0;           // the slots this workgroup's waves rank: [mineFirst, mineEnd)
     const int mineEnd = SPLIT ? (mineFirst + a.partSlots < a.slots ? mineFirst + a.partSlots : a.slots) : a.slots;
 
+    // under a capacity limit: where a key's counters are, and the first of the lane's
+    const bool fewKeys = a.numKeys <= kRowsFewKeys;
+    const int stride = fewKeys ? kRowsFewKeysStride : kRowsManyKeysStride;
+    const int counters = (lane & (fewKeys ? 7 : 3)) * stride;       // the lane's
+
     // pass 1, over the wave's whole sixteenth: per lane, ids below the key (unsigned compare: negative ids are above
     // every key) and ids equal to it, those ahead of the workgroup's own slots counted apart; which elements of its own
     // slots are equal is kept, four bits per slot, so that pass 2 needs no id any more
     if (kCapped) {
         for (int j = tid; j < key; j += kRowsThreads) {
-            s_hist[j] = 0;
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                if (c < 4 || fewKeys) {
+                    s_hist[c * stride + j] = 0;
+                }
+            }
         }
         __syncthreads();
     }
@@ -216,7 +237,7 @@ __global__ __launch_bounds__(kRowsThreads, 8) void ep_route_rows_kernel(RouteRow
                     if (!kCapped) {
                         less += below ? 1 : 0;
                     } else if (below && e < inTable) {
-                        atomicAdd(&s_hist[id[u][e]], 1);
+                        atomicAdd(&s_hist[counters + id[u][e]], 1);
                     }
                     mine |= id[u][e] == key ? 1u << e : 0u;
                 }
@@ -240,10 +261,20 @@ __global__ __launch_bounds__(kRowsThreads, 8) void ep_route_rows_kernel(RouteRow
     __syncthreads();
     int capped = 0;             // rows of the keys below
     if (kCapped) {
-        for (int j = lane; j < key; j += kWave) {
-            capped += min(s_hist[j], a.capacity);
+        for (int j = tid; j < key; j += kRowsThreads) {
+            int count = 0;
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                count += c < 4 || fewKeys ? s_hist[c * stride + j] : 0;
+            }
+            capped += min(count, a.capacity);
         }
         capped = WaveSum(capped);
+        if (lane == 0) {
+            s_capped[wave] = capped;
+        }
+        __syncthreads();
+        capped = WaveSum(lane < kRowsWaves ? s_capped[lane] : 0);
     }
     // elements beyond the table read as id 0: below every other key, equal to key 0
     const int beyond = kRowsWaves * a.slots * kRowsSlotRoutes - n;
@@ -503,6 +534,8 @@ bool RouteRowsPays(int64_t routes, int64_t numKeys, bool rowsAhead, bool readsRo
 // 50.7 and 39.9, 16384 x 1024 x top-4 72.7 and 65.4, 32768 x 1024 x top-1 82.7 and 54.6, 60000 x 512 122.6 and 68.9.
 // Capacity limits, whose histogram grows with the routes: 518 x 2048 x top-8 of 64 18.4 -> 14.2, with flags (no place launch)
 // 22.1 -> 17.2; 1729 x top-5 of 128 24.3 -> 20.8; 16 384 routes of 64 33.1 -> 30.0, of 512 35.0 -> 33.1, block fp8 23.0 and 22.9;
+// where every token goes to the same experts (with one counter a key) 8192 x 1024 x top-2 of 512 18.9 -> 16.3 (38.7), 16384 x 512 x
+// top-1 20.4 -> 18.3 (39.5), 4096 x 1024 x top-4 of 8 19.6 -> 17.5 (27.9);
 // 32 768 routes of 128 55.1 and 54.9, block fp8 29.7 and 31.3, of 512 56.4 and 58.4; 65 536 routes 102.4 and 104.0, 53.2 and 58.0.
 bool RouteRowsLimitPays(int64_t routes, int64_t numKeys, int64_t capacity)
 {
