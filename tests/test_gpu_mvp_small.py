@@ -39,3 +39,24 @@ def test_dispatch(bs, h, k, e, invalid, plain, int8, nums_type):
             assert np.array_equal(got["recv_counts"], want["recv_counts"])
             if quant != ep.Q_NONE:
                 assert np.array_equal(got["scales"][:want["rows"], 0], want["dyn_scales"][:want["rows"]])
+
+
+@pytest.mark.parametrize("bs,h,k", [(384, 16384, 2), (383, 16384, 2), (1537, 8192, 1), (1540, 8184, 1)])
+def test_rows_on_both_sides_of_those_that_are_kept(bs, h, k):
+    """24 MiB of rows of whole lines and more are written through and kept, others stream."""
+    e = 16
+    rng = np.random.default_rng(bs + h)
+    ids = ids_for(rng, bs, k, e, invalid=0.02)
+    xt, xb = x_for(rng, bs, h, ep.DT_FP16)
+    with Session() as s:
+        out = alloc_dispatch_outputs(bs, h, k, e)
+        counts = torch.full((1,), -1, dtype=torch.int32, device=DEV)
+        for _ in range(2):
+            assert ep.dispatch_v2(xt, to_dev(ids), s.comm, bs, h, k, e, out["expand_x"], out["assist"], out["token_nums"],
+                                  counts, ep.DT_FP16, s.stream) == 0
+        s.sync()
+        assert ep.last_kernel_name(s.comm, ep.K_SCATTER) == SMALL
+        got = fetch(out, "recv_counts", counts)
+    want = O.mvp_dispatch(O.Case(1, bs, h, k, e, dtype=O.DT_FP16), 0, xb[None], ids[None])
+    check_dispatch(got, want)
+    assert np.array_equal(got["recv_counts"], want["recv_counts"])

@@ -186,6 +186,16 @@ static bool SmallMvpFits(const SmallDispatchLaunch &l)
         (l.quantMode == TILEXR_EP_QUANT_NONE || (l.quantMode == TILEXR_EP_QUANT_TOKEN_INT8 && !l.inputBf16 && l.bs * l.topK * l.h <= (int64_t{3} << 20)));
 }
 
+// Many rows of whole lines are written through and stay in the memory-side cache, where Combine finds them.  Streamed, wide ones had
+// become slower than with the routing and scatter launches, us with those, streamed and kept: fp16 1000 x 16384 x top-1 of 64 32.1,
+// 34.2 and 29.6, 700 x top-2 30.0, 31.4 and 28.0, 512 x top-4 32.7, 33.4 and 30.2, 2048 x top-1 49.8, 50.2 and 48.0.  Level at
+// the line (256 x 6144 x top-8 17.4, 14.9 and 14.8, 240 x 7168 17.9, 15.5 and 15.5); rows that end within a line stream (2048 x
+// 16376 x top-1 56.4 and 51.2).
+static bool KeepsMvpRows(const SmallDispatchLaunch &l)
+{
+    return l.h % 64 == 0 && l.bs * l.topK * l.h * 2 >= (int64_t{24} << 20);
+}
+
 bool SmallDispatchFits(const SmallDispatchLaunch &l)
 {
     return (!l.mvp || SmallMvpFits(l)) && l.bs * l.topK <= kSmallRoutes && l.numExperts <= kMaxKeys && l.topK <= kMaxTopK && l.h % 8 == 0 &&
@@ -244,6 +254,8 @@ hipError_t LaunchSmallDispatch(const SmallDispatchLaunch &l)
                 constexpr int kV = decltype(vecsPerLane)::value;
                 if (LeavesRowsToL2(l)) {
                     launch(ep_dispatch_small_route_kernel<kV, 0, kIdsPerLane, false, TILEXR_EP_QUANT_NONE, true, false, true>, routes);
+                } else if (KeepsMvpRows(l)) {
+                    launch(ep_dispatch_small_route_kernel<kV, kAuxAgentScopeKept, kIdsPerLane, false, TILEXR_EP_QUANT_NONE, true, false, true>, routes);
                 } else {
                     launch(ep_dispatch_small_route_kernel<kV, kAuxNonTemporal, kIdsPerLane, false, TILEXR_EP_QUANT_NONE, true, false, true>, routes);
                 }
