@@ -111,6 +111,18 @@ def test_sums_in_the_order_of_the_rows(bs, h, k):
 def test_several_tokens_to_a_wave(bs, h, k, quant, dtype):
     """One or two slots and outputs of 47 MB and more: slices that end within a row, tokens that do not fill the last wave,
     lost rows, masked tokens, a shared expert; in places scales whose rows saturate in fp16, and NaN codes."""
+    _reduce_few(bs, h, k, quant, dtype, "ep_reduce_quant_few_kernel")
+
+
+@pytest.mark.parametrize("bs,h,k,kernel", [
+    (3301, 7168, 1, "few_"), (3301, 7184, 1, ""), (3005, 7920, 2, ""), (3005, 7936, 2, "few_"), (1777, 13312, 2, "few_"),
+    (1777, 13328, 2, ""), (1777, 13440, 1, "few_")])
+def test_rows_that_end_within_a_line(bs, h, k, kernel):
+    """Both sides of the widths at which such rows take one token to a wave."""
+    _reduce_few(bs, h, k, ep.Q_TOKEN_INT8, ep.DT_BF16, f"ep_reduce_quant_{kernel}kernel")
+
+
+def _reduce_few(bs, h, k, quant, dtype, kernel):
     experts = 16
     rng = np.random.default_rng(bs + h + quant)
     ids = ids_for(rng, bs, k, experts)
@@ -134,7 +146,7 @@ def test_several_tokens_to_a_wave(bs, h, k, quant, dtype):
                                     expert_out_quant_mode=quant, expert_out_scales=args[3], expert_scales=args[4],
                                     active_mask=args[5], active_mask_type=ep.MASK_TOKEN, shared_expert_x=args[6]) == 0
         s.sync()
-        assert ep.last_kernel_name(s.comm, ep.K_REDUCE) == "ep_reduce_quant_few_kernel"
+        assert ep.last_kernel_name(s.comm, ep.K_REDUCE) == kernel
         got = bits16(y)
     want = O.mem_combine(O.Case(1, bs, h, k, experts, dtype=dtype, mask_type=ep.MASK_TOKEN), 0, payload[None], assist[None],
                          d["send_counts"][None], expert_scales=w, token_mask=mask, shared_expert_x=shared, in_quant=quant,

@@ -313,6 +313,10 @@ __global__ __launch_bounds__(kThreads, V == 1 ? (KB > 4 ? 5 : (FL == kFlagsMayWa
 // then and is done with them before its look-up, its rows and its stores, one after the other, have cost it three trips to
 // memory: the waves a compute unit holds are too few for that.  Here a wave takes a slice of 64 vectors of ROWS / SLOTS
 // neighbouring tokens: their look-ups together, their ROWS rows together, then token by token the sum and the store.
+// Groups of tokens are dealt to the XCDs in turn (workgroup b runs on XCD b % 8) and all slices of a group go to the same one, so
+// that a line in which a slice ends is fetched and put together in one L2: 5000 x 7184 x top-2 int8 71.6 -> 70.1 us, 5000 x 8176
+// 77.7 -> 75.6, 9000 x 6160 top-1 80.7 -> 78.4, rows of whole lines unchanged (16384 x 4096 x top-2 100.1 and 100.2).  XCDs with a
+// range of tokens each are no choice (100 -> 117.8).
 constexpr int kQuantFewRows = 4;
 
 template <int SLOTS, int INQ, bool BF16>
@@ -324,9 +328,10 @@ __global__ __launch_bounds__(kThreads) void ep_reduce_quant_few_kernel(ReduceArg
     const int lane = threadIdx.x % kWave;
     const int vecs = a.h / 16;
     const int b128 = (a.h + 127) / 128;
-    const int unit = static_cast<int>(blockIdx.x) * kWavesPerBlock + static_cast<int>(threadIdx.x) / kWave;
-    const int group = unit / a.colSlices;
-    const int idx = (unit - group * a.colSlices) * kWave + lane;
+    const int unit = static_cast<int>(blockIdx.x / kXcdCount) * kWavesPerBlock + static_cast<int>(threadIdx.x) / kWave;
+    const int round = unit / a.colSlices;
+    const int group = round * kXcdCount + static_cast<int>(blockIdx.x % kXcdCount);
+    const int idx = (unit - round * a.colSlices) * kWave + lane;
     const int firstToken = __builtin_amdgcn_readfirstlane(group * kTokens);
 
     // lane l < ROWS: slot l % SLOTS of token firstToken + l / SLOTS
@@ -426,7 +431,8 @@ template <int SLOTS, bool BF16>
 void LaunchQuantFew(const ReduceLaunch &l, const ReduceArgs &a)
 {
     constexpr int kTokens = kQuantFewRows / SLOTS;
-    const dim3 g(static_cast<unsigned>(((a.bs + kTokens - 1) / kTokens * a.colSlices + kWavesPerBlock - 1) / kWavesPerBlock));
+    const int rounds = ((a.bs + kTokens - 1) / kTokens + kXcdCount - 1) / kXcdCount;
+    const dim3 g(static_cast<unsigned>((rounds * a.colSlices + kWavesPerBlock - 1) / kWavesPerBlock * kXcdCount));
     if (l.inQuant == TILEXR_EP_QUANT_TOKEN_INT8) {
         hipLaunchKernelGGL((ep_reduce_quant_few_kernel<SLOTS, TILEXR_EP_QUANT_TOKEN_INT8, BF16>), g, dim3(kThreads), 0, l.stream, a);
     } else {
