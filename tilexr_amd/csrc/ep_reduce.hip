@@ -226,9 +226,9 @@ bool WaveUnits(const ReduceLaunch &l, int slices, int ranks)
 //     75.5 -> 74.0, 80.4 -> 75.7; 134 MB 16384 x 4096 103.6 -> 100.3, 104.4 -> 100.9; 164 MB 10000 x 8192 121.5 and 123.4,
 //     127.9 -> 125.8; 221 MB 13500 x 8192 179.1 and 181.7, 178.8 and 183.6
 // Rows that end within a 128-byte line gain less, since most slices' ends are within one too, and lose from 449 to 495 vectors,
-// where the last of eight slices is short and the other kernel's 512 are not, and beyond 832, where its 1024 are nearly full: 5000 x 7184 x top-2 67.4 and 70.1, 69.3 and 71.9; 9000 x 7184 top-1 89.1 and 92.1, 90.0
-// and 91.9; 5000 x 7696 top-2 72.4 and 74.2, 73.9 and 75.7; 16368 columns top-1 112.4 and 118.5, 113.5 and 118.3.  But 9000 x
-// 4112 top-1 62.1 -> 58.0, 66.4 -> 60.6; 8000 x 6160 top-2 90.2 and 91.0, 92.8 and 92.4; 6000 x 8016 top-1 70.1 and 70.9, 71.8 and
+// where the last of eight slices is short and the other kernel's 512 are not, and beyond 832, where its 1024 are nearly full:
+// 5000 x 7184 x top-2 67.4 and 70.1, 69.3 and 71.9; 9000 x 7184 top-1 89.1 and 92.1, 90.0 and 91.9; 5000 x 7696 top-2 72.4 and
+// 74.2, 73.9 and 75.7; 16368 columns top-1 112.4 and 118.5, 113.5 and 118.3.  But 9000 x 4112 top-1 62.1 -> 58.0, 66.4 -> 60.6; 8000 x 6160 top-2 90.2 and 91.0, 92.8 and 92.4; 6000 x 8016 top-1 70.1 and 70.9, 71.8 and
 // 71.6; 5000 x 9232 top-2 83.7 and 83.7, 92.8 -> 87.5; 5000 x 12304 top-1 83.2 and 84.5, 90.2 -> 85.9.
 bool QuantTakesFew(const ReduceLaunch &l)
 {
